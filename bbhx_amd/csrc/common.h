@@ -244,22 +244,24 @@ __device__ inline void sincos_small(double x, double* s, double* c)
     *c = ((k + 1) & 2) ? -cc : cc;
 }
 
-// e^{i theta} for large |theta| by table: theta reduced modulo 2 pi, then
-// r = j pi/64 + b with integer |j| <= 64 and |b| <= pi/128; e^{i j pi/64} from a
-// 129-entry table (built by fill_etab, normally in LDS) and e^{i b} from its
-// series to b^7 / b^6 (truncation < 1e-18 relative): ~24 operations against
-// ~35 for sincos_small after reduce_2pi, within a few ulp of it. Any theta (also NaN or inf)
-// gives an index in [0, 128].
+// e^{i theta} for large |theta| by table: theta = j pi/64 + b with integer j and
+// |b| <= pi/128 in one Cody-Waite step (pi/64 = HI + LO to ~107 bits; j is
+// rounded, and its low bits read, by adding 1.5 2^52); e^{i j pi/64} from a
+// table of one turn (tab[(j + 64) mod 128], normally in LDS) and e^{i b} from
+// its series to b^7 / b^6 (truncation < 1e-18 relative): 16 operations, within a
+// few ulp for |theta| up to ~1e13. Any theta (also NaN or inf) gives an index in
+// [0, 127].
 constexpr double PI64_HI = 0.04908738521234052;     // pi / 64 rounded
 constexpr double PI64_LO = 1.9135106236677393e-18;  // pi / 64 - PI64_HI
+constexpr double ROUND_MAGIC = 6755399441055744.0;  // 1.5 2^52
 template <class E>
 __device__ inline cd cexpi_tab(double theta, const E* __restrict__ tab)
 {
-    const double r = reduce_2pi(theta);
-    const double j = rint(r * 20.371832715762604);  // 64 / pi
-    double b = fma(-j, PI64_HI, r);
+    const double t = fma(theta, 20.371832715762604, ROUND_MAGIC + 64.0);  // 64 / pi
+    const double j = t - (ROUND_MAGIC + 64.0);
+    double b = fma(-j, PI64_HI, theta);
     b = fma(-j, PI64_LO, b);
-    const E e = tab[(int)j + 64];
+    const E e = tab[__double2loint(t) & 127];
     const double b2 = b * b;
     double ps = fma(b2, -1.0 / 5040.0, 1.0 / 120.0);
     ps = fma(b2, ps, -1.0 / 6.0);
@@ -270,6 +272,23 @@ __device__ inline cd cexpi_tab(double theta, const E* __restrict__ tab)
     return cd{e.x * cb - e.y * sb, e.y * cb + e.x * sb};
 }
 
+// The same from a table of 1024 entries (tab[j mod 1024] = e^{i j pi/512}, built
+// by fill_etab1k): |b| <= pi/1024, so the series end at b^5 / b^4 (truncation
+// < 2e-18). For persistent kernels, which fill its 16 KB of LDS once.
+template <class E>
+__device__ inline cd cexpi_tab1k(double theta, const E* __restrict__ tab)
+{
+    const double t = fma(theta, 8 * 20.371832715762604, ROUND_MAGIC);
+    const double j = t - ROUND_MAGIC;
+    double b = fma(-j, PI64_HI / 8, theta);
+    b = fma(-j, PI64_LO / 8, b);
+    const E e = tab[__double2loint(t) & 1023];
+    const double b2 = b * b;
+    const double sb = fma(b * b2, fma(b2, 1.0 / 120.0, -1.0 / 6.0), b);
+    const double cb = fma(b2, fma(b2, 1.0 / 24.0, -0.5), 1.0);
+    return cd{e.x * cb - e.y * sb, e.y * cb + e.x * sb};
+}
+
 // The table of cexpi_tab: tab[j] = (cos, sin)((j - 64) pi / 64), j = 0..128,
 // filled by threads tid = 0..nt-1 of a workgroup (a barrier must follow).
 __device__ inline void fill_etab(double2* tab, int tid, int nt)
@@ -277,6 +296,17 @@ __device__ inline void fill_etab(double2* tab, int tid, int nt)
     for (int j = tid; j < 129; j += nt) {
         double sn, cs;
         sincos_small(fma((double)(j - 64), PI64_HI, (double)(j - 64) * PI64_LO), &sn, &cs);
+        tab[j] = make_double2(cs, sn);
+    }
+}
+
+// The table of cexpi_tab1k, likewise
+__device__ inline void fill_etab1k(double2* tab, int tid, int nt)
+{
+    for (int j = tid; j < 1024; j += nt) {
+        const double k = j < 512 ? j : j - 1024;
+        double sn, cs;
+        sincos_small(fma(k, PI64_HI / 8, k * (PI64_LO / 8)), &sn, &cs);
         tab[j] = make_double2(cs, sn);
     }
 }

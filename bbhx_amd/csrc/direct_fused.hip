@@ -51,7 +51,8 @@ bool response_orbit_tab(const bbhx_response* r, resp::OrbitTab& o);
 struct bbhx_direct_plan {
     int device = -1;
     int B = 0, M = 0, N = 0, Lmax = 0;
-    int min_chunk = 0;   // smallest chunk the partial-sum buffer is sized for
+    int min_chunk = 0;   // smallest chunk a caller may ask for
+    int min_item = 0;    // dense bins of the smallest work item the buffers are sized for
     long S = 0;          // total sparse points
     long max_items = 0;  // bound on (binary, chunk) work items
     // device buffers
@@ -82,7 +83,7 @@ struct bbhx_direct_plan {
     int* loud_cnt = nullptr;             // (4,) loud count, its pass's next-item counter; the same for quiet
     int* route = nullptr;                // (B,) 1: the h_h estimate sends the binary to the FP64 pass
     int* split_cnt = nullptr;            // (max_items / 256 + 1,) loud entries per block of the order, scanned
-    int max_chunks = 0;           // absolute chunks of min_chunk bins
+    int max_chunks = 0;           // absolute chunks of min_item bins
 };
 
 namespace {
@@ -95,15 +96,26 @@ struct alignas(32) Cubic {
     double y, c1, c2, c3;
 };
 
+// Whether t(f) stays inside the observation window over a whole segment: then
+// (or if it stays outside) the dense pass need not evaluate t(f) bin by bin.
+enum SegWin : int { WIN_MIXED = 0, WIN_ALL = 1, WIN_NONE = 2 };
+
 // segment i of one (binary, mode): it covers x_lo <= f < x_hi (x_hi = x_lo for
-// the last knot, which starts no segment)
+// the last knot, which starts no segment). The cubics in the order A, phase,
+// T1..T3 re/im, t_f (seg_slot): the 288 B in front of t_f's are what a segment
+// inside the window needs.
 struct alignas(32) SegRec {
-    double x_lo, x_hi, pad0, pad1;
+    double x_lo, x_hi;
+    int win, pad0;  // SegWin
+    double pad1;
     Cubic q[NQ];
 };
 constexpr int RS = sizeof(SegRec) / sizeof(double);  // 40 doubles
 constexpr int RQ = 4;                                 // offset of q[0] in doubles
 static_assert(sizeof(SegRec) == 320, "segment record layout");
+constexpr int S_A = 0, S_PH = 1, S_T = 2, S_TF = 8;  // slots of q
+// slot of quantity q of the grid pass (A, phase, t_f, T1..T3 re/im)
+__host__ __device__ constexpr int seg_slot(int q) { return q < 2 ? q : (q == 2 ? S_TF : q - 1); }
 
 // Segment record of the FP32-bulk form: bounds and the phase and t(f) cubics
 // in FP64 (phases reach 1e8 rad, and t(f) decides the observation window
@@ -127,8 +139,9 @@ __device__ inline cd to_cd(cf a) { return mk((double)a.re, (double)a.im); }
 __device__ inline void zero(cd& a) { a = mk(0.0, 0.0); }
 __device__ inline void zero(cf& a) { a = cf{0.0f, 0.0f}; }
 
-__device__ inline const Cubic& cubic_of(const SegRec& r, int k) { return r.q[k]; }
-__device__ inline const Cubic& cubic_of(const Cubic (&c)[NQ], int k) { return c[k]; }
+// type of the mode sum of a record's form
+template <class Rec>
+using dense_sum = typename std::conditional<std::is_same<Rec, SegRecF>::value, cf, cd>::type;
 
 __global__ __launch_bounds__(64) void k_dir_setup(FusedRec* __restrict__ recs, const double* __restrict__ params, int B, ModeList modes,
                             int M, const double* __restrict__ qnm, int table_len, double dspin)
@@ -281,6 +294,22 @@ __global__ __launch_bounds__(64) void k_dir_grid(double* __restrict__ X, double*
     }
 }
 
+// SegWin of the cubic c over [0, h]: a cubic lies between the least and the
+// greatest of its four Bernstein coefficients there; the margin (1e-12 of the
+// terms' magnitudes, and 1 microsecond) covers the rounding of those and of the
+// bin-by-bin evaluation, so WIN_ALL and WIN_NONE are what every bin would find.
+__device__ inline int segment_window(const Cubic& c, double h, double ts, double te)
+{
+    const double t1 = c.c1 * h, t2 = c.c2 * (h * h), t3 = c.c3 * (h * h * h);
+    const double b1 = c.y + t1 * (1.0 / 3.0), b2 = c.y + (2.0 * t1 + t2) * (1.0 / 3.0), b3 = c.y + t1 + t2 + t3;
+    const double m = 1e-6 + 1e-12 * (fabs(c.y) + fabs(t1) + fabs(t2) + fabs(t3));
+    const double lo = fmin(fmin(c.y, b1), fmin(b2, b3)) - m, hi = fmax(fmax(c.y, b1), fmax(b2, b3)) + m;
+    if (!(m < 1e300)) return WIN_MIXED;  // not finite: bin by bin
+    if (lo >= ts && (hi <= te || te <= 0.0)) return WIN_ALL;
+    if (hi < ts || (te > 0.0 && lo > te)) return WIN_NONE;
+    return WIN_MIXED;
+}
+
 constexpr int DSPL_BLOCK = 8;  // rows loaded ahead of the recurrence in each sweep of k_dir_spline
 
 // Not-a-knot spline of one binary: lane s = mode * 9 + quantity runs the
@@ -289,18 +318,29 @@ constexpr int DSPL_BLOCK = 8;  // rows loaded ahead of the recurrence in each sw
 __global__ __launch_bounds__(64) void k_dir_spline(const double* __restrict__ X, const double* __restrict__ Yc,
                                                    double* __restrict__ Cf, double* __restrict__ Fs,
                                                    SegRecF* __restrict__ CfF, const long* __restrict__ off,
-                                                   const int* __restrict__ len, int M)
+                                                   const int* __restrict__ len, const double* __restrict__ t_start,
+                                                   const double* __restrict__ t_end, int M)
 {
     const int b = blockIdx.x;
     const int s = threadIdx.x;
     if (s >= M * NQ) return;
+    const double ts = t_start[b], te = t_end[b];
     const int m = s / NQ;
     const int n = len[b];
     const long base = off[b];
     // element i of this system
     auto xi = [&](int i) { return X[(base + i) * M + m]; };
     const int q = s - m * NQ;
-    auto at = [&](int i) { return ((base + i) * M + m) * RS + RQ + q * 4; };
+    auto at = [&](int i) { return ((base + i) * M + m) * RS + RQ + seg_slot(q) * 4; };
+    // the record's head (bounds and window), written by the lane of t_f
+    auto put_head = [&](int i, double x_lo, double x_hi, int win) {
+        SegRec* r = reinterpret_cast<SegRec*>(Cf) + ((base + i) * M + m);
+        r->x_lo = x_lo;
+        r->x_hi = x_hi;
+        r->win = win;
+        r->pad0 = 0;
+        r->pad1 = 0.0;
+    };
     auto yi = [&](int i) { return Yc[((base + i) * M + m) * NQ + q]; };
     // the forward sweep's d' of this quantity and the mode's c' (the same for
     // its nine quantities: it depends on the knots alone), NQ + 1 per (knot, mode)
@@ -391,7 +431,7 @@ __global__ __launch_bounds__(64) void k_dir_spline(const double* __restrict__ X,
     }
     double xn = xi(n - 1), yn = yi(n - 1);
     *reinterpret_cast<Cubic*>(Cf + at(n - 1)) = Cubic{yn, 0.0, 0.0, 0.0};
-    if (q == 0) *reinterpret_cast<Cubic*>(Cf + ((base + n - 1) * M + m) * RS) = Cubic{xn, xn, 0.0, 0.0};
+    if (q == 2) put_head(n - 1, xn, xn, WIN_MIXED);
     if (CfF) put_f(n - 1, xn, xn, yn, 0.0, 0.0, 0.0);
     for (int i0 = n - 2; i0 >= 0; i0 -= DSPL_BLOCK) {
       double dv[DSPL_BLOCK], cv[DSPL_BLOCK], xv[DSPL_BLOCK], yv[DSPL_BLOCK];
@@ -415,7 +455,7 @@ __global__ __launch_bounds__(64) void k_dir_spline(const double* __restrict__ X,
         const double c2 = (slope - si) * idx - t, c3 = t * idx;
         *reinterpret_cast<Cubic*>(Cf + at(i)) = Cubic{y_i, si, c2, c3};
         if (CfF) put_f(i, x_i, xn, y_i, si, c2, c3);
-        if (q == 0) *reinterpret_cast<Cubic*>(Cf + ((base + i) * M + m) * RS) = Cubic{x_i, xn, 0.0, 0.0};
+        if (q == 2) put_head(i, x_i, xn, segment_window(Cubic{y_i, si, c2, c3}, xn - x_i, ts, te));
         snext = si;
         xn = x_i;
         yn = y_i;
@@ -559,52 +599,51 @@ __global__ void k_dir_perm(int* __restrict__ perm, int* __restrict__ cnt, const 
     perm[atomicAdd(&cnt[item_chunk(band, B, it, chunk, b)], 1)] = it;
 }
 
-// h[ch] += conj(T_ch A e^{i phase}) of one mode at x = f - x_i into its segment, if
-// t_start <= tf <= t_end (t_end <= 0: no upper limit) (WaveformBuild.cu:48-60, :80-143)
-template <class Q>
-__device__ inline void add_mode(cd h[3], const Q& q, double x, double ts, double te, const double2* tab)
+// h[ch] += conj(T_ch A e^{i phase}) of one mode at x = f - x_i into its segment
+// (WaveformBuild.cu:48-60, :80-143)
+__device__ inline void add_mode(cd h[3], const Cubic* q, double x, const double2* tab)
 {
-    const double x2 = x * x, x3 = x * x2;
-    auto ev = [&](int k) {
-        const Cubic c = cubic_of(q, k);
-        return c.y + c.c1 * x + c.c2 * x2 + c.c3 * x3;
-    };
-    const double tf = ev(2);
-    if ((tf >= ts) && ((tf <= te) || (te <= 0.0))) {
-        const cd ap = ev(0) * cexpi_tab(ev(1), tab);
-        h[0] += conj(mk(ev(3), ev(4)) * ap);
-        h[1] += conj(mk(ev(5), ev(6)) * ap);
-        h[2] += conj(mk(ev(7), ev(8)) * ap);
+    auto ev = [&](int k) { return fma(fma(fma(q[k].c3, x, q[k].c2), x, q[k].c1), x, q[k].y); };
+    const cd ap = ev(S_A) * cexpi_tab1k(ev(S_PH), tab);
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        const double tr = ev(S_T + 2 * c), ti = ev(S_T + 2 * c + 1);
+        h[c].re = fma(tr, ap.re, fma(-ti, ap.im, h[c].re));
+        h[c].im = fma(-tr, ap.im, fma(-ti, ap.re, h[c].im));
     }
+}
+
+// t_start <= t_f <= t_end (t_end <= 0: no upper limit) at x into a segment whose
+// 'win' does not say so already (WaveformBuild.cu:50)
+__device__ inline bool bin_in_window(const Cubic& c, double x, double ts, double te)
+{
+    const double tf = fma(fma(fma(c.c3, x, c.c2), x, c.c1), x, c.y);
+    return (tf >= ts) && ((tf <= te) || (te <= 0.0));
+}
+
+// add_mode where the window may cut the segment: q is the record at rc with all
+// but t_f's cubic loaded
+__device__ inline void add_mode_window(cd h[3], const SegRec& q, const SegRec* rc, double x, double ts, double te,
+                                       const double2* tab)
+{
+    if (q.win != WIN_ALL && (q.win == WIN_NONE || !bin_in_window(rc->q[S_TF], x, ts, te))) return;
+    add_mode(h, q.q, x, tab);
 }
 
 // Segment of one lane's dense frequency f in the grid of one mode, searched by
 // that lane, and its contribution (lanes of a wavefront in many different
-// segments). The record at the FP32 log2 estimate is read with its bounds and
-// all nine cubics in one round of loads; the index then moves until
-// x_lo <= f < x_hi or leaves [0, L - 2] (no contribution, WaveformBuild.cu:92-93).
-__device__ inline void mode_per_lane(cd h[3], const SegRec* __restrict__ rm, int M, int L, double f, int i, double ts,
-                                     double te, const double2* tab)
+// segments): from the FP32 log2 estimate the index moves until x_lo <= f < x_hi
+// or leaves [0, L - 2] (no contribution, WaveformBuild.cu:92-93).
+template <class Rec>
+__device__ inline void mode_per_lane(dense_sum<Rec> h[3], const Rec* __restrict__ rm, int M, int L,
+                                     double f, int i, double ts, double te, const double2* tab)
 {
-    const SegRec* r = rm + (long)i * M;
-    double2 bnd = *reinterpret_cast<const double2*>(r);
-    Cubic cq[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; q++) cq[q] = r->q[q];
-    // keeps the compiler from sinking these loads below the bounds check
-    // (which would serialise two rounds of memory latency)
-#pragma unroll
-    for (int q = 0; q < NQ; q++) asm volatile("" ::"v"(cq[q].y), "v"(cq[q].c1), "v"(cq[q].c2), "v"(cq[q].c3));
-    if (!(bnd.x <= f && f < bnd.y)) {
-        // the estimate missed (rounding near a knot): walk to the segment holding f
-        while (f < bnd.x && i > 0) bnd = *reinterpret_cast<const double2*>(rm + (long)--i * M);
-        while (f >= bnd.y && i < L - 2) bnd = *reinterpret_cast<const double2*>(rm + (long)++i * M);
-        if (!(bnd.x <= f && f < bnd.y)) return;
-        r = rm + (long)i * M;
-#pragma unroll
-        for (int q = 0; q < NQ; q++) cq[q] = r->q[q];
-    }
-    add_mode(h, cq, f - bnd.x, ts, te, tab);
+    double2 bnd = *reinterpret_cast<const double2*>(rm + (long)i * M);
+    while (f < bnd.x && i > 0) bnd = *reinterpret_cast<const double2*>(rm + (long)--i * M);
+    while (f >= bnd.y && i < L - 2) bnd = *reinterpret_cast<const double2*>(rm + (long)++i * M);
+    if (!(bnd.x <= f && f < bnd.y)) return;
+    const Rec* rc = rm + (long)i * M;
+    add_mode_window(h, *rc, rc, f - bnd.x, ts, te, tab);
 }
 
 // e^{i phase} in FP32 from an FP64 phase: the phase in revolutions reduced to
@@ -626,10 +665,11 @@ __device__ inline cf cexpi_f32(double phase, float* corr)
     return cf{c, s};
 }
 
-// add_mode of the FP32-bulk form: t(f) and the phase evaluated in FP64 (the
+// add_mode_window of the FP32-bulk form: t(f) and the phase evaluated in FP64 (the
 // same expressions as the FP64 form, so the window decision is identical),
 // the other seven cubics and the mode sum in FP32.
-__device__ inline void add_mode(cf h[3], const SegRecF& q, double x, double ts, double te, const double2*)
+__device__ inline void add_mode_window(cf h[3], const SegRecF& q, const SegRecF*, double x, double ts, double te,
+                                       const double2*)
 {
     const double x2 = x * x, x3 = x * x2;
     const double tf = q.tf[0] + q.tf[1] * x + q.tf[2] * x2 + q.tf[3] * x3;
@@ -651,28 +691,6 @@ __device__ inline void add_mode(cf h[3], const SegRecF& q, double x, double ts, 
     }
 }
 
-// mode_per_lane of the FP32-bulk form: the whole 192-B record in one round of loads
-__device__ inline void mode_per_lane(cf h[3], const SegRecF* __restrict__ rm, int M, int L, double f, int i,
-                                     double ts, double te, const double2*)
-{
-    SegRecF rec = rm[(long)i * M];
-    // keeps the compiler from sinking these loads below the bounds check
-#pragma unroll
-    for (int k = 0; k < 4; k++) asm volatile("" ::"v"(rec.ph[k]), "v"(rec.tf[k]));
-#pragma unroll
-    for (int k = 0; k < 7; k++) asm volatile("" ::"v"(rec.q[k][0]), "v"(rec.q[k][1]), "v"(rec.q[k][2]), "v"(rec.q[k][3]));
-    if (!(rec.x_lo <= f && f < rec.x_hi)) {
-        double2 bnd = make_double2(rec.x_lo, rec.x_hi);
-        while (f < bnd.x && i > 0) bnd = *reinterpret_cast<const double2*>(rm + (long)--i * M);
-        while (f >= bnd.y && i < L - 2) bnd = *reinterpret_cast<const double2*>(rm + (long)++i * M);
-        if (!(bnd.x <= f && f < bnd.y)) return;
-        rec = rm[(long)i * M];
-    }
-    add_mode(h, rec, f - rec.x_lo, ts, te, nullptr);
-}
-
-constexpr int RB = 2;  // iterations of 64 dense bins per block of a wavefront
-
 // ---------------------------------------------------------------- adjoint helpers
 
 // Adjoint record of one (knot, mode): for each of the nine quantities, the
@@ -688,25 +706,20 @@ __device__ inline int adj_q(int j) { return j < 2 ? j : j + 1; }
 // y, c1, c2, c3 each) of one mode at one dense bin, given
 // Lam_c = 4 w_c (d~_c - h~_c) (d logL = Re sum_c conj(Lam_c) dh_c with
 // h_c = sum_m conj(T_c A e^{i phase}); Likelihood.cu:357-375 differentiated).
-template <class Q>
-__device__ inline bool mode_adjoint(double cb[32], const Q& q, double x, double ts, double te, const cd Lam[3],
+__device__ inline bool mode_adjoint(double cb[32], const SegRec& q, double x, double ts, double te, const cd Lam[3],
                                     const double2* tab)
 {
+    if (q.win == WIN_NONE || (q.win == WIN_MIXED && !bin_in_window(q.q[S_TF], x, ts, te))) return false;
     const double x2 = x * x, x3 = x * x2;
-    auto ev = [&](int k) {
-        const Cubic c = cubic_of(q, k);
-        return c.y + c.c1 * x + c.c2 * x2 + c.c3 * x3;
-    };
-    const double tf = ev(2);
-    if (!((tf >= ts) && ((tf <= te) || (te <= 0.0)))) return false;
-    const double A = ev(0);
-    const cd E = cexpi_tab(ev(1), tab);
+    auto ev = [&](int k) { return fma(fma(fma(q.q[k].c3, x, q.q[k].c2), x, q.q[k].c1), x, q.q[k].y); };
+    const double A = ev(S_A);
+    const cd E = cexpi_tab1k(ev(S_PH), tab);
     const cd AE = A * E;
     double a[8];
     cd P = mk(0.0, 0.0);
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-        const cd T = mk(ev(3 + 2 * c), ev(4 + 2 * c));
+        const cd T = mk(ev(S_T + 2 * c), ev(S_T + 2 * c + 1));
         P += Lam[c] * T;
         const cd LAE = Lam[c] * AE;
         a[2 + 2 * c] = LAE.re;
@@ -769,30 +782,75 @@ __device__ inline void mode_adjoint_per_lane(double* __restrict__ Ym, const SegR
     for (int j = 0; j < 32; j++) unsafeAtomicAdd(y + adj_q(j >> 2) * 4 + (j & 3), cb[j]);
 }
 
-// Persistent dense-band kernel: partial[it] = (Re, Im of sum conj(d~) h~, sum |h~|^2, 0)
+// Persistent dense-band kernel, each wavefront taking work items of its own (the
+// wavefronts of a workgroup share the table of e^{i theta} and no barrier):
+// partial[it] = (Re, Im of sum conj(d~) h~, sum |h~|^2, 0)
 // over the dense bins of work item it, where h~ = w h (Likelihood.cu:357-375).
 //
-// Each wavefront takes a contiguous share of the work item's bins, in blocks of
-// RB x 64 consecutive bins (lane l: bins kb + 64 r + l), and sums the modes of a
+// A work item's bins go in blocks of RB x 64 consecutive bins (lane l: bins kb + 64 r + l), and sums the modes of a
 // block mode by mode. The segment of bin f in a mode's grid is
-// searchsorted(x, f, 'right') - 1 (waveformbuild.py:139-156). Dense bins are
-// much finer than the sparse grid over most of a band, so the lanes of an
-// iteration usually share one or two segments: a wavefront-uniform walker then
-// holds the current segment, reads its record once with scalar loads (bounds and
-// the nine cubics) and evaluates every lane whose f lies in [x_lo, x_hi), moving
-// to the next segment until all lanes are placed. The comparisons are the exact
-// FP64 ones against the stored knots, so the segment of every bin is the one
-// searchsorted gives. Where an iteration spans more than three segments (low
-// frequencies, short segments) each lane searches its own (mode_per_lane).
+// searchsorted(x, f, 'right') - 1 (waveformbuild.py:139-156), found with the
+// exact FP64 comparisons x_lo <= f < x_hi against the stored knots.
+//
+// Dense bins are much finer than the sparse grid over most of a band, so a block
+// usually lies in the segment that the mode's previous block ended in (kept in
+// lane m of 'curv'): a wavefront-uniform walker reads its record in one round of
+// scalar loads, evaluates every bin in [x_lo, x_hi) (t_f only where 'win' leaves
+// the window open) and moves to the next segment until all bins are placed. After
+// WALK_STEPS segments (low frequencies, where a block spans many) each lane left
+// over searches its own (mode_per_lane).
+//
+// Bound by FP64 issue: 55 vector instructions per (bin, mode) evaluation (24 of
+// the eight cubics, 14 of e^{i phase}, 12 of the mode sum), about 77 with the
+// walker and the inner products, vector units 82 % busy. 1024 uneven templates,
+// 1.58 M bins: 44.3 -> 20 ms (145 instructions per evaluation before, 65 %
+// busy: two rounds of scalar loads per segment and iteration, t_f for every bin,
+// a copy of one coefficient per cubic and bin, a 24-operation e^{i phase}).
+// RB = 4 measured best: the whole step 25.9 (RB = 2), 24.9 (3), 24.5 ms (4);
+// fewer iterations pay the record loads and the walker more often.
 //
 // ADJ: also the adjoint pass of the direct log-likelihood's gradient: after the
 // mode sum of a block, Lam = 4 w (d~ - h~) per bin and channel, then the modes
 // again, each bin's coefficient adjoints (mode_adjoint) summed over the lanes
 // that share a segment (reduce32) and added to the segment's adjoint record.
-// FP64 forms: at least 4 wavefronts per SIMD (at most 128 VGPRs), measured
-// faster than the 3 that the unconstrained register allocation gives, despite a
-// few spilled registers in the rarely taken per-lane path; FP32-bulk form: at
-// least 6 (at most 80 VGPRs), measured 6 % faster than its unconstrained 5
+// FP64 forms: at least 4 wavefronts per SIMD (at most 128 VGPRs); FP32-bulk
+// form: at least 6 (at most 80 VGPRs)
+
+constexpr int DENSE_RB = 4;  // iterations of 64 dense bins per block of a wavefront
+
+// A record at a wavefront-uniform address, its bounds and cubics (t_f's apart)
+// loaded in one round: the statements keep the compiler from sinking the
+// cubics' loads below the bounds check, which would serialise two rounds of
+// memory latency.
+__device__ inline SegRec load_uniform(const SegRec* rc)
+{
+    SegRec q;
+    q.x_lo = rc->x_lo;
+    q.x_hi = rc->x_hi;
+    q.win = rc->win;
+#pragma unroll
+    for (int k = 0; k < S_TF; k++) q.q[k] = rc->q[k];
+#pragma unroll
+    for (int k = 0; k < S_TF; k++)
+        asm volatile("" ::"s"(q.q[k].y), "s"(q.q[k].c1), "s"(q.q[k].c2), "s"(q.q[k].c3));
+    // an instruction takes one scalar operand: the c2 are copied to vector
+    // registers here, once for the iterations that share the record, where each
+    // cubic would otherwise copy one of its first two coefficients for every bin
+#pragma unroll
+    for (int k = 0; k < S_TF; k++) asm volatile("" : "+v"(q.q[k].c2));
+    return q;
+}
+__device__ inline SegRecF load_uniform(const SegRecF* rc) { return *rc; }
+
+// Steps of the walker before the lanes left over search for themselves.
+constexpr int WALK_STEPS = 4;
+
+// segment of f in a log-spaced grid, from an FP32 log2 (within one or two)
+__device__ inline int segment_estimate(double f, double glo, double gis, int L)
+{
+    return (int)fmin(fmax(((double)__log2f((float)f) - glo) * gis, 0.0), (double)(L - 2));
+}
+
 template <bool ADJ, class Rec>
 __global__ __launch_bounds__(256) __attribute__((
     amdgpu_waves_per_eu(std::is_same<Rec, SegRecF>::value ? 6 : 4, 8))) void k_dir_like_t(double* __restrict__ partial, double* __restrict__ Yadj,
@@ -808,103 +866,113 @@ __global__ __launch_bounds__(256) __attribute__((
                                                   int B, int M, int chunk)
 {
     static_assert(!ADJ || std::is_same<Rec, SegRec>::value, "the adjoint pass reads FP64 records");
-    using HT = typename std::conditional<std::is_same<Rec, SegRecF>::value, cf, cd>::type;
-    __shared__ double red[3][256 / 64];
-    __shared__ int s_next;
-    __shared__ double2 s_tab[129];
+    constexpr bool F32 = std::is_same<Rec, SegRecF>::value;
+    constexpr int RB = ADJ ? 2 : DENSE_RB;
+    using HT = dense_sum<Rec>;
+    __shared__ double2 s_tab[F32 ? 1 : 1024];
     const int nitems = total[0];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nw = blockDim.x >> 6;
-    if constexpr (!std::is_same<Rec, SegRecF>::value) fill_etab(s_tab, tid, blockDim.x);  // before the first barrier
+    const int lane = threadIdx.x & 63;
+    if constexpr (!F32) {
+        fill_etab1k(s_tab, threadIdx.x, blockDim.x);
+        __syncthreads();
+    }
     for (;;) {
-        // the next item in the chunk-major order (dynamic: the items running at
-        // any time stay a window of consecutive entries, i.e. the same chunks)
-        if (tid == 0) s_next = atomicAdd(next, 1);
-        __syncthreads();
-        const int pi = s_next;
-        __syncthreads();
+        // the wavefront's next item in the chunk-major order (dynamic: the items
+        // running at any time stay a window of consecutive entries, i.e. the same
+        // dense bins). The barrier (no instruction) is convergent: without one in
+        // this block the compiler may thread the branch on lane 0 with one at the
+        // end of the loop, and the other lanes would go round it on their own
+        __builtin_amdgcn_wave_barrier();
+        int pi = 0;
+        if (lane == 0) pi = atomicAdd(next, 1);
+        pi = __builtin_amdgcn_readfirstlane(pi);
         if (pi >= nitems) break;
         const int it = perm[pi];
         int b;
         const int g = item_chunk(band, B, it, chunk, b);
-        const int st = band[3 * b];
-        const int k0 = max(st, g * chunk);
-        const int k1 = min(band[3 * b + 1], (g + 1) * chunk);
+        const int kw0 = max(band[3 * b], g * chunk), kw1 = min(band[3 * b + 1], (g + 1) * chunk);
         const long base = off[b];
         const int L = len[b];
         const double ts = t_start[b], te = t_end[b];
-        // this wavefront's share: a multiple of 64 bins
-        const int per = (((k1 - k0 + nw - 1) / nw) + 63) & ~63;
-        const int kw0 = k0 + wv * per, kw1 = min(k1, kw0 + per);
         double a0 = 0.0, a1 = 0.0, a2 = 0.0;
+        // lane m: the segment that mode m's last block ended in; -1: not known,
+        // -2: a degenerate grid, no segment holds any f
+        int curv = -1;
+        if (lane < M && !(grid_istep[b * M + lane] > 0.0)) curv = -2;
         for (int kb = kw0; kb < kw1; kb += RB * 64) {
-            double f[RB], lf[RB];
+            double f[RB];
             HT h[RB][3];
 #pragma unroll
             for (int r = 0; r < RB; r++) {
-                const int k = kb + 64 * r + lane;
-                f[r] = k < kw1 ? freqs[k] : 0.0;
-                lf[r] = (double)__log2f((float)f[r]);
+                // bins past the item repeat its last one (not summed below)
+                f[r] = freqs[min((unsigned)(kb + 64 * r + lane), (unsigned)(kw1 - 1))];
 #pragma unroll
                 for (int ch = 0; ch < 3; ch++) zero(h[r][ch]);
             }
             for (int m = 0; m < M; m++) {
-                const double gis = grid_istep[b * M + m];
-                if (!(gis > 0.0)) continue;  // degenerate grid: no segment holds any f
-                const double glo = grid_lo[b * M + m];
+                int cur = __builtin_amdgcn_readlane(curv, m);
+                if (cur == -2) continue;
                 const Rec* rm = R + base * M + m;
-                int cur = -1;  // the walker's segment (wavefront-uniform); -1: not placed
-#pragma unroll
-                for (int r = 0; r < RB; r++) {
-                    bool pending = kb + 64 * r + lane < kw1;
-                    const unsigned long long pm = __ballot(pending);
-                    if (pm == 0) break;  // later iterations are past the share too
-                    const int est = (int)fmin(fmax((lf[r] - glo) * gis, 0.0), (double)(L - 2));
-                    const int e_first = __builtin_amdgcn_readlane(est, __builtin_ctzll(pm));
-                    const int e_last = __builtin_amdgcn_readlane(est, 63 - __builtin_clzll(pm));
-                    if (e_last - e_first > 2) {
-                        if (pending) mode_per_lane(h[r], rm, M, L, f[r], est, ts, te, s_tab);
-                        cur = -1;
-                        continue;
-                    }
-                    if (cur < 0) cur = e_first;
-                    // the walker moves down only while a pending lane lies below the current
-                    // segment, up only past lanes it has placed: in a sorted grid every step
-                    // makes progress; the bound only guards against an unsorted one
-                    for (int guard = 2 * L + 8; guard > 0; guard--) {
-                        if (__ballot(pending) == 0) break;
-                        const Rec* rc = rm + (long)cur * M;
-                        const double xlo = rc->x_lo, xhi = rc->x_hi;
-                        const bool below = pending && f[r] < xlo;
-                        if (__ballot(below) != 0) {
-                            if (cur == 0) pending = pending && !below;  // left of the grid
-                            else cur--;
-                            continue;
-                        }
-                        const bool in = pending && f[r] < xhi;
-                        if (in) add_mode(h[r], *rc, f[r] - xlo, ts, te, s_tab);
-                        pending = pending && !in;
-                        if (__ballot(pending) != 0) {
-                            if (cur == L - 2) pending = false;  // right of the grid
-                            else cur++;
-                        }
-                    }
+                if (cur < 0) {
+                    const int est = segment_estimate(f[0], grid_lo[b * M + m], grid_istep[b * M + m], L);
+                    cur = __builtin_amdgcn_readfirstlane(est);
                 }
+                bool todo[RB];
+#pragma unroll
+                for (int r = 0; r < RB; r++) todo[r] = kb + 64 * r + lane < kw1;
+                // lanes below the current segment send the walker down, else lanes
+                // above it up; a sorted block needs one step per segment it spans
+                bool open = true;
+                for (int step = 0; step < WALK_STEPS; step++) {
+                    cur = __builtin_amdgcn_readfirstlane(cur);
+                    const Rec* rc = rm + (unsigned)(cur * M);
+                    const Rec q = load_uniform(rc);
+                    bool rest = false;
+#pragma unroll
+                    for (int r = 0; r < RB; r++) {
+                        const bool in = todo[r] && f[r] >= q.x_lo && f[r] < q.x_hi;
+                        if (in) add_mode_window(h[r], q, rc, f[r] - q.x_lo, ts, te, s_tab);
+                        todo[r] = todo[r] && !in;
+                        rest = rest || todo[r];
+                    }
+                    if (!__any(rest)) { open = false; break; }
+                    bool below = false, above = false;
+#pragma unroll
+                    for (int r = 0; r < RB; r++) {
+                        below = below || (todo[r] && f[r] < q.x_lo);
+                        above = above || (todo[r] && f[r] >= q.x_hi);
+                    }
+                    if (__any(below) && cur > 0) cur--;
+                    else if (__any(above) && cur < L - 2) cur++;
+                    else { open = false; break; }  // beyond the grid's ends: no contribution
+                }
+                if (open) {
+#pragma unroll
+                    for (int r = 0; r < RB; r++)
+                        if (todo[r])
+                            mode_per_lane(h[r], rm, M, L, f[r],
+                                          segment_estimate(f[r], grid_lo[b * M + m], grid_istep[b * M + m], L), ts, te,
+                                          s_tab);
+                    cur = -1;
+                }
+                curv = lane == m ? cur : curv;
             }
+            // bins past the item repeat its last one with weight 0 (no branch, so
+            // that the loads of all iterations can go ahead of the arithmetic)
 #pragma unroll
             for (int r = 0; r < RB; r++) {
-                const int k = kb + 64 * r + lane;
-                if (k < kw1) {
+                const bool mine = kb + 64 * r + lane < kw1;
+                const unsigned k = min((unsigned)(kb + 64 * r + lane), (unsigned)(kw1 - 1));
 #pragma unroll
-                    for (int ch = 0; ch < 3; ch++) {
-                        const double w = wts[(long)ch * N + k];
-                        const cd ht = to_cd(h[r][ch]) * w;
-                        const cd d = dch[(long)ch * N + k];
-                        const cd dh = conj(d) * ht;
-                        a0 += dh.re;
-                        a1 += dh.im;
-                        a2 += ht.re * ht.re + ht.im * ht.im;
-                        if constexpr (ADJ) h[r][ch] = (4.0 * w) * (d - ht);  // Lam
-                    }
+                for (int ch = 0; ch < 3; ch++) {
+                    const double wk = (wts + (long)ch * N)[k];
+                    const cd d = (dch + (long)ch * N)[k];
+                    const double w = mine ? wk : 0.0;
+                    const cd ht = to_cd(h[r][ch]) * w;
+                    a0 = fma(d.re, ht.re, fma(d.im, ht.im, a0));
+                    a1 = fma(d.re, ht.im, fma(-d.im, ht.re, a1));
+                    a2 = fma(ht.re, ht.re, fma(ht.im, ht.im, a2));
+                    if constexpr (ADJ) h[r][ch] = (4.0 * w) * (d - ht);  // Lam
                 }
             }
             if constexpr (ADJ) {
@@ -920,7 +988,8 @@ __global__ __launch_bounds__(256) __attribute__((
                         bool pending = kb + 64 * r + lane < kw1;
                         const unsigned long long pm = __ballot(pending);
                         if (pm == 0) break;
-                        const int est = (int)fmin(fmax((lf[r] - glo) * gis, 0.0), (double)(L - 2));
+                        const double lf = (double)__log2f((float)f[r]);
+                        const int est = (int)fmin(fmax((lf - glo) * gis, 0.0), (double)(L - 2));
                         const int e_first = __builtin_amdgcn_readlane(est, __builtin_ctzll(pm));
                         const int e_last = __builtin_amdgcn_readlane(est, 63 - __builtin_clzll(pm));
                         if (e_last - e_first > 2) {
@@ -962,29 +1031,12 @@ __global__ __launch_bounds__(256) __attribute__((
                 }
             }
         }
-        // block reduction in a fixed order
         a0 = wsum(a0);
         a1 = wsum(a1);
         a2 = wsum(a2);
-        if (lane == 0) {
-            red[0][wv] = a0;
-            red[1][wv] = a1;
-            red[2][wv] = a2;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-            for (int w = 0; w < nw; w++) {
-                s0 += red[0][w];
-                s1 += red[1][w];
-                s2 += red[2][w];
-            }
-            partial[4 * (long)it] = s0;
-            partial[4 * (long)it + 1] = s1;
-            partial[4 * (long)it + 2] = s2;
-            partial[4 * (long)it + 3] = 0.0;
-        }
-        __syncthreads();
+        // every lane holds the sums: lanes l, l + 4, ... write the same value l
+        const int c = lane & 3;
+        partial[4 * (long)it + c] = c == 0 ? a0 : (c == 1 ? a1 : (c == 2 ? a2 : 0.0));
     }
 }
 
@@ -1350,6 +1402,27 @@ void plan_free(bbhx_direct_plan* p)
 
 }  // namespace
 
+// ---- dense bins per work item
+//
+// A work item is what one wavefront takes: a caller's chunk (bins per workgroup
+// and pass) split over the workgroup's wavefronts, and less than that for a small
+// batch, so that there are several items per wavefront slot (4 per SIMD, 4096)
+// for the dynamic order to balance, down to ITEM_MIN bins (one block of the FP64
+// kernel). Plans of up to SMALL_ITEMS such items have buffers for them. 16
+// templates of 65536 bins: 1.78 -> 1.14 ms for the whole step (64 items of 16384
+// bins left most of the chip idle). At 1024 templates of 1.58 M bins the item size
+// does not matter (items of 4096, 8192 and 16384 bins: 25.4, 25.5 and 26.3 ms).
+constexpr long ITEM_MIN = 256, SMALL_ITEMS = 1L << 18, ITEMS_WANTED = 4 * 4096;
+
+static int item_bins(const bbhx_direct_plan* p, int chunk, int block)
+{
+    long n = chunk / (block / 64);
+    const long fine = (long)p->B * p->N / ITEMS_WANTED;  // the whole data set of every binary over that many items
+    n = std::min(n, std::max(fine, ITEM_MIN));
+    n = (n + ITEM_MIN - 1) / ITEM_MIN * ITEM_MIN;
+    return (int)std::max(n, (long)p->min_item);
+}
+
 extern "C" int bbhx_hip_direct_plan_create(bbhx_direct_plan** out, int numBinAll, const int* lengths_host,
                                            int numModes, int data_length, int min_chunk)
 {
@@ -1374,8 +1447,11 @@ extern "C" int bbhx_hip_direct_plan_create(bbhx_direct_plan** out, int numBinAll
     p->N = data_length;
     p->Lmax = Lmax;
     p->min_chunk = min_chunk;
+    // small batches are cut finer than the caller's chunks (item_bins)
+    p->min_item = (long)numBinAll * data_length <= ITEM_MIN * SMALL_ITEMS ? std::min(min_chunk, (int)ITEM_MIN)
+                                                                         : min_chunk;
     p->S = S;
-    p->max_items = (long)numBinAll * ((data_length + min_chunk - 1) / min_chunk) + numBinAll;
+    p->max_items = (long)numBinAll * ((data_length + p->min_item - 1) / p->min_item) + numBinAll;
     if (p->max_items > 2147483647L) {
         delete p;
         return ERR_ARGS;
@@ -1394,7 +1470,7 @@ extern "C" int bbhx_hip_direct_plan_create(bbhx_direct_plan** out, int numBinAll
     p->band = dalloc<int>((size_t)numBinAll * 3, ok);
     p->total = dalloc<int>(1, ok);
     p->partial = dalloc<double>((size_t)p->max_items * 4, ok);
-    p->max_chunks = (data_length + min_chunk - 1) / min_chunk;
+    p->max_chunks = (data_length + p->min_item - 1) / p->min_item;
     p->perm = dalloc<int>((size_t)p->max_items, ok);
     p->cnt = dalloc<int>((size_t)p->max_chunks + 1, ok);
     p->next = dalloc<int>(1, ok);
@@ -1460,6 +1536,7 @@ int direct_launch(bbhx_direct_plan* p, double* d_h, double* h_h, double* grad, i
 {
     if (!p) return ERR_ARGS;
     if (chunk < p->min_chunk || (block != 64 && block != 128 && block != 256) || grid < 1) return ERR_ARGS;
+    chunk = item_bins(p, chunk, block);
     int dev = -1;
     (void)hipGetDevice(&dev);
     if (dev != p->device || numModes != p->M) return ERR_ARGS;
@@ -1486,14 +1563,15 @@ int direct_launch(bbhx_direct_plan* p, double* d_h, double* h_h, double* grad, i
     // the FP32-bulk form (not for the gradient, whose adjoint pass reads the FP64 records)
     const bool f32 = !grad && p->precision == 1;
     hipLaunchKernelGGL(k_dir_spline, dim3(B), dim3(64), 0, st, p->X, p->Yc, p->Cf, p->Fs,
-                       f32 ? static_cast<SegRecF*>(p->CfF) : nullptr, p->off, p->len, M);
+                       f32 ? static_cast<SegRecF*>(p->CfF) : nullptr, p->off, p->len, t_start, t_end, M);
     hipLaunchKernelGGL(k_dir_band, dim3(1), dim3(1024), 0, st, p->band, p->total, p->X, p->off, p->len, dataFreqs,
                        p->N, B, M, chunk);
-    const int nchunks = (p->N + chunk - 1) / chunk;  // <= max_chunks since chunk >= min_chunk
+    const int nchunks = (p->N + chunk - 1) / chunk;  // <= max_chunks since chunk >= min_item
     hipLaunchKernelGGL(k_dir_cnt_zero, dim3(ceil_div(nchunks + 1, 256)), dim3(256), 0, st, p->cnt, nchunks + 1,
                        p->next);
     // one lane per possible work item (those past the batch's count exit)
-    const int item_blocks = ceil_div(p->max_items, 256);
+    const long items = std::min(p->max_items, (long)B * nchunks + B);
+    const int item_blocks = ceil_div(items, 256);
     hipLaunchKernelGGL(k_dir_cnt, dim3(item_blocks), dim3(256), 0, st, p->cnt, p->band, p->total, B, chunk);
     hipLaunchKernelGGL(k_dir_cnt_scan, dim3(1), dim3(1024), 0, st, p->cnt, nchunks);
     hipLaunchKernelGGL(k_dir_perm, dim3(item_blocks), dim3(256), 0, st, p->perm, p->cnt, p->band, p->total, B, chunk);
@@ -1517,7 +1595,7 @@ int direct_launch(bbhx_direct_plan* p, double* d_h, double* h_h, double* grad, i
         hipLaunchKernelGGL(k_dir_route, dim3(B), dim3(64), 0, st, p->route, p->X, p->Yc, p->off, p->len, t_start,
                            t_end, dataFreqs, noiseFactors, p->N, M);
         hipLaunchKernelGGL(k_dir_loud_zero, dim3(1), dim3(64), 0, st, p->loud_cnt);
-        const int split_blocks = ceil_div(p->max_items, SPLIT_BLOCK);  // <= max_items / 256 + 1
+        const int split_blocks = ceil_div(items, SPLIT_BLOCK);  // <= max_items / 256 + 1
         hipLaunchKernelGGL(k_dir_split_count, dim3(split_blocks), dim3(SPLIT_BLOCK), 0, st, p->split_cnt, p->perm,
                            p->total, p->band, B, p->route);
         hipLaunchKernelGGL(k_dir_cnt_scan, dim3(1), dim3(1024), 0, st, p->split_cnt, split_blocks);
