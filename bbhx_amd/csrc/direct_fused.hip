@@ -33,7 +33,6 @@
 //   k_dir_reduce  one wavefront per binary: its partials in a fixed order (deterministic)
 
 #include <algorithm>
-#include <type_traits>
 #include <vector>
 
 #include "bbhx_hip.h"
@@ -75,14 +74,6 @@ struct bbhx_direct_plan {
     double* Yadj = nullptr;              // (S, M, 9, 4) adjoint records
     bbhx::gradk::GradRec* grecs = nullptr;  // (B, M) records with tangents
     double* gpart = nullptr;             // (B, M, 11) per-mode gradients
-    // FP32-bulk form (bbhx_hip_direct_plan_set_precision)
-    int precision = 0;                   // 0: FP64, 1: FP32 bulk, FP64 phase and t(f)
-    void* CfF = nullptr;                 // (S, M) 192-B segment records of that form
-    int* loud = nullptr;                 // (max_items,) work items of the binaries evaluated in FP64
-    int* quiet = nullptr;                // (max_items,) work items of the binaries evaluated in FP32
-    int* loud_cnt = nullptr;             // (4,) loud count, its pass's next-item counter; the same for quiet
-    int* route = nullptr;                // (B,) 1: the h_h estimate sends the binary to the FP64 pass
-    int* split_cnt = nullptr;            // (max_items / 256 + 1,) loud entries per block of the order, scanned
     int max_chunks = 0;           // absolute chunks of min_item bins
 };
 
@@ -116,32 +107,6 @@ static_assert(sizeof(SegRec) == 320, "segment record layout");
 constexpr int S_A = 0, S_PH = 1, S_T = 2, S_TF = 8;  // slots of q
 // slot of quantity q of the grid pass (A, phase, t_f, T1..T3 re/im)
 __host__ __device__ constexpr int seg_slot(int q) { return q < 2 ? q : (q == 2 ? S_TF : q - 1); }
-
-// Segment record of the FP32-bulk form: bounds and the phase and t(f) cubics
-// in FP64 (phases reach 1e8 rad, and t(f) decides the observation window
-// exactly as in the FP64 form), amplitude and the six transfer-function parts
-// (T1..T3 re, im) in FP32.
-struct alignas(64) SegRecF {
-    double x_lo, x_hi;
-    double ph[4];    // y, c1, c2, c3
-    double tf[4];
-    float q[7][4];   // A, T1 re, T1 im, T2 re, T2 im, T3 re, T3 im: y, c1, c2, c3
-};
-static_assert(sizeof(SegRecF) == 192, "FP32-bulk segment record layout");
-
-// single-precision complex (the mode sum of the FP32-bulk form)
-struct cf {
-    float re, im;
-};
-
-__device__ inline cd to_cd(cd a) { return a; }
-__device__ inline cd to_cd(cf a) { return mk((double)a.re, (double)a.im); }
-__device__ inline void zero(cd& a) { a = mk(0.0, 0.0); }
-__device__ inline void zero(cf& a) { a = cf{0.0f, 0.0f}; }
-
-// type of the mode sum of a record's form
-template <class Rec>
-using dense_sum = typename std::conditional<std::is_same<Rec, SegRecF>::value, cf, cd>::type;
 
 __global__ __launch_bounds__(64) void k_dir_setup(FusedRec* __restrict__ recs, const double* __restrict__ params, int B, ModeList modes,
                             int M, const double* __restrict__ qnm, int table_len, double dspin)
@@ -317,7 +282,7 @@ constexpr int DSPL_BLOCK = 8;  // rows loaded ahead of the recurrence in each sw
 // consecutive lanes read consecutive quantities of the same knot.
 __global__ __launch_bounds__(64) void k_dir_spline(const double* __restrict__ X, const double* __restrict__ Yc,
                                                    double* __restrict__ Cf, double* __restrict__ Fs,
-                                                   SegRecF* __restrict__ CfF, const long* __restrict__ off,
+                                                   const long* __restrict__ off,
                                                    const int* __restrict__ len, const double* __restrict__ t_start,
                                                    const double* __restrict__ t_end, int M)
 {
@@ -345,32 +310,6 @@ __global__ __launch_bounds__(64) void k_dir_spline(const double* __restrict__ X,
     // the forward sweep's d' of this quantity and the mode's c' (the same for
     // its nine quantities: it depends on the knots alone), NQ + 1 per (knot, mode)
     auto fs = [&](int i) { return ((base + i) * M + m) * (NQ + 1); };
-    // the FP32-bulk record of point i (CfF != nullptr): this lane's quantity
-    auto put_f = [&](int i, double x_lo, double x_hi, double c0, double c1, double c2, double c3) {
-        SegRecF& rf = CfF[(base + i) * M + m];
-        if (q == 1) {
-            rf.ph[0] = c0;
-            rf.ph[1] = c1;
-            rf.ph[2] = c2;
-            rf.ph[3] = c3;
-        } else if (q == 2) {
-            rf.tf[0] = c0;
-            rf.tf[1] = c1;
-            rf.tf[2] = c2;
-            rf.tf[3] = c3;
-        } else {
-            const int k = q == 0 ? 0 : q - 2;
-            rf.q[k][0] = (float)c0;
-            rf.q[k][1] = (float)c1;
-            rf.q[k][2] = (float)c2;
-            rf.q[k][3] = (float)c3;
-        }
-        if (q == 0) {
-            rf.x_lo = x_lo;
-            rf.x_hi = x_hi;
-        }
-    };
-
     // The forward sweep writes only d' and c' (80 B per (knot, mode), the
     // wavefront's lanes consecutive) to the scratch Fs; the backward sweep
     // writes every record once, in whole 32-B groups.
@@ -432,7 +371,6 @@ __global__ __launch_bounds__(64) void k_dir_spline(const double* __restrict__ X,
     double xn = xi(n - 1), yn = yi(n - 1);
     *reinterpret_cast<Cubic*>(Cf + at(n - 1)) = Cubic{yn, 0.0, 0.0, 0.0};
     if (q == 2) put_head(n - 1, xn, xn, WIN_MIXED);
-    if (CfF) put_f(n - 1, xn, xn, yn, 0.0, 0.0, 0.0);
     for (int i0 = n - 2; i0 >= 0; i0 -= DSPL_BLOCK) {
       double dv[DSPL_BLOCK], cv[DSPL_BLOCK], xv[DSPL_BLOCK], yv[DSPL_BLOCK];
 #pragma unroll
@@ -454,7 +392,6 @@ __global__ __launch_bounds__(64) void k_dir_spline(const double* __restrict__ X,
         const double t = (si + snext - 2 * slope) * idx;
         const double c2 = (slope - si) * idx - t, c3 = t * idx;
         *reinterpret_cast<Cubic*>(Cf + at(i)) = Cubic{y_i, si, c2, c3};
-        if (CfF) put_f(i, x_i, xn, y_i, si, c2, c3);
         if (q == 2) put_head(i, x_i, xn, segment_window(Cubic{y_i, si, c2, c3}, xn - x_i, ts, te));
         snext = si;
         xn = x_i;
@@ -634,61 +571,15 @@ __device__ inline void add_mode_window(cd h[3], const SegRec& q, const SegRec* r
 // that lane, and its contribution (lanes of a wavefront in many different
 // segments): from the FP32 log2 estimate the index moves until x_lo <= f < x_hi
 // or leaves [0, L - 2] (no contribution, WaveformBuild.cu:92-93).
-template <class Rec>
-__device__ inline void mode_per_lane(dense_sum<Rec> h[3], const Rec* __restrict__ rm, int M, int L,
+__device__ inline void mode_per_lane(cd h[3], const SegRec* __restrict__ rm, int M, int L,
                                      double f, int i, double ts, double te, const double2* tab)
 {
     double2 bnd = *reinterpret_cast<const double2*>(rm + (long)i * M);
     while (f < bnd.x && i > 0) bnd = *reinterpret_cast<const double2*>(rm + (long)--i * M);
     while (f >= bnd.y && i < L - 2) bnd = *reinterpret_cast<const double2*>(rm + (long)++i * M);
     if (!(bnd.x <= f && f < bnd.y)) return;
-    const Rec* rc = rm + (long)i * M;
+    const SegRec* rc = rm + (long)i * M;
     add_mode_window(h, *rc, rc, f - bnd.x, ts, te, tab);
-}
-
-// e^{i phase} in FP32 from an FP64 phase: the phase in revolutions reduced to
-// [-1/2, 1/2] in FP64 (for |phase| <= 1e9 rad the product and the rounding cost
-// < 2e-8 rad), then the hardware single-precision cosine and sine, which take
-// their argument in revolutions (error <= 1.3e-7). Their magnitude falls short
-// of 1 by ~3e-8 on average, a bias that does not average out over the dense
-// bins (it scales every template); *corr receives delta = (1 - c^2 - s^2) / 2,
-// formed in FP64 (products of two floats are exact there; in FP32 the sum
-// near 1 cannot resolve it), and the caller scales by 1 + delta.
-__device__ inline cf cexpi_f32(double phase, float* corr)
-{
-    double rev = phase * 0.15915494309189535;  // 1 / (2 pi)
-    rev -= rint(rev);
-    const float r = (float)rev;
-    const float c = __builtin_amdgcn_cosf(r), s = __builtin_amdgcn_sinf(r);
-    const double cd_ = c, sd_ = s;
-    *corr = (float)(-0.5 * fma(cd_, cd_, fma(sd_, sd_, -1.0)));
-    return cf{c, s};
-}
-
-// add_mode_window of the FP32-bulk form: t(f) and the phase evaluated in FP64 (the
-// same expressions as the FP64 form, so the window decision is identical),
-// the other seven cubics and the mode sum in FP32.
-__device__ inline void add_mode_window(cf h[3], const SegRecF& q, const SegRecF*, double x, double ts, double te,
-                                       const double2*)
-{
-    const double x2 = x * x, x3 = x * x2;
-    const double tf = q.tf[0] + q.tf[1] * x + q.tf[2] * x2 + q.tf[3] * x3;
-    if ((tf >= ts) && ((tf <= te) || (te <= 0.0))) {
-        float corr;
-        const cf E = cexpi_f32(q.ph[0] + q.ph[1] * x + q.ph[2] * x2 + q.ph[3] * x3, &corr);
-        const float xf = (float)x, xf2 = xf * xf, xf3 = xf2 * xf;
-        auto ev = [&](int k) { return q.q[k][0] + q.q[k][1] * xf + q.q[k][2] * xf2 + q.q[k][3] * xf3; };
-        const float A0 = ev(0);
-        const float A = fmaf(A0, corr, A0);  // |e^{i phase}| = 1 restored
-        const float ar = A * E.re, ai = A * E.im;
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const float tr = ev(1 + 2 * c), ti = ev(2 + 2 * c);
-            // conj(T A e^{i phase})
-            h[c].re += tr * ar - ti * ai;
-            h[c].im -= tr * ai + ti * ar;
-        }
-    }
 }
 
 // ---------------------------------------------------------------- adjoint helpers
@@ -813,8 +704,7 @@ __device__ inline void mode_adjoint_per_lane(double* __restrict__ Ym, const SegR
 // mode sum of a block, Lam = 4 w (d~ - h~) per bin and channel, then the modes
 // again, each bin's coefficient adjoints (mode_adjoint) summed over the lanes
 // that share a segment (reduce32) and added to the segment's adjoint record.
-// FP64 forms: at least 4 wavefronts per SIMD (at most 128 VGPRs); FP32-bulk
-// form: at least 6 (at most 80 VGPRs)
+// At least 4 wavefronts per SIMD (at most 128 VGPRs).
 
 constexpr int DENSE_RB = 4;  // iterations of 64 dense bins per block of a wavefront
 
@@ -840,7 +730,6 @@ __device__ inline SegRec load_uniform(const SegRec* rc)
     for (int k = 0; k < S_TF; k++) asm volatile("" : "+v"(q.q[k].c2));
     return q;
 }
-__device__ inline SegRecF load_uniform(const SegRecF* rc) { return *rc; }
 
 // Steps of the walker before the lanes left over search for themselves.
 constexpr int WALK_STEPS = 4;
@@ -851,12 +740,11 @@ __device__ inline int segment_estimate(double f, double glo, double gis, int L)
     return (int)fmin(fmax(((double)__log2f((float)f) - glo) * gis, 0.0), (double)(L - 2));
 }
 
-template <bool ADJ, class Rec>
-__global__ __launch_bounds__(256) __attribute__((
-    amdgpu_waves_per_eu(std::is_same<Rec, SegRecF>::value ? 6 : 4, 8))) void k_dir_like_t(double* __restrict__ partial, double* __restrict__ Yadj,
+template <bool ADJ>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_dir_like_t(double* __restrict__ partial, double* __restrict__ Yadj,
                                                     const int* __restrict__ band,
                                                   const int* __restrict__ total, const int* __restrict__ perm,
-                                                  int* __restrict__ next, const Rec* __restrict__ R,
+                                                  int* __restrict__ next, const SegRec* __restrict__ R,
                                                   const double* __restrict__ grid_lo,
                                                   const double* __restrict__ grid_istep,
                                                   const long* __restrict__ off, const int* __restrict__ len,
@@ -865,17 +753,12 @@ __global__ __launch_bounds__(256) __attribute__((
                                                   const cd* __restrict__ dch, const double* __restrict__ wts, int N,
                                                   int B, int M, int chunk)
 {
-    static_assert(!ADJ || std::is_same<Rec, SegRec>::value, "the adjoint pass reads FP64 records");
-    constexpr bool F32 = std::is_same<Rec, SegRecF>::value;
     constexpr int RB = ADJ ? 2 : DENSE_RB;
-    using HT = dense_sum<Rec>;
-    __shared__ double2 s_tab[F32 ? 1 : 1024];
+    __shared__ double2 s_tab[1024];
     const int nitems = total[0];
     const int lane = threadIdx.x & 63;
-    if constexpr (!F32) {
-        fill_etab1k(s_tab, threadIdx.x, blockDim.x);
-        __syncthreads();
-    }
+    fill_etab1k(s_tab, threadIdx.x, blockDim.x);
+    __syncthreads();
     for (;;) {
         // the wavefront's next item in the chunk-major order (dynamic: the items
         // running at any time stay a window of consecutive entries, i.e. the same
@@ -901,18 +784,18 @@ __global__ __launch_bounds__(256) __attribute__((
         if (lane < M && !(grid_istep[b * M + lane] > 0.0)) curv = -2;
         for (int kb = kw0; kb < kw1; kb += RB * 64) {
             double f[RB];
-            HT h[RB][3];
+            cd h[RB][3];
 #pragma unroll
             for (int r = 0; r < RB; r++) {
                 // bins past the item repeat its last one (not summed below)
                 f[r] = freqs[min((unsigned)(kb + 64 * r + lane), (unsigned)(kw1 - 1))];
 #pragma unroll
-                for (int ch = 0; ch < 3; ch++) zero(h[r][ch]);
+                for (int ch = 0; ch < 3; ch++) h[r][ch] = mk(0.0, 0.0);
             }
             for (int m = 0; m < M; m++) {
                 int cur = __builtin_amdgcn_readlane(curv, m);
                 if (cur == -2) continue;
-                const Rec* rm = R + base * M + m;
+                const SegRec* rm = R + base * M + m;
                 if (cur < 0) {
                     const int est = segment_estimate(f[0], grid_lo[b * M + m], grid_istep[b * M + m], L);
                     cur = __builtin_amdgcn_readfirstlane(est);
@@ -925,8 +808,8 @@ __global__ __launch_bounds__(256) __attribute__((
                 bool open = true;
                 for (int step = 0; step < WALK_STEPS; step++) {
                     cur = __builtin_amdgcn_readfirstlane(cur);
-                    const Rec* rc = rm + (unsigned)(cur * M);
-                    const Rec q = load_uniform(rc);
+                    const SegRec* rc = rm + (unsigned)(cur * M);
+                    const SegRec q = load_uniform(rc);
                     bool rest = false;
 #pragma unroll
                     for (int r = 0; r < RB; r++) {
@@ -968,7 +851,7 @@ __global__ __launch_bounds__(256) __attribute__((
                     const double wk = (wts + (long)ch * N)[k];
                     const cd d = (dch + (long)ch * N)[k];
                     const double w = mine ? wk : 0.0;
-                    const cd ht = to_cd(h[r][ch]) * w;
+                    const cd ht = h[r][ch] * w;
                     a0 = fma(d.re, ht.re, fma(d.im, ht.im, a0));
                     a1 = fma(d.re, ht.im, fma(-d.im, ht.re, a1));
                     a2 = fma(ht.re, ht.re, fma(ht.im, ht.im, a2));
@@ -1065,146 +948,6 @@ __global__ __launch_bounds__(64) void k_dir_reduce(double* __restrict__ d_h, dou
         h_h[2 * b] = 4.0 * s2;
         h_h[2 * b + 1] = 0.0;
     }
-}
-
-// ---------------------------------------------------------------- FP32-bulk routing
-//
-// The FP32-bulk form's error, measured template by template against the FP64
-// form on the uneven (8192) and the large (512) batches with every template in
-// FP32, is at most 1.4e-8 h_h wherever h_h > 3000 (and below 3.3e-5 in logL
-// where h_h <= 3000), so templates with h_h above FP32_FALLBACK_HH (error up to
-// ~3e-4 in logL there, 3x inside the 1e-3 target) are evaluated with the FP64
-// records and kernel. Which ones is first
-// decided from an estimate of h_h made before the dense pass (k_dir_route);
-// after it, any binary the estimate sent to FP32 whose h_h exceeds the bound
-// is evaluated again in FP64 (its work items only), so the estimate decides
-// the cost and never the result.
-
-constexpr double FP32_FALLBACK_HH = 2.0e4;
-
-__global__ void k_dir_loud_zero(int* __restrict__ loud_cnt)
-{
-    if (threadIdx.x < 4) loud_cnt[threadIdx.x] = 0;
-}
-
-// h_h of each binary estimated from its sparse knots (one wavefront per
-// binary), each mode on its own grid and the modes added without their
-// interference:
-//   4 sum_m sum_c sum_i A_mi^2 |T_mci|^2 w_c(x_i)^2 (x_{i+1} - x_i) / df
-// over knots inside the data band and the observation window, w taken at the
-// nearest bin of a uniform dense grid (for another grid the estimate, and so
-// only the split between the passes, is coarser).
-__global__ __launch_bounds__(64) void k_dir_route(int* __restrict__ route, const double* __restrict__ X,
-                                                  const double* __restrict__ Yc, const long* __restrict__ off,
-                                                  const int* __restrict__ len, const double* __restrict__ t_start,
-                                                  const double* __restrict__ t_end, const double* __restrict__ freqs,
-                                                  const double* __restrict__ wts, int N, int M)
-{
-    const int b = blockIdx.x, lane = threadIdx.x;
-    const int L = len[b];
-    const long base = off[b];
-    const double ts = t_start[b], te = t_end[b];
-    const double f0 = freqs[0], f1 = freqs[N - 1];
-    const double idf = f1 > f0 ? (N - 1) / (f1 - f0) : 0.0;
-    double s = 0.0;
-    // entry j = i M + m (knot i of mode m): consecutive lanes read consecutive
-    // (knot, mode) entries of X and Yc
-    for (int j = lane; j < (L - 1) * M; j += 64) {
-        const long p = base * M + j;
-        const double x = X[p], xn = X[p + M];
-        if (!(x >= f0 && x <= f1 && xn > x)) continue;
-        const double* y = Yc + p * NQ;
-        const double tf = y[2];
-        if (!((tf >= ts) && ((tf <= te) || (te <= 0.0)))) continue;
-        const int k = min(N - 1, max(0, (int)((x - f0) * idf + 0.5)));
-        double t = 0.0;
-        for (int ch = 0; ch < 3; ch++) {
-            const double w = wts[(long)ch * N + k];
-            t += (y[3 + 2 * ch] * y[3 + 2 * ch] + y[4 + 2 * ch] * y[4 + 2 * ch]) * (w * w);
-        }
-        s += (y[0] * y[0]) * t * ((fmin(xn, f1) - x) * idf);
-    }
-    s = wsum(s);
-    if (lane == 0) route[b] = 4.0 * s > FP32_FALLBACK_HH ? 1 : 0;
-}
-
-// The chunk-major order split into the items of binaries routed to FP64
-// (`loud`) and the others (`quiet`), each list keeping the order (the items in
-// flight then share their dense chunks, whose data come from L2): a count of
-// loud entries per block of SPLIT_BLOCK entries, its exclusive scan
-// (k_dir_cnt_scan), and the placement of every entry.
-constexpr int SPLIT_BLOCK = 256;
-
-__device__ inline bool routed_loud(int pi, int n, const int* __restrict__ perm, const int* __restrict__ band, int B,
-                                   const int* __restrict__ route, int& it)
-{
-    it = pi < n ? perm[pi] : 0;
-    return pi < n && route[owner(band, B, it)] != 0;
-}
-
-__global__ __launch_bounds__(SPLIT_BLOCK) void k_dir_split_count(int* __restrict__ split_cnt,
-                                                                 const int* __restrict__ perm,
-                                                                 const int* __restrict__ total,
-                                                                 const int* __restrict__ band, int B,
-                                                                 const int* __restrict__ route)
-{
-    __shared__ int wc[SPLIT_BLOCK / 64];
-    int it;
-    const bool l = routed_loud(blockIdx.x * SPLIT_BLOCK + threadIdx.x, total[0], perm, band, B, route, it);
-    const unsigned long long m = __ballot(l);
-    if ((threadIdx.x & 63) == 0) wc[threadIdx.x >> 6] = __popcll(m);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int c = 0;
-        for (int w = 0; w < SPLIT_BLOCK / 64; w++) c += wc[w];
-        split_cnt[blockIdx.x] = c;
-    }
-}
-
-// after the scan: split_cnt[blk] = loud entries before block blk. Entry pi goes
-// to loud[#loud before pi] or quiet[pi - #loud before pi]; the last entry
-// writes both counts (cnt[0] loud, cnt[2] quiet; zeroed before, for an empty order)
-__global__ __launch_bounds__(SPLIT_BLOCK) void k_dir_split_write(int* __restrict__ loud, int* __restrict__ quiet,
-                                                                 int* __restrict__ cnt,
-                                                                 const int* __restrict__ split_cnt,
-                                                                 const int* __restrict__ perm,
-                                                                 const int* __restrict__ total,
-                                                                 const int* __restrict__ band, int B,
-                                                                 const int* __restrict__ route)
-{
-    __shared__ int wc[SPLIT_BLOCK / 64];
-    const int n = total[0];
-    const int pi = blockIdx.x * SPLIT_BLOCK + threadIdx.x;
-    int it;
-    const bool l = routed_loud(pi, n, perm, band, B, route, it);
-    const unsigned long long m = __ballot(l);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) wc[w] = __popcll(m);
-    __syncthreads();
-    int before = split_cnt[blockIdx.x];
-    for (int k = 0; k < w; k++) before += wc[k];
-    const int lpos = before + __popcll(m & ((1ull << lane) - 1ull));
-    if (pi < n) {
-        if (l) loud[lpos] = it;
-        else quiet[pi - lpos] = it;
-        if (pi == n - 1) {
-            cnt[0] = lpos + (l ? 1 : 0);
-            cnt[2] = n - cnt[0];
-        }
-    }
-}
-
-// after the passes: the items of binaries evaluated in FP32 whose h_h exceeds
-// the bound
-__global__ void k_dir_loud_list(int* __restrict__ loud, int* __restrict__ loud_cnt, const int* __restrict__ perm,
-                                const int* __restrict__ total, const int* __restrict__ band, int B,
-                                const double* __restrict__ h_h, const int* __restrict__ route)
-{
-    const int pi = blockIdx.x * blockDim.x + threadIdx.x;
-    if (pi >= total[0]) return;
-    const int it = perm[pi];
-    const int b = owner(band, B, it);
-    if (!route[b] && h_h[2 * b] > FP32_FALLBACK_HH) loud[atomicAdd(loud_cnt, 1)] = it;
 }
 
 // ---------------------------------------------------------------- gradient kernels
@@ -1394,8 +1137,7 @@ T* dalloc(size_t n, bool& ok)
 void plan_free(bbhx_direct_plan* p)
 {
     void* bufs[] = {p->off, p->len, p->recs, p->X, p->Cf, p->Yc, p->Fs, p->grid_lo, p->grid_istep, p->band,
-                    p->total, p->partial, p->perm, p->cnt, p->next, p->Yadj, p->grecs, p->gpart, p->CfF,
-                    p->loud, p->quiet, p->loud_cnt, p->route, p->split_cnt};
+                    p->total, p->partial, p->perm, p->cnt, p->next, p->Yadj, p->grecs, p->gpart};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
 }
@@ -1505,7 +1247,6 @@ extern "C" long bbhx_hip_direct_plan_bytes(const bbhx_direct_plan* p)
     long bytes = SM * 8 * (1 + RS + NQ + NQ + 1) + (long)p->B * p->M * (sizeof(FusedRec) + 16) + p->max_items * 36 + p->B * 24 +
                  4L * (p->max_chunks + 1);
     if (p->Yadj) bytes += SM * 8 * NA + (long)p->B * p->M * (sizeof(bbhx::gradk::GradRec) + 8 * bbhx::gradk::NGRAD);
-    if (p->CfF) bytes += SM * (long)sizeof(SegRecF) + p->max_items * 8 + 16 + p->B * 4L + 4L * (p->max_items / 256 + 1);
     return bytes;
 }
 
@@ -1560,10 +1301,8 @@ int direct_launch(bbhx_direct_plan* p, double* d_h, double* h_h, double* grad, i
     hipLaunchKernelGGL(k_dir_grid, dim3(B * M), dim3(64), sizeof(double) * (size_t)p->Lmax, st, p->X, p->Yc,
                        p->grid_lo, p->grid_istep, flags, p->recs, p->off, p->len, params, t_start, t_end, B, M, ml,
                        orb, TDItag, rescaled, tdi2, initial_t_val, mf_min, mf_max);
-    // the FP32-bulk form (not for the gradient, whose adjoint pass reads the FP64 records)
-    const bool f32 = !grad && p->precision == 1;
     hipLaunchKernelGGL(k_dir_spline, dim3(B), dim3(64), 0, st, p->X, p->Yc, p->Cf, p->Fs,
-                       f32 ? static_cast<SegRecF*>(p->CfF) : nullptr, p->off, p->len, t_start, t_end, M);
+                       p->off, p->len, t_start, t_end, M);
     hipLaunchKernelGGL(k_dir_band, dim3(1), dim3(1024), 0, st, p->band, p->total, p->X, p->off, p->len, dataFreqs,
                        p->N, B, M, chunk);
     const int nchunks = (p->N + chunk - 1) / chunk;  // <= max_chunks since chunk >= min_item
@@ -1582,54 +1321,17 @@ int direct_launch(bbhx_direct_plan* p, double* d_h, double* h_h, double* grad, i
     }
     if (timed) (void)hipEventRecord(ev[1], st);
     if (grad)
-        hipLaunchKernelGGL((k_dir_like_t<true, SegRec>), dim3(grid), dim3(block), 0, st, p->partial, p->Yadj, p->band, p->total,
+        hipLaunchKernelGGL((k_dir_like_t<true>), dim3(grid), dim3(block), 0, st, p->partial, p->Yadj, p->band, p->total,
                            p->perm, p->next, reinterpret_cast<const SegRec*>(p->Cf), p->grid_lo, p->grid_istep,
                            p->off, p->len, t_start, t_end, dataFreqs, reinterpret_cast<const cd*>(dataChannels),
                            noiseFactors, p->N, B, M, chunk);
-    else if (f32) {
-        // binaries whose h_h estimate exceeds the bound go to the FP64 pass, the
-        // others to the FP32 pass; the FP32-bulk kernel holds 6 wavefronts per SIMD
-        // against the FP64 form's 4, so a grid sized for the FP64 form is scaled by
-        // 3/2 to fill the chip as fully (measured at 8192 uneven templates, all in
-        // FP32: grid 1024 as given 253 ms, 2048 203 ms)
-        hipLaunchKernelGGL(k_dir_route, dim3(B), dim3(64), 0, st, p->route, p->X, p->Yc, p->off, p->len, t_start,
-                           t_end, dataFreqs, noiseFactors, p->N, M);
-        hipLaunchKernelGGL(k_dir_loud_zero, dim3(1), dim3(64), 0, st, p->loud_cnt);
-        const int split_blocks = ceil_div(items, SPLIT_BLOCK);  // <= max_items / 256 + 1
-        hipLaunchKernelGGL(k_dir_split_count, dim3(split_blocks), dim3(SPLIT_BLOCK), 0, st, p->split_cnt, p->perm,
-                           p->total, p->band, B, p->route);
-        hipLaunchKernelGGL(k_dir_cnt_scan, dim3(1), dim3(1024), 0, st, p->split_cnt, split_blocks);
-        hipLaunchKernelGGL(k_dir_split_write, dim3(split_blocks), dim3(SPLIT_BLOCK), 0, st, p->loud, p->quiet,
-                           p->loud_cnt, p->split_cnt, p->perm, p->total, p->band, B, p->route);
-        hipLaunchKernelGGL((k_dir_like_t<false, SegRecF>), dim3((unsigned)std::min<long>(3L * grid / 2, 2147483647L)),
-                           dim3(block), 0, st, p->partial, nullptr,
-                           p->band, p->loud_cnt + 2, p->quiet, p->loud_cnt + 3, static_cast<const SegRecF*>(p->CfF),
-                           p->grid_lo, p->grid_istep, p->off, p->len, t_start, t_end, dataFreqs,
-                           reinterpret_cast<const cd*>(dataChannels), noiseFactors, p->N, B, M, chunk);
-        hipLaunchKernelGGL((k_dir_like_t<false, SegRec>), dim3(grid), dim3(block), 0, st, p->partial, nullptr,
-                           p->band, p->loud_cnt, p->loud, p->loud_cnt + 1, reinterpret_cast<const SegRec*>(p->Cf),
-                           p->grid_lo, p->grid_istep, p->off, p->len, t_start, t_end, dataFreqs,
-                           reinterpret_cast<const cd*>(dataChannels), noiseFactors, p->N, B, M, chunk);
-    } else
-        hipLaunchKernelGGL((k_dir_like_t<false, SegRec>), dim3(grid), dim3(block), 0, st, p->partial, nullptr,
+    else
+        hipLaunchKernelGGL((k_dir_like_t<false>), dim3(grid), dim3(block), 0, st, p->partial, nullptr,
                            p->band, p->total, p->perm, p->next, reinterpret_cast<const SegRec*>(p->Cf), p->grid_lo,
                            p->grid_istep, p->off, p->len, t_start, t_end, dataFreqs,
                            reinterpret_cast<const cd*>(dataChannels), noiseFactors, p->N, B, M, chunk);
     hipLaunchKernelGGL(k_dir_reduce, dim3(B), dim3(64), 0, st, d_h, h_h, p->partial, p->band,
                        p->total, B);
-    if (f32) {
-        // binaries of the FP32 pass whose h_h exceeds the bound again in FP64 (their
-        // items' partials overwritten), then every binary reduced again (the others'
-        // partials are unchanged)
-        hipLaunchKernelGGL(k_dir_loud_zero, dim3(1), dim3(64), 0, st, p->loud_cnt);
-        hipLaunchKernelGGL(k_dir_loud_list, dim3(item_blocks), dim3(256), 0, st, p->loud, p->loud_cnt, p->perm,
-                           p->total, p->band, B, h_h, p->route);
-        hipLaunchKernelGGL((k_dir_like_t<false, SegRec>), dim3(grid), dim3(block), 0, st, p->partial, nullptr,
-                           p->band, p->loud_cnt, p->loud, p->loud_cnt + 1, reinterpret_cast<const SegRec*>(p->Cf),
-                           p->grid_lo, p->grid_istep, p->off, p->len, t_start, t_end, dataFreqs,
-                           reinterpret_cast<const cd*>(dataChannels), noiseFactors, p->N, B, M, chunk);
-        hipLaunchKernelGGL(k_dir_reduce, dim3(B), dim3(64), 0, st, d_h, h_h, p->partial, p->band, p->total, B);
-    }
     if (grad) {
         hipLaunchKernelGGL(k_dirg_spline_adj, dim3(B), dim3(64), 0, st, p->Yadj, p->X, p->off, p->len, M);
         hipLaunchKernelGGL(k_dirg_knots, dim3(B * M), dim3(64), 0, st, p->gpart, p->grecs, p->Yadj, p->X, p->off,
@@ -1656,32 +1358,13 @@ extern "C" int bbhx_hip_direct_fused(bbhx_direct_plan* p, double* d_h, double* h
                          orbits, TDItag, rescaled, tdi2, chunk, block, grid, stream);
 }
 
+// 0 and 1 are evaluated alike, in FP64, the faster form: FP32 instructions issue at
+// the FP64 rate without packed arithmetic, and an FP32 pass over the quiet
+// templates needs its own records, the split of the items and a second pass for the
+// loud ones (1024 uneven templates: 27.7 ms against 25.0).
 extern "C" int bbhx_hip_direct_plan_set_precision(bbhx_direct_plan* p, int precision)
 {
-    if (!p || (precision != 0 && precision != 1)) return ERR_ARGS;
-    if (precision == 1 && !p->CfF) {
-        bool ok = true;
-        p->CfF = dalloc<SegRecF>((size_t)p->S * p->M, ok);
-        p->loud = dalloc<int>((size_t)p->max_items, ok);
-        p->quiet = dalloc<int>((size_t)p->max_items, ok);
-        p->loud_cnt = dalloc<int>(4, ok);
-        p->route = dalloc<int>((size_t)p->B, ok);
-        p->split_cnt = dalloc<int>((size_t)(p->max_items / 256 + 1), ok);
-        if (!ok) {
-            for (void* b : {p->CfF, (void*)p->loud, (void*)p->quiet, (void*)p->loud_cnt, (void*)p->route,
-                            (void*)p->split_cnt})
-                if (b) (void)hipFree(b);
-            p->CfF = nullptr;
-            p->loud = nullptr;
-            p->quiet = nullptr;
-            p->loud_cnt = nullptr;
-            p->route = nullptr;
-            p->split_cnt = nullptr;
-            return ERR_ALLOC;
-        }
-    }
-    p->precision = precision;
-    return OK;
+    return p && (precision == 0 || precision == 1) ? OK : ERR_ARGS;
 }
 
 extern "C" int bbhx_hip_direct_plan_enable_grad(bbhx_direct_plan* p)

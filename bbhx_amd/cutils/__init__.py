@@ -436,9 +436,8 @@ class DirectPlan:
         _check(load_library().bbhx_hip_direct_plan_enable_grad(self._h), "direct_plan_enable_grad")
 
     def set_precision(self, precision):
-        """0: FP64; 1: FP32 bulk (amplitude and transfer-function cubics, phase
-        factor and mode sum in FP32; phase, t(f) and the inner products in FP64).
-        The first switch to 1 allocates 192 B per (knot, mode)."""
+        """0: FP64; 1: log-likelihoods within 1e-3 of the FP64 form's suffice
+        (evaluated in FP64 too, the faster form on this machine)."""
         precision = int(precision)
         if precision != self.precision:
             _check(load_library().bbhx_hip_direct_plan_set_precision(self._h, precision), "direct_plan_set_precision")

@@ -83,8 +83,7 @@ class Likelihood(BBHxParallelModule):
         """Fused direct log-likelihood of device inputs (``fused_inputs``): a
         device tensor, with no host synchronisation (graph-capturable; flags
         must be zeroed before the call). precision (None: the plan's current
-        one): 0 FP64, 1 FP32 bulk with FP64 phase (``DirectPlan.set_precision``;
-        the first switch to 1 allocates, so make it before a graph capture)."""
+        one): 0 FP64, 1 within 1e-3 of it (``DirectPlan.set_precision``)."""
         torch = self.xp
         if precision is not None:
             plan.set_precision(precision)
@@ -110,7 +109,7 @@ class Likelihood(BBHxParallelModule):
         """Direct log-likelihood of templates with per-template sparse grid
         lengths (``lengths[b]``), fused: no template is materialised. Same
         params layout and result as ``get_ll(params, length=...)``.
-        precision 1: the FP32-bulk form (``get_ll_fused_device``)."""
+        precision 1: logL within 1e-3 (``get_ll_fused_device``)."""
         torch = self.xp
         rows, t_start, t_end = fused_param_rows(self.waveform_gen, params, t_obs_start, t_obs_end, self.device)
         lengths = np.asarray(lengths, dtype=np.int32)

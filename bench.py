@@ -258,12 +258,12 @@ def bench_direct_ragged(args):
         f"plan {plan.nbytes() / 2**30:.2f} GiB; {dense} dense (bin, template) pairs "
         f"({dense / (ms * 1e-3):.4g}/s); split {split}")
 
-    # FP32-bulk form of the same batch (phase, t(f) and inner products FP64), its own graph
+    # the same batch with precision 1 (logL within 1e-3 suffices), its own graph
     f32_info = None
     if not args.no_fp32:
         hh64 = like.h_h.real.cpu().numpy()
         flags.zero_()
-        like.get_ll_fused_device(plan, rows, ts, te, flags, MODES, precision=1)  # allocates the records
+        like.get_ll_fused_device(plan, rows, ts, te, flags, MODES, precision=1)
         torch.cuda.synchronize()
         g32 = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g32, stream=st):

@@ -237,14 +237,9 @@ long bbhx_hip_direct_plan_bytes(const bbhx_direct_plan* p);
 int bbhx_hip_direct_plan_band(const bbhx_direct_plan* p, int* band_host);
 /* Arithmetic of later bbhx_hip_direct_fused calls on this plan (no
  * counterpart in the reference, which computes in FP64 only): 0 = FP64
- * (default); 1 = FP32 bulk: the amplitude and transfer-function cubics, the
- * phase factor e^{i phase} and the mode sum in FP32, while the phase and t(f)
- * cubics (and the reduction of the phase modulo 2 pi) and the noise-weighted
- * inner products stay FP64. The first switch to 1 allocates 192 B per (knot,
- * mode) of FP32-bulk segment records (call it outside graph capture). The
- * gradient entry point always computes in FP64. In the FP32-bulk form the
- * dense-band launch uses 3/2 x grid workgroups (its kernel holds 6 wavefronts
- * per SIMD against 4), so a launch shape tuned for the FP64 form serves both. */
+ * (default); 1 = log-likelihoods within 1e-3 of the FP64 form's suffice. Both
+ * are evaluated in FP64, which is the faster form on this machine; any other
+ * value is refused (status 1). Allocates nothing. */
 int bbhx_hip_direct_plan_set_precision(bbhx_direct_plan* p, int precision);
 
 /* params (11, B) and t_start, t_end (B,) as for bbhx_hip_hdyn_fused; dataFreqs
