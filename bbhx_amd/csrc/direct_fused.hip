@@ -16,10 +16,10 @@
 //                 (phenomhm.py:208-224, :509-614), then amplitude, phase, t(f)
 //                 and the TDI response on the refitted grid (phenomhm.py:487-507,
 //                 Response.cu), written compact: nine values per (knot, mode)
-//   k_dir_spline  one wavefront per binary, one lane per (mode, quantity):
-//                 not-a-knot spline coefficients (Interpolate.cu:15-359) from
-//                 the compact values (forward sweep into the scratch Fs, then
-//                 each record's (y, c1, c2, c3) written together, once)
+//   k_dir_spline  one workgroup per block of a (binary, mode)'s knots, one lane
+//                 per knot: not-a-knot spline coefficients (Interpolate.cu:15-359)
+//                 of the nine quantities by parallel cyclic reduction, from the
+//                 compact values; each record written once
 //   k_dir_band    dense band [st, et) of each binary (waveformbuild.py:139-156)
 //                 and the exclusive prefix of its chunks of dense bins (chunks
 //                 aligned to absolute multiples of the chunk size)
@@ -61,7 +61,6 @@ struct bbhx_direct_plan {
     double* X = nullptr;   // (S, M)
     double* Cf = nullptr;  // (S, M, RS): segment records (bounds, value and cubic coefficients)
     double* Yc = nullptr;  // (S, M, NQ): the grid pass's nine values per knot, compact
-    double* Fs = nullptr;  // (S, M, NQ + 1): the spline's forward sweep, d' of each quantity, then c'
     double* grid_lo = nullptr;    // (B, M) log2 of the first refitted grid point
     double* grid_istep = nullptr; // (B, M) 1 / log2 step (0 for a degenerate grid)
     int* band = nullptr;          // (B, 3): st, et, chunk_begin
@@ -275,128 +274,192 @@ __device__ inline int segment_window(const Cubic& c, double h, double ts, double
     return WIN_MIXED;
 }
 
-constexpr int DSPL_BLOCK = 8;  // rows loaded ahead of the recurrence in each sweep of k_dir_spline
+// ---------------------------------------------------------------- tridiagonal solves
+//
+// The spline's systems (and their transposes) are solved by parallel cyclic
+// reduction, one knot per lane and all quantities of a (binary, mode) together:
+// with every row scaled to a unit diagonal, a step at distance d replaces the
+// couplings to rows i -+ d by ones to rows i -+ 2d. The rows are diagonally
+// dominant by two or more (the couplings' magnitudes add up to at most half of the
+// diagonal), so the couplings fall from 1/2 to at most 1/4, 1/16, 1/256, 2^-16,
+// 2^-32 and 2^-64 in six steps, after which each row is its solution. What lies
+// farther than that does not count either, so a grid longer than a workgroup is cut
+// into blocks that overlap by SPL_W rows on each side: a solution forgets by a
+// factor of about 0.27 per row (0.5 at worst) what a block's end leaves out, and
+// on a log-spaced grid over 4 decades the end's slopes, steeper by at most
+// r^(11/3) per row (r = the knots' ratio), weigh (0.28 r^(11/3))^48 < 1e-16 there.
+//
+// Bound by the steps' exchange through LDS for few templates (16 of 1024 knots: 25
+// us), by the records' writes (320 B per (knot, mode)) for many (1024 uneven ones,
+// 9.4 M records: 1.7 ms; 64 of 4096 knots: 0.2 ms). Thomas sweeps, one lane per (mode,
+// quantity), are one chain over all knots: 537 us, 3.1 ms and 2.24 ms.
+constexpr int SPL_W = 48;
+constexpr int SPL_STEPS = 6;
 
-// Not-a-knot spline of one binary: lane s = mode * 9 + quantity runs the
-// Thomas algorithm over the binary's L knots (the system of spline.hip);
-// consecutive lanes read consecutive quantities of the same knot.
-__global__ __launch_bounds__(64) void k_dir_spline(const double* __restrict__ X, const double* __restrict__ Yc,
-                                                   double* __restrict__ Cf, double* __restrict__ Fs,
-                                                   const long* __restrict__ off,
-                                                   const int* __restrict__ len, const double* __restrict__ t_start,
-                                                   const double* __restrict__ t_end, int M)
+// Rows per block = lanes of a workgroup (384 and 512 overlap less and measured the
+// same at 1024 uneven templates, slower for few).
+constexpr int SPL_T = 256;
+constexpr int SPL_U = SPL_T - 2 * SPL_W;  // rows between the starts of two blocks
+__host__ __device__ inline int spline_blocks(int n) { return n <= SPL_T ? 1 : 1 + (n - SPL_T + SPL_U - 1) / SPL_U; }
+
+// Solves x_i + a x_{i-1} + c x_{i+1} = r_i for NR right sides over the rows of a
+// workgroup (row t = threadIdx.x; rows outside it are left out); sh: (NR + 2)
+// SPL_T doubles of LDS, free on entry and on exit.
+template <int NR>
+__device__ inline void pcr_solve(double a, double c, double (&r)[NR], double* sh, int t)
 {
-    const int b = blockIdx.x;
-    const int s = threadIdx.x;
-    if (s >= M * NQ) return;
-    const double ts = t_start[b], te = t_end[b];
-    const int m = s / NQ;
-    const int n = len[b];
-    const long base = off[b];
-    // element i of this system
-    auto xi = [&](int i) { return X[(base + i) * M + m]; };
-    const int q = s - m * NQ;
-    auto at = [&](int i) { return ((base + i) * M + m) * RS + RQ + seg_slot(q) * 4; };
-    // the record's head (bounds and window), written by the lane of t_f
-    auto put_head = [&](int i, double x_lo, double x_hi, int win) {
-        SegRec* r = reinterpret_cast<SegRec*>(Cf) + ((base + i) * M + m);
-        r->x_lo = x_lo;
-        r->x_hi = x_hi;
-        r->win = win;
-        r->pad0 = 0;
-        r->pad1 = 0.0;
-    };
-    auto yi = [&](int i) { return Yc[((base + i) * M + m) * NQ + q]; };
-    // the forward sweep's d' of this quantity and the mode's c' (the same for
-    // its nine quantities: it depends on the knots alone), NQ + 1 per (knot, mode)
-    auto fs = [&](int i) { return ((base + i) * M + m) * (NQ + 1); };
-    // The forward sweep writes only d' and c' (80 B per (knot, mode), the
-    // wavefront's lanes consecutive) to the scratch Fs; the backward sweep
-    // writes every record once, in whole 32-B groups.
-    auto put_fwd = [&](int i, double d, double c) {
-        Fs[fs(i) + q] = d;
-        if (q == 0) Fs[fs(i) + NQ] = c;
-    };
-    double x0 = xi(0), x1 = xi(1), x2 = xi(2);
-    double y0 = yi(0), y1 = yi(1), y2 = yi(2);
-    double cprev, dprev;
-    {
-        double dx1 = x1 - x0, dx2 = x2 - x1, dd = x2 - x0;
-        double s1 = (y1 - y0) / dx1, s2 = (y2 - y1) / dx2;
-        double bb = ((dx1 + 2 * dd) * dx2 * s1 + dx1 * dx1 * s2) / dd;
-        cprev = dd / dx2;
-        dprev = bb / dx2;
-        put_fwd(0, dprev, cprev);
-    }
-    // each sweep loads DSPL_BLOCK rows ahead of its recurrence (one memory
-    // latency per block) and divides once per row
-    double xa = x0, xb = x1, ya = y0, yb = y1;
-    for (int i0 = 1; i0 < n - 1; i0 += DSPL_BLOCK) {
-        double xv[DSPL_BLOCK], yv[DSPL_BLOCK];
+    constexpr int T = SPL_T;
+    for (int k = 0, d = 1; k < SPL_STEPS; k++, d *= 2) {
+        sh[t] = a;
+        sh[T + t] = c;
 #pragma unroll
-        for (int u = 0; u < DSPL_BLOCK; u++) {
-            const int i = i0 + u;
-            xv[u] = i < n - 1 ? xi(i + 1) : 0.0;
-            yv[u] = i < n - 1 ? yi(i + 1) : 0.0;
+        for (int q = 0; q < NR; q++) sh[(2 + q) * T + t] = r[q];
+        __syncthreads();
+        const bool lo = t >= d, hi = t + d < T;
+        const int tl = lo ? t - d : t, th = hi ? t + d : t;
+        // couplings to rows outside the block are dropped
+        const double fl = lo ? a : 0.0, fh = hi ? c : 0.0;
+        const double ib = rcp_pos(1.0 - fl * sh[T + tl] - fh * sh[th]);
+        a = -(fl * sh[tl]) * ib;
+        c = -(fh * sh[T + th]) * ib;
+#pragma unroll
+        for (int q = 0; q < NR; q++) r[q] = (r[q] - fl * sh[(2 + q) * T + tl] - fh * sh[(2 + q) * T + th]) * ib;
+        __syncthreads();
+    }
+}
+
+// The rows of one workgroup of a spline kernel: block 'blk' of (binary b, mode m).
+struct SplineRows {
+    int b, m, n, first, row0, row1;  // loaded rows [first, first + T), results for [row0, row1)
+    bool any;
+};
+__device__ inline SplineRows spline_rows(const int* __restrict__ len, int M, int nbmax)
+{
+    constexpr int T = SPL_T;
+    SplineRows w;
+    const int blk = blockIdx.x % nbmax, bm = blockIdx.x / nbmax;
+    w.b = bm / M;
+    w.m = bm % M;
+    w.n = len[w.b];
+    const int nb = spline_blocks(w.n);
+    w.any = blk < nb;
+    w.first = blk * SPL_U;
+    w.row0 = blk == 0 ? 0 : w.first + SPL_W;
+    w.row1 = blk == nb - 1 ? w.n : w.first + T - SPL_W;
+    return w;
+}
+
+// Not-a-knot splines of the nine quantities of one (binary, mode) (the system of
+// spline.hip), one lane per knot. The two end rows are folded into their
+// neighbours, which leaves every row dominant: s_0 = (b_0 - (h_0 + h_1) s_1) / h_1.
+__global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void k_dir_spline(const double* __restrict__ X, const double* __restrict__ Yc,
+                                                    SegRec* __restrict__ Cf, const long* __restrict__ off,
+                                                    const int* __restrict__ len, const double* __restrict__ t_start,
+                                                    const double* __restrict__ t_end, int M, int nbmax)
+{
+    constexpr int T = SPL_T;
+    __shared__ __align__(16) double sh[(NQ + 2) * T];
+    __shared__ double ends[2][NQ];  // right sides of the two end rows
+    const int t = threadIdx.x;
+    const SplineRows w = spline_rows(len, M, nbmax);
+    if (!w.any) return;
+    const int i = w.first + t, n = w.n;
+    const long base = off[w.b];
+    const bool row = i < n;
+    const long p = (base + (row ? i : n - 1)) * M + w.m;
+    const double x = X[p];
+    double y[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) y[q] = Yc[p * NQ + q];
+    sh[t] = x;
+#pragma unroll
+    for (int q = 0; q < NQ; q++) sh[(1 + q) * T + t] = y[q];
+    __syncthreads();
+    const int tl = t > 0 ? t - 1 : 0, th = t + 1 < T ? t + 1 : t;
+    const double hl = x - sh[tl], xr = sh[th], hr = xr - x;
+    const double il = rcp_pos(hl), ir = rcp_pos(hr);
+    // rows to solve: the interior ones with both neighbours in the block
+    const bool solve = i > 0 && i < n - 1 && t > 0 && t + 1 < T;
+    const bool low = solve && i == 1, high = solve && i == n - 2;
+    const double d = hl + hr;
+    double a = low ? 0.0 : hr, c = high ? 0.0 : hl;
+    double diag = 2.0 * d;
+    if (low) diag -= d;
+    if (high) diag -= d;
+    const double id = rcp_pos(d), ib = rcp_pos(diag);
+    a = solve ? a * ib : 0.0;
+    c = solve ? c * ib : 0.0;
+    double mr[NQ], r[NQ];
+    // right sides of the end rows, as multiples of the slopes on either side
+    const double e0l = (hl + 2.0 * d) * hr * id, e0r = hl * hl * id;
+    const double e1l = hr * hr * id, e1r = (2.0 * d + hr) * hl * id;
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+        const double ml = (y[q] - sh[(1 + q) * T + tl]) * il;
+        mr[q] = (sh[(1 + q) * T + th] - y[q]) * ir;
+        double v = 3.0 * (hr * ml + hl * mr[q]);
+        if (low) {
+            ends[0][q] = e0l * ml + e0r * mr[q];
+            v -= ends[0][q];
         }
-#pragma unroll
-        for (int u = 0; u < DSPL_BLOCK; u++) {
-            const int i = i0 + u;
-            if (i >= n - 1) break;
-            const double xc = xv[u], yc = yv[u];
-            const double ex1 = xb - xa, ex2 = xc - xb;
-            const double t1 = (yb - ya) / ex1, t2 = (yc - yb) / ex2;
-            const double rhs = 3.0 * (ex2 * t1 + ex1 * t2);
-            const double diag = 2 * (ex1 + ex2), lo = ex2, up = ex1;
-            const double im = 1.0 / (diag - lo * cprev);
-            cprev = up * im;
-            dprev = (rhs - lo * dprev) * im;
-            put_fwd(i, dprev, cprev);
-            xa = xb;
-            xb = xc;
-            ya = yb;
-            yb = yc;
+        if (high) {
+            ends[1][q] = e1l * ml + e1r * mr[q];
+            v -= ends[1][q];
         }
+        r[q] = solve ? v * ib : 0.0;
     }
-    double snext;  // the last row's slope, the start of the backward sweep
-    {
-        const double xm3 = xi(n - 3), xm2 = xi(n - 2), xm1 = xi(n - 1);
-        const double ym3 = yi(n - 3), ym2 = yi(n - 2), ym1 = yi(n - 1);
-        const double ex1 = xm2 - xm3, ex2 = xm1 - xm2, ed = xm1 - xm3;
-        const double t1 = (ym2 - ym3) / ex1, t2 = (ym1 - ym2) / ex2;
-        const double rhs = ((ex2 * ex2 * t1 + (2 * ed + ex2) * ex1 * t2) / ed);
-        const double mm = ex1 - ed * cprev;
-        snext = (rhs - ed * dprev) / mm;
+    __syncthreads();
+    pcr_solve(a, c, r, sh, t);
+    // slopes to the neighbours, the end ones from their rows
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+        if (i != 0 && i < n - 1) sh[q * T + t] = r[q];
+        if (low) sh[q * T + t - 1] = (ends[0][q] - d * r[q]) * ir;
+        if (high) sh[q * T + t + 1] = (ends[1][q] - d * r[q]) * il;
     }
-    double xn = xi(n - 1), yn = yi(n - 1);
-    *reinterpret_cast<Cubic*>(Cf + at(n - 1)) = Cubic{yn, 0.0, 0.0, 0.0};
-    if (q == 2) put_head(n - 1, xn, xn, WIN_MIXED);
-    for (int i0 = n - 2; i0 >= 0; i0 -= DSPL_BLOCK) {
-      double dv[DSPL_BLOCK], cv[DSPL_BLOCK], xv[DSPL_BLOCK], yv[DSPL_BLOCK];
+    __syncthreads();
+    const bool end = i == n - 1;
+    int win = WIN_MIXED;
+    Cubic k[NQ];
 #pragma unroll
-      for (int u = 0; u < DSPL_BLOCK; u++) {
-          const int i = i0 - u;
-          dv[u] = i >= 0 ? Fs[fs(i) + q] : 0.0;
-          cv[u] = i >= 0 ? Fs[fs(i) + NQ] : 0.0;
-          xv[u] = i >= 0 ? xi(i) : 0.0;
-          yv[u] = i >= 0 ? yi(i) : 0.0;
-      }
+    for (int q = 0; q < NQ; q++) {
+        const double s = sh[q * T + t], sn = sh[q * T + th];
+        const double u = (s + sn - 2.0 * mr[q]) * ir;
+        k[q] = end ? Cubic{y[q], 0.0, 0.0, 0.0} : Cubic{y[q], s, (mr[q] - s) * ir - u, u * ir};
+        if (q == 2 && !end) win = segment_window(k[q], hr, t_start[w.b], t_end[w.b]);
+    }
+    __syncthreads();
+    // The records leave through LDS, 16 of a wavefront's at a time, so that a
+    // store covers whole records (written by their own lanes, 16 B to a line each,
+    // the kernel waits on the number of requests: 2.1 against 1.7 ms at 1024)
+    constexpr int PER = 16, PITCH = RS + 2;  // doubles, padded against bank conflicts
+    static_assert(4 * PER * PITCH <= (NQ + 2) * T, "the records of a workgroup's wavefronts fit in sh");
+    const int lane = t & 63, i0 = w.first + (t & ~63);
+    double* own = sh + (t >> 6) * PER * PITCH;
+    for (int g = 0; g < 64; g += PER) {
+        if (lane >= g && lane < g + PER) {
+            double* o = own + (lane - g) * PITCH;
+            o[0] = x;
+            o[1] = end ? x : xr;
+            o[2] = __hiloint2double(0, win);
+            o[3] = 0.0;
 #pragma unroll
-      for (int u = 0; u < DSPL_BLOCK; u++) {
-        const int i = i0 - u;
-        if (i < 0) break;
-        const double si = dv[u] - cv[u] * snext;
-        const double x_i = xv[u], y_i = yv[u];
-        const double idx = 1.0 / (xn - x_i);
-        const double slope = (yn - y_i) * idx;
-        const double t = (si + snext - 2 * slope) * idx;
-        const double c2 = (slope - si) * idx - t, c3 = t * idx;
-        *reinterpret_cast<Cubic*>(Cf + at(i)) = Cubic{y_i, si, c2, c3};
-        if (q == 2) put_head(i, x_i, xn, segment_window(Cubic{y_i, si, c2, c3}, xn - x_i, ts, te));
-        snext = si;
-        xn = x_i;
-        yn = y_i;
-      }
+            for (int q = 0; q < NQ; q++) {
+                double* v = o + RQ + 4 * seg_slot(q);
+                v[0] = k[q].y;
+                v[1] = k[q].c1;
+                v[2] = k[q].c2;
+                v[3] = k[q].c3;
+            }
+        }
+        __syncthreads();
+        for (int e = lane; e < PER * RS / 2; e += 64) {
+            const int j = e / (RS / 2), c = e - j * (RS / 2);
+            const int ij = i0 + g + j;
+            if (ij >= w.row0 && ij < w.row1)
+                reinterpret_cast<double2*>(Cf + (base + ij) * M + w.m)[c] = *reinterpret_cast<const double2*>(own + j * PITCH + 2 * c);
+        }
+        __syncthreads();
     }
 }
 
@@ -1136,7 +1199,7 @@ T* dalloc(size_t n, bool& ok)
 
 void plan_free(bbhx_direct_plan* p)
 {
-    void* bufs[] = {p->off, p->len, p->recs, p->X, p->Cf, p->Yc, p->Fs, p->grid_lo, p->grid_istep, p->band,
+    void* bufs[] = {p->off, p->len, p->recs, p->X, p->Cf, p->Yc, p->grid_lo, p->grid_istep, p->band,
                     p->total, p->partial, p->perm, p->cnt, p->next, p->Yadj, p->grecs, p->gpart};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
@@ -1206,7 +1269,6 @@ extern "C" int bbhx_hip_direct_plan_create(bbhx_direct_plan** out, int numBinAll
     p->X = dalloc<double>(SM, ok);
     p->Cf = dalloc<double>(SM * RS, ok);
     p->Yc = dalloc<double>(SM * NQ, ok);
-    p->Fs = dalloc<double>(SM * (NQ + 1), ok);
     p->grid_lo = dalloc<double>((size_t)numBinAll * numModes, ok);
     p->grid_istep = dalloc<double>((size_t)numBinAll * numModes, ok);
     p->band = dalloc<int>((size_t)numBinAll * 3, ok);
@@ -1244,7 +1306,7 @@ extern "C" long bbhx_hip_direct_plan_bytes(const bbhx_direct_plan* p)
 {
     if (!p) return -1;
     const long SM = p->S * p->M;
-    long bytes = SM * 8 * (1 + RS + NQ + NQ + 1) + (long)p->B * p->M * (sizeof(FusedRec) + 16) + p->max_items * 36 + p->B * 24 +
+    long bytes = SM * 8 * (1 + RS + NQ) + (long)p->B * p->M * (sizeof(FusedRec) + 16) + p->max_items * 36 + p->B * 24 +
                  4L * (p->max_chunks + 1);
     if (p->Yadj) bytes += SM * 8 * NA + (long)p->B * p->M * (sizeof(bbhx::gradk::GradRec) + 8 * bbhx::gradk::NGRAD);
     return bytes;
@@ -1301,8 +1363,8 @@ int direct_launch(bbhx_direct_plan* p, double* d_h, double* h_h, double* grad, i
     hipLaunchKernelGGL(k_dir_grid, dim3(B * M), dim3(64), sizeof(double) * (size_t)p->Lmax, st, p->X, p->Yc,
                        p->grid_lo, p->grid_istep, flags, p->recs, p->off, p->len, params, t_start, t_end, B, M, ml,
                        orb, TDItag, rescaled, tdi2, initial_t_val, mf_min, mf_max);
-    hipLaunchKernelGGL(k_dir_spline, dim3(B), dim3(64), 0, st, p->X, p->Yc, p->Cf, p->Fs,
-                       p->off, p->len, t_start, t_end, M);
+    const int nbmax = spline_blocks(p->Lmax);
+    hipLaunchKernelGGL(k_dir_spline, dim3((unsigned)((long)B * M * nbmax)), dim3(SPL_T), 0, st, p->X, p->Yc, reinterpret_cast<SegRec*>(p->Cf), p->off, p->len, t_start, t_end, M, nbmax);
     hipLaunchKernelGGL(k_dir_band, dim3(1), dim3(1024), 0, st, p->band, p->total, p->X, p->off, p->len, dataFreqs,
                        p->N, B, M, chunk);
     const int nchunks = (p->N + chunk - 1) / chunk;  // <= max_chunks since chunk >= min_item

@@ -1,5 +1,5 @@
-"""The dense pass of the fused direct likelihood at the sizes where its blocks,
-work items and segment search have edges, against the FP64 CPU oracle run
+"""The dense pass and the splines of the fused direct likelihood at the sizes where
+their blocks, work items and segment search have edges, against the FP64 CPU oracle run
 template by template.
 
 Tolerance: |delta logL| <= 1e-6 + 1e-8 (|d_h| + h_h). Both sides are FP64; the
@@ -24,6 +24,9 @@ CASES = {
     # segments of thousands of bins, and several segments to a bin
     "short_grids": (20001, "uniform", [4, 5, 7, 33], (16384, 1024, 256), (0.0, 1.0), MODES),
     "long_grids": (3001, "uniform", [4096, 3000], (4096, 1024, 256), (0.0, 1.0), MODES),
+    # the spline's row blocks of 256 knots, one more every 160
+    "spline_blocks": (2001, "uniform", [6, 255, 256, 257, 258, 415, 416, 417, 576, 577], (16384, 1024, 256), (0.0, 1.0),
+                      MODES),
     # items that are not a multiple of a block, the last one short
     "odd_chunk": (9001, "uniform", [500, 256], (1000, 1000, 256), (0.0, 1.0), MODES),
     # uneven data frequencies; blocks that start below the grid and end above it
