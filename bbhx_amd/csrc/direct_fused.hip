@@ -656,25 +656,23 @@ constexpr int NA = NQ * 4;  // 36 doubles
 // (t_f carries none: the observation window is held fixed)
 __device__ inline int adj_q(int j) { return j < 2 ? j : j + 1; }
 
-// d logL with respect to the 32 segment coefficients (A, phase, T1..T3 re/im;
-// y, c1, c2, c3 each) of one mode at one dense bin, given
-// Lam_c = 4 w_c (d~_c - h~_c) (d logL = Re sum_c conj(Lam_c) dh_c with
-// h_c = sum_m conj(T_c A e^{i phase}); Likelihood.cu:357-375 differentiated).
-__device__ inline bool mode_adjoint(double cb[32], const SegRec& q, double x, double ts, double te, const cd Lam[3],
-                                    const double2* tab)
+// Adjoints of the eight interpolated quantities of one mode at one dense bin (A,
+// phase, T1..T3 re/im), given Lam_c = 4 w_c (d~_c - h~_c) (d logL =
+// Re sum_c conj(Lam_c) dh_c with h_c = sum_m conj(T_c A e^{i phase});
+// Likelihood.cu:357-375 differentiated). The adjoint of coefficient p of a
+// quantity's cubic is its adjoint times x^p.
+__device__ inline void mode_adjoint(double (&a)[8], const Cubic* q, double x, const cd Lam[3], const double2* tab)
 {
-    if (q.win == WIN_NONE || (q.win == WIN_MIXED && !bin_in_window(q.q[S_TF], x, ts, te))) return false;
-    const double x2 = x * x, x3 = x * x2;
-    auto ev = [&](int k) { return fma(fma(fma(q.q[k].c3, x, q.q[k].c2), x, q.q[k].c1), x, q.q[k].y); };
+    auto ev = [&](int k) { return fma(fma(fma(q[k].c3, x, q[k].c2), x, q[k].c1), x, q[k].y); };
     const double A = ev(S_A);
     const cd E = cexpi_tab1k(ev(S_PH), tab);
     const cd AE = A * E;
-    double a[8];
     cd P = mk(0.0, 0.0);
 #pragma unroll
     for (int c = 0; c < 3; c++) {
         const cd T = mk(ev(S_T + 2 * c), ev(S_T + 2 * c + 1));
-        P += Lam[c] * T;
+        P.re = fma(Lam[c].re, T.re, fma(-Lam[c].im, T.im, P.re));
+        P.im = fma(Lam[c].re, T.im, fma(Lam[c].im, T.re, P.im));
         const cd LAE = Lam[c] * AE;
         a[2 + 2 * c] = LAE.re;
         a[3 + 2 * c] = -LAE.im;
@@ -682,41 +680,54 @@ __device__ inline bool mode_adjoint(double cb[32], const SegRec& q, double x, do
     const cd PE = P * E;
     a[0] = PE.re;
     a[1] = -A * PE.im;
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        cb[4 * j] = a[j];
-        cb[4 * j + 1] = a[j] * x;
-        cb[4 * j + 2] = a[j] * x2;
-        cb[4 * j + 3] = a[j] * x3;
-    }
-    return true;
 }
 
-// One step of reduce32: lanes whose bit BIT is set keep the upper H values,
-// the others the lower H, and each adds what its partner (lane ^ BIT) sends.
-template <int H, int BIT>
-__device__ inline void halve(double v[32], int lane)
+// v of the lane whose index differs in the bits of a quad permutation
+template <int CTRL>
+__device__ inline double quad_swap(double v)
 {
-    const bool up = (lane & BIT) != 0;
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+// 4 x 4 transpose within each quad of lanes: v[s] of lane i <- v[i] of lane s
+__device__ inline void quad_transpose(double (&v)[4], int lane)
+{
+    const bool odd = (lane & 1) != 0, up = (lane & 2) != 0;
 #pragma unroll
-    for (int j = 0; j < H; j++) {
-        const double send = up ? v[j] : v[j + H];
-        const double keep = up ? v[j + H] : v[j];
-        v[j] = keep + __shfl_xor(send, BIT, 64);
+    for (int k = 0; k < 4; k += 2) {
+        const double t0 = quad_swap<0xB1>(v[k]), t1 = quad_swap<0xB1>(v[k + 1]);  // lanes 1 0 3 2
+        v[k] = odd ? t1 : v[k];
+        v[k + 1] = odd ? v[k + 1] : t0;
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const double t0 = quad_swap<0x4E>(v[k]), t2 = quad_swap<0x4E>(v[k + 2]);  // lanes 2 3 0 1
+        v[k] = up ? t2 : v[k];
+        v[k + 2] = up ? v[k + 2] : t0;
     }
 }
 
-// Sum of v[0..32) over the 64 lanes of a wavefront by recursive halving (each
-// step exchanges half of the remaining values with the partner lane): lane l
-// returns the total of value l >> 1 (31 exchanges instead of 32 x 6).
-__device__ inline double reduce32(double v[32], int lane)
+// Sums over the bins of a wavefront of (quantity adjoint) x (power of x): an
+// (8 x bins) (bins x 4) product on the matrix cores, four blocks of 4 x 4 x 4
+// (v_mfma_f64_4x4x4: lane i + 4 b + 16 k gives A[i][k] and B[k][i] of block b and
+// holds D[k][i]). The quad of lanes 4 Q + s gives, in step s, the four quantities
+// and the four powers of one bin, that of lane 4 Q + s: a transpose within quads,
+// no exchange through LDS. acc[g] of lane j + 4 b + 16 i: quantity i + 4 g, power
+// j, the bins of block b.
+__device__ inline void adjoint_accumulate(double (&acc)[2], const double (&a)[8], double x, int lane)
 {
-    halve<16, 32>(v, lane);
-    halve<8, 16>(v, lane);
-    halve<4, 8>(v, lane);
-    halve<2, 4>(v, lane);
-    halve<1, 2>(v, lane);
-    return v[0] + __shfl_xor(v[0], 1, 64);
+    double v0[4] = {a[0], a[1], a[2], a[3]}, v1[4] = {a[4], a[5], a[6], a[7]};
+    double w[4] = {1.0, x, x * x, x * (x * x)};
+    quad_transpose(v0, lane);
+    quad_transpose(v1, lane);
+    quad_transpose(w, lane);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        acc[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(v0[k], w[k], acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f64_4x4x4f64(v1[k], w[k], acc[1], 0, 0, 0);
+    }
 }
 
 // adjoint of one lane's bin for one mode, segment searched by the lane (as
@@ -729,11 +740,18 @@ __device__ inline void mode_adjoint_per_lane(double* __restrict__ Ym, const SegR
     while (f < bnd.x && i > 0) bnd = *reinterpret_cast<const double2*>(rm + (long)--i * M);
     while (f >= bnd.y && i < L - 2) bnd = *reinterpret_cast<const double2*>(rm + (long)++i * M);
     if (!(bnd.x <= f && f < bnd.y)) return;
-    double cb[32];
-    if (!mode_adjoint(cb, *(rm + (long)i * M), f - bnd.x, ts, te, Lam, tab)) return;
+    const SegRec* rc = rm + (long)i * M;
+    const double x = f - bnd.x;
+    if (rc->win != WIN_ALL && (rc->win == WIN_NONE || !bin_in_window(rc->q[S_TF], x, ts, te))) return;
+    double a[8];
+    mode_adjoint(a, rc->q, x, Lam, tab);
     double* y = Ym + (long)i * M * NA;
 #pragma unroll
-    for (int j = 0; j < 32; j++) unsafeAtomicAdd(y + adj_q(j >> 2) * 4 + (j & 3), cb[j]);
+    for (int k = 0; k < 8; k++) {
+        double v = a[k];
+#pragma unroll
+        for (int c = 0; c < 4; c++, v *= x) unsafeAtomicAdd(y + adj_q(k) * 4 + c, v);
+    }
 }
 
 // Persistent dense-band kernel, each wavefront taking work items of its own (the
@@ -765,11 +783,17 @@ __device__ inline void mode_adjoint_per_lane(double* __restrict__ Ym, const SegR
 //
 // ADJ: also the adjoint pass of the direct log-likelihood's gradient: after the
 // mode sum of a block, Lam = 4 w (d~ - h~) per bin and channel, then the modes
-// again, each bin's coefficient adjoints (mode_adjoint) summed over the lanes
-// that share a segment (reduce32) and added to the segment's adjoint record.
-// At least 4 wavefronts per SIMD (at most 128 VGPRs).
+// again, each bin's quantity adjoints (mode_adjoint) contracted over the bins
+// that share a segment (adjoint_accumulate) and added to the segment's adjoint record
+// where the walker leaves it. At least 4 wavefronts per SIMD (at most 128 VGPRs), 3
+// with the adjoint pass, which takes one iteration per block: it holds Lam as well,
+// and more iterations spill (256 uneven templates of 1.58 M bins, 1, 2, 3 and 4 of
+// them: 23.4, 24.1, 33 and 37 ms). Bound by FP64 issue, some 1.2 x the forward's
+// instructions for the second pass over the modes. 32 sums over the wavefront by
+// exchanges between lanes in place of the matrix product, and a record loaded per
+// lane: 43.5 ms.
 
-constexpr int DENSE_RB = 4;  // iterations of 64 dense bins per block of a wavefront
+constexpr int DENSE_RB = 4, ADJ_RB = 1;  // iterations of 64 dense bins per block of a wavefront
 
 // A record at a wavefront-uniform address, its bounds and cubics (t_f's apart)
 // loaded in one round: the statements keep the compiler from sinking the
@@ -803,8 +827,50 @@ __device__ inline int segment_estimate(double f, double glo, double gis, int L)
     return (int)fmin(fmax(((double)__log2f((float)f) - glo) * gis, 0.0), (double)(L - 2));
 }
 
+// The walker over one mode's segments for a block of RB x 64 bins. 'cur': the
+// segment to start from (-1: not known); returns the one it ended in, or -1 if bins
+// are left over (todo) for their lanes to search. todo[r] says on entry whether
+// the lane holds a bin.
+//   guess(f)             segment near f
+//   visit(r, in, q, rc)  lanes 'in' of iteration r lie in segment q (record rc)
+//   leave(i)             segment i is done
+template <int RB, class Guess, class Visit, class Leave>
+__device__ inline int walk_block(int cur, const SegRec* rm, int M, int L, const double (&f)[RB], bool (&todo)[RB],
+                                 Guess guess, Visit visit, Leave leave)
+{
+    if (cur < 0) cur = __builtin_amdgcn_readfirstlane(guess(f[0]));
+    // lanes below the current segment send the walker down, else lanes above it up;
+    // a sorted block needs one step per segment it spans
+    bool open = true;
+    for (int step = 0; step < WALK_STEPS; step++) {
+        cur = __builtin_amdgcn_readfirstlane(cur);
+        const SegRec* rc = rm + (unsigned)(cur * M);
+        const SegRec q = load_uniform(rc);
+        bool rest = false;
+#pragma unroll
+        for (int r = 0; r < RB; r++) {
+            const bool in = todo[r] && f[r] >= q.x_lo && f[r] < q.x_hi;
+            visit(r, in, q, rc);
+            todo[r] = todo[r] && !in;
+            rest = rest || todo[r];
+        }
+        leave(cur);
+        if (!__any(rest)) { open = false; break; }
+        bool below = false, above = false;
+#pragma unroll
+        for (int r = 0; r < RB; r++) {
+            below = below || (todo[r] && f[r] < q.x_lo);
+            above = above || (todo[r] && f[r] >= q.x_hi);
+        }
+        if (__any(below) && cur > 0) cur--;
+        else if (__any(above) && cur < L - 2) cur++;
+        else { open = false; break; }  // beyond the grid's ends: no contribution
+    }
+    return open ? -1 : cur;
+}
+
 template <bool ADJ>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_dir_like_t(double* __restrict__ partial, double* __restrict__ Yadj,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADJ ? 3 : 4, 8))) void k_dir_like_t(double* __restrict__ partial, double* __restrict__ Yadj,
                                                     const int* __restrict__ band,
                                                   const int* __restrict__ total, const int* __restrict__ perm,
                                                   int* __restrict__ next, const SegRec* __restrict__ R,
@@ -816,7 +882,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
                                                   const cd* __restrict__ dch, const double* __restrict__ wts, int N,
                                                   int B, int M, int chunk)
 {
-    constexpr int RB = ADJ ? 2 : DENSE_RB;
+    constexpr int RB = ADJ ? ADJ_RB : DENSE_RB;
     __shared__ double2 s_tab[1024];
     const int nitems = total[0];
     const int lane = threadIdx.x & 63;
@@ -846,6 +912,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         int curv = -1;
         if (lane < M && !(grid_istep[b * M + lane] > 0.0)) curv = -2;
         for (int kb = kw0; kb < kw1; kb += RB * 64) {
+            const int curs = curv;  // where the modes' walkers start, for the adjoint pass
             double f[RB];
             cd h[RB][3];
 #pragma unroll
@@ -859,47 +926,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
                 int cur = __builtin_amdgcn_readlane(curv, m);
                 if (cur == -2) continue;
                 const SegRec* rm = R + base * M + m;
-                if (cur < 0) {
-                    const int est = segment_estimate(f[0], grid_lo[b * M + m], grid_istep[b * M + m], L);
-                    cur = __builtin_amdgcn_readfirstlane(est);
-                }
+                // loads the grid's parameters only where they are needed
+                auto guess = [&](double fr) {
+                    return segment_estimate(fr, grid_lo[b * M + m], grid_istep[b * M + m], L);
+                };
                 bool todo[RB];
 #pragma unroll
                 for (int r = 0; r < RB; r++) todo[r] = kb + 64 * r + lane < kw1;
-                // lanes below the current segment send the walker down, else lanes
-                // above it up; a sorted block needs one step per segment it spans
-                bool open = true;
-                for (int step = 0; step < WALK_STEPS; step++) {
-                    cur = __builtin_amdgcn_readfirstlane(cur);
-                    const SegRec* rc = rm + (unsigned)(cur * M);
-                    const SegRec q = load_uniform(rc);
-                    bool rest = false;
-#pragma unroll
-                    for (int r = 0; r < RB; r++) {
-                        const bool in = todo[r] && f[r] >= q.x_lo && f[r] < q.x_hi;
+                cur = walk_block<RB>(
+                    cur, rm, M, L, f, todo, guess,
+                    [&](int r, bool in, const SegRec& q, const SegRec* rc) {
                         if (in) add_mode_window(h[r], q, rc, f[r] - q.x_lo, ts, te, s_tab);
-                        todo[r] = todo[r] && !in;
-                        rest = rest || todo[r];
-                    }
-                    if (!__any(rest)) { open = false; break; }
-                    bool below = false, above = false;
-#pragma unroll
-                    for (int r = 0; r < RB; r++) {
-                        below = below || (todo[r] && f[r] < q.x_lo);
-                        above = above || (todo[r] && f[r] >= q.x_hi);
-                    }
-                    if (__any(below) && cur > 0) cur--;
-                    else if (__any(above) && cur < L - 2) cur++;
-                    else { open = false; break; }  // beyond the grid's ends: no contribution
-                }
-                if (open) {
+                    },
+                    [](int) {});
+                if (cur < 0) {
 #pragma unroll
                     for (int r = 0; r < RB; r++)
-                        if (todo[r])
-                            mode_per_lane(h[r], rm, M, L, f[r],
-                                          segment_estimate(f[r], grid_lo[b * M + m], grid_istep[b * M + m], L), ts, te,
-                                          s_tab);
-                    cur = -1;
+                        if (todo[r]) mode_per_lane(h[r], rm, M, L, f[r], guess(f[r]), ts, te, s_tab);
                 }
                 curv = lane == m ? cur : curv;
             }
@@ -923,56 +966,53 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
             }
             if constexpr (ADJ) {
                 for (int m = 0; m < M; m++) {
-                    const double gis = grid_istep[b * M + m];
-                    if (!(gis > 0.0)) continue;
-                    const double glo = grid_lo[b * M + m];
+                    int cur = __builtin_amdgcn_readlane(curs, m);
+                    if (cur == -2) continue;
                     const SegRec* rm = R + base * M + m;
+                    auto guess = [&](double fr) {
+                        return segment_estimate(fr, grid_lo[b * M + m], grid_istep[b * M + m], L);
+                    };
                     double* Ym = Yadj + (base * M + m) * (long)NA;
-                    int cur = -1;
+                    bool todo[RB];
 #pragma unroll
-                    for (int r = 0; r < RB; r++) {
-                        bool pending = kb + 64 * r + lane < kw1;
-                        const unsigned long long pm = __ballot(pending);
-                        if (pm == 0) break;
-                        const double lf = (double)__log2f((float)f[r]);
-                        const int est = (int)fmin(fmax((lf - glo) * gis, 0.0), (double)(L - 2));
-                        const int e_first = __builtin_amdgcn_readlane(est, __builtin_ctzll(pm));
-                        const int e_last = __builtin_amdgcn_readlane(est, 63 - __builtin_clzll(pm));
-                        if (e_last - e_first > 2) {
-                            if (pending) mode_adjoint_per_lane(Ym, rm, M, L, f[r], est, ts, te, h[r], s_tab);
-                            cur = -1;
-                            continue;
-                        }
-                        if (cur < 0) cur = e_first;
-                        for (int guard = 2 * L + 8; guard > 0; guard--) {
-                            if (__ballot(pending) == 0) break;
-                            const SegRec* rc = rm + (long)cur * M;
-                            const double xlo = rc->x_lo, xhi = rc->x_hi;
-                            const bool below = pending && f[r] < xlo;
-                            if (__ballot(below) != 0) {
-                                if (cur == 0) pending = pending && !below;
-                                else cur--;
-                                continue;
-                            }
-                            const bool in = pending && f[r] < xhi;
-                            double cb[32];
+                    for (int r = 0; r < RB; r++) todo[r] = kb + 64 * r + lane < kw1;
+                    double acc[2] = {0.0, 0.0};
+                    bool used = false;
+                    cur = walk_block<RB>(
+                        cur, rm, M, L, f, todo, guess,
+                        [&](int r, bool in, const SegRec& q, const SegRec* rc) {
+                            const double x = in ? f[r] - q.x_lo : 0.0;
+                            in = in && (q.win == WIN_ALL || (q.win == WIN_MIXED && bin_in_window(rc->q[S_TF], x, ts, te)));
+                            if (!__any(in)) return;
+                            used = true;
+                            // every lane evaluates (the others at x = 0), so that a block
+                            // within the segment needs no selection
+                            double a[8];
+                            mode_adjoint(a, q.q, x, h[r], s_tab);
+                            if (!__all(in)) {
 #pragma unroll
-                            for (int j = 0; j < 32; j++) cb[j] = 0.0;
-                            bool used = false;
-                            if (in) used = mode_adjoint(cb, *rc, f[r] - xlo, ts, te, h[r], s_tab);
-                            if (__ballot(used) != 0) {
-                                const double tot = reduce32(cb, lane);
-                                if ((lane & 1) == 0) {
-                                    const int j = lane >> 1;
-                                    unsafeAtomicAdd(Ym + (long)cur * M * NA + adj_q(j >> 2) * 4 + (j & 3), tot);
-                                }
+                                for (int k = 0; k < 8; k++) a[k] = in ? a[k] : 0.0;
                             }
-                            pending = pending && !in;
-                            if (__ballot(pending) != 0) {
-                                if (cur == L - 2) pending = false;
-                                else cur++;
+                            adjoint_accumulate(acc, a, x, lane);
+                        },
+                        [&](int i) {
+                            if (!used) return;
+                            // the four blocks of bins, then one lane per coefficient
+                            double* y = Ym + (long)i * M * NA;
+#pragma unroll
+                            for (int g = 0; g < 2; g++) {
+                                double v = acc[g];
+                                v += __shfl_xor(v, 4, 64);
+                                v += __shfl_xor(v, 8, 64);
+                                if ((lane & 12) == 0) unsafeAtomicAdd(y + adj_q(4 * g + (lane >> 4)) * 4 + (lane & 3), v);
+                                acc[g] = 0.0;
                             }
-                        }
+                            used = false;
+                        });
+                    if (cur < 0) {
+#pragma unroll
+                        for (int r = 0; r < RB; r++)
+                            if (todo[r]) mode_adjoint_per_lane(Ym, rm, M, L, f[r], guess(f[r]), ts, te, h[r], s_tab);
                     }
                 }
             }
