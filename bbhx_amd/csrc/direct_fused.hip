@@ -648,8 +648,7 @@ __device__ inline void mode_per_lane(cd h[3], const SegRec* __restrict__ rm, int
 // ---------------------------------------------------------------- adjoint helpers
 
 // Adjoint record of one (knot, mode): for each of the nine quantities, the
-// adjoints of its segment's (y, c1, c2, c3); after k_dirg_spline_adj, slot 0
-// of each quantity holds the adjoint of the quantity's value at the knot.
+// adjoints of its segment's (y, c1, c2, c3).
 constexpr int NA = NQ * 4;  // 36 doubles
 
 // quantity of adjoint j (0..7): A, phase, then the six transfer-function parts
@@ -1071,103 +1070,122 @@ __global__ __launch_bounds__(64) void k_dirg_setup(gradk::GradRec* __restrict__ 
     gradk::grad_setup_one(grecs[idx], params, B, b, modes.ell[mi], modes.mm[mi], qnm, table_len, dspin);
 }
 
-// Adjoint of the not-a-knot spline construction (the system of k_dir_spline):
-// segment-coefficient adjoints -> adjoints of the knot values. One wavefront
-// per binary, one lane per (mode, quantity) system (t_f excluded). In the
-// record of knot i, quantity q: slots 0..3 hold the coefficient adjoints of
-// segment i on entry; the passes reuse them (0: value adjoint, 1: slope
-// adjoint then z, 2, 3: the transposed solve's c', d'); slot 0 holds the
-// knot-value adjoint on exit.
-__global__ __launch_bounds__(64) void k_dirg_spline_adj(double* __restrict__ Yadj, const double* __restrict__ X,
-                                                        const long* __restrict__ off, const int* __restrict__ len,
-                                                        int M)
+// Adjoint of the not-a-knot spline construction (k_dir_spline): segment-coefficient
+// adjoints (Yadj) -> adjoints Ya (S, M, NQ) of the knot values, of one (binary, mode)
+// and the eight quantities that have them, one lane per knot, in the blocks of
+// k_dir_spline. Row j of the transposed system couples by h_{j-2} and h_{j+1} against
+// 2 (h_{j-1} + h_j) (h_i: interval i); the end rows are folded like the system's
+// (z_0 = s_0 / h_1 - z_1, and the same at the other end). A solution forgets like
+// the system's own, the inverse being the transpose.
+//
+// Bound by the records' reads (288 B per (knot, mode), one lane's at a time) and the
+// exchanges: 256 uneven templates, 2.36 M records: 0.66 ms (0.16 ms at the rate of a
+// copy). Thomas sweeps, one lane per (mode, quantity): 8.7 ms.
+__global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void k_dirg_spline_adj(
+    double* __restrict__ Ya, const double* __restrict__ Yadj, const double* __restrict__ X, const long* __restrict__ off,
+    const int* __restrict__ len, int M, int nbmax)
 {
-    const int b = blockIdx.x;
-    const int s = threadIdx.x;
-    if (s >= M * 8) return;
-    const int m = s / 8, q = adj_q(s % 8);
-    const int n = len[b];
-    const long base = off[b];
-    auto xi = [&](int i) { return X[(base + i) * M + m]; };
-    auto Y = [&](int i) { return Yadj + ((base + i) * M + m) * (long)NA + q * 4; };
-    // pass 1: segment coefficients -> value and slope adjoints (carry into knot i + 1)
-    double cy = 0.0, cs = 0.0;
-    for (int i = 0; i < n - 1; i++) {
-        double* y = Y(i);
-        const double c0 = y[0], c1 = y[1], c2 = y[2], c3 = y[3];
-        const double dx = xi(i + 1) - xi(i);
-        const double tb = -c2 + c3 / dx;
-        const double slb = c2 / dx - 2.0 * tb / dx;
-        y[0] = cy + c0 - slb / dx;
-        y[1] = cs + c1 - c2 / dx + tb / dx;
-        cy = slb / dx;
-        cs = tb / dx;
+    constexpr int T = SPL_T, NA8 = 8;
+    __shared__ double sh[(NA8 + 2) * T];
+    const int t = threadIdx.x;
+    const SplineRows w = spline_rows(len, M, nbmax);
+    if (!w.any) return;
+    const int i = w.first + t, n = w.n;
+    const long base = off[w.b];
+    const bool row = i < n, seg = i < n - 1;  // knot i, segment i
+    const long p = (base + (row ? i : n - 1)) * M + w.m;
+    const double x = X[p];
+    sh[t] = x;
+    __syncthreads();
+    auto at = [&](int d) { return min(max(t + d, 0), T - 1); };
+    // h[k]: interval i - 2 + k
+    double h[4], xk = sh[at(-2)];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const double xn = sh[at(k - 1)];
+        h[k] = xn - xk;
+        xk = xn;
     }
-    {
-        double* y = Y(n - 1);
-        y[0] = cy;
-        y[1] = cs;
+    const double ih = rcp_pos(h[2]);
+    // this segment's share of the value and slope adjoints of its two knots
+    double yb[NA8], sb[NA8], cy[NA8];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NA8; q++) {
+        const double* c = Yadj + p * NA + adj_q(q) * 4;
+        const double tb = (c[3] * ih - c[2]) * ih, sl = c[2] * ih - 2.0 * tb;
+        cy[q] = seg ? sl * ih : 0.0;
+        yb[q] = seg ? c[0] - cy[q] : 0.0;
+        sb[q] = seg ? c[1] - c[2] * ih + tb : 0.0;
+        sh[q * T + t] = seg ? tb : 0.0;
     }
-    // pass 2: A^T z = slope adjoints (A: the tridiagonal matrix of the slopes)
-    auto Aij = [&](int i, int j) -> double {
-        if (i == 0) return j == 0 ? xi(2) - xi(1) : (j == 1 ? xi(2) - xi(0) : 0.0);
-        if (i == n - 1) return j == n - 2 ? xi(n - 1) - xi(n - 3) : (j == n - 1 ? xi(n - 2) - xi(n - 3) : 0.0);
-        if (j == i - 1) return xi(i + 1) - xi(i);
-        if (j == i) return 2.0 * (xi(i + 1) - xi(i - 1));
-        if (j == i + 1) return xi(i) - xi(i - 1);
-        return 0.0;
-    };
-    double cprev = 0.0, dprev = 0.0;
-    for (int i = 0; i < n; i++) {
-        double* y = Y(i);
-        const double bdiag = Aij(i, i);
-        double den, d;
-        if (i == 0) {
-            den = bdiag;
-            d = y[1] / den;
-        } else {
-            const double a = Aij(i - 1, i);
-            den = bdiag - a * cprev;
-            d = (y[1] - a * dprev) / den;
-        }
-        const double c = i < n - 1 ? Aij(i + 1, i) / den : 0.0;
-        y[2] = c;
-        y[3] = d;
-        cprev = c;
-        dprev = d;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NA8; q++)
+        if (t > 0) sb[q] += sh[q * T + t - 1];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NA8; q++) sh[q * T + t] = cy[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NA8; q++)
+        if (t > 0) yb[q] += sh[q * T + t - 1];
+    __syncthreads();
+    // the transposed system; rows with all their neighbours in the block
+    const bool solve = i > 0 && i < n - 1 && t > 0 && t + 1 < T && (i == 1 || t > 1) && (i == n - 2 || t + 2 < T);
+    const bool low = solve && i == 1, high = solve && i == n - 2;
+    const double d = h[1] + h[2];
+    const double diag = 2.0 * d - (low ? d : 0.0) - (high ? d : 0.0), ib = rcp_pos(diag);
+    const double a = solve && !low ? h[0] * ib : 0.0, c = solve && !high ? h[3] * ib : 0.0;
+    double z[NA8];
+#pragma unroll
+    for (int q = 0; q < NA8; q++) sh[q * T + t] = sb[q];
+    __syncthreads();
+    const double iel = rcp_pos(h[2]), ieh = rcp_pos(h[1]);  // pivots of the end rows
+#pragma unroll
+    for (int q = 0; q < NA8; q++) {
+        double v = sb[q];
+        if (low) v -= d * (sh[q * T + t - 1] * iel);
+        if (high) v -= d * (sh[q * T + t + 1] * ieh);
+        z[q] = solve ? v * ib : 0.0;
     }
-    double znext = Y(n - 1)[3];
-    Y(n - 1)[1] = znext;
-    for (int i = n - 2; i >= 0; i--) {
-        double* y = Y(i);
-        znext = y[3] - y[2] * znext;
-        y[1] = znext;
+    double zl[NA8];  // the end rows' own terms, by their neighbours
+#pragma unroll
+    for (int q = 0; q < NA8; q++) zl[q] = low ? sh[q * T + t - 1] * iel : (high ? sh[q * T + t + 1] * ieh : 0.0);
+    // (a grid of four knots has two such rows, in different lanes)
+    __syncthreads();
+    pcr_solve(a, c, z, sh, t);
+#pragma unroll
+    for (int q = 0; q < NA8; q++) {
+        if (i != 0 && i < n - 1) sh[q * T + t] = z[q];
+        if (low) sh[q * T + t - 1] = zl[q] - z[q];
+        if (high) sh[q * T + t + 1] = zl[q] - z[q];
     }
-    // pass 3: value adjoints += R^T z (R: the right-hand side's dependence on the values)
-    {
-        const double dx1 = xi(1) - xi(0), dx2 = xi(2) - xi(1), dd = xi(2) - xi(0);
-        const double a1 = (dx1 + 2.0 * dd) * dx2 / (dd * dx1), a2 = dx1 * dx1 / (dd * dx2);
-        const double z0 = Y(0)[1];
-        Y(0)[0] += -a1 * z0;
-        Y(1)[0] += (a1 - a2) * z0;
-        Y(2)[0] += a2 * z0;
+    __syncthreads();
+    // adjoint of the segment's slope (y_{i+1} - y_i) / h_i from the right sides of rows
+    // i and i + 1 (3 (h_r m_l + h_l m_r)) and of the end rows
+    double k0 = i > 0 && i < n - 1 ? 3.0 * h[1] : 0.0;      // row i
+    double k1 = i + 1 < n - 1 ? 3.0 * h[3] : 0.0;           // row i + 1
+    double km = 0.0, k2 = 0.0;                              // rows i - 1, i + 2
+    if (i == 0) k0 = (h[2] + 2.0 * (h[2] + h[3])) * h[3] * rcp_pos(h[2] + h[3]);
+    if (i == 1) km = h[1] * h[1] * rcp_pos(h[1] + h[2]);
+    if (i == n - 3) k2 = h[3] * h[3] * rcp_pos(h[2] + h[3]);
+    if (i == n - 2) k1 = (2.0 * (h[1] + h[2]) + h[2]) * h[1] * rcp_pos(h[1] + h[2]);
+#pragma unroll
+    for (int q = 0; q < NA8; q++) {
+        double g = k0 * sh[q * T + t] + k1 * sh[q * T + at(1)];
+        if (i == 1) g += km * sh[q * T + t - 1];
+        if (i == n - 3) g += k2 * sh[q * T + at(2)];
+        cy[q] = seg ? g * ih : 0.0;
     }
-    for (int i = 1; i < n - 1; i++) {
-        const double e1 = xi(i) - xi(i - 1), e2 = xi(i + 1) - xi(i);
-        const double b1 = 3.0 * e2 / e1, b2 = 3.0 * e1 / e2;
-        const double zi = Y(i)[1];
-        Y(i - 1)[0] += -b1 * zi;
-        Y(i)[0] += (b1 - b2) * zi;
-        Y(i + 1)[0] += b2 * zi;
-    }
-    {
-        const double e1 = xi(n - 2) - xi(n - 3), e2 = xi(n - 1) - xi(n - 2), ed = xi(n - 1) - xi(n - 3);
-        const double c1 = e2 * e2 / (ed * e1), c2 = (2.0 * ed + e2) * e1 / (ed * e2);
-        const double zn = Y(n - 1)[1];
-        Y(n - 3)[0] += -c1 * zn;
-        Y(n - 2)[0] += (c1 - c2) * zn;
-        Y(n - 1)[0] += c2 * zn;
-    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NA8; q++) sh[q * T + t] = cy[q];
+    __syncthreads();
+    if (!row || i < w.row0 || i >= w.row1) return;
+#pragma unroll
+    for (int q = 0; q < NA8; q++)
+        Ya[p * NQ + adj_q(q)] = yb[q] - cy[q] + (i > 0 ? sh[q * T + t - 1] : 0.0);
 }
 
 // Knot-level contraction: one wavefront per (binary, mode), lane per knot; the
@@ -1175,7 +1193,7 @@ __global__ __launch_bounds__(64) void k_dirg_spline_adj(double* __restrict__ Yad
 // tangents at the knot's frequency (grad_point_core, no window rule: the
 // window acts on the dense bins). partial[(b M + m) 11 + p].
 __global__ __launch_bounds__(64) void k_dirg_knots(double* __restrict__ gpart, const gradk::GradRec* __restrict__ grecs,
-                                                   const double* __restrict__ Yadj, const double* __restrict__ X,
+                                                   const double* __restrict__ Ya, const double* __restrict__ X,
                                                    const long* __restrict__ off, const int* __restrict__ len,
                                                    const double* __restrict__ params, int B, int M,
                                                    resp::OrbitTab orb, int TDItag, int rescaled, int tdi2,
@@ -1199,10 +1217,10 @@ __global__ __launch_bounds__(64) void k_dirg_knots(double* __restrict__ gpart, c
     for (int p = 0; p < gradk::NGRAD; p++) acc[p] = 0.0;
     for (int i = threadIdx.x; i < n; i += 64) {
         const long rec = (base + i) * M + m;
-        const double* y = Yadj + rec * NA;
-        const double aA = y[0 * 4], aPh = y[1 * 4];
+        const double* y = Ya + rec * NQ;
+        const double aA = y[0], aPh = y[1];
         cd Wt[3];
-        for (int c = 0; c < 3; c++) Wt[c] = mk(y[(3 + 2 * c) * 4], -y[(4 + 2 * c) * 4]);
+        for (int c = 0; c < 3; c++) Wt[c] = mk(y[3 + 2 * c], -y[4 + 2 * c]);
         auto weights = [&](const cd*, cd, double, cd W[3], double& a_A, double& a_Ph) {
             for (int c = 0; c < 3; c++) W[c] = Wt[c];
             a_A = aA;
@@ -1435,8 +1453,10 @@ int direct_launch(bbhx_direct_plan* p, double* d_h, double* h_h, double* grad, i
     hipLaunchKernelGGL(k_dir_reduce, dim3(B), dim3(64), 0, st, d_h, h_h, p->partial, p->band,
                        p->total, B);
     if (grad) {
-        hipLaunchKernelGGL(k_dirg_spline_adj, dim3(B), dim3(64), 0, st, p->Yadj, p->X, p->off, p->len, M);
-        hipLaunchKernelGGL(k_dirg_knots, dim3(B * M), dim3(64), 0, st, p->gpart, p->grecs, p->Yadj, p->X, p->off,
+        // the knot values' adjoints take the place of the values, which are not read again
+        hipLaunchKernelGGL(k_dirg_spline_adj, dim3((unsigned)((long)B * M * nbmax)), dim3(SPL_T), 0, st, p->Yc,
+                           p->Yadj, p->X, p->off, p->len, M, nbmax);
+        hipLaunchKernelGGL(k_dirg_knots, dim3(B * M), dim3(64), 0, st, p->gpart, p->grecs, p->Yc, p->X, p->off,
                            p->len, params, B, M, orb, TDItag, rescaled, tdi2, initial_t_val);
         hipLaunchKernelGGL(k_dirg_reduce, dim3(ceil_div((long)B * gradk::NGRAD, 256)), dim3(256), 0, st, grad,
                            p->gpart, B, M);
