@@ -10,7 +10,7 @@
 // per quantity [y, c1, c2, c3], so that one segment of one quantity is 32
 // contiguous bytes and one record read both checks and evaluates the segment):
 //   k_dir_setup   one lane per (binary, mode): coefficient records
-//   k_dir_grid    one wavefront per (binary, mode): default grid
+//   k_dir_grid    one workgroup per (binary, mode): default grid
 //                 Mf in [mf_min, mf_max] * m / 2, t(f) there, the crossings of
 //                 t = 0 and t = Tobs, the grid refitted to that window
 //                 (phenomhm.py:208-224, :509-614), then amplitude, phase, t(f)
@@ -144,8 +144,17 @@ __device__ inline double wmax_d(double v)
     return v;
 }
 
-// One 64-lane wavefront per (binary, mode). LDS: t(f) of the default grid (L_b doubles).
-__global__ __launch_bounds__(64) void k_dir_grid(double* __restrict__ X, double* __restrict__ Yc,
+// One workgroup per (binary, mode), one lane per knot of each pass. LDS: t(f) of the
+// default grid (L_b doubles).
+//
+// Bound by the FP64 work of a knot, some 4000 instructions over both grids, at the
+// two wavefronts per SIMD that its 251 VGPRs leave (three and four spill: 1.41 and
+// 1.92 ms). 16 templates of 1024 knots: 33 us, 1024 uneven ones: 0.95 ms. One
+// wavefront per (binary, mode): 78 us, a chain of 16 knots per lane and pass, and
+// 1.18 ms, as the LDS for the longest grid then allows five wavefronts per CU. 512
+// lanes: 30 us and 1.18 ms.
+constexpr int GRID_T = 256;
+__global__ __launch_bounds__(GRID_T) void k_dir_grid(double* __restrict__ X, double* __restrict__ Yc,
                                                  double* __restrict__ grid_lo, double* __restrict__ grid_istep,
                                                  int* __restrict__ flags, const FusedRec* __restrict__ recs,
                                                  const long* __restrict__ off, const int* __restrict__ len,
@@ -156,9 +165,11 @@ __global__ __launch_bounds__(64) void k_dir_grid(double* __restrict__ X, double*
                                                  double initial_t_val, double mf_min, double mf_max)
 {
     extern __shared__ double tfs[];
+    __shared__ double2 s_t[GRID_T / 64];
+    __shared__ int4 s_n[GRID_T / 64];
     const int bm = blockIdx.x;
     const int b = bm / M, m = bm % M;
-    const int lane = threadIdx.x;
+    const int t = threadIdx.x, T = blockDim.x;
     const int L = len[b];
     const long base = off[b];
     const FusedRec& r = recs[bm];
@@ -169,7 +180,7 @@ __global__ __launch_bounds__(64) void k_dir_grid(double* __restrict__ X, double*
 
     // default grid (phenomhm.py:208-224) and t(f) on it; the frequencies go to X for now
     const double lo = log10(mf_min), hi = log10(mf_max), step = (hi - lo) / (L - 1);
-    for (int i = lane; i < L; i += 64) {
+    for (int i = t; i < L; i += T) {
         const double f = logspace_pt(lo, step, hi, i, L) / Msec * mm / 2;
         double amp, phase, tf;
         phm::phm_eval(r.w, f, amp, phase, tf);
@@ -181,17 +192,17 @@ __global__ __launch_bounds__(64) void k_dir_grid(double* __restrict__ X, double*
     // window search (phenomhm.py:520-614): the single segment where t crosses 0 / Tobs
     double tmin = 1e300, tmax = -1e300;
     int n0 = 0, nT = 0, s0 = -1, sT = -1;
-    for (int i = lane; i < L; i += 64) {
-        const double t = tfs[i];
-        tmin = fmin(tmin, t);
-        tmax = fmax(tmax, t);
+    for (int i = t; i < L; i += T) {
+        const double t0 = tfs[i];
+        tmin = fmin(tmin, t0);
+        tmax = fmax(tmax, t0);
         if (i + 1 < L) {
             const double t1 = tfs[i + 1];
-            if ((0.0 < t1) && (0.0 > t)) {
+            if ((0.0 < t1) && (0.0 > t0)) {
                 n0++;
                 s0 = i;
             }
-            if ((Tobs < t1) && (Tobs > t)) {
+            if ((Tobs < t1) && (Tobs > t0)) {
                 nT++;
                 sT = i;
             }
@@ -203,6 +214,20 @@ __global__ __launch_bounds__(64) void k_dir_grid(double* __restrict__ X, double*
     nT = wsum_i(nT);
     s0 = wmax_i(s0);
     sT = wmax_i(sT);
+    if ((t & 63) == 0) {
+        s_t[t >> 6] = {tmin, tmax};
+        s_n[t >> 6] = {n0, nT, s0, sT};
+    }
+    __syncthreads();
+    for (int w = 0; w < T / 64; w++) {
+        if (w == t >> 6) continue;
+        tmin = fmin(tmin, s_t[w].x);
+        tmax = fmax(tmax, s_t[w].y);
+        n0 += s_n[w].x;
+        nT += s_n[w].y;
+        s0 = max(s0, s_n[w].z);
+        sT = max(sT, s_n[w].w);
+    }
     const double* xf = X + base * M + m;
     double f_min = xf[0], f_max = xf[(long)(L - 1) * M];
     int flag = 0;
@@ -222,18 +247,18 @@ __global__ __launch_bounds__(64) void k_dir_grid(double* __restrict__ X, double*
             f_max = (y2 - y1) / (x2 - x1) * (Tobs - x1) + y1;
         }
     }
-    if (lane == 0 && flag) atomicOr(&flags[b], flag);
+    if (t == 0 && flag) atomicOr(&flags[b], flag);
     __syncthreads();  // every lane has read the default grid before it is overwritten
 
     // refitted grid and the nine quantities on it
     const double lo2 = log10(f_min), hi2 = log10(f_max), step2 = (hi2 - lo2) / (L - 1);
-    if (lane == 0) {
+    if (t == 0) {
         // log2 units: the dense kernel estimates the segment from an FP32 log2
         grid_lo[bm] = lo2 * LOG2_10;
         grid_istep[bm] = step2 > 0.0 ? 1.0 / (step2 * LOG2_10) : 0.0;
     }
     const double dt_shift = t_ref - initial_t_val;
-    for (int i = lane; i < L; i += 64) {
+    for (int i = t; i < L; i += T) {
         const double f = logspace_pt(lo2, step2, hi2, i, L);
         double amp, phase, tf;
         phm::phm_eval(r.w, f, amp, phase, tf);
@@ -1418,7 +1443,8 @@ int direct_launch(bbhx_direct_plan* p, double* d_h, double* h_h, double* grad, i
     hipLaunchKernelGGL(k_dir_setup, dim3(setup_blocks(B, M)), dim3(64), 0, st, p->recs, params, B,
                        ml, M, qnm,
                        table_len, dspin);
-    hipLaunchKernelGGL(k_dir_grid, dim3(B * M), dim3(64), sizeof(double) * (size_t)p->Lmax, st, p->X, p->Yc,
+    const int grid_t = std::min(GRID_T, (p->Lmax + 63) / 64 * 64);
+    hipLaunchKernelGGL(k_dir_grid, dim3(B * M), dim3(grid_t), sizeof(double) * (size_t)p->Lmax, st, p->X, p->Yc,
                        p->grid_lo, p->grid_istep, flags, p->recs, p->off, p->len, params, t_start, t_end, B, M, ml,
                        orb, TDItag, rescaled, tdi2, initial_t_val, mf_min, mf_max);
     const int nbmax = spline_blocks(p->Lmax);
