@@ -78,7 +78,186 @@ __global__ __launch_bounds__(INTERP_TILE) void k_interp_tdi(const InterpBin* __r
     out[2 * (long)d.len + i] = h[2];
 }
 
+// number of entries of the sorted a[0, n) that are <= v (n if v is not a number)
+__device__ inline int upper_bound(const double* __restrict__ a, int n, double v)
+{
+    int lo = 0, hi = n;
+    while (lo < hi) {
+        const int mid = lo + ((hi - lo) >> 1);
+        if (a[mid] > v) hi = mid;
+        else lo = mid + 1;
+    }
+    return lo;
+}
+
+// the same by a wavefront: 64 entries a round
+__device__ inline int wave_upper_bound(const double* __restrict__ a, int n, double v)
+{
+    const int lane = threadIdx.x & 63;
+    int lo = 0;
+    while (n > 0) {
+        const int step = (n + 63) >> 6;
+        const long p = (long)lane * step;
+        const int c = __popcll(__ballot(p < n && !(a[lo + (p < n ? p : 0)] > v)));
+        if (c == 0) break;
+        lo += (c - 1) * step + 1;
+        n = min(step, n - (c - 1) * step) - 1;
+    }
+    return lo;
+}
+
+// band[b] = [start, end) of the data grid that binary b's sparse grids cover: one
+// workgroup per binary, least and greatest of its n sparse frequencies
+__global__ __launch_bounds__(256) void k_interp_bands(int2* __restrict__ band, const double* __restrict__ freqs, long n,
+                                                      const double* __restrict__ dataFreqs, int N)
+{
+    __shared__ double s_lo[4], s_hi[4];
+    const double* x = freqs + (long)blockIdx.x * n;
+    double lo = x[0], hi = x[0];
+    auto least = [](double a, double b) { return (b < a || b != b) && a == a ? b : a; };  // not a number if any is
+    auto most = [](double a, double b) { return (b > a || b != b) && a == a ? b : a; };
+    for (long i = threadIdx.x; i < n; i += 256) {
+        lo = least(lo, x[i]);
+        hi = most(hi, x[i]);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        lo = least(lo, __shfl_xor(lo, o, 64));
+        hi = most(hi, __shfl_xor(hi, o, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        s_lo[threadIdx.x >> 6] = lo;
+        s_hi[threadIdx.x >> 6] = hi;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 128) return;
+    lo = s_lo[0];
+    hi = s_hi[0];
+    for (int w = 1; w < 4; w++) {
+        lo = least(lo, s_lo[w]);
+        hi = most(hi, s_hi[w]);
+    }
+    // one wavefront per end
+    const bool end = threadIdx.x >= 64;
+    const int k = wave_upper_bound(dataFreqs, N, end ? hi : lo);
+    if ((threadIdx.x & 63) == 0) (end ? band[blockIdx.x].y : band[blockIdx.x].x) = k;
+}
+
+// off[b]: bins of the bands before b's (one workgroup)
+__global__ __launch_bounds__(256) void k_interp_offsets(int64_t* __restrict__ off, const int2* __restrict__ band, int B)
+{
+    __shared__ int64_t part[256];
+    const int t = threadIdx.x, per = (B + 255) / 256, b0 = min(B, t * per), b1 = min(B, b0 + per);
+    int64_t sum = 0;
+    for (int b = b0; b < b1; b++) sum += max(0, band[b].y - band[b].x);
+    part[t] = sum;
+    __syncthreads();
+    int64_t run = 0;
+    for (int w = 0; w < t; w++) run += part[w];
+    for (int b = b0; b < b1; b++) {
+        off[b] = run;
+        run += max(0, band[b].y - band[b].x);
+    }
+}
+
+// Spline segment of every (binary, mode, dense bin): block -> (binary, mode, tile of
+// SEG_TILE bins). The grids are log-spaced, so the segment is estimated from an FP32
+// logarithm and checked, its neighbours next; whatever they do not hold is searched.
+// Bound by instruction issue, the estimate and its checks. Up to 38 M (binary, mode, bin): 0.11
+// ms (0.23 by a binary search per bin); torch's searchsorted and its conversions,
+// binary by binary: 0.49 ms and seven launches for each.
+constexpr int SEG_TILE = 1024;
+__global__ __launch_bounds__(256) void k_interp_segments(int* __restrict__ inds, const int2* __restrict__ band,
+                                                         const int64_t* __restrict__ off,
+                                                         const double* __restrict__ dataFreqs,
+                                                         const double* __restrict__ freqs, int M, int L, int tiles)
+{
+    const int tile = blockIdx.x % tiles, bm = blockIdx.x / tiles, b = bm / M, m = bm - b * M;
+    const int2 r = band[b];
+    const int len = r.y - r.x;
+    const double* x = freqs + (long)bm * L;
+    int* o = inds + off[b] * M + (long)m * len;
+    const int i0 = tile * SEG_TILE, n = min(len - i0, SEG_TILE);
+    const double x0 = x[0], x1 = x[L - 1];
+    const float g0 = __log2f((float)x0), gs = (float)(L - 1) / (__log2f((float)x1) - g0);
+    for (int i = threadIdx.x; i < n; i += 256) {
+        const double f = dataFreqs[r.x + i0 + i];
+        int k = -1;
+        if (L < 2) k = upper_bound(x, L, f) - 1;
+        else if (f >= x1) k = L - 1;
+        else if (!(f < x0)) {
+            k = (int)fminf(fmaxf((__log2f((float)f) - g0) * gs, 0.0f), (float)(L - 2));
+            if (f < x[k]) k = max(k - 1, 0);
+            else if (f >= x[k + 1]) k = min(k + 1, L - 2);
+            if (!(x[k] <= f && f < x[k + 1])) k = upper_bound(x, L, f) - 1;
+        }
+        o[i0 + i] = k;
+    }
+}
+
+// out[b][ch][k]: the template on b's band, zero elsewhere; block -> (binary, tile), one
+// pass over the output (bound by its writes; a fill, then a copy per binary, writes the
+// bands twice)
+__global__ __launch_bounds__(256) void k_fill_bands(double2* __restrict__ out, const double2* __restrict__ tmpl,
+                                                    const int2* __restrict__ band, const int64_t* __restrict__ off,
+                                                    int N, int tiles)
+{
+    const int tile = blockIdx.x % tiles, b = blockIdx.x / tiles;
+    if ((unsigned)tile * 256 + threadIdx.x >= (unsigned)N) return;
+    const int k = tile * 256 + threadIdx.x;
+    const int2 r = band[b];
+    const int len = r.y - r.x;
+    const bool in = k >= r.x && k < r.y;
+    const double2* t = tmpl + off[b] * 3 + (k - r.x);
+    double2* o = out + (long)b * 3 * N + k;
+#pragma unroll
+    for (int ch = 0; ch < 3; ch++) o[(long)ch * N] = in ? t[(long)ch * len] : make_double2(0.0, 0.0);
+}
+
 }  // namespace
+
+extern "C" int bbhx_hip_interp_bands(int* band, int64_t* off, const double* freqs, const double* dataFreqs, int length,
+                                     int data_length, int numBinAll, int numModes, void* stream)
+{
+    if (length < 1 || data_length < 0 || numBinAll < 0 || numModes < 1) return ERR_ARGS;
+    if (numBinAll == 0) return OK;
+    if (!band || !off || !freqs || (!dataFreqs && data_length > 0)) return ERR_ARGS;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    int2* r = reinterpret_cast<int2*>(band);
+    hipLaunchKernelGGL(k_interp_bands, dim3(numBinAll), dim3(256), 0, st, r, freqs, (long)numModes * length, dataFreqs,
+                       data_length);
+    hipLaunchKernelGGL(k_interp_offsets, dim3(1), dim3(256), 0, st, off, r, numBinAll);
+    return hipGetLastError() == hipSuccess ? OK : ERR_LAUNCH;
+}
+
+extern "C" int bbhx_hip_interp_segments(int* inds, const int* band, const int64_t* off, const double* freqs,
+                                        const double* dataFreqs, int length, int max_len, int numBinAll, int numModes,
+                                        void* stream)
+{
+    if (length < 1 || max_len < 0 || numBinAll < 0 || numModes < 1) return ERR_ARGS;
+    if (numBinAll == 0 || max_len == 0) return OK;
+    if (!inds || !band || !off || !freqs || !dataFreqs) return ERR_ARGS;
+    const int tiles = (int)(((long)max_len + SEG_TILE - 1) / SEG_TILE);
+    const long blocks = (long)numBinAll * numModes * tiles;
+    if (blocks > 2147483647L) return ERR_ARGS;
+    hipLaunchKernelGGL(k_interp_segments, dim3((unsigned)blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
+                       inds, reinterpret_cast<const int2*>(band), off, dataFreqs, freqs, numModes, length, tiles);
+    return hipGetLastError() == hipSuccess ? OK : ERR_LAUNCH;
+}
+
+extern "C" int bbhx_hip_fill_bands(double* out, const double* templates, const int* band, const int64_t* off,
+                                   int data_length, int numBinAll, void* stream)
+{
+    if (data_length < 0 || numBinAll < 0) return ERR_ARGS;
+    if (numBinAll == 0 || data_length == 0) return OK;
+    if (!out || !templates || !band || !off) return ERR_ARGS;
+    const int tiles = (int)(((long)data_length + 255) / 256);
+    const long blocks = (long)numBinAll * tiles;
+    if (blocks > 2147483647L) return ERR_ARGS;
+    hipLaunchKernelGGL(k_fill_bands, dim3((unsigned)blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
+                       reinterpret_cast<double2*>(out), reinterpret_cast<const double2*>(templates),
+                       reinterpret_cast<const int2*>(band), off, data_length, tiles);
+    return hipGetLastError() == hipSuccess ? OK : ERR_LAUNCH;
+}
 
 namespace bbhx {
 // Uploads a host table of per-binary descriptors to the table workspace.

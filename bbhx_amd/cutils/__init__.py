@@ -96,6 +96,9 @@ def load_library():
                                        C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _vp],
         "bbhx_hip_direct_plan_enable_grad": [_vp],
         "bbhx_hip_direct_plan_set_precision": [_vp, C.c_int],
+        "bbhx_hip_interp_bands": [_vp, _vp, _vp, _vp, C.c_int, C.c_int, C.c_int, C.c_int, _vp],
+        "bbhx_hip_interp_segments": [_vp, _vp, _vp, _vp, _vp, C.c_int, C.c_int, C.c_int, C.c_int, _vp],
+        "bbhx_hip_fill_bands": [_vp, _vp, _vp, _vp, C.c_int, C.c_int, _vp],
         "bbhx_hip_aet1_psd": [_vp, _vp, C.c_int64, C.c_double, C.c_double, C.c_double, _vp],
         "bbhx_hip_window_times": [_vp, _vp, _vp, _vp, C.c_int, C.c_double, C.c_double, _vp],
         "bbhx_hip_release_workspace": [],
@@ -122,7 +125,8 @@ def exported_symbols():
         "bbhx_hip_hdyn_fused_grad", "bbhx_hip_direct_plan_create", "bbhx_hip_direct_plan_destroy",
         "bbhx_hip_direct_plan_bytes", "bbhx_hip_direct_plan_band", "bbhx_hip_direct_fused", "bbhx_hip_hdyn_prep",
         "bbhx_hip_direct_fused_grad", "bbhx_hip_direct_plan_enable_grad", "bbhx_hip_direct_plan_set_precision",
-        "bbhx_hip_aet1_psd", "bbhx_hip_window_times", "bbhx_hip_release_workspace", "bbhx_hip_version", "bbhx_hip_timing_enable",
+        "bbhx_hip_aet1_psd", "bbhx_hip_interp_bands", "bbhx_hip_interp_segments", "bbhx_hip_fill_bands",
+        "bbhx_hip_window_times", "bbhx_hip_release_workspace", "bbhx_hip_version", "bbhx_hip_timing_enable",
         "bbhx_hip_timing_read",
     ]
 
@@ -287,6 +291,49 @@ def InterpTDI_wrap(templateChannels_ptrs, dataFreqs, freqs, propArrays, c1, c2, 
         _dev(c3, f64), tsp, tep, int(length), int(data_length), int(numBinAll), int(numModes), ipp, sp, lp,
         _stream())
     _check(st, "InterpTDI")
+
+
+def interp_bands(data_freqs, freqs):
+    """Dense band of each binary's sparse grids freqs (B, M, L): (band (B, 2) int32, off (B,) int64) on the device
+    (no reference counterpart in BBHxBackendMethods; see include/bbhx_hip.h)."""
+    torch = _torch()
+    f64 = torch.float64
+    B, M, L = (int(v) for v in freqs.shape)
+    band = torch.empty((B, 2), dtype=torch.int32, device=freqs.device)
+    off = torch.empty(B, dtype=torch.int64, device=freqs.device)
+    st = load_library().bbhx_hip_interp_bands(_dev(band), _dev(off), _dev(freqs, f64, "freqs"),
+                                              _dev(data_freqs, f64, "data_freqs"), L, int(data_freqs.numel()), B, M,
+                                              _stream())
+    _check(st, "interp_bands")
+    return band, off
+
+
+def interp_segments(data_freqs, freqs, band, off, lengths):
+    """Spline segment of every (mode, dense bin): one flat int32 tensor, (M, lengths[b]) of each binary after the
+    other; band, off from ``interp_bands``, lengths on the host (no reference counterpart in BBHxBackendMethods)."""
+    torch = _torch()
+    f64 = torch.float64
+    B, M, L = (int(v) for v in freqs.shape)
+    if len(lengths) != B or tuple(band.shape) != (B, 2) or off.numel() != B:
+        raise ValueError("band, off and lengths must have one entry per binary")
+    inds = torch.empty(M * int(np.sum(lengths, dtype=np.int64)), dtype=torch.int32, device=freqs.device)
+    st = load_library().bbhx_hip_interp_segments(
+        _dev(inds), _dev(band, torch.int32), _dev(off, torch.int64), _dev(freqs, f64, "freqs"),
+        _dev(data_freqs, f64, "data_freqs"), L, int(max(lengths, default=0)), B, M, _stream())
+    _check(st, "interp_segments")
+    return inds
+
+
+def fill_bands(out, templates, band, off):
+    """out (B, 3, N) <- the flat templates on their bands, zero elsewhere (no reference counterpart in
+    BBHxBackendMethods; see include/bbhx_hip.h)."""
+    c128 = _torch().complex128
+    B, nch, N = (int(v) for v in out.shape)
+    if nch != 3 or tuple(band.shape) != (B, 2) or off.numel() != B:
+        raise ValueError("out must be (B, 3, N), band and off have one entry per binary")
+    st = load_library().bbhx_hip_fill_bands(_dev(out, c128), _dev(templates, c128), _dev(band, _torch().int32),
+                                            _dev(off, _torch().int64), N, B, _stream())
+    _check(st, "fill_bands")
 
 
 def direct_sum_wrap(templateChannels, bbh_buffer, numBinAll, data_length, nChannels, numModes, t_start, t_end):
@@ -615,6 +662,9 @@ class BBHxHipBackend:
         self.DirectPlan = DirectPlan
         self.hdyn_prep = hdyn_prep
         self.aet1_psd = aet1_psd
+        self.interp_bands = interp_bands
+        self.interp_segments = interp_segments
+        self.fill_bands = fill_bands
         self.window_times = window_times
         self.direct_fused_grad = direct_fused_grad
         self.device = torch.device("cuda", torch.cuda.current_device())

@@ -42,22 +42,21 @@ class TemplateInterpFD(BBHxParallelModule):
         (searchsorted side='right' of the min/max sparse frequency,
         waveformbuild.py:139-156) and, per mode and dense bin, the spline segment
         searchsorted(x_bm, f, 'right') - 1 (:159-172)."""
-        torch = self.xp
-        B, M = freqs_shaped.shape[:2]
-        lo = freqs_shaped.amin(dim=(1, 2))
-        hi = freqs_shaped.amax(dim=(1, 2))
-        st = torch.searchsorted(data_freqs, lo, right=True)
-        et = torch.searchsorted(data_freqs, hi, right=True)
-        st_h = st.cpu().numpy().astype(np.int64)
-        et_h = et.cpu().numpy().astype(np.int64)
-        lengths = (et_h - st_h).astype(np.int32)
-        inds = []
-        for i in range(B):
-            seg = data_freqs[st_h[i]:et_h[i]]
-            vals = seg[None, :].expand(M, -1).contiguous()
-            k = torch.searchsorted(freqs_shaped[i].contiguous(), vals, right=True) - 1
-            inds.append(k.to(torch.int32).flatten().contiguous())
-        return st_h.astype(np.int32), lengths, inds
+        data_freqs, freqs_shaped = to_dev(data_freqs, self.device), to_dev(freqs_shaped, self.device)
+        # bands and bins before them, kept for placing the templates in the data grid
+        self._band, self._off = self.backend.interp_bands(data_freqs, freqs_shaped)
+        band = self._band.cpu().numpy()
+        lengths = np.maximum(band[:, 1] - band[:, 0], 0)
+        flat = self.backend.interp_segments(data_freqs, freqs_shaped, self._band, self._off, lengths)
+        inds = list(flat.split((lengths.astype(np.int64) * freqs_shaped.shape[1]).tolist()))
+        return band[:, 0].copy(), lengths, inds
+
+    def filled(self, n):
+        """The templates of the last call in a data grid of n bins, zero outside
+        their bands: (num_bin_all, 3, n)."""
+        out = self.xp.empty((self.num_bin_all, 3, n), dtype=self.xp.complex128, device=self.device)
+        self.backend.fill_bands(out, self._template_flat, self._band, self._off)
+        return out
 
     def __call__(self, data_freqs, interp_container, t_start, t_end, length, num_modes, num_channels):
         """Returns the list of (num_channels, n_b) complex templates (waveformbuild.py:89-239)."""
@@ -77,7 +76,9 @@ class TemplateInterpFD(BBHxParallelModule):
         self.inds = inds
         self.ptrs = np.asarray([a.data_ptr() for a in inds], dtype=np.int64)
         total = int(np.sum(self.lengths.astype(np.int64))) * num_channels
-        self._template_flat = torch.zeros(max(total, 1), dtype=torch.complex128, device=self.device)
+        # the kernel writes its three channels of every bin
+        alloc = torch.empty if num_channels == 3 else torch.zeros
+        self._template_flat = alloc(max(total, 1), dtype=torch.complex128, device=self.device)
         self.template_carrier = []
         off = 0
         for n in self.lengths:
@@ -203,9 +204,5 @@ class BBHWaveformFD(BBHxParallelModule):
                                                    self.interp_response.lengths):
                     data_out[:, int(start_i):int(start_i) + int(length_i)] += temp
                 return data_out.squeeze() if squeeze else data_out
-            data_out = torch.zeros((self.num_bin_all, 3, nf), dtype=torch.complex128, device=self.device)
-            for bin_i, (temp, start_i, length_i) in enumerate(zip(template_channels, self.interp_response.start_inds,
-                                                                  self.interp_response.lengths)):
-                data_out[bin_i, :, int(start_i):int(start_i) + int(length_i)] = temp
-            return data_out
+            return self.interp_response.filled(nf)
         return (template_channels, self.interp_response.start_inds, self.interp_response.lengths)

@@ -294,6 +294,23 @@ int bbhx_hip_hdyn_prep(double* dataConstants, double* totals, const double* data
                        const double* h0, const double* psd, int data_length, const double* nodes, int K, double df,
                        void* stream);
 
+/* The index arrays of bbhx_hip_InterpTDI on the device (the reference's Python forms
+ * them with searchsorted, binary by binary, waveformbuild.py:139-172). freqs (B, M,
+ * length) sparse grids, dataFreqs (data_length) ascending. interp_bands: band (B, 2) =
+ * [start, end) of the data grid that a binary's grids cover (entries above the
+ * least and up to the greatest sparse frequency), off (B) the bins of the
+ * bands before it. interp_segments: inds, (M, end - start) per binary at off[b] * M, the
+ * spline segment of each bin; max_len the longest band. fill_bands: out (B, 3,
+ * data_length) complex, the templates ((3, end - start) per binary at 3 * off[b]) on
+ * their bands and zero elsewhere. */
+int bbhx_hip_interp_bands(int* band, int64_t* off, const double* freqs, const double* dataFreqs, int length,
+                          int data_length, int numBinAll, int numModes, void* stream);
+int bbhx_hip_interp_segments(int* inds, const int* band, const int64_t* off, const double* freqs,
+                             const double* dataFreqs, int length, int max_len, int numBinAll, int numModes,
+                             void* stream);
+int bbhx_hip_fill_bands(double* out, const double* templates, const int* band, const int64_t* off, int data_length,
+                        int numBinAll, void* stream);
+
 /* Noise PSDs (3, n) of the A, E and T channels at n device frequencies: test-mass
  * acceleration acc (m s^-2 Hz^-1/2, shaped at 0.4 and 8 mHz), optical metrology oms
  * (m Hz^-1/2, shaped at 2 mHz), equal arms of armlength metres, first-generation
