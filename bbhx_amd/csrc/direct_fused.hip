@@ -1167,60 +1167,60 @@ __global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void
         Ya[p * NQ + adj_q(q)] = yb[q] - cy[q] + (i > 0 ? sh[q * T + t - 1] : 0.0);
 }
 
-// Knot-level contraction: one wavefront per (binary, mode), lane per knot; the
+// Knot-level contraction, a workgroup per (binary, mode) and GRAD_T knots; the
 // knot-value adjoints of A, phase and T weight the waveform's and response's
 // tangents at the knot's frequency (grad_point_core, no window rule: the
-// window acts on the dense bins). partial[(b M + m) 11 + p].
-__global__ __launch_bounds__(64) void k_dirg_knots(double* __restrict__ gpart, const gradk::GradRec* __restrict__ grecs,
-                                                   const double* __restrict__ Ya, const double* __restrict__ X,
-                                                   const long* __restrict__ off, const int* __restrict__ len,
-                                                   const double* __restrict__ params, int B, int M,
-                                                   resp::OrbitTab orb, int TDItag, int rescaled, int tdi2,
-                                                   double initial_t_val)
+// window acts on the dense bins). partial[((b M + m) nc + chunk) 11 + p].
+__global__ __launch_bounds__(gradk::GRAD_T) __attribute__((amdgpu_waves_per_eu(2))) void k_dirg_knots(
+    double* __restrict__ gpart, const gradk::GradRec* __restrict__ grecs, const double* __restrict__ Ya,
+    const double* __restrict__ X, const long* __restrict__ off, const int* __restrict__ len,
+    const double* __restrict__ params, int B, int M, int nc, resp::OrbitTab orb, int TDItag, int rescaled, int tdi2,
+    double initial_t_val)
 {
-    const int bm = blockIdx.x;
+    __shared__ gradk::GradShared sh;
+    const int bm = blockIdx.x / nc, chunk = blockIdx.x % nc;
     const int b = bm / M, m = bm % M;
+    const int n = len[b], i = chunk * gradk::GRAD_T + threadIdx.x;
+    if (chunk * gradk::GRAD_T >= n) return;
     Window win;
     win.t_ref = params[P_TREF * B + b];
     win.ts = 0.0;
     win.te = 0.0;
     win.dt_shift = win.t_ref - initial_t_val;
     const double dist = params[P_DIST * B + b];
-    const gradk::GradRec& G = grecs[bm];
-    const int n = len[b];
-    const long base = off[b];
-    __shared__ double2 tab[129];
-    etab_to_lds(tab);
-    __syncthreads();
+    const gradk::GradRec& G = gradk::grad_stage(sh, grecs + bm);
     double acc[gradk::NGRAD];
     for (int p = 0; p < gradk::NGRAD; p++) acc[p] = 0.0;
-    for (int i = threadIdx.x; i < n; i += 64) {
-        const long rec = (base + i) * M + m;
+    if (i < n) {
+        const long rec = (off[b] + i) * M + m;
         const double* y = Ya + rec * NQ;
-        const double aA = y[0], aPh = y[1];
-        cd Wt[3];
-        for (int c = 0; c < 3; c++) Wt[c] = mk(y[3 + 2 * c], -y[4 + 2 * c]);
         auto weights = [&](const cd*, cd, double, cd W[3], double& a_A, double& a_Ph) {
-            for (int c = 0; c < 3; c++) W[c] = Wt[c];
-            a_A = aA;
-            a_Ph = aPh;
+            for (int c = 0; c < 3; c++) W[c] = mk(y[3 + 2 * c], -y[4 + 2 * c]);
+            a_A = y[0];
+            a_Ph = y[1];
         };
-        gradk::grad_point_core(G, orb, X[rec], win, false, weights, TDItag, rescaled, tdi2, dist, acc, tab);
+        gradk::grad_point_core(G, orb, X[rec], win, false, weights, TDItag, rescaled, tdi2, dist, acc, sh.tab,
+                               sh.tan + threadIdx.x, blockDim.x);
     }
-    for (int p = 0; p < gradk::NGRAD; p++) acc[p] = wsum(acc[p]);
-    if (threadIdx.x == 0)
-        for (int p = 0; p < gradk::NGRAD; p++) gpart[(long)bm * gradk::NGRAD + p] = acc[p];
+    gradk::grad_sum(sh, acc, gpart + (long)blockIdx.x * gradk::NGRAD);
 }
 
-// grad[p B + b] = sum over modes, in mode order
-__global__ void k_dirg_reduce(double* __restrict__ grad, const double* __restrict__ gpart, int B, int M)
+// grad[p B + b] = sum over the modes and their chunks: one wavefront per binary
+__global__ __launch_bounds__(64) void k_dirg_reduce(double* __restrict__ grad, const double* __restrict__ gpart, const int* __restrict__ len,
+                              int B, int M, int nc)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= B * gradk::NGRAD) return;
-    const int p = t / B, b = t % B;
-    double s = 0.0;
-    for (int m = 0; m < M; m++) s += gpart[((long)b * M + m) * gradk::NGRAD + p];
-    grad[(long)p * B + b] = s;
+    const int b = blockIdx.x, n = gradk::grad_chunks(len[b]);
+    double acc[gradk::NGRAD];
+    for (int p = 0; p < gradk::NGRAD; p++) acc[p] = 0.0;
+    for (int e = threadIdx.x; e < M * n; e += 64) {
+        const int m = e / n, c = e - m * n;
+        const double* g = gpart + (((long)b * M + m) * nc + c) * gradk::NGRAD;
+        for (int p = 0; p < gradk::NGRAD; p++) acc[p] += g[p];
+    }
+    for (int p = 0; p < gradk::NGRAD; p++) {
+        const double v = wsum(acc[p]);
+        if (threadIdx.x == 0) grad[(long)p * B + b] = v;
+    }
 }
 
 template <class T>
@@ -1345,7 +1345,7 @@ extern "C" long bbhx_hip_direct_plan_bytes(const bbhx_direct_plan* p)
     const long SM = p->S * p->M;
     long bytes = SM * 8 * (1 + RS + NQ) + (long)p->B * p->M * (sizeof(FusedRec) + 16) + p->max_items * 36 + p->B * 24 +
                  4L * (p->max_chunks + 1);
-    if (p->Yadj) bytes += SM * 8 * NA + (long)p->B * p->M * (sizeof(bbhx::gradk::GradRec) + 8 * bbhx::gradk::NGRAD);
+    if (p->Yadj) bytes += SM * 8 * NA + (long)p->B * p->M * (sizeof(bbhx::gradk::GradRec) + 8 * bbhx::gradk::NGRAD * bbhx::gradk::grad_chunks(p->Lmax));
     return bytes;
 }
 
@@ -1436,10 +1436,11 @@ int direct_launch(bbhx_direct_plan* p, double* d_h, double* h_h, double* grad, i
         // the knot values' adjoints take the place of the values, which are not read again
         hipLaunchKernelGGL(k_dirg_spline_adj, dim3((unsigned)((long)B * M * nbmax)), dim3(SPL_T), 0, st, p->Yc,
                            p->Yadj, p->X, p->off, p->len, M, nbmax);
-        hipLaunchKernelGGL(k_dirg_knots, dim3(B * M), dim3(64), 0, st, p->gpart, p->grecs, p->Yc, p->X, p->off,
-                           p->len, params, B, M, orb, TDItag, rescaled, tdi2, initial_t_val);
-        hipLaunchKernelGGL(k_dirg_reduce, dim3(ceil_div((long)B * gradk::NGRAD, 256)), dim3(256), 0, st, grad,
-                           p->gpart, B, M);
+        const int nc = gradk::grad_chunks(p->Lmax);
+        hipLaunchKernelGGL(k_dirg_knots, dim3((unsigned)((long)B * M * nc)), dim3(gradk::grad_threads(p->Lmax)), 0, st,
+                           p->gpart, p->grecs, p->Yc, p->X, p->off, p->len, params, B, M, nc, orb, TDItag, rescaled, tdi2, initial_t_val);
+        hipLaunchKernelGGL(k_dirg_reduce, dim3(B), dim3(64), 0, st, grad,
+                           p->gpart, p->len, B, M, nc);
     }
     if (timed) (void)hipEventRecord(ev[2], st);
     return hipGetLastError() == hipSuccess ? OK : ERR_LAUNCH;
@@ -1476,7 +1477,7 @@ extern "C" int bbhx_hip_direct_plan_enable_grad(bbhx_direct_plan* p)
     bool ok = true;
     p->Yadj = dalloc<double>((size_t)p->S * p->M * NA, ok);
     p->grecs = dalloc<gradk::GradRec>((size_t)p->B * p->M, ok);
-    p->gpart = dalloc<double>((size_t)p->B * p->M * gradk::NGRAD, ok);
+    p->gpart = dalloc<double>((size_t)p->B * p->M * gradk::NGRAD * gradk::grad_chunks(p->Lmax), ok);
     if (!ok) {
         for (void* b : {(void*)p->Yadj, (void*)p->grecs, (void*)p->gpart})
             if (b) (void)hipFree(b);

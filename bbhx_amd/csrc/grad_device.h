@@ -509,7 +509,7 @@ __device__ inline bool grad_resp_part(const GradResp& R, const resp::OrbitTab& o
             dsm[j] = dsinc(am, cos_m, sm[j]);
             dsp[j] = dsinc(ap, cos_p, sp[j]);
         }
-    }
+        }
     // link L = 0: pair (23, 32) with e23; L = 1: (31, 13) with e31; L = 2: (12, 21) with e12
     const int ka[3] = {1, 2, 0}, kb[3] = {2, 0, 1};
     cd eL[3], gL[3];
@@ -610,7 +610,7 @@ __device__ inline bool grad_resp_part(const GradResp& R, const resp::OrbitTab& o
         Skv += ixeB * (kn[L] * vn[L]);
         Tu += egC * un[L] + egB * (up[ka[L]] + up[kb[L]]);
         Tv += egC * vn[L] + egB * (vp[ka[L]] + vp[kb[L]]);
-    }
+        }
     // Re of: Spsi = 2 (Yp SV - Yc SU), Sa = Tu - 2 (Yp Sku + Yc Skv),
     // Sb = Tv + 2 (Yp Skv - Yc Sku), Scos = dYp SU + dYc SV
     const double Spsi = 2.0 * (re_mul(R.Yp, SV) - re_mul(R.Yc, SU));
@@ -633,20 +633,84 @@ __device__ inline bool grad_resp_part(const GradResp& R, const resp::OrbitTab& o
     return true;
 }
 
+// The kernels that sum grad_point_core over the points of one (binary, mode) take a
+// workgroup of up to GRAD_T lanes per GRAD_T points, one point per lane.
+//
+// Bound by FP64 issue and latency at two wavefronts per SIMD. A loop over points in a lane
+// keeps the point-independent constants and record entries in registers, 460 VGPRs and
+// one wavefront per SIMD; straight-line code with the record in LDS needs 290, 256 with
+// a few spills. 1024 templates x 6 modes x 256 nodes: 272 -> 196 us (256 VGPRs for the
+// loop: 484; the straight line at one wavefront per SIMD: 298).
+constexpr int GRAD_T = 256;
+constexpr int GRAD_STASH = 3 * NI;
+__host__ __device__ inline int grad_chunks(int n) { return (n + GRAD_T - 1) / GRAD_T; }
+inline int grad_threads(int n) { return n < GRAD_T ? (n + 63) / 64 * 64 : GRAD_T; }
+
+struct GradShared {
+    double2 tab[129];
+    double rec[sizeof(GradRec) / sizeof(double)];
+    double tan[GRAD_STASH * GRAD_T];
+    double acc[NGRAD][GRAD_T / 64];
+};
+
+// the record and the e^{i theta} table into LDS
+__device__ inline const GradRec& grad_stage(GradShared& s, const GradRec* __restrict__ g)
+{
+    fused::etab_to_lds(s.tab);
+    const double* src = reinterpret_cast<const double*>(g);
+    for (int i = threadIdx.x; i < (int)(sizeof(GradRec) / sizeof(double)); i += blockDim.x) s.rec[i] = src[i];
+    __syncthreads();
+    return *reinterpret_cast<const GradRec*>(s.rec);
+}
+
+// out[p] = the workgroup's sum of acc[p], wavefront by wavefront
+__device__ inline void grad_sum(GradShared& s, const double acc[NGRAD], double* __restrict__ out)
+{
+    for (int p = 0; p < NGRAD; p++) {
+        const double v = fused::wsum(acc[p]);
+        if ((threadIdx.x & 63) == 0) s.acc[p][threadIdx.x >> 6] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x >= NGRAD) return;
+    double v = s.acc[threadIdx.x][0];
+    for (int w = 1; w < (int)blockDim.x >> 6; w++) v += s.acc[threadIdx.x][w];
+    out[threadIdx.x] = v;
+}
+
 // Both parts at one (frequency, mode): the waveform's values from the record
-// with tangents.
+// with tangents. The tangents wait in the lane's column of 'stash' (LDS, GRAD_STASH
+// rows of 'pitch') while the response is evaluated, which keeps both parts within 256
+// VGPRs.
 template <class Weights, class E>
 __device__ inline void grad_point_core(const GradRec& G, const resp::OrbitTab& o, double f, const fused::Window& win,
                                        bool use_window, Weights weights, int TDItag, int rescaled, int tdi2,
-                                       double dist, double acc[NGRAD], const E* __restrict__ tab)
+                                       double dist, double acc[NGRAD], const E* __restrict__ tab, double* stash,
+                                       int pitch)
 {
-    D4 A, Ph, Tf;
-    phm_eval_tan(G.w, f, A, Ph, Tf);
+    double Av, Phv, Tfv;
+    {
+        D4 A, Ph, Tf;
+        phm_eval_tan(G.w, f, A, Ph, Tf);
+        Av = A.v;
+        Phv = Ph.v;
+        Tfv = Tf.v;
+#pragma unroll
+        for (int k = 0; k < NI; k++) {
+            stash[3 * k * pitch] = Tf.d[k];
+            stash[(3 * k + 1) * pitch] = A.d[k];
+            stash[(3 * k + 2) * pitch] = Ph.d[k];
+        }
+    }
+    // keeps the tangents in the stash instead of the registers they came from
+    asm volatile("" ::: "memory");
     double a_t, a_A, a_phi;
-    if (!grad_resp_part(G.s, o, f, A.v, Ph.v, Tf.v, win, use_window, weights, TDItag, rescaled, tdi2, dist, acc, tab,
-                        a_t, a_A, a_phi))
+    if (!grad_resp_part(G.s, o, f, Av, Phv, Tfv, win, use_window, weights, TDItag, rescaled, tdi2, dist, acc, tab, a_t,
+                        a_A, a_phi))
         return;
-    for (int k = 0; k < NI; k++) acc[k] += a_t * Tf.d[k] + a_A * A.d[k] + a_phi * Ph.d[k];
+#pragma unroll
+    for (int k = 0; k < NI; k++)
+        acc[k] += a_t * stash[3 * k * pitch] + a_A * stash[(3 * k + 1) * pitch] +
+                  a_phi * stash[(3 * k + 2) * pitch];
 }
 
 

@@ -126,19 +126,20 @@ __device__ inline void adjoint_weights(cd* gs, const cd* rs, const NodeW* __rest
 // X = T A e^{i phi}), so that W_c = g_c A e^{i phi}, a_A = Re S, a_phi = -A Im S
 // with S = sum_c g_c T_c e^{i phi}.
 __device__ inline void grad_point(const GradRec& G, const resp::OrbitTab& o, double f, const Window& win,
-                                  const cd g[3], int TDItag, int rescaled, int tdi2, double dist, double acc[NGRAD],
-                                  const double2* tab)
+                                  const cd* __restrict__ gn, int K, int TDItag, int rescaled, int tdi2, double dist, double acc[NGRAD],
+                                  const double2* tab, double* stash, int pitch)
 {
     auto weights = [&](const cd T[3], cd E1, double Av, cd W[3], double& aA, double& aPh) {
         cd S1 = mk(0.0, 0.0);
         for (int c = 0; c < 3; c++) {
-            S1 += g[c] * T[c] * E1;
-            W[c] = (g[c] * E1) * Av;
+            const cd g = gn[c * K];
+            S1 += g * T[c] * E1;
+            W[c] = (g * E1) * Av;
         }
         aA = S1.re;
         aPh = -Av * S1.im;
     };
-    grad_point_core(G, o, f, win, true, weights, TDItag, rescaled, tdi2, dist, acc, tab);
+    grad_point_core(G, o, f, win, true, weights, TDItag, rescaled, tdi2, dist, acc, tab, stash, pitch);
 }
 
 // Forward pass and adjoint weights of one template (one wavefront): d_h, h_h
@@ -178,17 +179,16 @@ __global__ __launch_bounds__(64 * MAX_RESIDUAL_WAVES) __attribute__((amdgpu_wave
     }
 }
 
-// Gradient contributions of one (template, mode): one wavefront, lane l owns
-// nodes l, l+64, ... (the record is the same for the whole wavefront);
-// partial[(b * M + m) * 11 + p].
-__global__ __launch_bounds__(64) void k_grad_points(double* __restrict__ partial, const GradRec* __restrict__ grecs,
-                                                    const cd* __restrict__ gw, const double* __restrict__ params,
-                                                    const double* __restrict__ t_start,
-                                                    const double* __restrict__ t_end, int B, int M,
-                                                    const double* __restrict__ freqs, int K, resp::OrbitTab orb,
-                                                    int TDItag, int rescaled, int tdi2, double initial_t_val)
+// Gradient contributions of one (template, mode) and chunk of up to GRAD_T nodes:
+// partial[((b * M + m) * chunks + chunk) * 11 + p].
+__global__ __launch_bounds__(GRAD_T) __attribute__((amdgpu_waves_per_eu(2))) void k_grad_points(
+    double* __restrict__ partial, const GradRec* __restrict__ grecs, const cd* __restrict__ gw,
+    const double* __restrict__ params, const double* __restrict__ t_start, const double* __restrict__ t_end, int B,
+    int M, const double* __restrict__ freqs, int K, resp::OrbitTab orb, int TDItag, int rescaled, int tdi2,
+    double initial_t_val)
 {
-    const int bm = blockIdx.x;
+    __shared__ GradShared sh;
+    const int chunks = grad_chunks(K), bm = blockIdx.x / chunks, chunk = blockIdx.x % chunks;
     const int b = bm / M;
     Window win;
     win.t_ref = params[P_TREF * B + b];
@@ -196,30 +196,24 @@ __global__ __launch_bounds__(64) void k_grad_points(double* __restrict__ partial
     win.te = t_end[b];
     win.dt_shift = win.t_ref - initial_t_val;
     const double dist = params[P_DIST * B + b];
-    const GradRec& G = grecs[bm];
-    const cd* g_b = gw + (long)b * 3 * K;
-    __shared__ double2 tab[129];
-    etab_to_lds(tab);
-    __syncthreads();
+    const GradRec& G = grad_stage(sh, grecs + bm);
     double acc[NGRAD];
     for (int p = 0; p < NGRAD; p++) acc[p] = 0.0;
-    for (int j = threadIdx.x; j < K; j += 64) {
-        const cd g[3] = {g_b[j], g_b[K + j], g_b[2 * K + j]};
-        grad_point(G, orb, freqs[j], win, g, TDItag, rescaled, tdi2, dist, acc, tab);
-    }
-    for (int p = 0; p < NGRAD; p++) acc[p] = wsum(acc[p]);
-    if (threadIdx.x == 0)
-        for (int p = 0; p < NGRAD; p++) partial[(long)bm * NGRAD + p] = acc[p];
+    const int j = chunk * GRAD_T + threadIdx.x;
+    if (j < K)
+        grad_point(G, orb, freqs[j], win, gw + (long)b * 3 * K + j, K, TDItag, rescaled, tdi2, dist, acc, sh.tab,
+                   sh.tan + threadIdx.x, blockDim.x);
+    grad_sum(sh, acc, partial + (long)blockIdx.x * NGRAD);
 }
 
-// grad[p * B + b] = sum over modes, in mode order
-__global__ void k_grad_reduce(double* __restrict__ grad, const double* __restrict__ partial, int B, int M)
+// grad[p * B + b] = sum over the modes' chunks, in order
+__global__ void k_grad_reduce(double* __restrict__ grad, const double* __restrict__ partial, int B, int n)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= B * NGRAD) return;
     const int p = t / B, b = t % B;
     double s = 0.0;
-    for (int m = 0; m < M; m++) s += partial[((long)b * M + m) * NGRAD + p];
+    for (int m = 0; m < n; m++) s += partial[((long)b * n + m) * NGRAD + p];
     grad[(long)p * B + b] = s;
 }
 
@@ -272,10 +266,10 @@ extern "C" int bbhx_hip_hdyn_fused_grad(double* d_h, double* h_h, double* grad, 
     FusedRec* recs = reinterpret_cast<FusedRec*>(fws);
     NodeW* nw = reinterpret_cast<NodeW*>(fws + sizeof(FusedRec) * (size_t)nrec);
     GradRec* grecs = static_cast<GradRec*>(workspace_get(WS_GRAD, sizeof(GradRec) * (size_t)nrec, st));
-    // adjoint weights (B, 3, K) complex, then partial gradients (B, M, 11)
+    // adjoint weights (B, 3, K) complex, then partial gradients (B, M, chunks, 11)
     const size_t gw_bytes = sizeof(cd) * 3 * (size_t)K * numBinAll;
     char* scratch = static_cast<char*>(
-        workspace_get(WS_GRAD_AUX, gw_bytes + sizeof(double) * NGRAD * (size_t)nrec, st));
+        workspace_get(WS_GRAD_AUX, gw_bytes + sizeof(double) * NGRAD * (size_t)nrec * grad_chunks(K), st));
     if (!fws || !grecs || !scratch) return ERR_ALLOC;
     cd* gw = reinterpret_cast<cd*>(scratch);
     double* partial = reinterpret_cast<double*>(scratch + gw_bytes);
@@ -304,10 +298,11 @@ extern "C" int bbhx_hip_hdyn_fused_grad(double* d_h, double* h_h, double* grad, 
                        sizeof(cd) * 3 * (size_t)K, st, d_h, h_h, logL, d_d, gw, recs, params, t_start, t_end,
                        numBinAll, ml, numModes, freqs, nw, K, orb, TDItag, rescaled, tdi2, initial_t_val);
     if (hipStreamWaitEvent(st, side->join, 0) != hipSuccess) return ERR_LAUNCH;
-    hipLaunchKernelGGL(k_grad_points, dim3(nrec), dim3(64), 0, st, partial, grecs, gw, params, t_start, t_end,
+    const int chunks = grad_chunks(K);
+    hipLaunchKernelGGL(k_grad_points, dim3((unsigned)(nrec * (long)chunks)), dim3(grad_threads(K)), 0, st, partial, grecs, gw, params, t_start, t_end,
                        numBinAll, numModes, freqs, K, orb, TDItag, rescaled, tdi2, initial_t_val);
     hipLaunchKernelGGL(k_grad_reduce, dim3(ceil_div((long)numBinAll * NGRAD, 256)), dim3(256), 0, st, grad, partial,
-                       numBinAll, numModes);
+                       numBinAll, numModes * chunks);
     if (timed) (void)hipEventRecord(ev[2], st);
     return hipGetLastError() == hipSuccess ? OK : ERR_LAUNCH;
 }
