@@ -200,74 +200,148 @@ __device__ inline void node_weight(NodeW* __restrict__ nw, const double* __restr
 // whole wavefront is there, the pair is evaluated once: one PhenomHM
 // evaluation, the second mode's factor, and one response evaluation with the
 // two modes' Y factors weighted by their amplitudes.
+//
+// node_residual: r (out) of the node at frequency f (1 / h0: q, channel c's at q[c K]).
+// The modes k0 + kl, k0 + kd + kl, ... (k0, kd of the wavefront, kl of the lane); kd = 1:
+// all of them, in pairs where they go. One body for both, as its code, some 20 KB, is
+// fetched anew for each launch: with a second copy for kd > 1 16 templates took 36 us.
 template <class E>
-__device__ inline void residuals(cd* rs, const FusedRec* __restrict__ rb, const ModeList& ml, int M,
+__device__ inline void node_residual(cd out[3], const FusedRec* __restrict__ rb, int pairs, int M, int k0, int kd,
+                                     int kl, const Window& win, double f, const NodeW* __restrict__ q, int K,
+                                     const resp::OrbitTab& orb, int TDItag, int rescaled, int tdi2,
+                                     const E* __restrict__ tab)
+{
+    const resp::NodeResp nr = resp::resp_node(orb, f);
+    cd S[6];
+    for (int k = 0; k < 6; k++) S[k] = mk(0.0, 0.0);
+    for (int k = k0; k < M; k += kd) {
+        const FusedRec& r = rb[min(k + kl, M - 1)];
+        double amp, phase, tf, ad;
+        phm::phm_eval(r.w, f, amp, phase, tf, &ad);
+        // phenomhm.py:487-507: phase += 2 pi f (t_ref - t0); tf += t_ref
+        phase = phase + ((f * win.dt_shift) * 2) * PI;
+        tf = tf + win.t_ref;
+        cd G[6];
+        double dphi;
+        if (kd == 1 && (pairs >> k & 1)) {
+            const FusedRec& r2 = rb[k + 1];
+            const double Mf = f * r.w.M_sec;
+            const bool same = Mf <= fmin(fmin(r.w.fi, r2.w.fi), fmin(r.w.amp_fi, r2.w.amp_fi)) &&
+                              r.w.ai * Mf < phm::PHI_JOIN_INS;
+            if (__all(same)) {
+                const double amp2 = (ad * phm::hm_amp_factor(r2.w, Mf, r2.w.amp_Ai * Mf)) * r2.w.amp_scale;
+                const cd Yp = r.s.Yp * amp + r2.s.Yp * amp2, Yc = r.s.Yc * amp + r2.s.Yc * amp2;
+                resp::resp_links_y(r.s, Yp, Yc, orb, nr, f, tf, G, dphi, tab);
+                if (in_window(win, tf)) {
+                    const cd e = cexpi_tab(phase + dphi, tab);
+                    for (int i = 0; i < 6; i++) S[i] += G[i] * e;
+                }
+                k++;
+                continue;
+            }
+        }
+        resp::resp_links(r.s, orb, nr, f, tf, G, dphi, tab);
+        // The waveform phase multiplies the link terms after they are
+        // formed, not inside their exponentials: the TDI combination takes
+        // differences of nearly equal link terms at low frequency, so the
+        // link terms' relative phases must not carry the rounding of this
+        // large phase (1e4-1e7 rad). Modes outside the observation window
+        // contribute nothing (WaveformBuild.cu:50).
+        if (in_window(win, tf) && k + kl < M) {
+            const cd ap = amp * cexpi_tab(phase + dphi, tab);
+            for (int i = 0; i < 6; i++) S[i] += G[i] * ap;
+        }
+    }
+    cd T[3];
+    resp::tdi_combine(S, nr, TDItag, rescaled, tdi2, T);
+    // r = h / h0 with h = conj(T) (likelihood.py:603), as h (1 / h0)
+    for (int c = 0; c < 3; c++) out[c] = k0 + kl < M ? conj(T[c]) * q[c * K].q : mk(0.0, 0.0);
+}
+
+// Whether the R nodes left over are too many for their modes to be spread over T lanes
+__host__ __device__ inline bool residual_full(int R, int T) { return R > 32 && 2 * ((R + 63) & ~63) > T; }
+
+// Groups of wavefronts they are spread over, within the LDS of 1024 nodes
+__host__ __device__ inline int residual_groups(int R, int T, int K)
+{
+    const int fit = 1 + (1024 - K) / R, ng = T / ((R + 63) & ~63);
+    return ng < fit ? ng : fit;
+}
+
+// A pass takes as many nodes as the workgroup has lanes. Nodes left over for at most half
+// of them are evaluated with their modes spread over the other lanes, and the
+// (linear) residuals added: over the lanes of one wavefront, by exchanges, if at most 32
+// nodes are left, else over its wavefronts, through 'part' (LDS, see residual_lds).
+// 20011 templates of 257 nodes, where the last pass held one: 1155 -> 1016 us; 16 of
+// 128 nodes, two wavefronts' worth on eight: 27.9 -> 17.7 us. SPLIT: whether there
+// are such nodes (residual_split); the kernel that does not expect them is 3% faster
+// at 4096 templates of 128 nodes (117 against 120 us).
+template <bool SPLIT, class E>
+__device__ inline void residuals(cd* rs, cd* part, const FusedRec* __restrict__ rb, const ModeList& ml, int M,
                                  const Window& win, const double* __restrict__ freqs, const NodeW* __restrict__ nw,
                                  int K, const resp::OrbitTab& orb, int TDItag, int rescaled, int tdi2,
                                  const E* __restrict__ tab)
 {
-    for (int j = threadIdx.x; j < K; j += blockDim.x) {
-        const double f = freqs[j];
-        const resp::NodeResp nr = resp::resp_node(orb, f);
-        cd S[6];
-        for (int k = 0; k < 6; k++) S[k] = mk(0.0, 0.0);
-        for (int k = 0; k < M; k++) {
-            const FusedRec& r = rb[ml.order[k]];
-            double amp, phase, tf, ad;
-            phm::phm_eval(r.w, f, amp, phase, tf, &ad);
-            // phenomhm.py:487-507: phase += 2 pi f (t_ref - t0); tf += t_ref
-            phase = phase + ((f * win.dt_shift) * 2) * PI;
-            tf = tf + win.t_ref;
-            cd G[6];
-            double dphi;
-            if (ml.pair[k]) {
-                const FusedRec& r2 = rb[ml.order[k + 1]];
-                const double Mf = f * r.w.M_sec;
-                const bool same = Mf <= fmin(fmin(r.w.fi, r2.w.fi), fmin(r.w.amp_fi, r2.w.amp_fi)) &&
-                                  r.w.ai * Mf < phm::PHI_JOIN_INS;
-                if (__all(same)) {
-                    const double amp2 = (ad * phm::hm_amp_factor(r2.w, Mf, r2.w.amp_Ai * Mf)) * r2.w.amp_scale;
-                    const cd Yp = r.s.Yp * amp + r2.s.Yp * amp2, Yc = r.s.Yc * amp + r2.s.Yc * amp2;
-                    resp::resp_links_y(r.s, Yp, Yc, orb, nr, f, tf, G, dphi, tab);
-                    if (in_window(win, tf)) {
-                        const cd e = cexpi_tab(phase + dphi, tab);
-                        for (int q = 0; q < 6; q++) S[q] += G[q] * e;
-                    }
-                    k++;
-                    continue;
-                }
-            }
-            resp::resp_links(r.s, orb, nr, f, tf, G, dphi, tab);
-            // The waveform phase multiplies the link terms after they are
-            // formed, not inside their exponentials: the TDI combination takes
-            // differences of nearly equal link terms at low frequency, so the
-            // link terms' relative phases must not carry the rounding of this
-            // large phase (1e4-1e7 rad). Modes outside the observation window
-            // contribute nothing (WaveformBuild.cu:50).
-            if (in_window(win, tf)) {
-                const cd ap = amp * cexpi_tab(phase + dphi, tab);
-                for (int k = 0; k < 6; k++) S[k] += G[k] * ap;
-            }
+    const int t = threadIdx.x, T = blockDim.x;
+    int pairs = 0;
+    for (int k = 0; k < M; k++) pairs |= ml.pair[k] << k;
+    if constexpr (!SPLIT) {
+        for (int j = t; j < K; j += T) {
+            cd r[3];
+            node_residual(r, rb, pairs, M, 0, 1, 0, win, freqs[j], nw + j, K, orb, TDItag, rescaled, tdi2, tab);
+            for (int c = 0; c < 3; c++) rs[c * K + j] = r[c];
         }
-        cd T[3];
-        resp::tdi_combine(S, nr, TDItag, rescaled, tdi2, T);
-        // r = h / h0 with h = conj(T) (likelihood.py:603), as h (1 / h0)
-        for (int c = 0; c < 3; c++) rs[c * K + j] = conj(T[c]) * nw[c * K + j].q;
+        return;
+    }
+    for (int base = 0; base < K; base += T) {
+        const int R = K - base;
+        const bool full = residual_full(R, T), one = !full && R <= 32;
+        // lanes per group of modes, this lane's group and node, the number of groups
+        int rows = T, ng = 1;
+        if (one) {
+            rows = R > 1 ? 1 << (32 - __builtin_clz(R - 1)) : 1;
+            ng = 64 / rows;
+        } else if (!full) {
+            rows = (R + 63) & ~63;
+            ng = residual_groups(R, T, K);
+        }
+        const int g = t / rows, n = t - g * rows, j = base + min(n, R - 1);
+        cd r[3];
+        if (one ? t < 64 : g < ng && (n < R || !full))
+            node_residual(r, rb, pairs, M, one ? 0 : __builtin_amdgcn_readfirstlane(g), ng, one ? g : 0, win, freqs[j], nw + j, K, orb, TDItag, rescaled, tdi2, tab);
+        if (one) {
+            if (t < 64)
+                for (int o = rows; o < 64; o <<= 1)
+                    for (int c = 0; c < 3; c++) r[c] += mk(__shfl_xor(r[c].re, o, 64), __shfl_xor(r[c].im, o, 64));
+        } else if (ng > 1) {
+            if (g > 0 && g < ng && n < R)
+                for (int c = 0; c < 3; c++) part[((g - 1) * 3 + c) * R + n] = r[c];
+            __syncthreads();
+            if (t < R)
+                for (int i = 1; i < ng; i++)
+                    for (int c = 0; c < 3; c++) r[c] += part[((i - 1) * 3 + c) * R + n];
+        }
+        if (t < R)
+            for (int c = 0; c < 3; c++) rs[c * K + j] = r[c];
     }
 }
 
-// The records of one template copied into LDS ('srec', M of them) by the
+// The records of one template copied into LDS ('srec', M of them, in the order of
+// evaluation) by the
 // threads of a workgroup; a barrier must follow. The residual pass then reads
 // them with LDS loads (wave-uniform addresses, one broadcast each) instead of
 // scalar loads: measured 140 -> 129 us for 4096 templates x 128 nodes (the
 // scalar-load waits per mode, which the SGPR budget serialises, gone). The
 // copy itself costs about 3 us of the kernel at that size (measured by doing
 // it twice).
-__device__ inline void records_to_lds(FusedRec* srec, const FusedRec* __restrict__ rb, int M)
+__device__ inline void records_to_lds(FusedRec* srec, const FusedRec* __restrict__ rb, const ModeList& ml, int M)
 {
-    const double* src = reinterpret_cast<const double*>(rb);
-    double* dst = reinterpret_cast<double*>(srec);
-    for (int i = threadIdx.x; i < (int)(M * sizeof(FusedRec) / sizeof(double)); i += blockDim.x) dst[i] = src[i];
+    constexpr int W = sizeof(FusedRec) / sizeof(double);
+    for (int k = 0; k < M; k++) {
+        const double* src = reinterpret_cast<const double*>(rb + ml.order[k]);
+        double* dst = reinterpret_cast<double*>(srec + k);
+        for (int i = threadIdx.x; i < W; i += blockDim.x) dst[i] = src[i];
+    }
 }
 
 // The e^{i theta} table of cexpi_tab copied from constant memory into LDS
@@ -321,15 +395,34 @@ __device__ inline void node_sums(const cd* rs, const NodeW* __restrict__ nw, int
 
 // Wavefronts per template of the residual pass (workgroup of 64 x that many
 // threads): enough for about 2048 wavefronts in the launch (two per SIMD of
-// MI355X's 1024), at most one per 64 nodes and at most MAX_RESIDUAL_WAVES.
+// MI355X's 1024), at most one per mode and 64 nodes and at most MAX_RESIDUAL_WAVES.
 // The forward and the gradient's weights pass use the same count, so their
 // sums agree bit for bit.
-inline int residual_waves(int B, int K)
+inline int residual_waves(int B, int K, int M)
 {
     int nw = (2048 + B - 1) / B;
-    nw = nw < (K + 63) / 64 ? nw : (K + 63) / 64;
+    const int most = K > 32 ? (K + 63) / 64 * M : 1;
+    nw = nw < most ? nw : most;
     nw = nw < MAX_RESIDUAL_WAVES ? nw : MAX_RESIDUAL_WAVES;
     return nw > 1 ? nw : 1;
+}
+
+// Whether the last pass of that many wavefronts spreads its modes over the lanes
+inline bool residual_split(int waves, int K)
+{
+    int R = K;
+    while (residual_full(R, 64 * waves)) R -= 64 * waves;
+    return R > 0;
+}
+
+// LDS of the residual pass with that many wavefronts: rs, then part
+inline size_t residual_lds(int waves, int K)
+{
+    const int T = 64 * waves;
+    int R = K;
+    while (residual_full(R, T)) R -= T;
+    const int part = R > 32 ? (residual_groups(R, T, K) - 1) * R : 0;
+    return sizeof(cd) * 3 * (size_t)(K + part);
 }
 
 // Host helpers shared by the fused entry points (hdyn_fused.hip): three timing

@@ -57,7 +57,7 @@ __global__ __launch_bounds__(64) void k_fused_setup(FusedRec* __restrict__ recs,
     setup_split(recs, params, B, modes, M, qnm, table_len, dspin);
 }
 
-// One workgroup per template, of residual_waves(B, K) wavefronts (one at large
+// One workgroup per template, of residual_waves wavefronts (one at large
 // batches; several at small ones, so that the chip still holds two per SIMD).
 // Dynamic LDS holds the residuals r[3][K] of this template; static LDS its
 // records and the e^{i theta} table (the records read with LDS broadcast loads:
@@ -65,6 +65,7 @@ __global__ __launch_bounds__(64) void k_fused_setup(FusedRec* __restrict__ recs,
 // The register budget is capped so that two wavefronts share each SIMD (256
 // VGPRs each, no spills); capped at three per SIMD (168 VGPRs) values spill and
 // it takes twice as long.
+template <bool SPLIT>
 __global__ __launch_bounds__(64 * MAX_RESIDUAL_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void k_fused_eval(
     double* __restrict__ d_h, double* __restrict__ h_h, double* __restrict__ ll, double d_d,
     const FusedRec* __restrict__ recs, const double* __restrict__ params, const double* __restrict__ t_start,
@@ -82,9 +83,9 @@ __global__ __launch_bounds__(64 * MAX_RESIDUAL_WAVES) __attribute__((amdgpu_wave
     win.te = t_end[b];
     win.dt_shift = win.t_ref - initial_t_val;
     __shared__ FusedRec srec[MAX_MODES];
-    records_to_lds(srec, recs + (long)b * M, M);
+    records_to_lds(srec, recs + (long)b * M, ml, M);
     __syncthreads();
-    residuals(rs, srec, ml, M, win, freqs, nw, K, orb, TDItag, rescaled, tdi2, tab);
+    residuals<SPLIT>(rs, rs + 3 * K, srec, ml, M, win, freqs, nw, K, orb, TDItag, rescaled, tdi2, tab);
     __syncthreads();
     double sums[4];
     node_sums(rs, nw, K, sums);
@@ -217,8 +218,8 @@ int hdyn_fused_launch(FusedRec* recs, NodeW* nw, double* d_h, double* h_h, const
                        reinterpret_cast<const cd*>(h0), reinterpret_cast<const cd*>(dataConstants), K, jend);
     if (hipGetLastError() != hipSuccess) return ERR_LAUNCH;
     if (timed) (void)hipEventRecord(ev[1], st);
-    const size_t lds = sizeof(cd) * 3 * (size_t)K;
-    hipLaunchKernelGGL(k_fused_eval, dim3(numBinAll), dim3(64 * residual_waves(numBinAll, K)), lds, st, d_h, h_h,
+    const int waves = residual_waves(numBinAll, K, numModes);
+    hipLaunchKernelGGL(residual_split(waves, K) ? k_fused_eval<true> : k_fused_eval<false>, dim3(numBinAll), dim3(64 * waves), residual_lds(waves, K), st, d_h, h_h,
                        logL, d_d, recs, params, t_start, t_end, numBinAll, ml, numModes, freqs, nw, K, orb, TDItag,
                        rescaled, tdi2, initial_t_val);
     if (timed) (void)hipEventRecord(ev[2], st);

@@ -145,6 +145,7 @@ __device__ inline void grad_point(const GradRec& G, const resp::OrbitTab& o, dou
 // Forward pass and adjoint weights of one template (one wavefront): d_h, h_h
 // as the forward kernel computes them, and gw[(b * 3 + c) * K + j] = the
 // complex weight g of node j, channel c.
+template <bool SPLIT>
 __global__ __launch_bounds__(64 * MAX_RESIDUAL_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void k_grad_weights(
     double* __restrict__ d_h, double* __restrict__ h_h, double* __restrict__ ll, double d_d, cd* __restrict__ gw,
     const FusedRec* __restrict__ recs, const double* __restrict__ params, const double* __restrict__ t_start,
@@ -162,9 +163,9 @@ __global__ __launch_bounds__(64 * MAX_RESIDUAL_WAVES) __attribute__((amdgpu_wave
     win.te = t_end[b];
     win.dt_shift = win.t_ref - initial_t_val;
     __shared__ FusedRec srec[MAX_MODES];
-    records_to_lds(srec, recs + (long)b * M, M);
+    records_to_lds(srec, recs + (long)b * M, ml, M);
     __syncthreads();
-    residuals(rs, srec, ml, M, win, freqs, nw, K, orb, TDItag, rescaled, tdi2, tab);
+    residuals<SPLIT>(rs, rs + 3 * K, srec, ml, M, win, freqs, nw, K, orb, TDItag, rescaled, tdi2, tab);
     __syncthreads();
     double sums[4];
     node_sums(rs, nw, K, sums);
@@ -294,8 +295,8 @@ extern "C" int bbhx_hip_hdyn_fused_grad(double* d_h, double* h_h, double* grad, 
                        reinterpret_cast<const cd*>(h0), reinterpret_cast<const cd*>(dataConstants), K, jend);
     if (hipGetLastError() != hipSuccess) return ERR_LAUNCH;
     if (timed) (void)hipEventRecord(ev[1], st);
-    hipLaunchKernelGGL(k_grad_weights, dim3(numBinAll), dim3(64 * residual_waves(numBinAll, K)),
-                       sizeof(cd) * 3 * (size_t)K, st, d_h, h_h, logL, d_d, gw, recs, params, t_start, t_end,
+    const int waves = residual_waves(numBinAll, K, numModes);
+    hipLaunchKernelGGL(residual_split(waves, K) ? k_grad_weights<true> : k_grad_weights<false>, dim3(numBinAll), dim3(64 * waves), residual_lds(waves, K), st, d_h, h_h, logL, d_d, gw, recs, params, t_start, t_end,
                        numBinAll, ml, numModes, freqs, nw, K, orb, TDItag, rescaled, tdi2, initial_t_val);
     if (hipStreamWaitEvent(st, side->join, 0) != hipSuccess) return ERR_LAUNCH;
     const int chunks = grad_chunks(K);
