@@ -105,6 +105,111 @@ inline int launch_status()
     return e == hipSuccess ? OK : ERR_LAUNCH;
 }
 
+// The glue between the evaluations, one launch each (with tensor operations they are
+// 9, 7 and some 45 launches and three waits of about 20 us each). The products and sums are
+// rounded one by one, as those operations round them.
+
+// The default grid Mf in [10^lo, 10^hi] m / 2 of every (binary, mode) (phenomhm.py:208-224)
+__global__ __launch_bounds__(EVAL_THREADS) void k_phm_default_grid(double* __restrict__ freqs,
+                                                                   const double* __restrict__ m1,
+                                                                   const double* __restrict__ m2,
+                                                                   const int* __restrict__ mms, double lo, double hi,
+                                                                   int M, int L, long n)
+{
+#pragma clang fp contract(off)
+    const long p = (long)blockIdx.x * EVAL_THREADS + threadIdx.x;
+    if (p >= n) return;
+    const long row = p / L;
+    const int i = (int)(p - row * L), b = (int)(row / M), m = (int)(row - (long)b * M);
+    const double step = (hi - lo) / (L - 1), y = i == L - 1 ? hi : lo + i * step;
+    freqs[p] = pow(10.0, y) / ((m1[b] + m2[b]) * MTSUN_SI) * mms[m] / 2.0;
+}
+
+// phase += 2 pi f (t_ref - t0), tf += t_ref (phenomhm.py:487-507)
+__global__ __launch_bounds__(EVAL_THREADS) void k_phm_time_shift(double* __restrict__ phase, double* __restrict__ tf,
+                                                                 const double* __restrict__ freqs,
+                                                                 const double* __restrict__ t_ref, double t0,
+                                                                 long per_bin, long n)
+{
+#pragma clang fp contract(off)
+    const long p = (long)blockIdx.x * EVAL_THREADS + threadIdx.x;
+    if (p >= n) return;
+    const double t = t_ref[p / per_bin];
+    phase[p] += freqs[p] * (t - t0) * 2.0 * PI;
+    tf[p] += t;
+}
+
+// The grid of each (binary, mode) refitted to 0 <= t(f) <= Tobs (phenomhm.py:520-600):
+// where t(f) crosses a bound inside the grid, the crossing frequency by linear
+// interpolation, else the grid's own end. One workgroup per row; *flag is raised if a
+// row that needs a bound does not cross it exactly once.
+__global__ __launch_bounds__(EVAL_THREADS) void k_phm_refit_grid(double* __restrict__ out, int* __restrict__ flag,
+                                                                 const double* __restrict__ tf,
+                                                                 const double* __restrict__ freqs,
+                                                                 const double* __restrict__ Tobs, int tobs_b,
+                                                                 int tobs_m, int M, int L)
+{
+#pragma clang fp contract(off)
+    constexpr int W = EVAL_THREADS / 64;
+    __shared__ double s_min[2][W], s_max[2][W];
+    __shared__ int s_hits[2], s_seg[2];
+    const int b = blockIdx.x / M, m = blockIdx.x - b * M;
+    const double* t = tf + (long)blockIdx.x * L;
+    const double* f = freqs + (long)blockIdx.x * L;
+    const double level[2] = {0.0, Tobs ? Tobs[(long)b * tobs_b + (long)m * tobs_m] : 1e300};
+    // not a number if any entry is
+    auto least = [](double a, double c) { return (c < a || c != c) && a == a ? c : a; };
+    auto most = [](double a, double c) { return (c > a || c != c) && a == a ? c : a; };
+    if (threadIdx.x < 2) s_hits[threadIdx.x] = s_seg[threadIdx.x] = 0;
+    __syncthreads();
+    double lo[2] = {t[0], f[0]}, hi[2] = {t[0], f[0]};
+    for (int i = threadIdx.x; i < L; i += EVAL_THREADS) {
+        const double ti = t[i], fi = f[i];
+        lo[0] = least(lo[0], ti);
+        hi[0] = most(hi[0], ti);
+        lo[1] = least(lo[1], fi);
+        hi[1] = most(hi[1], fi);
+        if (i + 1 < L) {
+            const double tn = t[i + 1];
+            for (int e = 0; e < 2; e++)
+                if (level[e] < tn && level[e] > ti) {
+                    atomicAdd(&s_hits[e], 1);
+                    s_seg[e] = i;
+                }
+        }
+    }
+    for (int q = 0; q < 2; q++) {
+        for (int o = 32; o > 0; o >>= 1) {
+            lo[q] = least(lo[q], __shfl_xor(lo[q], o, 64));
+            hi[q] = most(hi[q], __shfl_xor(hi[q], o, 64));
+        }
+        if ((threadIdx.x & 63) == 0) {
+            s_min[q][threadIdx.x >> 6] = lo[q];
+            s_max[q][threadIdx.x >> 6] = hi[q];
+        }
+    }
+    __syncthreads();
+    for (int q = 0; q < 2; q++)
+        for (int w = 0; w < W; w++) {
+            lo[q] = least(lo[q], s_min[q][w]);
+            hi[q] = most(hi[q], s_max[q][w]);
+        }
+    double end[2] = {lo[1], hi[1]};
+    const bool fix[2] = {lo[0] < level[0], hi[0] > level[1]};
+    for (int e = 0; e < 2; e++) {
+        if (!fix[e]) continue;
+        if (s_hits[e] != 1) {
+            if (threadIdx.x == 0) atomicOr(flag, 1);
+            continue;
+        }
+        const int k = s_seg[e];
+        end[e] = (f[k + 1] - f[k]) / (t[k + 1] - t[k]) * (level[e] - t[k]) + f[k];
+    }
+    const double y0 = log10(end[0]), y1 = log10(end[1]), step = (y1 - y0) / (L - 1);
+    for (int i = threadIdx.x; i < L; i += EVAL_THREADS)
+        out[(long)blockIdx.x * L + i] = pow(10.0, i == L - 1 ? y1 : y0 + i * step);
+}
+
 }  // namespace
 
 extern "C" {
@@ -174,6 +279,45 @@ int bbhx_hip_waveform_amp_phase(double* waveformOut, const int* ells, const int*
                            0, S(stream), waveformOut, recs, freqs, numModes, length,
                            (long)numBinAll * numModes * length);
     }
+    return launch_status();
+}
+
+int bbhx_hip_phm_default_grid(double* freqs, const double* m1, const double* m2, const int* mms, double log10_lo,
+                              double log10_hi, int length, int numModes, int numBinAll, void* stream)
+{
+    if (length < 1 || numModes < 1 || numBinAll < 0) return ERR_ARGS;
+    if (numBinAll == 0) return OK;
+    if (!freqs || !m1 || !m2 || !mms) return ERR_ARGS;
+    const long n = (long)numBinAll * numModes * length;
+    if (ceil_div(n, EVAL_THREADS) > 2147483647L) return ERR_ARGS;
+    hipLaunchKernelGGL(k_phm_default_grid, dim3((unsigned)ceil_div(n, EVAL_THREADS)), dim3(EVAL_THREADS), 0, S(stream),
+                       freqs, m1, m2, mms, log10_lo, log10_hi, numModes, length, n);
+    return launch_status();
+}
+
+int bbhx_hip_phm_time_shift(double* waveformOut, const double* freqs, const double* t_ref, double t0, int length,
+                            int numModes, int numBinAll, void* stream)
+{
+    if (length < 1 || numModes < 1 || numBinAll < 0) return ERR_ARGS;
+    if (numBinAll == 0) return OK;
+    if (!waveformOut || !freqs || !t_ref) return ERR_ARGS;
+    const long n = (long)numBinAll * numModes * length;
+    if (ceil_div(n, EVAL_THREADS) > 2147483647L) return ERR_ARGS;
+    hipLaunchKernelGGL(k_phm_time_shift, dim3((unsigned)ceil_div(n, EVAL_THREADS)), dim3(EVAL_THREADS), 0, S(stream),
+                       waveformOut + n, waveformOut + 2 * n, freqs, t_ref, t0, (long)numModes * length, n);
+    return launch_status();
+}
+
+int bbhx_hip_phm_refit_grid(double* new_freqs, int* flag, const double* tf, const double* freqs, const double* Tobs,
+                            int tobs_stride_bin, int tobs_stride_mode, int length, int numModes, int numBinAll,
+                            void* stream)
+{
+    if (length < 1 || numModes < 1 || numBinAll < 0) return ERR_ARGS;
+    if (numBinAll == 0) return OK;
+    if (!new_freqs || !flag || !tf || !freqs) return ERR_ARGS;
+    if ((long)numBinAll * numModes > 2147483647L) return ERR_ARGS;
+    hipLaunchKernelGGL(k_phm_refit_grid, dim3((unsigned)(numBinAll * numModes)), dim3(EVAL_THREADS), 0, S(stream),
+                       new_freqs, flag, tf, freqs, Tobs, tobs_stride_bin, tobs_stride_mode, numModes, length);
     return launch_status();
 }
 

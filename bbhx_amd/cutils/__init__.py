@@ -96,6 +96,9 @@ def load_library():
                                        C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _vp],
         "bbhx_hip_direct_plan_enable_grad": [_vp],
         "bbhx_hip_direct_plan_set_precision": [_vp, C.c_int],
+        "bbhx_hip_phm_default_grid": [_vp, _vp, _vp, _vp, C.c_double, C.c_double, C.c_int, C.c_int, C.c_int, _vp],
+        "bbhx_hip_phm_time_shift": [_vp, _vp, _vp, C.c_double, C.c_int, C.c_int, C.c_int, _vp],
+        "bbhx_hip_phm_refit_grid": [_vp, _vp, _vp, _vp, _vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _vp],
         "bbhx_hip_interp_bands": [_vp, _vp, _vp, _vp, C.c_int, C.c_int, C.c_int, C.c_int, _vp],
         "bbhx_hip_interp_segments": [_vp, _vp, _vp, _vp, _vp, C.c_int, C.c_int, C.c_int, C.c_int, _vp],
         "bbhx_hip_fill_bands": [_vp, _vp, _vp, _vp, C.c_int, C.c_int, _vp],
@@ -125,6 +128,7 @@ def exported_symbols():
         "bbhx_hip_hdyn_fused_grad", "bbhx_hip_direct_plan_create", "bbhx_hip_direct_plan_destroy",
         "bbhx_hip_direct_plan_bytes", "bbhx_hip_direct_plan_band", "bbhx_hip_direct_fused", "bbhx_hip_hdyn_prep",
         "bbhx_hip_direct_fused_grad", "bbhx_hip_direct_plan_enable_grad", "bbhx_hip_direct_plan_set_precision",
+        "bbhx_hip_phm_default_grid", "bbhx_hip_phm_time_shift", "bbhx_hip_phm_refit_grid",
         "bbhx_hip_aet1_psd", "bbhx_hip_interp_bands", "bbhx_hip_interp_segments", "bbhx_hip_fill_bands",
         "bbhx_hip_window_times", "bbhx_hip_release_workspace", "bbhx_hip_version", "bbhx_hip_timing_enable",
         "bbhx_hip_timing_read",
@@ -215,6 +219,50 @@ def get_phenomd_ringdown_frequencies(fringdown, fdamp, m1, m2, chi1z, chi2z, num
         _dev(fringdown, f64), _dev(fdamp, f64), _dev(m1, f64), _dev(m2, f64), _dev(chi1z, f64), _dev(chi2z, f64),
         int(numBinAll), *[_dev(t, f64) for t in tabs], float(dspin), n, _stream())
     _check(st, "get_phenomd_ringdown_frequencies")
+
+
+def phm_default_grid(m1, m2, mms, log10_lo, log10_hi, length):
+    """Default sparse grid, flat (B, M, length), from device masses and mode numbers (no reference counterpart in
+    BBHxBackendMethods; see include/bbhx_hip.h)."""
+    torch = _torch()
+    f64 = torch.float64
+    B, M = int(m1.numel()), int(mms.numel())
+    freqs = torch.empty(B * M * int(length), dtype=f64, device=m1.device)
+    st = load_library().bbhx_hip_phm_default_grid(_dev(freqs), _dev(m1, f64), _dev(m2, f64), _dev(mms, torch.int32),
+                                                  float(log10_lo), float(log10_hi), int(length), M, B, _stream())
+    _check(st, "phm_default_grid")
+    return freqs
+
+
+def phm_time_shift(waveform, freqs, t_ref, t0, length, num_modes):
+    """Shift phase and tf of the (amp, phase, tf) buffer by t_ref (no reference counterpart in BBHxBackendMethods)."""
+    f64 = _torch().float64
+    B = int(t_ref.numel())
+    n = B * int(num_modes) * int(length)
+    _need(freqs, n, "freqs")
+    if waveform.numel() < 3 * n:
+        raise ValueError(f"waveform must hold at least {3 * n} elements, got {waveform.numel()}")
+    st = load_library().bbhx_hip_phm_time_shift(_dev(waveform, f64), _dev(freqs, f64), _dev(t_ref, f64), float(t0),
+                                                int(length), int(num_modes), B, _stream())
+    _check(st, "phm_time_shift")
+
+
+def phm_refit_grid(tf, freqs, Tobs):
+    """(grids (B, M, L) refitted to 0 <= tf <= Tobs, flag): flag[0] != 0 if one crosses a bound more than once or
+    not at all. tf, freqs (B, M, L); Tobs (B,), (B, M) or None (no reference counterpart in BBHxBackendMethods)."""
+    torch = _torch()
+    f64 = torch.float64
+    B, M, L = (int(v) for v in freqs.shape)
+    if tuple(tf.shape) != (B, M, L) or (Tobs is not None and tuple(Tobs.shape) not in ((B,), (B, M))):
+        raise ValueError("tf must be (B, M, L) like freqs, Tobs (B,) or (B, M)")
+    out = torch.empty_like(freqs)
+    flag = torch.zeros(1, dtype=torch.int32, device=freqs.device)
+    per_mode = Tobs is not None and Tobs.ndim == 2
+    st = load_library().bbhx_hip_phm_refit_grid(
+        _dev(out), _dev(flag), _dev(tf, f64), _dev(freqs, f64), None if Tobs is None else _dev(Tobs, f64),
+        M if per_mode else 1, 1 if per_mode else 0, L, M, B, _stream())
+    _check(st, "phm_refit_grid")
+    return out, flag
 
 
 class pyFastLISAResponse:
@@ -662,6 +710,9 @@ class BBHxHipBackend:
         self.DirectPlan = DirectPlan
         self.hdyn_prep = hdyn_prep
         self.aet1_psd = aet1_psd
+        self.phm_default_grid = phm_default_grid
+        self.phm_time_shift = phm_time_shift
+        self.phm_refit_grid = phm_refit_grid
         self.interp_bands = interp_bands
         self.interp_segments = interp_segments
         self.fill_bands = fill_bands

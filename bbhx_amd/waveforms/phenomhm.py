@@ -12,7 +12,7 @@ import numpy as np
 from scipy.interpolate import CubicSpline
 
 from ..utils.arrays import as_np1d, np_logspace_rows, to_dev
-from ..utils.constants import MSUN_SI, MTSUN_SI
+from ..utils.constants import MSUN_SI
 from ..utils.parallelbase import BBHxParallelModule
 from .ringdownphenomd import QNMData_a, QNMData_fdamp, QNMData_fring, dspin
 
@@ -108,13 +108,8 @@ class PhenomHMAmpPhase(BBHxParallelModule):
 
     def _initialize_freqs(self, m1, m2, mms):
         """Default grid Mf in [mf_min, mf_max] * m/2 (phenomhm.py:208-224)."""
-        torch = self.xp
-        M_tot_sec = to_dev((m1 + m2) * MTSUN_SI, self.device)
-        lo = torch.tensor(np.log10(self.mf_min), dtype=torch.float64, device=self.device)
-        hi = torch.tensor(np.log10(self.mf_max), dtype=torch.float64, device=self.device)
-        base = np_logspace_rows(lo, hi, self.length)
-        self.freqs = (base[None, None, :] / M_tot_sec[:, None, None] * mms.to(torch.float64)[None, :, None]
-                      / 2).flatten()
+        self.freqs = self.backend.phm_default_grid(m1, m2, mms, np.log10(self.mf_min), np.log10(self.mf_max),
+                                                   self.length)
 
     @property
     def amp(self):
@@ -189,7 +184,7 @@ class PhenomHMAmpPhase(BBHxParallelModule):
             self.waveform_carrier = out_buffer
 
         if freqs is None:
-            self._initialize_freqs(m1, m2, mms)
+            self._initialize_freqs(m1_d, m2_d, mms)
         else:
             freqs = to_dev(freqs, dev)
             if freqs.ndim == 1:
@@ -224,12 +219,9 @@ class PhenomHMAmpPhase(BBHxParallelModule):
                           self.run_phenomd)
 
         # phase += 2 pi f (t_ref - t0); tf += t_ref (phenomhm.py:487-507)
-        tref_d = to_dev(t_ref, dev)
-        temp = self.freqs_shaped * (tref_d[:, None, None] - self.initial_t_val) * 2 * np.pi
-        npp = self.num_per_param
-        self.waveform_carrier[npp: 2 * npp] += temp.flatten()
-        self.waveform_carrier[2 * npp: 3 * npp] += tref_d[:, None, None].expand(
-            num_bin_all, num_modes, self.length).flatten()
+        tref_d = to_dev(np.repeat(t_ref, num_bin_all) if t_ref.size == 1 else t_ref, dev)
+        self.backend.phm_time_shift(self.waveform_carrier, self._freqs, tref_d, self.initial_t_val, self.length,
+                                    num_modes)
 
     @staticmethod
     def tobs_grid(Tobs, B, M, device):
@@ -288,8 +280,11 @@ class PhenomHMAmpPhase(BBHxParallelModule):
         if direct:
             return
         Tobs_t = self.tobs_grid(Tobs, self.num_bin_all, self.num_modes, self.device)
-        f_min, f_max = self.window_bounds(self.tf, self.freqs_shaped, Tobs_t)
-        new_freqs = np_logspace_rows(torch.log10(f_min), torch.log10(f_max), self.length)
+        new_freqs, flag = self.backend.phm_refit_grid(self.tf, self.freqs_shaped, Tobs_t)
+        if flag.item():
+            # raises, or fits what crosses the bounds once in all
+            f_min, f_max = self.window_bounds(self.tf, self.freqs_shaped, Tobs_t)
+            new_freqs = np_logspace_rows(torch.log10(f_min), torch.log10(f_max), self.length)
         tmp_kwargs = kwargs.copy()
         tmp_kwargs["freqs"] = new_freqs
         self.run_wave(*args, **tmp_kwargs)

@@ -294,6 +294,23 @@ int bbhx_hip_hdyn_prep(double* dataConstants, double* totals, const double* data
                        const double* h0, const double* psd, int data_length, const double* nodes, int K, double df,
                        void* stream);
 
+/* What the reference's Python does between its waveform kernel's two runs with array
+ * operations. phm_default_grid: freqs (B, M, length), 10^y / ((m1 + m2) MTSUN) * mm / 2
+ * for y evenly from log10_lo to log10_hi, masses in solar masses on the device
+ * (phenomhm.py:208-224). phm_time_shift: phase += 2 pi f (t_ref - t0), tf += t_ref in
+ * the (amp, phase, tf) buffer (phenomhm.py:487-507). phm_refit_grid: new_freqs, the
+ * grids refitted to 0 <= tf <= Tobs (phenomhm.py:520-600); Tobs on the device, entry
+ * (b, m) at b * tobs_stride_bin + m * tobs_stride_mode, or null for no upper bound; *flag
+ * (device, zeroed by the caller) is set if a grid does not cross a bound exactly once
+ * (its new grid is then of no use). */
+int bbhx_hip_phm_default_grid(double* freqs, const double* m1, const double* m2, const int* mms, double log10_lo,
+                              double log10_hi, int length, int numModes, int numBinAll, void* stream);
+int bbhx_hip_phm_time_shift(double* waveformOut, const double* freqs, const double* t_ref, double t0, int length,
+                            int numModes, int numBinAll, void* stream);
+int bbhx_hip_phm_refit_grid(double* new_freqs, int* flag, const double* tf, const double* freqs, const double* Tobs,
+                            int tobs_stride_bin, int tobs_stride_mode, int length, int numModes, int numBinAll,
+                            void* stream);
+
 /* The index arrays of bbhx_hip_InterpTDI on the device (the reference's Python forms
  * them with searchsorted, binary by binary, waveformbuild.py:139-172). freqs (B, M,
  * length) sparse grids, dataFreqs (data_length) ascending. interp_bands: band (B, 2) =
