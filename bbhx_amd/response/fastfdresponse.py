@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import numpy as np
 
-from ..utils.arrays import as_np1d, to_dev
+from ..utils.arrays import as_np1d, rows_to_dev, to_dev
 from ..utils.orbits import EqualArmlengthOrbits
 from ..utils.parallelbase import BBHxParallelModule
 
@@ -172,11 +172,14 @@ class LISATDIResponse(BBHxParallelModule):
     def _mode_arrays(self, modes):
         torch = self.xp
         if modes is None:
+            self.modes = [(int(ell), int(mm)) for ell, mm in zip(self.ells_default.cpu().tolist(),
+                                                                 self.mms_default.cpu().tolist())]
             return self.ells_default, self.mms_default
-        ells_h = np.asarray([ell for ell, mm in modes], dtype=np.int32)
-        mms_h = np.asarray([mm for ell, mm in modes], dtype=np.int32)
-        self._sanity_check_modes(ells_h, mms_h)
-        return torch.as_tensor(ells_h, device=self.device), torch.as_tensor(mms_h, device=self.device)
+        lm = np.asarray([[ell for ell, mm in modes], [mm for ell, mm in modes]], dtype=np.int32)
+        self._sanity_check_modes(lm[0], lm[1])
+        self.modes = list(zip(lm[0].tolist(), lm[1].tolist()))
+        lm = torch.as_tensor(lm, device=self.device)
+        return lm[0], lm[1]
 
     def __call__(self, freqs, inc, lam, beta, psi, phi_ref, length, modes=None, phase=None, tf=None,
                  out_buffer=None, adjust_phase=True, direct=False):
@@ -186,9 +189,8 @@ class LISATDIResponse(BBHxParallelModule):
         ``phase`` and ``tf`` are given; with the latter the shifted phase is
         written back into ``phase`` when ``adjust_phase``."""
         dev = self.device
-        inc, lam, beta, psi, phi_ref = (to_dev(as_np1d(v), dev) for v in (inc, lam, beta, psi, phi_ref))
+        inc, lam, beta, psi, phi_ref = rows_to_dev([as_np1d(v) for v in (inc, lam, beta, psi, phi_ref)], dev)
         ells, mms = self._mode_arrays(modes)
-        self.modes = [(int(ell), int(mm)) for ell, mm in zip(ells.cpu().tolist(), mms.cpu().tolist())]
         B, M, L = int(inc.numel()), int(ells.numel()), int(length)
         self.length, self.num_modes, self.num_bin_all = L, M, B
         self.num_per_bin = L * M
@@ -225,8 +227,8 @@ class LISATDIResponse(BBHxParallelModule):
             self.response_carrier[ia * n:(ia + 1) * n] = phase_d.flatten()
             self.response_carrier[(ia + 1) * n:(ia + 2) * n] = tf_d.flatten()
         elif not direct:
-            tfv = self.tf
-            self.check_orbit_coverage(float(tfv.min()), float(tfv.max()), t_lo, t_hi)
+            tf_min, tf_max = self.xp.stack(self.xp.aminmax(self.tf)).tolist()
+            self.check_orbit_coverage(tf_min, tf_max, t_lo, t_hi)
 
         self.response_gen(self.response_carrier, ells, mms, self.freqs, phi_ref, inc, lam, beta, psi,
                           self.TDItag_int, self.rescaled, self.tdi2, self.order_fresnel_stencil, M, L, B, ia)

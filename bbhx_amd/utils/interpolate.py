@@ -29,10 +29,11 @@ class CubicSplineInterpolant(BBHxParallelModule):
         self.length = length
         self.reshape_shape = (num_interp_params, num_bin_all, num_modes, length)
         self.x_reshape_shape = (num_bin_all, num_modes, length)
-        B = torch.zeros(ninterps * length, dtype=torch.float64, device=self.device)
-        self.c1 = upper_diag = torch.zeros_like(B)
-        self.c2 = diag = torch.zeros_like(B)
-        self.c3 = lower_diag = torch.zeros_like(B)
+        # the kernel writes every entry
+        B = torch.empty(ninterps * length, dtype=torch.float64, device=self.device)
+        self.c1 = upper_diag = torch.empty_like(B)
+        self.c2 = diag = torch.empty_like(B)
+        self.c3 = lower_diag = torch.empty_like(B)
         self.y = y_all
         self.B = B
         self.interpolate_arrays(x, y_all, B, upper_diag, diag, lower_diag, length, num_interp_params, num_modes,

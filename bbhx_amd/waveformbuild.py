@@ -13,7 +13,7 @@ import warnings
 import numpy as np
 
 from .response.fastfdresponse import LISATDIResponse
-from .utils.arrays import as_np1d, to_dev
+from .utils.arrays import as_np1d, rows_to_dev, to_dev
 from .utils.constants import YRSID_SI
 from .utils.interpolate import CubicSplineInterpolant
 from .utils.parallelbase import BBHxParallelModule
@@ -168,7 +168,8 @@ class BBHWaveformFD(BBHxParallelModule):
                           modes=self.amp_phase_gen.modes, direct=direct)
 
         self.out_buffer_final = out_buffer.reshape(9, self.num_bin_all, self.num_modes, self.length)
-        t_start_d, t_end_d = to_dev(t_start, self.device), to_dev(t_end, self.device)
+        if direct:
+            t_start_d, t_end_d = rows_to_dev([t_start, t_end], self.device)
 
         if direct and compress:
             templateChannels = torch.zeros(self.num_bin_all * 3 * self.length, dtype=torch.complex128,

@@ -11,7 +11,7 @@ from __future__ import annotations
 import numpy as np
 from scipy.interpolate import CubicSpline
 
-from ..utils.arrays import as_np1d, np_logspace_rows, to_dev
+from ..utils.arrays import as_np1d, np_logspace_rows, rows_to_dev, to_dev
 from ..utils.constants import MSUN_SI
 from ..utils.parallelbase import BBHxParallelModule
 from .ringdownphenomd import QNMData_a, QNMData_fdamp, QNMData_fring, dspin
@@ -140,17 +140,19 @@ class PhenomHMAmpPhase(BBHxParallelModule):
     def _modes_to_arrays(self, modes):
         torch = self.xp
         if modes is not None:
-            ells = np.asarray([ell for ell, mm in modes], dtype=np.int32)
-            mms = np.asarray([mm for ell, mm in modes], dtype=np.int32)
+            lm = np.asarray([[ell for ell, mm in modes], [mm for ell, mm in modes]], dtype=np.int32)
             self.modes = modes
-            self._sanity_check_modes(ells, mms)
-            return (torch.as_tensor(ells, device=self.device), torch.as_tensor(mms, device=self.device))
+            self._sanity_check_modes(lm[0], lm[1])
+            lm = torch.as_tensor(lm, device=self.device)
+            return lm[0], lm[1]
         self.modes = self.allowable_modes
         return self.ells_default, self.mms_default
 
-    def run_wave(self, m1, m2, chi1z, chi2z, distance, phi_ref, f_ref, t_ref, length, freqs=None,
-                 out_buffer=None, modes=None):
-        """Generate amplitude, phase and t(f) (phenomhm.py:270-507)."""
+    def _prepare(self, m1, m2, chi1z, chi2z, distance, phi_ref, f_ref, t_ref, length, freqs=None,
+                 out_buffer=None, modes=None, Tobs=None):
+        """What the runs of one call share: the checked parameters on the device
+        (with Tobs, if it has one entry per binary) and the ringdown frequencies.
+        Returns them, and the arguments freqs and out_buffer."""
         torch = self.xp
         m1, m2, chi1z, chi2z = as_np1d(m1), as_np1d(m2), as_np1d(chi1z), as_np1d(chi2z)
         distance, phi_ref, f_ref, t_ref = as_np1d(distance), as_np1d(phi_ref), as_np1d(f_ref), as_np1d(t_ref)
@@ -171,11 +173,28 @@ class PhenomHMAmpPhase(BBHxParallelModule):
         self.num_per_param = self.length * num_modes * num_bin_all
         self.num_per_bin = self.length * num_modes
 
-        dev = self.device
-        m1_d, m2_d = to_dev(m1, dev), to_dev(m2, dev)
-        chi1_d, chi2_d = to_dev(chi1z, dev), to_dev(chi2z, dev)
-        dist_d, fref_d = to_dev(distance, dev), to_dev(f_ref, dev)
+        if t_ref.size == 1:
+            t_ref = np.repeat(t_ref, num_bin_all)
+        rows = [m1, m2, chi1z, chi2z, distance, f_ref, t_ref, m1 * MSUN_SI, m2 * MSUN_SI]
+        per_bin = isinstance(Tobs, np.ndarray) and Tobs.shape == (num_bin_all,)
+        rows = rows_to_dev(rows + [Tobs] if per_bin else rows, self.device)
+        m1_d, m2_d, chi1_d, chi2_d = rows[:4]
 
+        frd, fdm = (torch.empty(num_bin_all, dtype=torch.float64, device=self.device) for _ in range(2))
+        self.phenomd_ringdown_freqs(frd, fdm, m1_d, m2_d, chi1_d, chi2_d, num_bin_all, self.y_rd, self.c1_rd,
+                                    self.c2_rd, self.c3_rd, self.y_dm, self.c1_dm, self.c2_dm, self.c3_dm, self.dspin)
+        if not self.run_phenomd:
+            hm = torch.empty((2, num_bin_all, num_modes), dtype=torch.float64, device=self.device)
+            self.phenomhm_ringdown_freqs(hm[0], hm[1], m1_d, m2_d, chi1_d, chi2_d, ells, mms, num_modes, num_bin_all)
+            frd = torch.cat([hm[0], frd[:, None]], dim=1).flatten()
+            fdm = torch.cat([hm[1], fdm[:, None]], dim=1).flatten()
+        self.fringdown, self.fdamp = frd, fdm
+        return (rows, ells.contiguous(), mms.contiguous()), freqs, out_buffer
+
+    def _evaluate(self, inputs, freqs, out_buffer):
+        """One run of the prepared inputs on freqs (None: the default grid)."""
+        (m1_d, m2_d, chi1_d, chi2_d, dist_d, fref_d, tref_d, m1_SI, m2_SI, *_), ells, mms = inputs
+        num_bin_all, num_modes = self.num_bin_all, self.num_modes
         if out_buffer is None:
             self._initialize_waveform_container()
         else:
@@ -186,7 +205,7 @@ class PhenomHMAmpPhase(BBHxParallelModule):
         if freqs is None:
             self._initialize_freqs(m1_d, m2_d, mms)
         else:
-            freqs = to_dev(freqs, dev)
+            freqs = to_dev(freqs, self.device)
             if freqs.ndim == 1:
                 self.freqs = freqs.reshape(1, 1, -1).expand(num_bin_all, num_modes, -1).contiguous().flatten()
             elif freqs.ndim == 3:
@@ -197,31 +216,19 @@ class PhenomHMAmpPhase(BBHxParallelModule):
         if self._freqs.numel() != self.num_per_param:
             raise ValueError("freqs do not match (num_bin_all, num_modes, length).")
 
-        m1_SI, m2_SI = m1_d * MSUN_SI, m2_d * MSUN_SI
-
-        fringdown = torch.zeros(num_modes * num_bin_all, dtype=torch.float64, device=dev)
-        fdamp = torch.zeros_like(fringdown)
-        self.phenomd_ringdown_freqs(fringdown, fdamp, m1_d, m2_d, chi1_d, chi2_d, num_bin_all, self.y_rd,
-                                    self.c1_rd, self.c2_rd, self.c3_rd, self.y_dm, self.c1_dm, self.c2_dm,
-                                    self.c3_dm, self.dspin)
-        if not self.run_phenomd:
-            append_frd = fringdown[:num_bin_all].clone()
-            append_fdm = fdamp[:num_bin_all].clone()
-            self.phenomhm_ringdown_freqs(fringdown, fdamp, m1_d, m2_d, chi1_d, chi2_d, ells, mms, num_modes,
-                                         num_bin_all)
-            fringdown = torch.cat([fringdown.reshape(-1, num_modes), append_frd[:, None]], dim=1).flatten().contiguous()
-            fdamp = torch.cat([fdamp.reshape(-1, num_modes), append_fdm[:, None]], dim=1).flatten().contiguous()
-        self.fringdown, self.fdamp = fringdown, fdamp
-
         # inside the kernel t_ref and phi_ref are zero
-        self.waveform_gen(self.waveform_carrier, ells.contiguous(), mms.contiguous(), self._freqs, m1_SI, m2_SI,
-                          chi1_d, chi2_d, dist_d, fref_d, num_modes, self.length, num_bin_all, fringdown, fdamp,
-                          self.run_phenomd)
+        self.waveform_gen(self.waveform_carrier, ells, mms, self._freqs, m1_SI, m2_SI, chi1_d, chi2_d, dist_d, fref_d,
+                          num_modes, self.length, num_bin_all, self.fringdown, self.fdamp, self.run_phenomd)
 
         # phase += 2 pi f (t_ref - t0); tf += t_ref (phenomhm.py:487-507)
-        tref_d = to_dev(np.repeat(t_ref, num_bin_all) if t_ref.size == 1 else t_ref, dev)
         self.backend.phm_time_shift(self.waveform_carrier, self._freqs, tref_d, self.initial_t_val, self.length,
                                     num_modes)
+
+    def run_wave(self, m1, m2, chi1z, chi2z, distance, phi_ref, f_ref, t_ref, length, freqs=None,
+                 out_buffer=None, modes=None):
+        """Generate amplitude, phase and t(f) (phenomhm.py:270-507)."""
+        self._evaluate(*self._prepare(m1, m2, chi1z, chi2z, distance, phi_ref, f_ref, t_ref, length, freqs=freqs,
+                                      out_buffer=out_buffer, modes=modes))
 
     @staticmethod
     def tobs_grid(Tobs, B, M, device):
@@ -276,15 +283,18 @@ class PhenomHMAmpPhase(BBHxParallelModule):
         """Run the waveform; unless ``direct``, refit each (binary, mode) grid to
         the part with 0 <= t(f) <= Tobs and run again (phenomhm.py:509-614)."""
         torch = self.xp
-        self.run_wave(*args, **kwargs)
+        inputs, freqs, out_buffer = self._prepare(*args, Tobs=Tobs, **kwargs)
+        self._evaluate(inputs, freqs, out_buffer)
         if direct:
             return
-        Tobs_t = self.tobs_grid(Tobs, self.num_bin_all, self.num_modes, self.device)
+        if len(inputs[0]) > 9:
+            Tobs_t = inputs[0][9]
+        else:
+            Tobs_t = self.tobs_grid(Tobs, self.num_bin_all, self.num_modes, self.device)
         new_freqs, flag = self.backend.phm_refit_grid(self.tf, self.freqs_shaped, Tobs_t)
         if flag.item():
             # raises, or fits what crosses the bounds once in all
+            Tobs_t = self.tobs_grid(Tobs, self.num_bin_all, self.num_modes, self.device)
             f_min, f_max = self.window_bounds(self.tf, self.freqs_shaped, Tobs_t)
             new_freqs = np_logspace_rows(torch.log10(f_min), torch.log10(f_max), self.length)
-        tmp_kwargs = kwargs.copy()
-        tmp_kwargs["freqs"] = new_freqs
-        self.run_wave(*args, **tmp_kwargs)
+        self._evaluate(inputs, new_freqs, self.waveform_carrier)
