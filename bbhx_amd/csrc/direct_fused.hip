@@ -866,16 +866,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADJ ? 3 : 4
     const int lane = threadIdx.x & 63;
     fill_etab1k(s_tab, threadIdx.x, blockDim.x);
     __syncthreads();
-    for (;;) {
-        // the wavefront's next item in the chunk-major order (dynamic: the items
-        // running at any time stay a window of consecutive entries, i.e. the same
-        // dense bins). The barrier (no instruction) is convergent: without one in
-        // this block the compiler may thread the branch on lane 0 with one at the
-        // end of the loop, and the other lanes would go round it on their own
+    // The wavefront's items in the chunk-major order: the first by its number, the
+    // following from a counter (dynamic: the items running at any time stay a window of
+    // consecutive entries, i.e. the same dense bins). The counter takes some 8 ns per
+    // wavefront, so with none left beyond the first ones it is not asked: 16 templates of
+    // 65536 bins, 8192 wavefronts for 4096 items: 180 -> 72 us.
+    const int waves = gridDim.x * (blockDim.x >> 6);
+    int pi = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+    for (bool first = true;; first = false) {
+        // The barrier (no instruction) is convergent: without one in this block the
+        // compiler may thread the branch on lane 0 with one at the end of the loop, and
+        // the other lanes would go round it on their own
         __builtin_amdgcn_wave_barrier();
-        int pi = 0;
-        if (lane == 0) pi = atomicAdd(next, 1);
-        pi = __builtin_amdgcn_readfirstlane(pi);
+        if (!first) {
+            if (waves >= nitems) break;
+            pi = 0;
+            if (lane == 0) pi = atomicAdd(next, 1);
+            pi = waves + __builtin_amdgcn_readfirstlane(pi);
+        }
         if (pi >= nitems) break;
         const int it = perm[pi];
         int b;
@@ -885,10 +893,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADJ ? 3 : 4
         const int L = len[b];
         const double ts = t_start[b], te = t_end[b];
         double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-        // lane m: the segment that mode m's last block ended in; -1: not known,
-        // -2: a degenerate grid, no segment holds any f
+        // lane m: the segment that mode m's last block ended in (at first an estimate);
+        // -1: not known, -2: a degenerate grid, no segment holds any f
         int curv = -1;
-        if (lane < M && !(grid_istep[b * M + lane] > 0.0)) curv = -2;
+        if (lane < M) {
+            const double gis = grid_istep[b * M + lane];
+            curv = gis > 0.0 ? segment_estimate(freqs[kw0], grid_lo[b * M + lane], gis, L) : -2;
+        }
         for (int kb = kw0; kb < kw1; kb += RB * 64) {
             const int curs = curv;  // where the modes' walkers start, for the adjoint pass
             double f[RB];
@@ -1248,20 +1259,24 @@ void plan_free(bbhx_direct_plan* p)
 //
 // A work item is what one wavefront takes: a caller's chunk (bins per workgroup
 // and pass) split over the workgroup's wavefronts, and less than that for a small
-// batch, so that there are several items per wavefront slot (4 per SIMD, 4096)
-// for the dynamic order to balance, down to ITEM_MIN bins (one block of the FP64
-// kernel). Plans of up to SMALL_ITEMS such items have buffers for them. 16
-// templates of 65536 bins: 1.78 -> 1.14 ms for the whole step (64 items of 16384
-// bins left most of the chip idle). At 1024 templates of 1.58 M bins the item size
-// does not matter (items of 4096, 8192 and 16384 bins: 25.4, 25.5 and 26.3 ms).
-constexpr long ITEM_MIN = 256, SMALL_ITEMS = 1L << 18, ITEMS_WANTED = 4 * 4096;
+// batch, down to ITEM_MIN bins (half a block). Up to FEW bins in all, as many items as
+// wavefronts in a launch of the default grid, ITEMS_ONCE, each with a first item and
+// no other, as the counter of the following ones takes 8 ns a time; above, twice as
+// many, for the dynamic order to balance. Plans of up to SMALL_ITEMS such items have
+// buffers for them. The whole call with at least 256 bins and 16384 items at any
+// size, and with this rule: 16 templates of 65536 bins 321 and 303 us, 48 of them 440
+// and 395, 64 499 and 433; with ITEMS_ONCE at 128 and 256 of them 630 became 657 and
+// 1005 became 1174 us. At 1024 templates of 1.58 M bins the item size does not
+// matter (items of 4096, 8192 and 16384 bins: 25.4, 25.5 and 26.3 ms).
+constexpr long ITEM_MIN = 128, SMALL_ITEMS = 1L << 19, ITEMS_ONCE = 8192, FEW = ITEMS_ONCE * 512;
 
 static int item_bins(const bbhx_direct_plan* p, int chunk, int block)
 {
     long n = chunk / (block / 64);
-    const long fine = (long)p->B * p->N / ITEMS_WANTED;  // the whole data set of every binary over that many items
+    const long all = (long)p->B * p->N;  // the whole data set of every binary
+    const long fine = all / (all <= FEW ? ITEMS_ONCE : 2 * ITEMS_ONCE);
     n = std::min(n, std::max(fine, ITEM_MIN));
-    n = (n + ITEM_MIN - 1) / ITEM_MIN * ITEM_MIN;
+    n = n <= ITEM_MIN ? ITEM_MIN : (n + 255) / 256 * 256;  // half a block, or whole ones
     return (int)std::max(n, (long)p->min_item);
 }
 
