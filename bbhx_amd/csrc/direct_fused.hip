@@ -25,8 +25,8 @@
 //                 aligned to absolute multiples of the chunk size)
 //   k_dir_cnt_zero, k_dir_cnt, k_dir_cnt_scan, k_dir_perm
 //                 chunk-major execution order of the work items (counting sort)
-//   k_dir_like    persistent: workgroups loop over the (binary, chunk) work
-//                 items in that order; each thread evaluates dense bins (spline segment per
+//   k_dir_like    persistent: wavefronts take the (binary, chunk) work
+//                 items in that order; each lane evaluates dense bins (spline segment per
 //                 mode, WaveformBuild.cu:80-143, window and mode sum :48-60)
 //                 and accumulates the noise-weighted inner products
 //                 (Likelihood.cu:357-471); one partial sum per work item
@@ -737,8 +737,8 @@ __device__ inline void mode_adjoint_per_lane(double* __restrict__ Ym, const SegR
 // partial[it] = (Re, Im of sum conj(d~) h~, sum |h~|^2, 0)
 // over the dense bins of work item it, where h~ = w h (Likelihood.cu:357-375).
 //
-// A work item's bins go in blocks of RB x 64 consecutive bins (lane l: bins kb + 64 r + l), and sums the modes of a
-// block mode by mode. The segment of bin f in a mode's grid is
+// A work item's bins go in blocks of RB x 64 consecutive bins (lane l: bins
+// kb + 64 r + l), the modes of a block summed mode by mode. The segment of bin f in a mode's grid is
 // searchsorted(x, f, 'right') - 1 (waveformbuild.py:139-156), found with the
 // exact FP64 comparisons x_lo <= f < x_hi against the stored knots.
 //
