@@ -162,9 +162,10 @@ __global__ __launch_bounds__(256) void k_interp_offsets(int64_t* __restrict__ of
 // Spline segment of every (binary, mode, dense bin): block -> (binary, mode, tile of
 // SEG_TILE bins). The grids are log-spaced, so the segment is estimated from an FP32
 // logarithm and checked, its neighbours next; whatever they do not hold is searched.
-// Bound by instruction issue, the estimate and its checks. Up to 38 M (binary, mode, bin): 0.11
-// ms (0.23 by a binary search per bin); torch's searchsorted and its conversions,
-// binary by binary: 0.49 ms and seven launches for each.
+// Bound by instruction issue, the estimate and its checks, and the writes. Up to 38 M
+// (binary, mode, bin): 0.062 ms (0.112 with a lane's bins one after another, 0.23 by a
+// binary search per bin); torch's searchsorted and its conversions, binary by binary:
+// 0.49 ms and seven launches for each.
 constexpr int SEG_TILE = 1024;
 __global__ __launch_bounds__(256) void k_interp_segments(int* __restrict__ inds, const int2* __restrict__ band,
                                                          const int64_t* __restrict__ off,
@@ -177,20 +178,39 @@ __global__ __launch_bounds__(256) void k_interp_segments(int* __restrict__ inds,
     const double* x = freqs + (long)bm * L;
     int* o = inds + off[b] * M + (long)m * len;
     const int i0 = tile * SEG_TILE, n = min(len - i0, SEG_TILE);
+    if (L < 2) {
+        for (int i = threadIdx.x; i < n; i += 256) o[i0 + i] = upper_bound(x, L, dataFreqs[r.x + i0 + i]) - 1;
+        return;
+    }
+    if (n <= 0) return;
     const double x0 = x[0], x1 = x[L - 1];
     const float g0 = __log2f((float)x0), gs = (float)(L - 1) / (__log2f((float)x1) - g0);
-    for (int i = threadIdx.x; i < n; i += 256) {
-        const double f = dataFreqs[r.x + i0 + i];
-        int k = -1;
-        if (L < 2) k = upper_bound(x, L, f) - 1;
-        else if (f >= x1) k = L - 1;
-        else if (!(f < x0)) {
-            k = (int)fminf(fmaxf((__log2f((float)f) - g0) * gs, 0.0f), (float)(L - 2));
-            if (f < x[k]) k = max(k - 1, 0);
-            else if (f >= x[k + 1]) k = min(k + 1, L - 2);
-            if (!(x[k] <= f && f < x[k + 1])) k = upper_bound(x, L, f) - 1;
+    // the estimates' bounds of all of the lane's bins first, so that their loads overlap
+    constexpr int U = SEG_TILE / 256;
+    double f[U], xa[U], xb[U];
+    int k[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) f[u] = dataFreqs[r.x + i0 + min((int)threadIdx.x + 256 * u, n - 1)];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        k[u] = (int)fminf(fmaxf((__log2f((float)f[u]) - g0) * gs, 0.0f), (float)(L - 2));
+        xa[u] = x[k[u]];
+        xb[u] = x[k[u] + 1];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const int i = threadIdx.x + 256 * u;
+        if (i >= n) return;
+        int j = k[u];
+        if (!(xa[u] <= f[u] && f[u] < xb[u])) {
+            if (f[u] >= x1) j = L - 1;
+            else if (f[u] < x0) j = -1;
+            else {
+                j = f[u] < xa[u] ? max(j - 1, 0) : min(j + 1, L - 2);
+                if (!(x[j] <= f[u] && f[u] < x[j + 1])) j = upper_bound(x, L, f[u]) - 1;
+            }
         }
-        o[i0 + i] = k;
+        o[i0 + i] = j;
     }
 }
 
