@@ -464,4 +464,20 @@ __host__ __device__ inline cd mul_i(cd a) { return cd{-a.im, a.re}; }
 
 inline int ceil_div(long a, long b) { return int((a + b - 1) / b); }
 
+// HIP takes fewer than 2^32 work-items per dimension of a grid: rows of 'blocks'
+// workgroups of 'threads' lanes each, in as few launches as that allows;
+// launch(first row, grid) makes one.
+constexpr long GRID_LANES = (1L << 32) - 1;
+template <class Launch>
+inline int launch_rows(long rows, long blocks, int threads, Launch launch)
+{
+    const long most = GRID_LANES / threads / blocks;
+    if (most < 1) return ERR_ARGS;
+    for (long r = 0; r < rows; r += most) {
+        launch(r, dim3((unsigned)((rows - r < most ? rows - r : most) * blocks)));
+        if (hipGetLastError() != hipSuccess) return ERR_LAUNCH;
+    }
+    return OK;
+}
+
 }  // namespace bbhx

@@ -18,8 +18,6 @@
 // sweeps took 206 and 159 us (a wavefront per system, 64 row blocks), 2.4 and 6.6 ms (a lane
 // per system).
 
-#include <algorithm>
-
 #include "bbhx_hip.h"
 #include "common.h"
 #include "spline_device.h"
@@ -30,19 +28,20 @@ namespace {
 
 constexpr int SPL_NR = 3;  // systems of one set of knots per workgroup
 
-// Workgroup g of the launch: block g % nb of the knots of set sub0 + g / nb % nsets,
-// quantities NR (g / nb / nsets) and following of P; system = quantity * nsub + set.
+// Workgroup g of the launch: block g % nb of the knots of item e = e0 + g / nb, which is
+// set e % nsub and the quantities NR (e / nsub) and following of P; system =
+// quantity * nsub + set.
 template <int NR>
 __global__ __launch_bounds__(SPL_T) void k_spline(const double* __restrict__ x, const double* __restrict__ y,
                                                   double* __restrict__ Bs, double* __restrict__ c1,
                                                   double* __restrict__ c2, double* __restrict__ c3, int n, int nsub,
-                                                  int P, int nb, int sub0, int nsets)
+                                                  int P, int nb, int e0)
 {
     constexpr int T = SPL_T;
     __shared__ double sh[(NR + 2) * T];
     __shared__ double ends[2][NR];  // right sides of the two end rows
     const int t = threadIdx.x;
-    const int blk = blockIdx.x % nb, g = blockIdx.x / nb, sub = sub0 + g % nsets, q0 = g / nsets * NR;
+    const int blk = blockIdx.x % nb, e = e0 + blockIdx.x / nb, sub = e % nsub, q0 = e / nsub * NR;
     const int first = blk * SPL_U, i = first + t, iy = min(i, n - 1);
     const int row0 = blk == 0 ? 0 : first + SPL_W, row1 = blk == nb - 1 ? n : first + T - SPL_W;
     const double xi = x[(long)sub * n + iy];
@@ -127,15 +126,9 @@ extern "C" int bbhx_hip_interpolate(const double* freqs, const double* propArray
     const int nsub = numModes * numBinAll, nb = spline_blocks(length);
     const bool one = numInterpParams < SPL_NR;
     const int groups = one ? numInterpParams : (numInterpParams + SPL_NR - 1) / SPL_NR;
-    // sets of knots per launch, within the limit of its grid
-    const int per = (int)std::max(1L, std::min((long)nsub, (1L << 30) / nb / groups));
-    for (int s0 = 0; s0 < nsub; s0 += per) {
-        const int sets = std::min(per, nsub - s0);
-        const dim3 grid((unsigned)((long)sets * nb * groups));
+    return launch_rows((long)nsub * groups, nb, SPL_T, [&](long e0, dim3 grid) {
         hipLaunchKernelGGL(one ? k_spline<1> : k_spline<SPL_NR>, grid, dim3(SPL_T), 0,
                            reinterpret_cast<hipStream_t>(stream), freqs, propArrays, B, upper_diag, diag, lower_diag,
-                           length, nsub, numInterpParams, nb, s0, sets);
-        if (hipGetLastError() != hipSuccess) return ERR_LAUNCH;
-    }
-    return OK;
+                           length, nsub, numInterpParams, nb, (int)e0);
+    });
 }
