@@ -388,7 +388,7 @@ __global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void
         r[q] = solve ? v * ib : 0.0;
     }
     __syncthreads();
-    pcr_solve(a, c, r, sh, t);
+    pcr_solve(a, c, r, sh, t, 0, T);
     // slopes to the neighbours, the end ones from their rows
 #pragma unroll
     for (int q = 0; q < NQ; q++) {
@@ -1144,7 +1144,7 @@ __global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void
     for (int q = 0; q < NA8; q++) zl[q] = low ? sh[q * T + t - 1] * iel : (high ? sh[q * T + t + 1] * ieh : 0.0);
     // (a grid of four knots has two such rows, in different lanes)
     __syncthreads();
-    pcr_solve(a, c, z, sh, t);
+    pcr_solve(a, c, z, sh, t, 0, T);
 #pragma unroll
     for (int q = 0; q < NA8; q++) {
         if (i != 0 && i < n - 1) sh[q * T + t] = z[q];

@@ -29,20 +29,29 @@ namespace {
 constexpr int SPL_NR = 3;  // systems of one set of knots per workgroup
 
 // Workgroup g of the launch: block g % nb of the knots of item e = e0 + g / nb, which is
-// set e % nsub and the quantities NR (e / nsub) and following of P; system =
-// quantity * nsub + set.
-template <int NR>
+// the G sets from G (e % packs) on and the quantities NR (e / packs) and following of P;
+// system = quantity * nsub + set. PACK: sets of at most half a workgroup's lanes, which take
+// n lanes each, one after another. With a workgroup for each of them, 100000 sets of 4, 16
+// and 64 knots and nine quantities took 1036, 1040 and 1066 us instead of 29, 119 and 465
+// (a lane per system, by a Thomas sweep: 76, 1287 and 4922). Otherwise G = 1, in a kernel of
+// its own, without the room for the sets' end rows.
+template <int NR, bool PACK>
 __global__ __launch_bounds__(SPL_T) void k_spline(const double* __restrict__ x, const double* __restrict__ y,
                                                   double* __restrict__ Bs, double* __restrict__ c1,
                                                   double* __restrict__ c2, double* __restrict__ c3, int n, int nsub,
-                                                  int P, int nb, int e0)
+                                                  int P, int nb, int G, int e0)
 {
     constexpr int T = SPL_T;
     __shared__ double sh[(NR + 2) * T];
-    __shared__ double ends[2][NR];  // right sides of the two end rows
+    __shared__ double ends[2][NR][PACK ? T / 3 : 1];  // right sides of the sets' two end rows
     const int t = threadIdx.x;
-    const int blk = blockIdx.x % nb, e = e0 + blockIdx.x / nb, sub = e % nsub, q0 = e / nsub * NR;
-    const int first = blk * SPL_U, i = first + t, iy = min(i, n - 1);
+    const int blk = blockIdx.x % nb, e = e0 + blockIdx.x / nb, packs = PACK ? (nsub - 1) / G + 1 : nsub;
+    const int set0 = PACK ? e % packs * G : e % packs, q0 = e / packs * NR;
+    // this lane's set in the workgroup and its lanes
+    const int s = PACK ? t / n : 0, t0 = s * n, t1 = PACK ? t0 + n : T;
+    const bool any = !PACK || (s < G && set0 + s < nsub);
+    const int sub = any ? set0 + s : set0;
+    const int first = blk * SPL_U, i = any ? first + t - t0 : n, iy = min(i, n - 1);
     const int row0 = blk == 0 ? 0 : first + SPL_W, row1 = blk == nb - 1 ? n : first + T - SPL_W;
     const double xi = x[(long)sub * n + iy];
     long at[NR];
@@ -79,24 +88,24 @@ __global__ __launch_bounds__(SPL_T) void k_spline(const double* __restrict__ x, 
         mr[q] = (sh[(1 + q) * T + th] - v[q]) * ir;
         double w = 3.0 * (hr * ml + hl * mr[q]);
         if (low) {
-            ends[0][q] = e0l * ml + e0r * mr[q];
-            w -= ends[0][q];
+            ends[0][q][s] = e0l * ml + e0r * mr[q];
+            w -= ends[0][q][s];
         }
         if (high) {
-            ends[1][q] = e1l * ml + e1r * mr[q];
-            w -= ends[1][q];
+            ends[1][q][s] = e1l * ml + e1r * mr[q];
+            w -= ends[1][q][s];
         }
         if (parabola) w = hr * ml + hl * mr[q];
         r[q] = solve ? w * ib : 0.0;
     }
     __syncthreads();
-    pcr_solve(a, c, r, sh, t);
+    pcr_solve(a, c, r, sh, t, t0, t1);
     // slopes to the neighbours, the end ones from their rows
 #pragma unroll
     for (int q = 0; q < NR; q++) {
         if (i != 0 && i < n - 1) sh[q * T + t] = r[q];
-        if (low) sh[q * T + t - 1] = (ends[0][q] - d * r[q]) * ir;
-        if (high) sh[q * T + t + 1] = (ends[1][q] - d * r[q]) * il;
+        if (low) sh[q * T + t - 1] = (ends[0][q][s] - d * r[q]) * ir;
+        if (high) sh[q * T + t + 1] = (ends[1][q][s] - d * r[q]) * il;
     }
     __syncthreads();
     if (i < row0 || i >= row1) return;
@@ -104,10 +113,10 @@ __global__ __launch_bounds__(SPL_T) void k_spline(const double* __restrict__ x, 
 #pragma unroll
     for (int q = 0; q < NR; q++) {
         if (q0 + q >= P) break;
-        const double s = sh[q * T + t], u = (s + sh[q * T + th] - 2.0 * mr[q]) * ir;
-        Bs[at[q]] = s;
-        c1[at[q]] = end ? 0.0 : s;
-        c2[at[q]] = end ? 0.0 : (mr[q] - s) * ir - u;
+        const double sl = sh[q * T + t], u = (sl + sh[q * T + th] - 2.0 * mr[q]) * ir;
+        Bs[at[q]] = sl;
+        c1[at[q]] = end ? 0.0 : sl;
+        c2[at[q]] = end ? 0.0 : (mr[q] - sl) * ir - u;
         c3[at[q]] = end ? 0.0 : u * ir;
     }
 }
@@ -124,11 +133,14 @@ extern "C" int bbhx_hip_interpolate(const double* freqs, const double* propArray
     long nsys = (long)numInterpParams * numModes * numBinAll;
     if (nsys > 2147483647L) return ERR_ARGS;
     const int nsub = numModes * numBinAll, nb = spline_blocks(length);
-    const bool one = numInterpParams < SPL_NR;
+    const bool one = numInterpParams < SPL_NR, pack = length <= SPL_T / 2;
     const int groups = one ? numInterpParams : (numInterpParams + SPL_NR - 1) / SPL_NR;
-    return launch_rows((long)nsub * groups, nb, SPL_T, [&](long e0, dim3 grid) {
-        hipLaunchKernelGGL(one ? k_spline<1> : k_spline<SPL_NR>, grid, dim3(SPL_T), 0,
+    const int G = pack ? SPL_T / length : 1;
+    const auto kernel = one ? (pack ? k_spline<1, true> : k_spline<1, false>)
+                            : (pack ? k_spline<SPL_NR, true> : k_spline<SPL_NR, false>);
+    return launch_rows((long)((nsub - 1) / G + 1) * groups, nb, SPL_T, [&](long e0, dim3 grid) {
+        hipLaunchKernelGGL(kernel, grid, dim3(SPL_T), 0,
                            reinterpret_cast<hipStream_t>(stream), freqs, propArrays, B, upper_diag, diag, lower_diag,
-                           length, nsub, numInterpParams, nb, (int)e0);
+                           length, nsub, numInterpParams, nb, G, (int)e0);
     });
 }

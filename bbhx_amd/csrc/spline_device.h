@@ -26,11 +26,11 @@ constexpr int SPL_T = 256;
 constexpr int SPL_U = SPL_T - 2 * SPL_W;  // rows between the starts of two blocks
 __host__ __device__ inline int spline_blocks(int n) { return n <= SPL_T ? 1 : 1 + (n - SPL_T + SPL_U - 1) / SPL_U; }
 
-// Solves x_i + a x_{i-1} + c x_{i+1} = r_i for NR right sides over the rows of a
-// workgroup (row t = threadIdx.x; rows outside it are left out); sh: (NR + 2)
-// SPL_T doubles of LDS, free on entry and on exit.
+// Solves x_i + a x_{i-1} + c x_{i+1} = r_i for NR right sides over rows [t0, t1) of a
+// workgroup (this lane's row t = threadIdx.x among them; rows outside are left out); sh:
+// (NR + 2) SPL_T doubles of LDS, free on entry and on exit.
 template <int NR>
-__device__ inline void pcr_solve(double a, double c, double (&r)[NR], double* sh, int t)
+__device__ inline void pcr_solve(double a, double c, double (&r)[NR], double* sh, int t, int t0, int t1)
 {
     constexpr int T = SPL_T;
     for (int k = 0, d = 1; k < SPL_STEPS; k++, d *= 2) {
@@ -39,9 +39,9 @@ __device__ inline void pcr_solve(double a, double c, double (&r)[NR], double* sh
 #pragma unroll
         for (int q = 0; q < NR; q++) sh[(2 + q) * T + t] = r[q];
         __syncthreads();
-        const bool lo = t >= d, hi = t + d < T;
+        const bool lo = t - d >= t0, hi = t + d < t1;
         const int tl = lo ? t - d : t, th = hi ? t + d : t;
-        // couplings to rows outside the block are dropped
+        // couplings to rows outside are dropped
         const double fl = lo ? a : 0.0, fh = hi ? c : 0.0;
         const double ib = rcp_pos(1.0 - fl * sh[T + tl] - fh * sh[th]);
         a = -(fl * sh[tl]) * ib;

@@ -37,7 +37,7 @@ class Library:
 
 def interpolate(lib, n, params, sets):
     p = [C.c_void_p(4096)] * 6
-    return lib.call("interpolate", *p, n, params, 1, sets, None, args_of="k_spline", nargs=11)
+    return lib.call("interpolate", *p, n, params, 1, sets, None, args_of="k_spline", nargs=12)
 
 
 CASES = {"interpolate": interpolate}

@@ -37,12 +37,15 @@ def launches(result, kernel):
 
 
 def test_spline_grids(record):
-    """Every (set of knots, group of quantities) has its workgroups, whatever the number of sets."""
-    sizes = [(300, 9, 4_000_000), (16, 9, 6_000_000), (16, 1, 40_000_000), (1 << 28, 2, 3)]
+    """Every (set of knots, group of quantities) has its workgroups, whatever the number of
+    sets; short sets share them."""
+    sizes = [(300, 9, 4_000_000), (129, 9, 6_000_000), (128, 9, 6_000_001), (4, 9, 6_000_000), (3, 1, 40_000_000),
+             (1 << 28, 2, 3)]
     for (n, params, sets), r in zip(sizes, record(*[("interpolate", *s) for s in sizes])):
         blocks = 1 if n <= 256 else 1 + -(-(n - 256) // 160)
         done = 0
         for grid, block, args in launches(r, "k_spline"):
-            assert args[10] & 0xFFFFFFFF == done and grid[0] % blocks == 0
+            assert args[11] & 0xFFFFFFFF == done and grid[0] % blocks == 0
             done += grid[0] // blocks
-        assert done == sets * (-(-params // 3) if params >= 3 else params)
+        packs = -(-sets // (256 // n)) if n <= 128 else sets
+        assert done == packs * (-(-params // 3) if params >= 3 else params)
