@@ -33,6 +33,8 @@
 //   k_dir_reduce  one wavefront per binary: its partials in a fixed order (deterministic)
 
 #include <algorithm>
+#include <memory>
+#include <new>
 #include <vector>
 
 #include "bbhx_hip.h"
@@ -48,6 +50,13 @@ namespace bbhx {
 bool response_orbit_tab(const bbhx_response* r, resp::OrbitTab& o);
 }
 
+// A part of a plan's work table: the entries of one launch
+struct TablePart {
+    int threads = 0;  // lanes per workgroup
+    int lmax = 0;     // longest grid
+    long first = 0, count = 0;
+};
+
 struct bbhx_direct_plan {
     int device = -1;
     int B = 0, M = 0, N = 0, Lmax = 0;
@@ -58,6 +67,17 @@ struct bbhx_direct_plan {
     // device buffers
     long* off = nullptr;   // (B,) first point of each binary
     int* len = nullptr;    // (B,)
+    std::vector<int> lengths;  // the same on the host
+    // Work tables of the launches whose workgroups go by grid length: laid out for the
+    // longest grid, most of them start for nothing in an uneven batch. 4096 templates of 64
+    // knots and one of 4096, as many workgroups for each of them and the tables: k_dirg_knots
+    // 10.4 and 0.42 ms, k_dir_grid 0.65 and 0.29, k_dirg_spline_adj 0.55 and 0.41.
+    int* grid_b = nullptr;     // (B,) binaries by size of their k_dir_grid workgroup
+    int2* spl = nullptr;       // {b M + m, block} of each workgroup of the spline kernels
+    int4* knots = nullptr;     // {b M + m, first knot, row of gpart} of each of k_dirg_knots'
+    int* gpart_b = nullptr;    // (B + 1,) first row of gpart of each binary
+    TablePart grid_parts[3], knot_parts[4];
+    long nspl = 0, nknots = 0;
     FusedRec* recs = nullptr;
     double* X = nullptr;   // (S, M)
     double* Cf = nullptr;  // (S, M, RS): segment records (bounds, value and cubic coefficients)
@@ -73,7 +93,7 @@ struct bbhx_direct_plan {
     // gradient buffers (bbhx_hip_direct_plan_enable_grad)
     double* Yadj = nullptr;              // (S, M, 9, 4) adjoint records
     bbhx::gradk::GradRec* grecs = nullptr;  // (B, M) records with tangents
-    double* gpart = nullptr;             // (B, M, 11) per-mode gradients
+    double* gpart = nullptr;             // (rows, 11) gradients of the workgroups of k_dirg_knots
     int max_chunks = 0;           // absolute chunks of min_item bins
 };
 
@@ -158,8 +178,8 @@ constexpr int GRID_T = 256;
 __global__ __launch_bounds__(GRID_T) void k_dir_grid(double* __restrict__ X, double* __restrict__ Yc,
                                                  double* __restrict__ grid_lo, double* __restrict__ grid_istep,
                                                  int* __restrict__ flags, const FusedRec* __restrict__ recs,
-                                                 const long* __restrict__ off, const int* __restrict__ len,
-                                                 const double* __restrict__ params,
+                                                 const int* __restrict__ bins, const long* __restrict__ off,
+                                                 const int* __restrict__ len, const double* __restrict__ params,
                                                  const double* __restrict__ t_start,
                                                  const double* __restrict__ t_end, int B, int M, ModeList modes,
                                                  resp::OrbitTab orb, int TDItag, int rescaled, int tdi2,
@@ -168,8 +188,7 @@ __global__ __launch_bounds__(GRID_T) void k_dir_grid(double* __restrict__ X, dou
     extern __shared__ double tfs[];
     __shared__ double2 s_t[GRID_T / 64];
     __shared__ int4 s_n[GRID_T / 64];
-    const int bm = blockIdx.x;
-    const int b = bm / M, m = bm % M;
+    const int b = bins[blockIdx.x / M], m = blockIdx.x % M, bm = b * M + m;
     const int t = threadIdx.x, T = blockDim.x;
     const int L = len[b];
     const long base = off[b];
@@ -307,21 +326,20 @@ __device__ inline int segment_window(const Cubic& c, double h, double ts, double
 // 9.4 M records: 1.7 ms; 64 of 4096 knots: 0.2 ms). Thomas sweeps, one lane per (mode,
 // quantity), are one chain over all knots: 537 us, 3.1 ms and 2.24 ms.
 
-// The rows of one workgroup of a spline kernel: block 'blk' of (binary b, mode m).
+// The rows of one workgroup of a spline kernel: block 'blk' of (binary b, mode m), by
+// its entry of the plan's table.
 struct SplineRows {
     int b, m, n, first, row0, row1;  // loaded rows [first, first + T), results for [row0, row1)
-    bool any;
 };
-__device__ inline SplineRows spline_rows(const int* __restrict__ len, int M, int nbmax)
+__device__ inline SplineRows spline_rows(const int2* __restrict__ spl, const int* __restrict__ len, int M)
 {
     constexpr int T = SPL_T;
     SplineRows w;
-    const int blk = blockIdx.x % nbmax, bm = blockIdx.x / nbmax;
+    const int bm = spl[blockIdx.x].x, blk = spl[blockIdx.x].y;
     w.b = bm / M;
     w.m = bm % M;
     w.n = len[w.b];
     const int nb = spline_blocks(w.n);
-    w.any = blk < nb;
     w.first = blk * SPL_U;
     w.row0 = blk == 0 ? 0 : w.first + SPL_W;
     w.row1 = blk == nb - 1 ? w.n : w.first + T - SPL_W;
@@ -332,16 +350,16 @@ __device__ inline SplineRows spline_rows(const int* __restrict__ len, int M, int
 // spline.hip), one lane per knot. The two end rows are folded into their
 // neighbours, which leaves every row dominant: s_0 = (b_0 - (h_0 + h_1) s_1) / h_1.
 __global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void k_dir_spline(const double* __restrict__ X, const double* __restrict__ Yc,
-                                                    SegRec* __restrict__ Cf, const long* __restrict__ off,
-                                                    const int* __restrict__ len, const double* __restrict__ t_start,
-                                                    const double* __restrict__ t_end, int M, int nbmax)
+                                                    SegRec* __restrict__ Cf, const int2* __restrict__ spl,
+                                                    const long* __restrict__ off, const int* __restrict__ len,
+                                                    const double* __restrict__ t_start,
+                                                    const double* __restrict__ t_end, int M)
 {
     constexpr int T = SPL_T;
     __shared__ __align__(16) double sh[(NQ + 2) * T];
     __shared__ double ends[2][NQ];  // right sides of the two end rows
     const int t = threadIdx.x;
-    const SplineRows w = spline_rows(len, M, nbmax);
-    if (!w.any) return;
+    const SplineRows w = spline_rows(spl, len, M);
     const int i = w.first + t, n = w.n;
     const long base = off[w.b];
     const bool row = i < n;
@@ -1072,14 +1090,13 @@ __global__ __launch_bounds__(64) void k_dirg_setup(gradk::GradRec* __restrict__ 
 // exchanges: 256 uneven templates, 2.36 M records: 0.66 ms (0.16 ms at the rate of a
 // copy). Thomas sweeps, one lane per (mode, quantity): 8.7 ms.
 __global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void k_dirg_spline_adj(
-    double* __restrict__ Ya, const double* __restrict__ Yadj, const double* __restrict__ X, const long* __restrict__ off,
-    const int* __restrict__ len, int M, int nbmax)
+    double* __restrict__ Ya, const double* __restrict__ Yadj, const double* __restrict__ X,
+    const int2* __restrict__ spl, const long* __restrict__ off, const int* __restrict__ len, int M)
 {
     constexpr int T = SPL_T, NA8 = 8;
     __shared__ double sh[(NA8 + 2) * T];
     const int t = threadIdx.x;
-    const SplineRows w = spline_rows(len, M, nbmax);
-    if (!w.any) return;
+    const SplineRows w = spline_rows(spl, len, M);
     const int i = w.first + t, n = w.n;
     const long base = off[w.b];
     const bool row = i < n, seg = i < n - 1;  // knot i, segment i
@@ -1178,21 +1195,21 @@ __global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void
         Ya[p * NQ + adj_q(q)] = yb[q] - cy[q] + (i > 0 ? sh[q * T + t - 1] : 0.0);
 }
 
-// Knot-level contraction, a workgroup per (binary, mode) and GRAD_T knots; the
+// Knot-level contraction, a workgroup per (binary, mode) and up to GRAD_T knots, by its
+// entry of the plan's table; the
 // knot-value adjoints of A, phase and T weight the waveform's and response's
 // tangents at the knot's frequency (grad_point_core, no window rule: the
-// window acts on the dense bins). partial[((b M + m) nc + chunk) 11 + p].
+// window acts on the dense bins).
 __global__ __launch_bounds__(gradk::GRAD_T) __attribute__((amdgpu_waves_per_eu(2))) void k_dirg_knots(
     double* __restrict__ gpart, const gradk::GradRec* __restrict__ grecs, const double* __restrict__ Ya,
-    const double* __restrict__ X, const long* __restrict__ off, const int* __restrict__ len,
-    const double* __restrict__ params, int B, int M, int nc, resp::OrbitTab orb, int TDItag, int rescaled, int tdi2,
-    double initial_t_val)
+    const double* __restrict__ X, const int4* __restrict__ knots, const long* __restrict__ off,
+    const int* __restrict__ len, const double* __restrict__ params, int B, int M, resp::OrbitTab orb, int TDItag,
+    int rescaled, int tdi2, double initial_t_val)
 {
     __shared__ gradk::GradShared sh;
-    const int bm = blockIdx.x / nc, chunk = blockIdx.x % nc;
-    const int b = bm / M, m = bm % M;
-    const int n = len[b], i = chunk * gradk::GRAD_T + threadIdx.x;
-    if (chunk * gradk::GRAD_T >= n) return;
+    const int4 w = knots[blockIdx.x];
+    const int bm = w.x, b = bm / M, m = bm % M;
+    const int n = len[b], i = w.y + threadIdx.x;
     Window win;
     win.t_ref = params[P_TREF * B + b];
     win.ts = 0.0;
@@ -1213,21 +1230,18 @@ __global__ __launch_bounds__(gradk::GRAD_T) __attribute__((amdgpu_waves_per_eu(2
         gradk::grad_point_core(G, orb, X[rec], win, false, weights, TDItag, rescaled, tdi2, dist, acc, sh.tab,
                                sh.tan + threadIdx.x, blockDim.x);
     }
-    gradk::grad_sum(sh, acc, gpart + (long)blockIdx.x * gradk::NGRAD);
+    gradk::grad_sum(sh, acc, gpart + (long)w.z * gradk::NGRAD);
 }
 
-// grad[p B + b] = sum over the modes and their chunks: one wavefront per binary
-__global__ __launch_bounds__(64) void k_dirg_reduce(double* __restrict__ grad, const double* __restrict__ gpart, const int* __restrict__ len,
-                              int B, int M, int nc)
+// grad[p B + b] = sum over the binary's rows of gpart: one wavefront per binary
+__global__ __launch_bounds__(64) void k_dirg_reduce(double* __restrict__ grad, const double* __restrict__ gpart,
+                                                    const int* __restrict__ gpart_b, int B)
 {
-    const int b = blockIdx.x, n = gradk::grad_chunks(len[b]);
+    const int b = blockIdx.x, r1 = gpart_b[b + 1];
     double acc[gradk::NGRAD];
     for (int p = 0; p < gradk::NGRAD; p++) acc[p] = 0.0;
-    for (int e = threadIdx.x; e < M * n; e += 64) {
-        const int m = e / n, c = e - m * n;
-        const double* g = gpart + (((long)b * M + m) * nc + c) * gradk::NGRAD;
-        for (int p = 0; p < gradk::NGRAD; p++) acc[p] += g[p];
-    }
+    for (int r = gpart_b[b] + threadIdx.x; r < r1; r += 64)
+        for (int p = 0; p < gradk::NGRAD; p++) acc[p] += gpart[(long)r * gradk::NGRAD + p];
     for (int p = 0; p < gradk::NGRAD; p++) {
         const double v = wsum(acc[p]);
         if (threadIdx.x == 0) grad[(long)p * B + b] = v;
@@ -1248,9 +1262,68 @@ T* dalloc(size_t n, bool& ok)
 void plan_free(bbhx_direct_plan* p)
 {
     void* bufs[] = {p->off, p->len, p->recs, p->X, p->Cf, p->Yc, p->grid_lo, p->grid_istep, p->band,
-                    p->total, p->partial, p->perm, p->cnt, p->next, p->Yadj, p->grecs, p->gpart};
+                    p->total, p->partial, p->perm, p->cnt, p->next, p->Yadj, p->grecs, p->gpart, p->grid_b,
+                    p->spl, p->knots, p->gpart_b};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
+}
+
+// a host table on the device
+template <class T>
+T* upload(const std::vector<T>& v, bool& ok)
+{
+    T* d = dalloc<T>(v.size(), ok);
+    ok = ok && (v.empty() || hipMemcpy(d, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice) == hipSuccess);
+    return d;
+}
+
+// Binaries by the lanes that k_dir_grid takes for their knots, 64, 128 or GRID_T, and the
+// blocks of the spline kernels; false: more of these than a table holds.
+bool lay_out_forward(bbhx_direct_plan* p, std::vector<int>& grid_b, std::vector<int2>& spl)
+{
+    for (int c = 0; c < 3; c++) {
+        TablePart& part = p->grid_parts[c];
+        part.threads = 64 << c;
+        part.first = (long)grid_b.size();
+        for (int b = 0; b < p->B; b++) {
+            const int n = p->lengths[b];
+            if (std::min(GRID_T, n <= 64 ? 64 : (n <= 128 ? 128 : GRID_T)) != part.threads) continue;
+            grid_b.push_back(b);
+            part.lmax = std::max(part.lmax, n);
+        }
+        part.count = (long)grid_b.size() - part.first;
+    }
+    for (int b = 0; b < p->B; b++)
+        for (int m = 0; m < p->M; m++)
+            for (int blk = 0; blk < spline_blocks(p->lengths[b]); blk++) spl.push_back({b * p->M + m, blk});
+    p->nspl = (long)spl.size();
+    return p->nspl <= 2147483647L;
+}
+
+// The workgroups of k_dirg_knots, by their lanes; false: as above.
+bool lay_out_knots(bbhx_direct_plan* p, std::vector<int4>& knots, std::vector<int>& gpart_b)
+{
+    long rows = 0;
+    for (int b = 0; b < p->B; b++) {
+        gpart_b.push_back((int)rows);
+        rows += (long)p->M * gradk::grad_chunks(p->lengths[b]);
+        if (rows > 2147483647L) return false;
+    }
+    gpart_b.push_back((int)rows);
+    for (int c = 0; c < 4; c++) {
+        TablePart& part = p->knot_parts[c];
+        part.threads = 64 * (c + 1);
+        part.first = (long)knots.size();
+        for (int b = 0; b < p->B; b++) {
+            const int n = p->lengths[b], chunks = gradk::grad_chunks(n);
+            if (gradk::grad_threads(n) != part.threads) continue;
+            for (int m = 0; m < p->M; m++)
+                for (int k = 0; k < chunks; k++)
+                    knots.push_back({b * p->M + m, k * part.threads, gpart_b[b] + m * chunks + k, 0});
+        }
+        part.count = (long)knots.size() - part.first;
+    }
+    return true;
 }
 
 }  // namespace
@@ -1280,12 +1353,9 @@ static int item_bins(const bbhx_direct_plan* p, int chunk, int block)
     return (int)std::max(n, (long)p->min_item);
 }
 
-extern "C" int bbhx_hip_direct_plan_create(bbhx_direct_plan** out, int numBinAll, const int* lengths_host,
-                                           int numModes, int data_length, int min_chunk)
+static int plan_create(bbhx_direct_plan** out, int numBinAll, const int* lengths_host, int numModes, int data_length,
+                       int min_chunk)
 {
-    if (!out || numBinAll < 1 || !lengths_host || numModes < 1 || numModes > MAX_MODES || data_length < 1 ||
-        min_chunk < 64)
-        return ERR_ARGS;
     std::vector<long> off(numBinAll);
     long S = 0;
     int Lmax = 0;
@@ -1297,8 +1367,9 @@ extern "C" int bbhx_hip_direct_plan_create(bbhx_direct_plan** out, int numBinAll
     }
     // the default-grid t(f) of one (binary, mode) lives in LDS
     if ((size_t)Lmax * sizeof(double) > 48 * 1024) return ERR_ARGS;
-    auto* p = new bbhx_direct_plan;
+    auto p = std::make_unique<bbhx_direct_plan>();
     (void)hipGetDevice(&p->device);
+    p->lengths.assign(lengths_host, lengths_host + numBinAll);
     p->B = numBinAll;
     p->M = numModes;
     p->N = data_length;
@@ -1309,12 +1380,14 @@ extern "C" int bbhx_hip_direct_plan_create(bbhx_direct_plan** out, int numBinAll
                                                                          : min_chunk;
     p->S = S;
     p->max_items = (long)numBinAll * ((data_length + p->min_item - 1) / p->min_item) + numBinAll;
-    if (p->max_items > 2147483647L) {
-        delete p;
-        return ERR_ARGS;
-    }
+    if (p->max_items > 2147483647L) return ERR_ARGS;
+    std::vector<int> grid_b;
+    std::vector<int2> spl;
+    if (!lay_out_forward(p.get(), grid_b, spl)) return ERR_ARGS;
     bool ok = true;
     const size_t SM = (size_t)S * numModes;
+    p->grid_b = upload(grid_b, ok);
+    p->spl = upload(spl, ok);
     p->off = dalloc<long>(numBinAll, ok);
     p->len = dalloc<int>(numBinAll, ok);
     p->recs = dalloc<FusedRec>((size_t)numBinAll * numModes, ok);
@@ -1331,20 +1404,30 @@ extern "C" int bbhx_hip_direct_plan_create(bbhx_direct_plan** out, int numBinAll
     p->cnt = dalloc<int>((size_t)p->max_chunks + 1, ok);
     p->next = dalloc<int>(1, ok);
     if (!ok) {
-        plan_free(p);
-        delete p;
+        plan_free(p.get());
         return ERR_ALLOC;
     }
     if (hipMemcpy(p->off, off.data(), sizeof(long) * numBinAll, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(p->len, lengths_host, sizeof(int) * numBinAll, hipMemcpyHostToDevice) != hipSuccess) {
-        plan_free(p);
-        delete p;
+        plan_free(p.get());
         return ERR_LAUNCH;
     }
-    *out = p;
+    *out = p.release();
     return OK;
 }
 
+extern "C" int bbhx_hip_direct_plan_create(bbhx_direct_plan** out, int numBinAll, const int* lengths_host,
+                                           int numModes, int data_length, int min_chunk)
+{
+    if (!out || numBinAll < 1 || !lengths_host || numModes < 1 || numModes > MAX_MODES || data_length < 1 ||
+        min_chunk < 64)
+        return ERR_ARGS;
+    try {
+        return plan_create(out, numBinAll, lengths_host, numModes, data_length, min_chunk);
+    } catch (const std::bad_alloc&) {
+        return ERR_ALLOC;
+    }
+}
 extern "C" int bbhx_hip_direct_plan_destroy(bbhx_direct_plan* p)
 {
     if (!p) return ERR_ARGS;
@@ -1358,9 +1441,10 @@ extern "C" long bbhx_hip_direct_plan_bytes(const bbhx_direct_plan* p)
 {
     if (!p) return -1;
     const long SM = p->S * p->M;
-    long bytes = SM * 8 * (1 + RS + NQ) + (long)p->B * p->M * (sizeof(FusedRec) + 16) + p->max_items * 36 + p->B * 24 +
-                 4L * (p->max_chunks + 1);
-    if (p->Yadj) bytes += SM * 8 * NA + (long)p->B * p->M * (sizeof(bbhx::gradk::GradRec) + 8 * bbhx::gradk::NGRAD * bbhx::gradk::grad_chunks(p->Lmax));
+    long bytes = SM * 8 * (1 + RS + NQ) + (long)p->B * p->M * (sizeof(FusedRec) + 16) + p->max_items * 36 + p->B * 28 +
+                 8 * p->nspl + 4L * (p->max_chunks + 1);
+    if (p->Yadj)
+        bytes += SM * 8 * NA + (long)p->B * p->M * sizeof(gradk::GradRec) + p->B * 4 + p->nknots * (16 + 8 * gradk::NGRAD);
     return bytes;
 }
 
@@ -1412,12 +1496,22 @@ int direct_launch(bbhx_direct_plan* p, double* d_h, double* h_h, double* grad, i
     hipLaunchKernelGGL(k_dir_setup, dim3(setup_blocks(B, M)), dim3(64), 0, st, p->recs, params, B,
                        ml, M, qnm,
                        table_len, dspin);
-    const int grid_t = std::min(GRID_T, (p->Lmax + 63) / 64 * 64);
-    hipLaunchKernelGGL(k_dir_grid, dim3(B * M), dim3(grid_t), sizeof(double) * (size_t)p->Lmax, st, p->X, p->Yc,
-                       p->grid_lo, p->grid_istep, flags, p->recs, p->off, p->len, params, t_start, t_end, B, M, ml,
-                       orb, TDItag, rescaled, tdi2, initial_t_val, mf_min, mf_max);
-    const int nbmax = spline_blocks(p->Lmax);
-    hipLaunchKernelGGL(k_dir_spline, dim3((unsigned)((long)B * M * nbmax)), dim3(SPL_T), 0, st, p->X, p->Yc, reinterpret_cast<SegRec*>(p->Cf), p->off, p->len, t_start, t_end, M, nbmax);
+    int rc = OK;
+    for (const TablePart& part : p->grid_parts) {
+        if (rc != OK) return rc;
+        rc = launch_rows(part.count, M, part.threads, [&](long r, dim3 g) {
+            hipLaunchKernelGGL(k_dir_grid, g, dim3(part.threads), sizeof(double) * (size_t)part.lmax, st, p->X, p->Yc,
+                               p->grid_lo, p->grid_istep, flags, p->recs, p->grid_b + part.first + r, p->off, p->len,
+                               params, t_start, t_end, B, M, ml, orb, TDItag, rescaled, tdi2, initial_t_val, mf_min,
+                               mf_max);
+        });
+    }
+    if (rc == OK)
+        rc = launch_rows(p->nspl, 1, SPL_T, [&](long r, dim3 g) {
+            hipLaunchKernelGGL(k_dir_spline, g, dim3(SPL_T), 0, st, p->X, p->Yc, reinterpret_cast<SegRec*>(p->Cf),
+                               p->spl + r, p->off, p->len, t_start, t_end, M);
+        });
+    if (rc != OK) return rc;
     hipLaunchKernelGGL(k_dir_band, dim3(1), dim3(1024), 0, st, p->band, p->total, p->X, p->off, p->len, dataFreqs,
                        p->N, B, M, chunk);
     const int nchunks = (p->N + chunk - 1) / chunk;  // <= max_chunks since chunk >= min_item
@@ -1449,13 +1543,20 @@ int direct_launch(bbhx_direct_plan* p, double* d_h, double* h_h, double* grad, i
                        p->total, B);
     if (grad) {
         // the knot values' adjoints take the place of the values, which are not read again
-        hipLaunchKernelGGL(k_dirg_spline_adj, dim3((unsigned)((long)B * M * nbmax)), dim3(SPL_T), 0, st, p->Yc,
-                           p->Yadj, p->X, p->off, p->len, M, nbmax);
-        const int nc = gradk::grad_chunks(p->Lmax);
-        hipLaunchKernelGGL(k_dirg_knots, dim3((unsigned)((long)B * M * nc)), dim3(gradk::grad_threads(p->Lmax)), 0, st,
-                           p->gpart, p->grecs, p->Yc, p->X, p->off, p->len, params, B, M, nc, orb, TDItag, rescaled, tdi2, initial_t_val);
-        hipLaunchKernelGGL(k_dirg_reduce, dim3(B), dim3(64), 0, st, grad,
-                           p->gpart, p->len, B, M, nc);
+        rc = launch_rows(p->nspl, 1, SPL_T, [&](long r, dim3 g) {
+            hipLaunchKernelGGL(k_dirg_spline_adj, g, dim3(SPL_T), 0, st, p->Yc, p->Yadj, p->X, p->spl + r, p->off,
+                               p->len, M);
+        });
+        for (const TablePart& part : p->knot_parts) {
+            if (rc != OK) return rc;
+            rc = launch_rows(part.count, 1, part.threads, [&](long r, dim3 g) {
+                hipLaunchKernelGGL(k_dirg_knots, g, dim3(part.threads), 0, st, p->gpart, p->grecs, p->Yc, p->X,
+                                   p->knots + part.first + r, p->off, p->len, params, B, M, orb, TDItag, rescaled,
+                                   tdi2, initial_t_val);
+            });
+        }
+        if (rc != OK) return rc;
+        hipLaunchKernelGGL(k_dirg_reduce, dim3(B), dim3(64), 0, st, grad, p->gpart, p->gpart_b, B);
     }
     if (timed) (void)hipEventRecord(ev[2], st);
     return hipGetLastError() == hipSuccess ? OK : ERR_LAUNCH;
@@ -1485,23 +1586,40 @@ extern "C" int bbhx_hip_direct_plan_set_precision(bbhx_direct_plan* p, int preci
     return p && (precision == 0 || precision == 1) ? OK : ERR_ARGS;
 }
 
-extern "C" int bbhx_hip_direct_plan_enable_grad(bbhx_direct_plan* p)
+static int plan_enable_grad(bbhx_direct_plan* p)
 {
-    if (!p) return ERR_ARGS;
-    if (p->Yadj) return OK;
     bool ok = true;
+    std::vector<int4> knots;
+    std::vector<int> gpart_b;
+    if (!lay_out_knots(p, knots, gpart_b)) return ERR_ARGS;
+    p->nknots = (long)knots.size();
     p->Yadj = dalloc<double>((size_t)p->S * p->M * NA, ok);
     p->grecs = dalloc<gradk::GradRec>((size_t)p->B * p->M, ok);
-    p->gpart = dalloc<double>((size_t)p->B * p->M * gradk::NGRAD * gradk::grad_chunks(p->Lmax), ok);
+    p->gpart = dalloc<double>(knots.size() * gradk::NGRAD, ok);
+    p->knots = upload(knots, ok);
+    p->gpart_b = upload(gpart_b, ok);
     if (!ok) {
-        for (void* b : {(void*)p->Yadj, (void*)p->grecs, (void*)p->gpart})
+        for (void* b : {(void*)p->Yadj, (void*)p->grecs, (void*)p->gpart, (void*)p->knots, (void*)p->gpart_b})
             if (b) (void)hipFree(b);
         p->Yadj = nullptr;
         p->grecs = nullptr;
         p->gpart = nullptr;
+        p->knots = nullptr;
+        p->gpart_b = nullptr;
         return ERR_ALLOC;
     }
     return OK;
+}
+
+extern "C" int bbhx_hip_direct_plan_enable_grad(bbhx_direct_plan* p)
+{
+    if (!p) return ERR_ARGS;
+    if (p->Yadj) return OK;
+    try {
+        return plan_enable_grad(p);
+    } catch (const std::bad_alloc&) {
+        return ERR_ALLOC;
+    }
 }
 
 extern "C" int bbhx_hip_direct_fused_grad(bbhx_direct_plan* p, double* d_h, double* h_h, double* grad, int* flags,

@@ -7,6 +7,8 @@ import json
 import sys
 from pathlib import Path
 
+import numpy as np
+
 ROOT = Path(__file__).resolve().parent.parent
 sys.path.insert(0, str(ROOT))
 
@@ -25,6 +27,8 @@ class Library:
         """Status of an entry point; its launches as (kernel, grid, block, args)."""
         self.rec.recorder_clear(args_of.encode(), nargs)
         status = getattr(self.lib, "bbhx_hip_" + name)(*args)
+        if not self.rec.recorder_count():
+            return status
         self.launches = []
         for i in range(self.rec.recorder_count()):
             g = (C.c_uint64 * 6)()
@@ -40,13 +44,50 @@ def interpolate(lib, n, params, sets):
     return lib.call("interpolate", *p, n, params, 1, sets, None, args_of="k_spline", nargs=12)
 
 
-CASES = {"interpolate": interpolate}
+def direct(lib, groups, modes, bins, kernel, table, width, grad=False):
+    """A direct call on templates of (count, length) groups; also the entries of the work
+    table that argument ``table`` of the kernel's launches points to, ``width`` ints each."""
+    p = C.c_void_p(4096)
+    ints = lambda v: np.ascontiguousarray(v, dtype=np.int32).ctypes.data_as(C.POINTER(C.c_int))
+    lengths = np.concatenate([np.full(n, length, dtype=np.int32) for n, length in groups])
+    resp, plan = C.c_void_p(), C.c_void_p()
+    links = ints([12, 23, 31, 13, 32, 21])
+    assert lib.call("response_create", C.byref(resp)) == 0
+    assert lib.call("response_add_orbits", resp, 1e4, 100, p, p, p, links, links, links, 2.5e9) == 0
+    status = lib.call("direct_plan_create", C.byref(plan), len(lengths), ints(lengths), modes, bins, 1024)
+    if status == 0 and grad:
+        status = lib.call("direct_plan_enable_grad", plan)
+    if status:
+        return status
+    lm = np.array([(2, 2), (2, 1), (3, 3), (3, 2), (4, 4), (4, 3)][:modes], dtype=np.int32).T.copy()
+    out = [p] * (4 if grad else 3)
+    status = lib.call("direct_fused_grad" if grad else "direct_fused", plan, *out, p, p, p, ints(lm[0]), ints(lm[1]),
+                      modes, p, p, p, p, 1001, 2e-3, 0.0, 1e-4, 0.6, resp, 0, 0, 1, 16384, 256, 2048, None,
+                      args_of=kernel, nargs=table + 1)
+    rows = []
+    for k, grid, _, args in lib.launches:
+        if kernel in k:
+            buf = (C.c_int * (width * grid[0])).from_address(args[table])
+            rows.append(np.frombuffer(buf, dtype=np.int32).reshape(-1, width))
+    lib.extra = summary(np.concatenate(rows)) if rows else None
+    lib.call("direct_plan_destroy", plan)
+    return status
+
+
+def summary(table):
+    """A table's size, how many of its rows differ in the first two entries, and their range."""
+    key = table[:, 0].astype(np.int64) << 32 | table[:, 1]
+    return dict(size=len(table), distinct=len(np.unique(key)), low=table.min(0).tolist(), high=table.max(0).tolist())
+
+
+CASES = {"interpolate": interpolate, "direct": direct}
 
 
 if __name__ == "__main__":
     lib = Library(sys.argv[1])
     out = []
     for name, *args in json.loads(sys.argv[2]):
+        lib.launches, lib.extra = [], None
         status = CASES[name](lib, *args)
-        out.append(dict(status=status, launches=lib.launches))
+        out.append(dict(status=status, launches=lib.launches, table=lib.extra))
     print(json.dumps(out))

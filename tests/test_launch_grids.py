@@ -49,3 +49,43 @@ def test_spline_grids(record):
             done += grid[0] // blocks
         packs = -(-sets // (256 // n)) if n <= 128 else sets
         assert done == packs * (-(-params // 3) if params >= 3 else params)
+
+
+def spline_blocks(n):
+    return 1 if n <= 256 else 1 + -(-(n - 256) // 160)
+
+
+@pytest.mark.parametrize("groups,modes", [([(5, 64), (1, 4096), (3, 100)], 6), ([(1, 4), (2, 257)], 1),
+                                          ([(40, 300), (2, 256)], 3)])
+def test_direct_work_by_length(record, groups, modes):
+    """An uneven batch's launches hold the workgroups of its grids' own lengths and no others."""
+    cases = [("direct", groups, modes, 4096, *k) for k in
+             (("k_dir_spline", 3, 2), ("k_dirg_spline_adj", 3, 2, True), ("k_dirg_knots", 4, 4, True))]
+    spline, adj, knots = record(*cases)
+    work = modes * sum(n * spline_blocks(length) for n, length in groups)
+    binaries = sum(n for n, _ in groups)
+    for r in (spline, adj):
+        assert sum(g[0] for g, _, _ in launches(r, "k_dir_spline")) == work
+        assert r["table"] == dict(size=work, distinct=work, low=[0, 0],
+                                  high=[binaries * modes - 1, max(spline_blocks(n) for _, n in groups) - 1])
+    assert sum(g[0] for g, _, _ in launches(adj, "k_dirg_spline_adj")) == work
+    work = modes * sum(n * -(-length // 256) for n, length in groups)
+    assert sum(g[0] for g, _, _ in launches(knots, "k_dirg_knots")) == work
+    assert knots["table"]["size"] == knots["table"]["distinct"] == work
+    assert knots["table"]["high"][2] == work - 1
+    grid = {}
+    for n, length in groups:
+        lanes = 64 if length <= 64 else 128 if length <= 128 else 256
+        grid[lanes] = grid.get(lanes, 0) + n * modes
+    assert {b[0]: g[0] for g, b, _ in launches(spline, "k_dir_grid")} == grid
+
+
+def test_direct_grids_of_many_templates(record):
+    """More (template, mode) pairs than one launch of 256 lanes each holds."""
+    n = 2_900_000
+    forward, = record(("direct", [(n, 129)], 6, 1024, "k_dir_spline", 3, 2))
+    assert sum(g[0] for g, _, _ in launches(forward, "k_dir_grid")) == 6 * n
+    assert forward["table"] == dict(size=6 * n, distinct=6 * n, low=[0, 0], high=[6 * n - 1, 0])
+    grad, = record(("direct", [(n, 193)], 6, 1024, "k_dirg_knots", 4, 4, True))
+    assert sum(g[0] for g, _, _ in launches(grad, "k_dirg_knots")) == 6 * n
+    assert grad["table"]["distinct"] == 6 * n and grad["table"]["high"][2] == 6 * n - 1
