@@ -48,7 +48,7 @@ __global__ __launch_bounds__(SPL_T) void k_spline(const double* __restrict__ x, 
     const int blk = blockIdx.x % nb, e = e0 + blockIdx.x / nb, packs = PACK ? (nsub - 1) / G + 1 : nsub;
     const int set0 = PACK ? e % packs * G : e % packs, q0 = e / packs * NR;
     // this lane's set in the workgroup and its lanes
-    const int s = PACK ? t / n : 0, t0 = s * n, t1 = PACK ? t0 + n : T;
+    const int s = PACK ? t / n : 0, t0 = s * n, t1 = PACK ? min(t0 + n, T) : T;
     const bool any = !PACK || (s < G && set0 + s < nsub);
     const int sub = any ? set0 + s : set0;
     const int first = blk * SPL_U, i = any ? first + t - t0 : n, iy = min(i, n - 1);
