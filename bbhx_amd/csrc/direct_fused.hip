@@ -16,8 +16,8 @@
 //                 (phenomhm.py:208-224, :509-614), then amplitude, phase, t(f)
 //                 and the TDI response on the refitted grid (phenomhm.py:487-507,
 //                 Response.cu), written compact: nine values per (knot, mode)
-//   k_dir_spline  one workgroup per block of a (binary, mode)'s knots, one lane
-//                 per knot: not-a-knot spline coefficients (Interpolate.cu:15-359)
+//   k_dir_spline  one workgroup per block of a (binary, mode)'s knots, or for several
+//                 short grids, one lane per knot: not-a-knot spline coefficients (Interpolate.cu:15-359)
 //                 of the nine quantities by parallel cyclic reduction, from the
 //                 compact values; each record written once
 //   k_dir_band    dense band [st, et) of each binary (waveformbuild.py:139-156)
@@ -73,11 +73,11 @@ struct bbhx_direct_plan {
     // knots and one of 4096, as many workgroups for each of them and the tables: k_dirg_knots
     // 10.4 and 0.42 ms, k_dir_grid 0.65 and 0.29, k_dirg_spline_adj 0.55 and 0.41.
     int* grid_b = nullptr;     // (B,) binaries by size of their k_dir_grid workgroup
-    int2* spl = nullptr;       // {b M + m, block} of each workgroup of the spline kernels
+    int4* spl = nullptr;       // workgroups of the spline kernels (SplineRows): blocks, then packs
     int4* knots = nullptr;     // {b M + m, first knot, row of gpart} of each of k_dirg_knots'
     int* gpart_b = nullptr;    // (B + 1,) first row of gpart of each binary
     TablePart grid_parts[3], knot_parts[4];
-    long nspl = 0, nknots = 0;
+    long nspl = 0, nblocks = 0, nknots = 0;
     FusedRec* recs = nullptr;
     double* X = nullptr;   // (S, M)
     double* Cf = nullptr;  // (S, M, RS): segment records (bounds, value and cubic coefficients)
@@ -326,44 +326,60 @@ __device__ inline int segment_window(const Cubic& c, double h, double ts, double
 // 9.4 M records: 1.7 ms; 64 of 4096 knots: 0.2 ms). Thomas sweeps, one lane per (mode,
 // quantity), are one chain over all knots: 537 us, 3.1 ms and 2.24 ms.
 
-// The rows of one workgroup of a spline kernel: block 'blk' of (binary b, mode m), by
-// its entry of the plan's table.
-struct SplineRows {
-    int b, m, n, first, row0, row1;  // loaded rows [first, first + T), results for [row0, row1)
+// This lane's row in a spline kernel, by the workgroup's entry of the plan's table.
+// A block {b M + m, 1, T, block}: T rows of one (binary, mode). A pack {b M + m, sets, lanes
+// per set, 0}: whole grids of at most T / 2 knots, of (binary, mode) pairs from b M + m on,
+// side by side; with a workgroup for each of them, 16384 templates of 16 knots take 1.71
+// ms instead of 0.15 (a lane per (mode, quantity), by Thomas sweeps: 0.26).
+struct SplineRow {
+    int b, m, n, i, s;  // knot i of the n of (binary b, mode m); set s of the workgroup
+    int t0, t1;         // lanes of the set
+    int row0, row1;     // rows of the grid that this workgroup finishes
+    bool any, out;      // i is a row of the grid; one of those
 };
-__device__ inline SplineRows spline_rows(const int2* __restrict__ spl, const int* __restrict__ len, int M)
+template <bool PACK>
+__device__ inline SplineRow spline_row(const int4* __restrict__ spl, const int* __restrict__ len, int M)
 {
     constexpr int T = SPL_T;
-    SplineRows w;
-    const int bm = spl[blockIdx.x].x, blk = spl[blockIdx.x].y;
+    const int4 e = spl[blockIdx.x];
+    const int t = threadIdx.x;
+    SplineRow w;
+    w.s = PACK ? t / e.z : 0;
+    const bool set = !PACK || w.s < e.y;
+    const int bm = PACK && set ? e.x + w.s : e.x;
     w.b = bm / M;
     w.m = bm % M;
     w.n = len[w.b];
-    const int nb = spline_blocks(w.n);
-    w.first = blk * SPL_U;
-    w.row0 = blk == 0 ? 0 : w.first + SPL_W;
-    w.row1 = blk == nb - 1 ? w.n : w.first + T - SPL_W;
+    w.t0 = w.s * e.z;
+    w.t1 = PACK ? min(w.t0 + e.z, T) : T;
+    const int first = PACK ? 0 : e.w * SPL_U;
+    w.i = set ? first + t - w.t0 : w.n;
+    w.row0 = PACK || e.w == 0 ? 0 : first + SPL_W;
+    w.row1 = PACK || e.w == spline_blocks(w.n) - 1 ? w.n : first + T - SPL_W;
+    w.any = w.i < w.n;
+    w.out = w.i >= w.row0 && w.i < w.row1;
     return w;
 }
+constexpr int SPL_SETS = SPL_T / 4;  // sets of a pack
 
 // Not-a-knot splines of the nine quantities of one (binary, mode) (the system of
 // spline.hip), one lane per knot. The two end rows are folded into their
 // neighbours, which leaves every row dominant: s_0 = (b_0 - (h_0 + h_1) s_1) / h_1.
+template <bool PACK>
 __global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void k_dir_spline(const double* __restrict__ X, const double* __restrict__ Yc,
-                                                    SegRec* __restrict__ Cf, const int2* __restrict__ spl,
+                                                    SegRec* __restrict__ Cf, const int4* __restrict__ spl,
                                                     const long* __restrict__ off, const int* __restrict__ len,
                                                     const double* __restrict__ t_start,
                                                     const double* __restrict__ t_end, int M)
 {
     constexpr int T = SPL_T;
     __shared__ __align__(16) double sh[(NQ + 2) * T];
-    __shared__ double ends[2][NQ];  // right sides of the two end rows
+    __shared__ double ends[2][NQ][PACK ? SPL_SETS : 1];  // right sides of the sets' two end rows
     const int t = threadIdx.x;
-    const SplineRows w = spline_rows(spl, len, M);
-    const int i = w.first + t, n = w.n;
+    const SplineRow w = spline_row<PACK>(spl, len, M);
+    const int i = w.i, n = w.n, s = w.s;
     const long base = off[w.b];
-    const bool row = i < n;
-    const long p = (base + (row ? i : n - 1)) * M + w.m;
+    const long p = (base + (w.any ? i : n - 1)) * M + w.m;
     const double x = X[p];
     double y[NQ];
 #pragma unroll
@@ -396,23 +412,23 @@ __global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void
         mr[q] = (sh[(1 + q) * T + th] - y[q]) * ir;
         double v = 3.0 * (hr * ml + hl * mr[q]);
         if (low) {
-            ends[0][q] = e0l * ml + e0r * mr[q];
-            v -= ends[0][q];
+            ends[0][q][s] = e0l * ml + e0r * mr[q];
+            v -= ends[0][q][s];
         }
         if (high) {
-            ends[1][q] = e1l * ml + e1r * mr[q];
-            v -= ends[1][q];
+            ends[1][q][s] = e1l * ml + e1r * mr[q];
+            v -= ends[1][q][s];
         }
         r[q] = solve ? v * ib : 0.0;
     }
     __syncthreads();
-    pcr_solve(a, c, r, sh, t, 0, T);
+    pcr_solve(a, c, r, sh, t, w.t0, w.t1);
     // slopes to the neighbours, the end ones from their rows
 #pragma unroll
     for (int q = 0; q < NQ; q++) {
         if (i != 0 && i < n - 1) sh[q * T + t] = r[q];
-        if (low) sh[q * T + t - 1] = (ends[0][q] - d * r[q]) * ir;
-        if (high) sh[q * T + t + 1] = (ends[1][q] - d * r[q]) * il;
+        if (low) sh[q * T + t - 1] = (ends[0][q][s] - d * r[q]) * ir;
+        if (high) sh[q * T + t + 1] = (ends[1][q][s] - d * r[q]) * il;
     }
     __syncthreads();
     const bool end = i == n - 1;
@@ -420,9 +436,9 @@ __global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void
     Cubic k[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; q++) {
-        const double s = sh[q * T + t], sn = sh[q * T + th];
-        const double u = (s + sn - 2.0 * mr[q]) * ir;
-        k[q] = end ? Cubic{y[q], 0.0, 0.0, 0.0} : Cubic{y[q], s, (mr[q] - s) * ir - u, u * ir};
+        const double sl = sh[q * T + t], sn = sh[q * T + th];
+        const double u = (sl + sn - 2.0 * mr[q]) * ir;
+        k[q] = end ? Cubic{y[q], 0.0, 0.0, 0.0} : Cubic{y[q], sl, (mr[q] - sl) * ir - u, u * ir};
         if (q == 2 && !end) win = segment_window(k[q], hr, t_start[w.b], t_end[w.b]);
     }
     __syncthreads();
@@ -431,7 +447,9 @@ __global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void
     // the kernel waits on the number of requests: 2.1 against 1.7 ms at 1024)
     constexpr int PER = 16, PITCH = RS + 2;  // doubles, padded against bank conflicts
     static_assert(4 * PER * PITCH <= (NQ + 2) * T, "the records of a workgroup's wavefronts fit in sh");
-    const int lane = t & 63, i0 = w.first + (t & ~63);
+    const int lane = t & 63;
+    __shared__ long rec[PACK ? T : 1];  // the rows' records, -1: none
+    if (PACK) rec[t] = w.out ? p : -1;
     double* own = sh + (t >> 6) * PER * PITCH;
     for (int g = 0; g < 64; g += PER) {
         if (lane >= g && lane < g + PER) {
@@ -452,9 +470,10 @@ __global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void
         __syncthreads();
         for (int e = lane; e < PER * RS / 2; e += 64) {
             const int j = e / (RS / 2), c = e - j * (RS / 2);
-            const int ij = i0 + g + j;
-            if (ij >= w.row0 && ij < w.row1)
-                reinterpret_cast<double2*>(Cf + (base + ij) * M + w.m)[c] = *reinterpret_cast<const double2*>(own + j * PITCH + 2 * c);
+            const int ij = i - lane + g + j;
+            const long pj = PACK ? rec[(t & ~63) + g + j] : (ij >= w.row0 && ij < w.row1 ? (base + ij) * M + w.m : -1);
+            if (pj >= 0)
+                reinterpret_cast<double2*>(Cf + pj)[c] = *reinterpret_cast<const double2*>(own + j * PITCH + 2 * c);
         }
         __syncthreads();
     }
@@ -1089,18 +1108,19 @@ __global__ __launch_bounds__(64) void k_dirg_setup(gradk::GradRec* __restrict__ 
 // Bound by the records' reads (288 B per (knot, mode), one lane's at a time) and the
 // exchanges: 256 uneven templates, 2.36 M records: 0.66 ms (0.16 ms at the rate of a
 // copy). Thomas sweeps, one lane per (mode, quantity): 8.7 ms.
+template <bool PACK>
 __global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void k_dirg_spline_adj(
     double* __restrict__ Ya, const double* __restrict__ Yadj, const double* __restrict__ X,
-    const int2* __restrict__ spl, const long* __restrict__ off, const int* __restrict__ len, int M)
+    const int4* __restrict__ spl, const long* __restrict__ off, const int* __restrict__ len, int M)
 {
     constexpr int T = SPL_T, NA8 = 8;
     __shared__ double sh[(NA8 + 2) * T];
     const int t = threadIdx.x;
-    const SplineRows w = spline_rows(spl, len, M);
-    const int i = w.first + t, n = w.n;
+    const SplineRow w = spline_row<PACK>(spl, len, M);
+    const int i = w.i, n = w.n;
     const long base = off[w.b];
-    const bool row = i < n, seg = i < n - 1;  // knot i, segment i
-    const long p = (base + (row ? i : n - 1)) * M + w.m;
+    const bool seg = i < n - 1;  // segment i
+    const long p = (base + (w.any ? i : n - 1)) * M + w.m;
     const double x = X[p];
     sh[t] = x;
     __syncthreads();
@@ -1161,7 +1181,7 @@ __global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void
     for (int q = 0; q < NA8; q++) zl[q] = low ? sh[q * T + t - 1] * iel : (high ? sh[q * T + t + 1] * ieh : 0.0);
     // (a grid of four knots has two such rows, in different lanes)
     __syncthreads();
-    pcr_solve(a, c, z, sh, t, 0, T);
+    pcr_solve(a, c, z, sh, t, w.t0, w.t1);
 #pragma unroll
     for (int q = 0; q < NA8; q++) {
         if (i != 0 && i < n - 1) sh[q * T + t] = z[q];
@@ -1189,7 +1209,7 @@ __global__ __launch_bounds__(SPL_T) __attribute__((amdgpu_waves_per_eu(4))) void
 #pragma unroll
     for (int q = 0; q < NA8; q++) sh[q * T + t] = cy[q];
     __syncthreads();
-    if (!row || i < w.row0 || i >= w.row1) return;
+    if (!w.out) return;
 #pragma unroll
     for (int q = 0; q < NA8; q++)
         Ya[p * NQ + adj_q(q)] = yb[q] - cy[q] + (i > 0 ? sh[q * T + t - 1] : 0.0);
@@ -1278,8 +1298,8 @@ T* upload(const std::vector<T>& v, bool& ok)
 }
 
 // Binaries by the lanes that k_dir_grid takes for their knots, 64, 128 or GRID_T, and the
-// blocks of the spline kernels; false: more of these than a table holds.
-bool lay_out_forward(bbhx_direct_plan* p, std::vector<int>& grid_b, std::vector<int2>& spl)
+// workgroups of the spline kernels; false: more of these than a table holds.
+bool lay_out_forward(bbhx_direct_plan* p, std::vector<int>& grid_b, std::vector<int4>& spl)
 {
     for (int c = 0; c < 3; c++) {
         TablePart& part = p->grid_parts[c];
@@ -1294,8 +1314,19 @@ bool lay_out_forward(bbhx_direct_plan* p, std::vector<int>& grid_b, std::vector<
         part.count = (long)grid_b.size() - part.first;
     }
     for (int b = 0; b < p->B; b++)
-        for (int m = 0; m < p->M; m++)
-            for (int blk = 0; blk < spline_blocks(p->lengths[b]); blk++) spl.push_back({b * p->M + m, blk});
+        for (int m = 0; m < p->M && 2 * p->lengths[b] > SPL_T; m++)
+            for (int blk = 0; blk < spline_blocks(p->lengths[b]); blk++) spl.push_back({b * p->M + m, 1, SPL_T, blk});
+    p->nblocks = (long)spl.size();
+    for (int b = 0; b < p->B; b++)
+        for (int m = 0; m < p->M && 2 * p->lengths[b] <= SPL_T; m++) {
+            const int bm = b * p->M + m, n = p->lengths[b];
+            int4* last = (long)spl.size() > p->nblocks ? &spl.back() : nullptr;
+            if (last && last->x + last->y == bm && (last->y + 1) * std::max(last->z, n) <= SPL_T) {
+                last->y++;
+                last->z = std::max(last->z, n);
+            } else
+                spl.push_back({bm, 1, n, 0});
+        }
     p->nspl = (long)spl.size();
     return p->nspl <= 2147483647L;
 }
@@ -1382,7 +1413,7 @@ static int plan_create(bbhx_direct_plan** out, int numBinAll, const int* lengths
     p->max_items = (long)numBinAll * ((data_length + p->min_item - 1) / p->min_item) + numBinAll;
     if (p->max_items > 2147483647L) return ERR_ARGS;
     std::vector<int> grid_b;
-    std::vector<int2> spl;
+    std::vector<int4> spl;
     if (!lay_out_forward(p.get(), grid_b, spl)) return ERR_ARGS;
     bool ok = true;
     const size_t SM = (size_t)S * numModes;
@@ -1442,7 +1473,7 @@ extern "C" long bbhx_hip_direct_plan_bytes(const bbhx_direct_plan* p)
     if (!p) return -1;
     const long SM = p->S * p->M;
     long bytes = SM * 8 * (1 + RS + NQ) + (long)p->B * p->M * (sizeof(FusedRec) + 16) + p->max_items * 36 + p->B * 28 +
-                 8 * p->nspl + 4L * (p->max_chunks + 1);
+                 16 * p->nspl + 4L * (p->max_chunks + 1);
     if (p->Yadj)
         bytes += SM * 8 * NA + (long)p->B * p->M * sizeof(gradk::GradRec) + p->B * 4 + p->nknots * (16 + 8 * gradk::NGRAD);
     return bytes;
@@ -1463,6 +1494,16 @@ extern "C" int bbhx_hip_direct_plan_band(const bbhx_direct_plan* p, int* band_ho
 }
 
 namespace {
+
+// The launches of a spline kernel, for blocks and for packs
+template <class Kernel, class Launch>
+int spline_launches(const bbhx_direct_plan* p, Kernel blocks, Kernel packs, Launch launch)
+{
+    const int rc = launch_rows(p->nblocks, 1, SPL_T, [&](long r, dim3 g) { launch(blocks, p->spl + r, g); });
+    if (rc != OK) return rc;
+    return launch_rows(p->nspl - p->nblocks, 1, SPL_T,
+                       [&](long r, dim3 g) { launch(packs, p->spl + p->nblocks + r, g); });
+}
 
 // The launch sequence of the fused direct likelihood; with grad != nullptr
 // also its gradient (the plan's gradient buffers must exist).
@@ -1507,9 +1548,9 @@ int direct_launch(bbhx_direct_plan* p, double* d_h, double* h_h, double* grad, i
         });
     }
     if (rc == OK)
-        rc = launch_rows(p->nspl, 1, SPL_T, [&](long r, dim3 g) {
-            hipLaunchKernelGGL(k_dir_spline, g, dim3(SPL_T), 0, st, p->X, p->Yc, reinterpret_cast<SegRec*>(p->Cf),
-                               p->spl + r, p->off, p->len, t_start, t_end, M);
+        rc = spline_launches(p, k_dir_spline<false>, k_dir_spline<true>, [&](auto kernel, const int4* spl, dim3 g) {
+            hipLaunchKernelGGL(kernel, g, dim3(SPL_T), 0, st, p->X, p->Yc, reinterpret_cast<SegRec*>(p->Cf), spl,
+                               p->off, p->len, t_start, t_end, M);
         });
     if (rc != OK) return rc;
     hipLaunchKernelGGL(k_dir_band, dim3(1), dim3(1024), 0, st, p->band, p->total, p->X, p->off, p->len, dataFreqs,
@@ -1543,10 +1584,11 @@ int direct_launch(bbhx_direct_plan* p, double* d_h, double* h_h, double* grad, i
                        p->total, B);
     if (grad) {
         // the knot values' adjoints take the place of the values, which are not read again
-        rc = launch_rows(p->nspl, 1, SPL_T, [&](long r, dim3 g) {
-            hipLaunchKernelGGL(k_dirg_spline_adj, g, dim3(SPL_T), 0, st, p->Yc, p->Yadj, p->X, p->spl + r, p->off,
-                               p->len, M);
-        });
+        rc = spline_launches(p, k_dirg_spline_adj<false>, k_dirg_spline_adj<true>,
+                             [&](auto kernel, const int4* spl, dim3 g) {
+                                 hipLaunchKernelGGL(kernel, g, dim3(SPL_T), 0, st, p->Yc, p->Yadj, p->X, spl, p->off,
+                                                    p->len, M);
+                             });
         for (const TablePart& part : p->knot_parts) {
             if (rc != OK) return rc;
             rc = launch_rows(part.count, 1, part.threads, [&](long r, dim3 g) {

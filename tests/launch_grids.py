@@ -77,7 +77,8 @@ def direct(lib, groups, modes, bins, kernel, table, width, grad=False):
 def summary(table):
     """A table's size, how many of its rows differ in the first two entries, and their range."""
     key = table[:, 0].astype(np.int64) << 32 | table[:, 1]
-    return dict(size=len(table), distinct=len(np.unique(key)), low=table.min(0).tolist(), high=table.max(0).tolist())
+    out = dict(size=len(table), distinct=len(np.unique(key)), low=table.min(0).tolist(), high=table.max(0).tolist())
+    return dict(table=out, rows=table.tolist() if len(table) < 10000 else None)
 
 
 CASES = {"interpolate": interpolate, "direct": direct}
@@ -89,5 +90,5 @@ if __name__ == "__main__":
     for name, *args in json.loads(sys.argv[2]):
         lib.launches, lib.extra = [], None
         status = CASES[name](lib, *args)
-        out.append(dict(status=status, launches=lib.launches, table=lib.extra))
+        out.append(dict(status=status, launches=lib.launches, **(lib.extra or {})))
     print(json.dumps(out))

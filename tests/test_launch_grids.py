@@ -56,19 +56,28 @@ def spline_blocks(n):
 
 
 @pytest.mark.parametrize("groups,modes", [([(5, 64), (1, 4096), (3, 100)], 6), ([(1, 4), (2, 257)], 1),
-                                          ([(40, 300), (2, 256)], 3)])
+                                          ([(40, 300), (2, 129)], 3), ([(70, 4), (3, 128), (9, 5)], 6)])
 def test_direct_work_by_length(record, groups, modes):
     """An uneven batch's launches hold the workgroups of its grids' own lengths and no others."""
     cases = [("direct", groups, modes, 4096, *k) for k in
-             (("k_dir_spline", 3, 2), ("k_dirg_spline_adj", 3, 2, True), ("k_dirg_knots", 4, 4, True))]
+             (("k_dir_spline", 3, 4), ("k_dirg_spline_adj", 3, 4, True), ("k_dirg_knots", 4, 4, True))]
     spline, adj, knots = record(*cases)
-    work = modes * sum(n * spline_blocks(length) for n, length in groups)
-    binaries = sum(n for n, _ in groups)
-    for r in (spline, adj):
-        assert sum(g[0] for g, _, _ in launches(r, "k_dir_spline")) == work
-        assert r["table"] == dict(size=work, distinct=work, low=[0, 0],
-                                  high=[binaries * modes - 1, max(spline_blocks(n) for _, n in groups) - 1])
-    assert sum(g[0] for g, _, _ in launches(adj, "k_dirg_spline_adj")) == work
+    lengths = [length for n, length in groups for _ in range(n)]
+    for r, kernel in ((spline, "k_dir_spline"), (adj, "k_dirg_spline_adj")):
+        want = [(b * modes + m, k) for b, n in enumerate(lengths) if n > 128 for m in range(modes)
+                for k in range(spline_blocks(n))]
+        blocks = len(want)
+        rows, got = r["rows"], []
+        assert sum(g[0] for g, _, _ in launches(r, kernel)) == len(rows)
+        for first, sets, lanes, block in rows[:blocks]:
+            assert (sets, lanes) == (1, 256)
+            got.append((first, block))
+        want += [(b * modes + m, 0) for b, n in enumerate(lengths) if n <= 128 for m in range(modes)]
+        for first, sets, lanes, block in rows[blocks:]:
+            assert sets * lanes <= 256 and block == 0
+            assert lanes == max(lengths[(first + k) // modes] for k in range(sets))
+            got += [(first + k, 0) for k in range(sets)]
+        assert got == want
     work = modes * sum(n * -(-length // 256) for n, length in groups)
     assert sum(g[0] for g, _, _ in launches(knots, "k_dirg_knots")) == work
     assert knots["table"]["size"] == knots["table"]["distinct"] == work
@@ -80,12 +89,17 @@ def test_direct_work_by_length(record, groups, modes):
     assert {b[0]: g[0] for g, b, _ in launches(spline, "k_dir_grid")} == grid
 
 
+def test_short_direct_grids_share_workgroups(record):
+    r, = record(("direct", [(1000, 16)], 6, 1024, "k_dir_spline", 3, 4))
+    assert [g[0] for g, _, _ in launches(r, "k_dir_spline")] == [6000 // 16]
+
+
 def test_direct_grids_of_many_templates(record):
     """More (template, mode) pairs than one launch of 256 lanes each holds."""
     n = 2_900_000
-    forward, = record(("direct", [(n, 129)], 6, 1024, "k_dir_spline", 3, 2))
+    forward, = record(("direct", [(n, 129)], 6, 1024, "k_dir_spline", 3, 4))
     assert sum(g[0] for g, _, _ in launches(forward, "k_dir_grid")) == 6 * n
-    assert forward["table"] == dict(size=6 * n, distinct=6 * n, low=[0, 0], high=[6 * n - 1, 0])
+    assert forward["table"] == dict(size=6 * n, distinct=6 * n, low=[0, 1, 256, 0], high=[6 * n - 1, 1, 256, 0])
     grad, = record(("direct", [(n, 193)], 6, 1024, "k_dirg_knots", 4, 4, True))
     assert sum(g[0] for g, _, _ in launches(grad, "k_dirg_knots")) == 6 * n
     assert grad["table"]["distinct"] == 6 * n and grad["table"]["high"][2] == 6 * n - 1
