@@ -633,8 +633,10 @@ __device__ inline bool grad_resp_part(const GradResp& R, const resp::OrbitTab& o
     return true;
 }
 
-// The kernels that sum grad_point_core over the points of one (binary, mode) take a
-// workgroup of up to GRAD_T lanes per GRAD_T points, one point per lane.
+// The kernels that sum grad_point_core over the points of one (binary, mode) take one
+// point per lane, workgroups of up to GRAD_T lanes: as few as that allows, the wavefronts
+// spread evenly over them, as idle ones of a last workgroup would hold their registers
+// until the others are done.
 //
 // Bound by FP64 issue and latency at two wavefronts per SIMD. A loop over points in a lane
 // keeps the point-independent constants and record entries in registers, 460 VGPRs and
@@ -644,7 +646,7 @@ __device__ inline bool grad_resp_part(const GradResp& R, const resp::OrbitTab& o
 constexpr int GRAD_T = 256;
 constexpr int GRAD_STASH = 3 * NI;
 __host__ __device__ inline int grad_chunks(int n) { return (n + GRAD_T - 1) / GRAD_T; }
-inline int grad_threads(int n) { return n < GRAD_T ? (n + 63) / 64 * 64 : GRAD_T; }
+inline int grad_threads(int n) { return 64 * (((n + 63) / 64 - 1) / grad_chunks(n) + 1); }
 
 struct GradShared {
     double2 tab[129];

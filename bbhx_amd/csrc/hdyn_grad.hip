@@ -180,16 +180,16 @@ __global__ __launch_bounds__(64 * MAX_RESIDUAL_WAVES) __attribute__((amdgpu_wave
     }
 }
 
-// Gradient contributions of one (template, mode) and chunk of up to GRAD_T nodes:
-// partial[((b * M + m) * chunks + chunk) * 11 + p].
+// Gradient contributions of one (template, mode) and chunk of as many nodes as lanes,
+// the nc chunks from node k0 on in this launch: partial[((b * M + m) * chunks + c0 + chunk) * 11 + p].
 __global__ __launch_bounds__(GRAD_T) __attribute__((amdgpu_waves_per_eu(2))) void k_grad_points(
     double* __restrict__ partial, const GradRec* __restrict__ grecs, const cd* __restrict__ gw,
     const double* __restrict__ params, const double* __restrict__ t_start, const double* __restrict__ t_end, int B,
     int M, const double* __restrict__ freqs, int K, resp::OrbitTab orb, int TDItag, int rescaled, int tdi2,
-    double initial_t_val)
+    double initial_t_val, int k0, int c0, int nc)
 {
     __shared__ GradShared sh;
-    const int chunks = grad_chunks(K), bm = blockIdx.x / chunks, chunk = blockIdx.x % chunks;
+    const int bm = blockIdx.x / nc, chunk = blockIdx.x % nc;
     const int b = bm / M;
     Window win;
     win.t_ref = params[P_TREF * B + b];
@@ -200,11 +200,11 @@ __global__ __launch_bounds__(GRAD_T) __attribute__((amdgpu_waves_per_eu(2))) voi
     const GradRec& G = grad_stage(sh, grecs + bm);
     double acc[NGRAD];
     for (int p = 0; p < NGRAD; p++) acc[p] = 0.0;
-    const int j = chunk * GRAD_T + threadIdx.x;
+    const int j = k0 + chunk * blockDim.x + threadIdx.x;
     if (j < K)
         grad_point(G, orb, freqs[j], win, gw + (long)b * 3 * K + j, K, TDItag, rescaled, tdi2, dist, acc, sh.tab,
                    sh.tan + threadIdx.x, blockDim.x);
-    grad_sum(sh, acc, partial + (long)blockIdx.x * NGRAD);
+    grad_sum(sh, acc, partial + ((long)bm * grad_chunks(K) + c0 + chunk) * NGRAD);
 }
 
 // grad[p * B + b] = sum over the modes' chunks, in order
@@ -299,9 +299,21 @@ extern "C" int bbhx_hip_hdyn_fused_grad(double* d_h, double* h_h, double* grad, 
     hipLaunchKernelGGL(residual_split(waves, K) ? k_grad_weights<true> : k_grad_weights<false>, dim3(numBinAll), dim3(64 * waves), residual_lds(waves, K), st, d_h, h_h, logL, d_d, gw, recs, params, t_start, t_end,
                        numBinAll, ml, numModes, freqs, nw, K, orb, TDItag, rescaled, tdi2, initial_t_val);
     if (hipStreamWaitEvent(st, side->join, 0) != hipSuccess) return ERR_LAUNCH;
-    const int chunks = grad_chunks(K);
-    hipLaunchKernelGGL(k_grad_points, dim3((unsigned)(nrec * (long)chunks)), dim3(grad_threads(K)), 0, st, partial, grecs, gw, params, t_start, t_end,
-                       numBinAll, numModes, freqs, K, orb, TDItag, rescaled, tdi2, initial_t_val);
+    // Full workgroups and the nodes left over, if those fill none, in launches of their own
+    // where the first fill the chip several times (512 at once); fewer would just run one
+    // after the other. 2048 templates of 257 to 300 nodes: 457 us, 558 with the wavefronts
+    // spread evenly over the workgroups, 653 with idle ones in the last.
+    const int chunks = grad_chunks(K), full = K / GRAD_T, rest = K - full * GRAD_T;
+    auto points = [&](int k0, int c0, int nc, int threads) {
+        hipLaunchKernelGGL(k_grad_points, dim3((unsigned)(nrec * (long)nc)), dim3(threads), 0, st, partial, grecs, gw,
+                           params, t_start, t_end, numBinAll, numModes, freqs, K, orb, TDItag, rescaled, tdi2,
+                           initial_t_val, k0, c0, nc);
+    };
+    if (full > 0 && rest > 0 && rest <= GRAD_T - 64 && (long)nrec * full >= 4096) {
+        points(0, 0, full, GRAD_T);
+        points(full * GRAD_T, full, 1, grad_threads(rest));
+    } else
+        points(0, 0, chunks, grad_threads(K));
     hipLaunchKernelGGL(k_grad_reduce, dim3(ceil_div((long)numBinAll * NGRAD, 256)), dim3(256), 0, st, grad, partial,
                        numBinAll, numModes * chunks);
     if (timed) (void)hipEventRecord(ev[2], st);
