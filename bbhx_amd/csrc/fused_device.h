@@ -393,27 +393,29 @@ __device__ inline void node_sums(const cd* rs, const NodeW* __restrict__ nw, int
     }
 }
 
-// Wavefronts per template of the residual pass (workgroup of 64 x that many
-// threads): enough for about 2048 wavefronts in the launch (two per SIMD of
-// MI355X's 1024), at most one per mode and 64 nodes and at most MAX_RESIDUAL_WAVES.
-// One for up to 64 nodes, where a template's result so does not depend on the batch.
-// The forward and the gradient's weights pass use the same count, so their
-// sums agree bit for bit.
-inline int residual_waves(int B, int K, int M)
-{
-    int nw = (2048 + B - 1) / B;
-    const int most = K > 64 ? (K + 63) / 64 * M : 1;
-    nw = nw < most ? nw : most;
-    nw = nw < MAX_RESIDUAL_WAVES ? nw : MAX_RESIDUAL_WAVES;
-    return nw > 1 ? nw : 1;
-}
-
 // Whether the last pass of that many wavefronts spreads its modes over the lanes
 inline bool residual_split(int waves, int K)
 {
     int R = K;
     while (residual_full(R, 64 * waves)) R -= 64 * waves;
     return R > 0;
+}
+
+// Wavefronts per template of the residual pass (workgroup of 64 x that many
+// threads): enough for about 2048 wavefronts in the launch (two per SIMD of
+// MI355X's 1024), at most one per mode and 64 nodes (one per 64 nodes where the modes are
+// not spread, as the others would only wait) and at most MAX_RESIDUAL_WAVES.
+// One for up to 64 nodes, where a template's result so does not depend on the batch.
+// The forward and the gradient's weights pass use the same count, so their
+// sums agree bit for bit.
+inline int residual_waves(int B, int K, int M)
+{
+    int nw = (2048 + B - 1) / B;
+    const int nodes = (K + 63) / 64, most = K > 64 ? nodes * M : 1;
+    nw = nw < most ? nw : most;
+    nw = nw < MAX_RESIDUAL_WAVES ? nw : MAX_RESIDUAL_WAVES;
+    if (nw > nodes && !residual_split(nw, K)) nw = nodes;
+    return nw > 1 ? nw : 1;
 }
 
 // LDS of the residual pass with that many wavefronts: rs, then part

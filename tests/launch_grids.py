@@ -44,22 +44,43 @@ def interpolate(lib, n, params, sets):
     return lib.call("interpolate", *p, n, params, 1, sets, None, args_of="k_spline", nargs=12)
 
 
+def ints(v):
+    return np.ascontiguousarray(v, dtype=np.int32).ctypes.data_as(C.POINTER(C.c_int))
+
+
+def mode_list(modes):
+    return np.array([(2, 2), (2, 1), (3, 3), (3, 2), (4, 4), (4, 3)][:modes], dtype=np.int32).T.copy()
+
+
+def response(lib):
+    resp, p = C.c_void_p(), C.c_void_p(4096)
+    links = ints([12, 23, 31, 13, 32, 21])
+    assert lib.call("response_create", C.byref(resp)) == 0
+    assert lib.call("response_add_orbits", resp, 1e4, 100, p, p, p, links, links, links, 2.5e9) == 0
+    return resp
+
+
+def heterodyned(lib, batch, nodes, modes, grad=False):
+    p, lm, resp = C.c_void_p(4096), mode_list(modes), response(lib)
+    args = [*([p] * (6 if grad else 5)), batch, ints(lm[0]), ints(lm[1]), modes, p, p, p, nodes, p, 1001, 2e-3, 0.0,
+            resp, 0, 0, 1, 0]
+    if grad:
+        return lib.call("hdyn_fused_grad", *args, p, 0.0, None, args_of="k_grad_points", nargs=18)
+    return lib.call("hdyn_fused", *args, 0, p, 0.0, None)
+
+
 def direct(lib, groups, modes, bins, kernel, table, width, grad=False):
     """A direct call on templates of (count, length) groups; also the entries of the work
     table that argument ``table`` of the kernel's launches points to, ``width`` ints each."""
     p = C.c_void_p(4096)
-    ints = lambda v: np.ascontiguousarray(v, dtype=np.int32).ctypes.data_as(C.POINTER(C.c_int))
     lengths = np.concatenate([np.full(n, length, dtype=np.int32) for n, length in groups])
-    resp, plan = C.c_void_p(), C.c_void_p()
-    links = ints([12, 23, 31, 13, 32, 21])
-    assert lib.call("response_create", C.byref(resp)) == 0
-    assert lib.call("response_add_orbits", resp, 1e4, 100, p, p, p, links, links, links, 2.5e9) == 0
+    resp, plan = response(lib), C.c_void_p()
     status = lib.call("direct_plan_create", C.byref(plan), len(lengths), ints(lengths), modes, bins, 1024)
     if status == 0 and grad:
         status = lib.call("direct_plan_enable_grad", plan)
     if status:
         return status
-    lm = np.array([(2, 2), (2, 1), (3, 3), (3, 2), (4, 4), (4, 3)][:modes], dtype=np.int32).T.copy()
+    lm = mode_list(modes)
     out = [p] * (4 if grad else 3)
     status = lib.call("direct_fused_grad" if grad else "direct_fused", plan, *out, p, p, p, ints(lm[0]), ints(lm[1]),
                       modes, p, p, p, p, 1001, 2e-3, 0.0, 1e-4, 0.6, resp, 0, 0, 1, 16384, 256, 2048, None,
@@ -81,7 +102,7 @@ def summary(table):
     return dict(table=out, rows=table.tolist() if len(table) < 10000 else None)
 
 
-CASES = {"interpolate": interpolate, "direct": direct}
+CASES = {"interpolate": interpolate, "direct": direct, "heterodyned": heterodyned}
 
 
 if __name__ == "__main__":

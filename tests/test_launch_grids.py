@@ -103,3 +103,12 @@ def test_direct_grids_of_many_templates(record):
     grad, = record(("direct", [(n, 193)], 6, 1024, "k_dirg_knots", 4, 4, True))
     assert sum(g[0] for g, _, _ in launches(grad, "k_dirg_knots")) == 6 * n
     assert grad["table"]["distinct"] == 6 * n and grad["table"]["high"][2] == 6 * n - 1
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_heterodyned_wavefronts(record, grad):
+    """One wavefront per 64 nodes where the modes of the last nodes are not spread over others."""
+    sizes = [(16, 300, 6, 5), (16, 320, 1, 5), (16, 128, 6, 8), (16, 64, 6, 1), (16, 1000, 6, 8), (300, 448, 6, 7)]
+    for (batch, nodes, modes, waves), r in zip(sizes, record(*[("heterodyned", *s[:3], grad) for s in sizes])):
+        (grid, block, _), = launches(r, "k_grad_weights" if grad else "k_fused_eval")
+        assert (grid[0], block[0]) == (batch, 64 * waves)
