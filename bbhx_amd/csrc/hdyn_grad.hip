@@ -180,16 +180,17 @@ __global__ __launch_bounds__(64 * MAX_RESIDUAL_WAVES) __attribute__((amdgpu_wave
     }
 }
 
-// Gradient contributions of one (template, mode) and chunk of as many nodes as lanes,
-// the nc chunks from node k0 on in this launch: partial[((b * M + m) * chunks + c0 + chunk) * 11 + p].
+// Gradient contributions of one (template, mode), from bm0 on in this launch, and chunk of
+// as many nodes as lanes, nc of them from node k0 on:
+// partial[((b * M + m) * chunks + c0 + chunk) * 11 + p].
 __global__ __launch_bounds__(GRAD_T) __attribute__((amdgpu_waves_per_eu(2))) void k_grad_points(
     double* __restrict__ partial, const GradRec* __restrict__ grecs, const cd* __restrict__ gw,
     const double* __restrict__ params, const double* __restrict__ t_start, const double* __restrict__ t_end, int B,
     int M, const double* __restrict__ freqs, int K, resp::OrbitTab orb, int TDItag, int rescaled, int tdi2,
-    double initial_t_val, int k0, int c0, int nc)
+    double initial_t_val, int bm0, int k0, int c0, int nc)
 {
     __shared__ GradShared sh;
-    const int bm = blockIdx.x / nc, chunk = blockIdx.x % nc;
+    const int bm = bm0 + blockIdx.x / nc, chunk = blockIdx.x % nc;
     const int b = bm / M;
     Window win;
     win.t_ref = params[P_TREF * B + b];
@@ -305,15 +306,19 @@ extern "C" int bbhx_hip_hdyn_fused_grad(double* d_h, double* h_h, double* grad, 
     // spread evenly over the workgroups, 653 with idle ones in the last.
     const int chunks = grad_chunks(K), full = K / GRAD_T, rest = K - full * GRAD_T;
     auto points = [&](int k0, int c0, int nc, int threads) {
-        hipLaunchKernelGGL(k_grad_points, dim3((unsigned)(nrec * (long)nc)), dim3(threads), 0, st, partial, grecs, gw,
-                           params, t_start, t_end, numBinAll, numModes, freqs, K, orb, TDItag, rescaled, tdi2,
-                           initial_t_val, k0, c0, nc);
+        return launch_rows(nrec, nc, threads, [&](long bm0, dim3 g) {
+            hipLaunchKernelGGL(k_grad_points, g, dim3(threads), 0, st, partial, grecs, gw, params, t_start, t_end,
+                               numBinAll, numModes, freqs, K, orb, TDItag, rescaled, tdi2, initial_t_val, (int)bm0, k0,
+                               c0, nc);
+        });
     };
+    int rc;
     if (full > 0 && rest > 0 && rest <= GRAD_T - 64 && (long)nrec * full >= 4096) {
-        points(0, 0, full, GRAD_T);
-        points(full * GRAD_T, full, 1, grad_threads(rest));
+        rc = points(0, 0, full, GRAD_T);
+        if (rc == OK) rc = points(full * GRAD_T, full, 1, grad_threads(rest));
     } else
-        points(0, 0, chunks, grad_threads(K));
+        rc = points(0, 0, chunks, grad_threads(K));
+    if (rc != OK) return rc;
     hipLaunchKernelGGL(k_grad_reduce, dim3(ceil_div((long)numBinAll * NGRAD, 256)), dim3(256), 0, st, grad, partial,
                        numBinAll, numModes * chunks);
     if (timed) (void)hipEventRecord(ev[2], st);

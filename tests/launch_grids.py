@@ -65,7 +65,7 @@ def heterodyned(lib, batch, nodes, modes, grad=False):
     args = [*([p] * (6 if grad else 5)), batch, ints(lm[0]), ints(lm[1]), modes, p, p, p, nodes, p, 1001, 2e-3, 0.0,
             resp, 0, 0, 1, 0]
     if grad:
-        return lib.call("hdyn_fused_grad", *args, p, 0.0, None, args_of="k_grad_points", nargs=18)
+        return lib.call("hdyn_fused_grad", *args, p, 0.0, None, args_of="k_grad_points", nargs=19)
     return lib.call("hdyn_fused", *args, 0, p, 0.0, None)
 
 

@@ -112,3 +112,21 @@ def test_heterodyned_wavefronts(record, grad):
     for (batch, nodes, modes, waves), r in zip(sizes, record(*[("heterodyned", *s[:3], grad) for s in sizes])):
         (grid, block, _), = launches(r, "k_grad_weights" if grad else "k_fused_eval")
         assert (grid[0], block[0]) == (batch, 64 * waves)
+
+
+@pytest.mark.parametrize("batch,nodes,modes", [(3_000_000, 256, 6), (2_800_000, 300, 6), (17_000_000, 65, 1),
+                                               (100, 300, 6)])
+def test_heterodyned_gradient_of_many_templates(record, batch, nodes, modes):
+    """Every (template, mode)'s chunks of nodes are launched, whatever their number."""
+    r, = record(("heterodyned", batch, nodes, modes, True))
+    done = {}
+    for grid, block, args in launches(r, "k_grad_points"):
+        row0, node0, chunk0, chunks = (a & 0xFFFFFFFF for a in args[15:19])
+        rows, lanes = done.get((node0, chunk0, chunks), (0, block[0]))
+        assert row0 == rows and grid[0] % chunks == 0 and lanes == block[0]
+        done[node0, chunk0, chunks] = rows + grid[0] // chunks, lanes
+    node = chunk = 0
+    for (node0, chunk0, chunks), (rows, lanes) in done.items():
+        assert (node0, chunk0, rows) == (node, chunk, batch * modes)
+        node, chunk = node0 + chunks * lanes, chunk0 + chunks
+    assert nodes <= node < nodes + 256 and chunk == -(-nodes // 256)
