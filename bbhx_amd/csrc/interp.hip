@@ -159,8 +159,8 @@ __global__ __launch_bounds__(256) void k_interp_offsets(int64_t* __restrict__ of
     }
 }
 
-// Spline segment of every (binary, mode, dense bin): block -> (binary, mode, tile of
-// SEG_TILE bins). The grids are log-spaced, so the segment is estimated from an FP32
+// Spline segment of every (binary, mode, dense bin): block -> (binary, mode) from bm0 on,
+// tile of SEG_TILE bins. The grids are log-spaced, so the segment is estimated from an FP32
 // logarithm and checked, its neighbours next; whatever they do not hold is searched.
 // Bound by instruction issue, the estimate and its checks, and the writes. Up to 38 M
 // (binary, mode, bin): 0.062 ms (0.112 with a lane's bins one after another, 0.23 by a
@@ -170,9 +170,10 @@ constexpr int SEG_TILE = 1024;
 __global__ __launch_bounds__(256) void k_interp_segments(int* __restrict__ inds, const int2* __restrict__ band,
                                                          const int64_t* __restrict__ off,
                                                          const double* __restrict__ dataFreqs,
-                                                         const double* __restrict__ freqs, int M, int L, int tiles)
+                                                         const double* __restrict__ freqs, int M, int L, int tiles,
+                                                         int bm0)
 {
-    const int tile = blockIdx.x % tiles, bm = blockIdx.x / tiles, b = bm / M, m = bm - b * M;
+    const int tile = blockIdx.x % tiles, bm = bm0 + blockIdx.x / tiles, b = bm / M, m = bm - b * M;
     const int2 r = band[b];
     const int len = r.y - r.x;
     const double* x = freqs + (long)bm * L;
@@ -243,8 +244,11 @@ extern "C" int bbhx_hip_interp_bands(int* band, int64_t* off, const double* freq
     if (!band || !off || !freqs || (!dataFreqs && data_length > 0)) return ERR_ARGS;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     int2* r = reinterpret_cast<int2*>(band);
-    hipLaunchKernelGGL(k_interp_bands, dim3(numBinAll), dim3(256), 0, st, r, freqs, (long)numModes * length, dataFreqs,
-                       data_length);
+    const long n = (long)numModes * length;
+    const int rc = launch_rows(numBinAll, 1, 256, [&](long b0, dim3 grid) {
+        hipLaunchKernelGGL(k_interp_bands, grid, dim3(256), 0, st, r + b0, freqs + b0 * n, n, dataFreqs, data_length);
+    });
+    if (rc != OK) return rc;
     hipLaunchKernelGGL(k_interp_offsets, dim3(1), dim3(256), 0, st, off, r, numBinAll);
     return hipGetLastError() == hipSuccess ? OK : ERR_LAUNCH;
 }
@@ -257,11 +261,13 @@ extern "C" int bbhx_hip_interp_segments(int* inds, const int* band, const int64_
     if (numBinAll == 0 || max_len == 0) return OK;
     if (!inds || !band || !off || !freqs || !dataFreqs) return ERR_ARGS;
     const int tiles = (int)(((long)max_len + SEG_TILE - 1) / SEG_TILE);
-    const long blocks = (long)numBinAll * numModes * tiles;
-    if (blocks > 2147483647L) return ERR_ARGS;
-    hipLaunchKernelGGL(k_interp_segments, dim3((unsigned)blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
-                       inds, reinterpret_cast<const int2*>(band), off, dataFreqs, freqs, numModes, length, tiles);
-    return hipGetLastError() == hipSuccess ? OK : ERR_LAUNCH;
+    const long rows = (long)numBinAll * numModes;
+    if (rows > 2147483647L) return ERR_ARGS;
+    return launch_rows(rows, tiles, 256, [&](long bm0, dim3 grid) {
+        hipLaunchKernelGGL(k_interp_segments, grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream), inds,
+                           reinterpret_cast<const int2*>(band), off, dataFreqs, freqs, numModes, length, tiles,
+                           (int)bm0);
+    });
 }
 
 extern "C" int bbhx_hip_fill_bands(double* out, const double* templates, const int* band, const int64_t* off,
@@ -271,12 +277,12 @@ extern "C" int bbhx_hip_fill_bands(double* out, const double* templates, const i
     if (numBinAll == 0 || data_length == 0) return OK;
     if (!out || !templates || !band || !off) return ERR_ARGS;
     const int tiles = (int)(((long)data_length + 255) / 256);
-    const long blocks = (long)numBinAll * tiles;
-    if (blocks > 2147483647L) return ERR_ARGS;
-    hipLaunchKernelGGL(k_fill_bands, dim3((unsigned)blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
-                       reinterpret_cast<double2*>(out), reinterpret_cast<const double2*>(templates),
-                       reinterpret_cast<const int2*>(band), off, data_length, tiles);
-    return hipGetLastError() == hipSuccess ? OK : ERR_LAUNCH;
+    return launch_rows(numBinAll, tiles, 256, [&](long b0, dim3 grid) {
+        hipLaunchKernelGGL(k_fill_bands, grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
+                           reinterpret_cast<double2*>(out) + b0 * 3 * data_length,
+                           reinterpret_cast<const double2*>(templates), reinterpret_cast<const int2*>(band) + b0,
+                           off + b0, data_length, tiles);
+    });
 }
 
 namespace bbhx {

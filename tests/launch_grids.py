@@ -102,7 +102,16 @@ def summary(table):
     return dict(table=out, rows=table.tolist() if len(table) < 10000 else None)
 
 
-CASES = {"interpolate": interpolate, "direct": direct, "heterodyned": heterodyned}
+P = C.c_void_p(1 << 20)
+CALLS = {
+    "interp_bands": lambda lib, batch, modes, length: lib.call(
+        "interp_bands", P, P, P, P, length, 1000, batch, modes, None, args_of="k_interp_bands", nargs=5),
+    "interp_segments": lambda lib, batch, modes, longest: lib.call(
+        "interp_segments", P, P, P, P, P, 64, longest, batch, modes, None, args_of="k_interp_segments", nargs=9),
+    "fill_bands": lambda lib, batch, bins: lib.call(
+        "fill_bands", P, P, P, P, bins, batch, None, args_of="k_fill_bands", nargs=6),
+}
+CASES = {"interpolate": interpolate, "direct": direct, "heterodyned": heterodyned, **CALLS}
 
 
 if __name__ == "__main__":

@@ -130,3 +130,27 @@ def test_heterodyned_gradient_of_many_templates(record, batch, nodes, modes):
         assert (node0, chunk0, rows) == (node, chunk, batch * modes)
         node, chunk = node0 + chunks * lanes, chunk0 + chunks
     assert nodes <= node < nodes + 256 and chunk == -(-nodes // 256)
+
+
+def test_template_grids_of_many_binaries(record):
+    """Bands, segments and placement of batches beyond one launch: every binary's workgroups,
+    its arrays where they were."""
+    base = 1 << 20
+    bands, segments, fill = record(("interp_bands", 20_000_000, 2, 4), ("interp_segments", 1900, 6, 1_580_000),
+                                   ("fill_bands", 600, 12_600_000))
+    done = 0
+    for grid, _, args in launches(bands, "k_interp_bands"):
+        assert args[0] == base + 8 * done and args[1] == base + 8 * done * 2 * 4
+        done += grid[0]
+    assert done == 20_000_000
+    done, tiles = 0, -(-1_580_000 // 1024)
+    for grid, _, args in launches(segments, "k_interp_segments"):
+        assert args[8] & 0xFFFFFFFF == done and grid[0] % tiles == 0
+        done += grid[0] // tiles
+    assert done == 1900 * 6
+    done, tiles = 0, -(-12_600_000 // 256)
+    for grid, _, args in launches(fill, "k_fill_bands"):
+        assert args[0] == base + 16 * 3 * 12_600_000 * done and args[1] == base
+        assert args[2] == base + 8 * done and args[3] == base + 8 * done
+        done += grid[0] // tiles
+    assert done == 600
