@@ -114,10 +114,10 @@ __global__ __launch_bounds__(EVAL_THREADS) void k_phm_default_grid(double* __res
                                                                    const double* __restrict__ m1,
                                                                    const double* __restrict__ m2,
                                                                    const int* __restrict__ mms, double lo, double hi,
-                                                                   int M, int L, long n)
+                                                                   int M, int L, long p0, long n)
 {
 #pragma clang fp contract(off)
-    const long p = (long)blockIdx.x * EVAL_THREADS + threadIdx.x;
+    const long p = p0 + (long)blockIdx.x * EVAL_THREADS + threadIdx.x;
     if (p >= n) return;
     const long row = p / L;
     const int i = (int)(p - row * L), b = (int)(row / M), m = (int)(row - (long)b * M);
@@ -129,10 +129,10 @@ __global__ __launch_bounds__(EVAL_THREADS) void k_phm_default_grid(double* __res
 __global__ __launch_bounds__(EVAL_THREADS) void k_phm_time_shift(double* __restrict__ phase, double* __restrict__ tf,
                                                                  const double* __restrict__ freqs,
                                                                  const double* __restrict__ t_ref, double t0,
-                                                                 long per_bin, long n)
+                                                                 long per_bin, long p0, long n)
 {
 #pragma clang fp contract(off)
-    const long p = (long)blockIdx.x * EVAL_THREADS + threadIdx.x;
+    const long p = p0 + (long)blockIdx.x * EVAL_THREADS + threadIdx.x;
     if (p >= n) return;
     const double t = t_ref[p / per_bin];
     phase[p] += freqs[p] * (t - t0) * 2.0 * PI;
@@ -141,21 +141,21 @@ __global__ __launch_bounds__(EVAL_THREADS) void k_phm_time_shift(double* __restr
 
 // The grid of each (binary, mode) refitted to 0 <= t(f) <= Tobs (phenomhm.py:520-600):
 // where t(f) crosses a bound inside the grid, the crossing frequency by linear
-// interpolation, else the grid's own end. One workgroup per row; *flag is raised if a
+// interpolation, else the grid's own end. One workgroup per row, from r0 on; *flag is raised if a
 // row that needs a bound does not cross it exactly once.
 __global__ __launch_bounds__(EVAL_THREADS) void k_phm_refit_grid(double* __restrict__ out, int* __restrict__ flag,
                                                                  const double* __restrict__ tf,
                                                                  const double* __restrict__ freqs,
                                                                  const double* __restrict__ Tobs, int tobs_b,
-                                                                 int tobs_m, int M, int L)
+                                                                 int tobs_m, int M, int L, int r0)
 {
 #pragma clang fp contract(off)
     constexpr int W = EVAL_THREADS / 64;
     __shared__ double s_min[2][W], s_max[2][W];
     __shared__ int s_hits[2], s_seg[2];
-    const int b = blockIdx.x / M, m = blockIdx.x - b * M;
-    const double* t = tf + (long)blockIdx.x * L;
-    const double* f = freqs + (long)blockIdx.x * L;
+    const int row = r0 + blockIdx.x, b = row / M, m = row - b * M;
+    const double* t = tf + (long)row * L;
+    const double* f = freqs + (long)row * L;
     const double level[2] = {0.0, Tobs ? Tobs[(long)b * tobs_b + (long)m * tobs_m] : 1e300};
     // not a number if any entry is
     auto least = [](double a, double c) { return (c < a || c != c) && a == a ? c : a; };
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(EVAL_THREADS) void k_phm_refit_grid(double* __restr
     }
     const double y0 = log10(end[0]), y1 = log10(end[1]), step = (y1 - y0) / (L - 1);
     for (int i = threadIdx.x; i < L; i += EVAL_THREADS)
-        out[(long)blockIdx.x * L + i] = pow(10.0, i == L - 1 ? y1 : y0 + i * step);
+        out[(long)row * L + i] = pow(10.0, i == L - 1 ? y1 : y0 + i * step);
 }
 
 }  // namespace
@@ -289,10 +289,10 @@ int bbhx_hip_phm_default_grid(double* freqs, const double* m1, const double* m2,
     if (numBinAll == 0) return OK;
     if (!freqs || !m1 || !m2 || !mms) return ERR_ARGS;
     const long n = (long)numBinAll * numModes * length;
-    if (ceil_div(n, EVAL_THREADS) > 2147483647L) return ERR_ARGS;
-    hipLaunchKernelGGL(k_phm_default_grid, dim3((unsigned)ceil_div(n, EVAL_THREADS)), dim3(EVAL_THREADS), 0, S(stream),
-                       freqs, m1, m2, mms, log10_lo, log10_hi, numModes, length, n);
-    return launch_status();
+    return launch_rows((n + EVAL_THREADS - 1) / EVAL_THREADS, 1, EVAL_THREADS, [&](long r, dim3 grid) {
+        hipLaunchKernelGGL(k_phm_default_grid, grid, dim3(EVAL_THREADS), 0, S(stream), freqs, m1, m2, mms, log10_lo,
+                           log10_hi, numModes, length, r * EVAL_THREADS, n);
+    });
 }
 
 int bbhx_hip_phm_time_shift(double* waveformOut, const double* freqs, const double* t_ref, double t0, int length,
@@ -302,10 +302,10 @@ int bbhx_hip_phm_time_shift(double* waveformOut, const double* freqs, const doub
     if (numBinAll == 0) return OK;
     if (!waveformOut || !freqs || !t_ref) return ERR_ARGS;
     const long n = (long)numBinAll * numModes * length;
-    if (ceil_div(n, EVAL_THREADS) > 2147483647L) return ERR_ARGS;
-    hipLaunchKernelGGL(k_phm_time_shift, dim3((unsigned)ceil_div(n, EVAL_THREADS)), dim3(EVAL_THREADS), 0, S(stream),
-                       waveformOut + n, waveformOut + 2 * n, freqs, t_ref, t0, (long)numModes * length, n);
-    return launch_status();
+    return launch_rows((n + EVAL_THREADS - 1) / EVAL_THREADS, 1, EVAL_THREADS, [&](long r, dim3 grid) {
+        hipLaunchKernelGGL(k_phm_time_shift, grid, dim3(EVAL_THREADS), 0, S(stream), waveformOut + n,
+                           waveformOut + 2 * n, freqs, t_ref, t0, (long)numModes * length, r * EVAL_THREADS, n);
+    });
 }
 
 int bbhx_hip_phm_refit_grid(double* new_freqs, int* flag, const double* tf, const double* freqs, const double* Tobs,
@@ -315,10 +315,12 @@ int bbhx_hip_phm_refit_grid(double* new_freqs, int* flag, const double* tf, cons
     if (length < 1 || numModes < 1 || numBinAll < 0) return ERR_ARGS;
     if (numBinAll == 0) return OK;
     if (!new_freqs || !flag || !tf || !freqs) return ERR_ARGS;
-    if ((long)numBinAll * numModes > 2147483647L) return ERR_ARGS;
-    hipLaunchKernelGGL(k_phm_refit_grid, dim3((unsigned)(numBinAll * numModes)), dim3(EVAL_THREADS), 0, S(stream),
-                       new_freqs, flag, tf, freqs, Tobs, tobs_stride_bin, tobs_stride_mode, numModes, length);
-    return launch_status();
+    const long rows = (long)numBinAll * numModes;
+    if (rows > 2147483647L) return ERR_ARGS;
+    return launch_rows(rows, 1, EVAL_THREADS, [&](long r, dim3 grid) {
+        hipLaunchKernelGGL(k_phm_refit_grid, grid, dim3(EVAL_THREADS), 0, S(stream), new_freqs, flag, tf, freqs, Tobs,
+                           tobs_stride_bin, tobs_stride_mode, numModes, length, (int)r);
+    });
 }
 
 }  // extern "C"

@@ -110,6 +110,12 @@ CALLS = {
         "interp_segments", P, P, P, P, P, 64, longest, batch, modes, None, args_of="k_interp_segments", nargs=9),
     "fill_bands": lambda lib, batch, bins: lib.call(
         "fill_bands", P, P, P, P, bins, batch, None, args_of="k_fill_bands", nargs=6),
+    "phm_default_grid": lambda lib, batch, modes, length: lib.call(
+        "phm_default_grid", P, P, P, P, -4.0, -0.2, length, modes, batch, None, args_of="grid", nargs=10),
+    "phm_time_shift": lambda lib, batch, modes, length: lib.call(
+        "phm_time_shift", P, P, P, 0.0, length, modes, batch, None, args_of="shift", nargs=8),
+    "phm_refit_grid": lambda lib, batch, modes, length: lib.call(
+        "phm_refit_grid", P, P, P, P, None, 1, 0, length, modes, batch, None, args_of="refit", nargs=10),
 }
 CASES = {"interpolate": interpolate, "direct": direct, "heterodyned": heterodyned, **CALLS}
 

@@ -154,3 +154,22 @@ def test_template_grids_of_many_binaries(record):
         assert args[2] == base + 8 * done and args[3] == base + 8 * done
         done += grid[0] // tiles
     assert done == 600
+
+
+def test_waveform_grids_of_many_points(record):
+    """The waveform's frequency grids and time shift beyond one launch of a lane per point."""
+    batch, modes, length = 3_000_000, 6, 300
+    points = batch * modes * length
+    for what, kernel, at in (("phm_default_grid", "k_phm_default_grid", 8), ("phm_time_shift", "k_phm_time_shift", 6)):
+        r, = record((what, batch, modes, length))
+        done = 0
+        for grid, _, args in launches(r, kernel):
+            assert args[at:at + 2] == [256 * done, points]
+            done += grid[0]
+        assert done == -(-points // 256)
+    r, = record(("phm_refit_grid", batch, modes, length))
+    done = 0
+    for grid, _, args in launches(r, "k_phm_refit_grid"):
+        assert args[9] & 0xFFFFFFFF == done
+        done += grid[0]
+    assert done == batch * modes
