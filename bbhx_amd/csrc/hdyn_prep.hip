@@ -195,9 +195,9 @@ __global__ __launch_bounds__(192) void k_prep_totals(double* __restrict__ totals
 // Bound by the rows' writes and the sine and cosine. 2^20 frequencies: 12 us; numpy on
 // the host, powers and all: 118 ms.
 __global__ __launch_bounds__(256) void k_aet1_psd(double* __restrict__ S, const double* __restrict__ f, long n,
-                                                  double arm, double acc, double oms)
+                                                  double arm, double acc, double oms, long k0)
 {
-    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long k = k0 + (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
     const double fk = f[k], w = 2.0 * PI * fk, wc = w / C_SI, x = arm * wc;
     const double lo = 0.4e-3 / fk, hi = fk / 8e-3, op = 2e-3 / fk;
@@ -219,12 +219,13 @@ __global__ __launch_bounds__(256) void k_aet1_psd(double* __restrict__ S, const 
 extern "C" int bbhx_hip_aet1_psd(double* psd, const double* freqs, int64_t n, double armlength, double acc, double oms,
                                  void* stream)
 {
-    if (n < 0 || n > (int64_t)2147483647 * 256) return ERR_ARGS;
+    if (n < 0) return ERR_ARGS;
     if (n == 0) return OK;
     if (!psd || !freqs) return ERR_ARGS;
-    hipLaunchKernelGGL(k_aet1_psd, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                       reinterpret_cast<hipStream_t>(stream), psd, freqs, (long)n, armlength, acc, oms);
-    return hipGetLastError() == hipSuccess ? OK : ERR_LAUNCH;
+    return launch_rows((n + 255) / 256, 1, 256, [&](long r, dim3 grid) {
+        hipLaunchKernelGGL(k_aet1_psd, grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream), psd, freqs, (long)n,
+                           armlength, acc, oms, 256 * r);
+    });
 }
 
 extern "C" int bbhx_hip_hdyn_prep(double* dataConstants, double* totals, const double* dataFreqs,

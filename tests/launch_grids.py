@@ -116,6 +116,8 @@ CALLS = {
         "phm_time_shift", P, P, P, 0.0, length, modes, batch, None, args_of="shift", nargs=8),
     "phm_refit_grid": lambda lib, batch, modes, length: lib.call(
         "phm_refit_grid", P, P, P, P, None, 1, 0, length, modes, batch, None, args_of="refit", nargs=10),
+    "aet1_psd": lambda lib, n: lib.call(
+        "aet1_psd", P, P, n, 2.5e9, 3e-15, 1.5e-11, None, args_of="k_aet1_psd", nargs=7),
 }
 CASES = {"interpolate": interpolate, "direct": direct, "heterodyned": heterodyned, **CALLS}
 

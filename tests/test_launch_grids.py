@@ -173,3 +173,13 @@ def test_waveform_grids_of_many_points(record):
         assert args[9] & 0xFFFFFFFF == done
         done += grid[0]
     assert done == batch * modes
+
+
+def test_noise_of_many_frequencies(record):
+    n = 5_000_000_000
+    r, = record(("aet1_psd", n))
+    done = 0
+    for grid, _, args in launches(r, "k_aet1_psd"):
+        assert args[2] == n and args[6] == 256 * done
+        done += grid[0]
+    assert done == -(-n // 256)
