@@ -28,7 +28,7 @@ def to_dev(x, device, dtype=None):
 
 
 def rows_to_dev(rows, device):
-    """float64 tensors on ``device`` of several 1D numpy arrays, in one copy (a copy
+    """float64 tensors on ``device`` of several numpy arrays, flattened, in one copy (a copy
     of a few values waits some 40 us); views of one buffer, each 512-byte aligned."""
     import torch
 
@@ -36,7 +36,7 @@ def rows_to_dev(rows, device):
     starts = np.cumsum([0] + [-(-r.size // step) * step for r in rows])
     host = np.zeros(starts[-1])
     for s, r in zip(starts, rows):
-        host[s:s + r.size] = r
+        host[s:s + r.size] = r.ravel()
     buf = torch.as_tensor(host, device=device)
     return [buf[s:s + r.size] for s, r in zip(starts, rows)]
 

@@ -175,6 +175,8 @@ class PhenomHMAmpPhase(BBHxParallelModule):
 
         if t_ref.size == 1:
             t_ref = np.repeat(t_ref, num_bin_all)
+        elif t_ref.shape != (num_bin_all,):
+            raise ValueError("t_ref must have one entry, or one per binary.")
         rows = [m1, m2, chi1z, chi2z, distance, f_ref, t_ref, m1 * MSUN_SI, m2 * MSUN_SI]
         per_bin = isinstance(Tobs, np.ndarray) and Tobs.shape == (num_bin_all,)
         rows = rows_to_dev(rows + [Tobs] if per_bin else rows, self.device)
