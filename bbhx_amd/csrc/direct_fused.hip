@@ -1363,15 +1363,21 @@ bool lay_out_knots(bbhx_direct_plan* p, std::vector<int4>& knots, std::vector<in
 //
 // A work item is what one wavefront takes: a caller's chunk (bins per workgroup
 // and pass) split over the workgroup's wavefronts, and less than that for a small
-// batch, down to ITEM_MIN bins (half a block). Up to FEW bins in all, as many items as
-// wavefronts in a launch of the default grid, ITEMS_ONCE, each with a first item and
-// no other, as the counter of the following ones takes 8 ns a time; above, twice as
-// many, for the dynamic order to balance. Plans of up to SMALL_ITEMS such items have
-// buffers for them. The whole call with at least 256 bins and 16384 items at any
-// size, and with this rule: 16 templates of 65536 bins 321 and 303 us, 48 of them 440
-// and 395, 64 499 and 433; with ITEMS_ONCE at 128 and 256 of them 630 became 657 and
-// 1005 became 1174 us. At 1024 templates of 1.58 M bins the item size does not
-// matter (items of 4096, 8192 and 16384 bins: 25.4, 25.5 and 26.3 ms).
+// batch, down to ITEM_MIN bins (half a block). Up to FEW bins in all about ITEMS_ONCE
+// items, the wavefronts of the default launch on 256 CUs: if the bands hold no more than
+// that, each has a first item and no other, and the counter of the following ones, 8 ns
+// a time, is not asked. Above, twice as many, for the dynamic order to balance. Plans of
+// up to SMALL_ITEMS such items have buffers for them. The whole call with at least 256
+// bins and 16384 items at any size, and with this rule: 16 templates of 65536 bins 321 and
+// 303 us, 48 of them 440 and 395, 64 499 and 433; with ITEMS_ONCE at 128 and 256 of
+// them 630 became 657 and 1005 became 1174 us. At 1024 templates of 1.58 M bins the item
+// size does not matter (items of 4096, 8192 and 16384 bins: 25.4, 25.5 and 26.3 ms).
+//
+// The size does not follow the caller's launch: counted for its own wavefronts, 4096
+// instead of 8192 of them took 171 instead of 222 us for 16 such templates, but 861 instead
+// of 682 for 200 (fewer items balance worse), 2048 took 224 instead of 210 for 16. Nor does
+// it count the items of a whole data set exactly: 16 templates of 65537 bins, 8208 items at
+// most and 8192 at hand, 156 us, 171 with the next larger size.
 constexpr long ITEM_MIN = 128, SMALL_ITEMS = 1L << 19, ITEMS_ONCE = 8192, FEW = ITEMS_ONCE * 512;
 
 static int item_bins(const bbhx_direct_plan* p, int chunk, int block)
