@@ -258,45 +258,6 @@ def bench_direct_ragged(args):
         f"plan {plan.nbytes() / 2**30:.2f} GiB; {dense} dense (bin, template) pairs "
         f"({dense / (ms * 1e-3):.4g}/s); split {split}")
 
-    # the same batch with precision 1 (logL within 1e-3 suffices), its own graph
-    f32_info = None
-    if not args.no_fp32:
-        hh64 = like.h_h.real.cpu().numpy()
-        flags.zero_()
-        like.get_ll_fused_device(plan, rows, ts, te, flags, MODES, precision=1)
-        torch.cuda.synchronize()
-        g32 = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g32, stream=st):
-            flags.zero_()
-            out32 = like.get_ll_fused_device(plan, rows, ts, te, flags, MODES)
-        torch.cuda.synchronize()
-        g32.replay()
-        torch.cuda.synchronize()
-        ll32 = out32.cpu().numpy()
-        t0 = time.perf_counter()
-        for _ in range(args.steps):
-            g32.replay()
-        torch.cuda.synchronize()
-        t1 = time.perf_counter()
-        ms32 = (t1 - t0) * 1e3 / args.steps
-        timing_enable(True)
-        for _ in range(2):
-            flags.zero_()
-            like.get_ll_fused_device(plan, rows, ts, te, flags, MODES)
-        s32, e32, n32 = timing_read()
-        timing_enable(False)
-        plan.set_precision(0)
-        dll = np.abs(ll32 - eager)
-        f32_info = {"ms": ms32, "evals_per_s": B / (ms32 * 1e-3), "speedup_vs_fp64": ms / ms32,
-                    "setup_ms": s32 / max(n32, 1), "dense_ms": e32 / max(n32, 1),
-                    "max_abs_dlogL_vs_fp64": float(dll.max()), "median_abs_dlogL_vs_fp64": float(np.median(dll)),
-                    "max_rel_dlogL_vs_hh": float(np.max(dll / np.maximum(np.abs(hh64), 1.0))),
-                    "templates_within_1e-3": int(np.sum(dll < 1e-3)),
-                    "templates_in_fp64": int(np.sum(hh64 > 2.0e4))}
-        log(f"FP32 bulk: {ms32:.3f} ms/step ({ms / ms32:.2f}x the FP64 form), dense {e32 / max(n32, 1):.2f} ms; "
-            f"|dlogL| vs FP64 max {dll.max():.2e}, median {np.median(dll):.2e}; "
-            f"{int(np.sum(dll < 1e-3))}/{B} within 1e-3")
-
     # the unfused inner product (the reference's direct_like kernel, a10) on a few
     # templates materialised by the kernel-by-kernel path: HBM-bound, 168 B per
     # dense bin and template (h read 48 and written back noise-weighted 48, as the
@@ -437,7 +398,7 @@ def bench_direct_ragged(args):
                    "lengths_min": int(lengths.min()), "lengths_max": int(lengths.max()),
                    "lengths_sum": int(lengths.sum()), "dense_bins": int(f.size), "modes": 6, "tdi": "AET tdi2",
                    "launch": {k: tuned[k] for k in ("chunk", "block", "grid")}, "max_abs_dlogL_graph_vs_eager": diff,
-                   "dense_bin_templates": dense, **split, "fp32_bulk": f32_info, "gradient": grad_info,
+                   "dense_bin_templates": dense, **split, "gradient": grad_info,
                    "unfused_inner_product": unfused},
         "roofline": roofline,
         "cpu_baseline": cpu,
@@ -457,7 +418,6 @@ def main():
     ap.add_argument("--cpu-seconds", type=float, default=10.0)
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-grad", action="store_true", help="direct workloads: skip the gradient timing")
-    ap.add_argument("--no-fp32", action="store_true", help="direct workloads: skip the FP32-bulk form")
     ap.add_argument("--no-unfused", action="store_true",
                     help="direct workloads: skip the unfused inner-product (k_direct_like) bandwidth measurement")
     ap.add_argument("--launch", default="", help="direct workloads: fixed 'chunk,block,grid' instead of autotuning")
