@@ -1,10 +1,12 @@
 """Launch-shape autotuner for the fused direct likelihood of a ragged batch.
 
 The persistent dense-band kernel (k_dir_like) has three free shape parameters:
-the number of dense bins per work item (``chunk``), the threads per workgroup
-(``block``) and the number of persistent workgroups (``grid``). The best
-choice depends on the batch: many short bands favour small chunks (balance),
-few long bands large ones (less per-item overhead). ``tune_direct`` times
+the dense bins that a workgroup takes at a time (``chunk``; each of its wavefronts
+takes work items of its share of them), the threads per workgroup (``block``) and
+the number of persistent workgroups (``grid``). The best choice depends on the
+batch: many short bands favour small chunks (balance), few long bands large ones
+(less per-item overhead). Small batches are cut finer than any chunk here, so
+that only block and grid tell their candidates apart. ``tune_direct`` times
 every candidate on the caller's actual batch with device events on the
 current stream and returns the fastest; results are cached per
 (device, batch signature) for the life of the process and, if a path is given,

@@ -50,18 +50,6 @@ __host__ __device__ inline cd operator*(cd a, double s) { return cd{a.re * s, a.
 __host__ __device__ inline cd conj(cd a) { return cd{a.re, -a.im}; }
 __host__ __device__ inline cd& operator+=(cd& a, cd b) { a.re += b.re; a.im += b.im; return a; }
 
-// theta mod 2 pi in two Cody-Waite steps (2 pi = HI + LO to ~107 bits); exact
-// to the rounding of theta itself for |theta| up to ~1e13.
-__device__ inline double reduce_2pi(double theta)
-{
-    const double TWO_PI_HI = 6.283185307179586;
-    const double TWO_PI_LO = 2.4492935982947064e-16;
-    const double INV_TWO_PI = 0.15915494309189535;
-    double k = rint(theta * INV_TWO_PI);
-    double r = fma(-k, TWO_PI_HI, theta);
-    return fma(-k, TWO_PI_LO, r);
-}
-
 // 1/x for finite normal x != 0: the hardware reciprocal estimate refined by
 // two Newton steps e = 1 - x r, r += r e (within ~1 ulp of the rounded quotient).
 __device__ inline double rcp_pos(double x)
@@ -204,7 +192,7 @@ __device__ inline double scoef(double c)
     return c;
 }
 
-// sin and cos for |x| <= ~4 (e.g. after reduce_2pi): quadrant reduction by
+// sin and cos for |x| <= ~4: quadrant reduction by
 // pi/2 = HI + LO, then the Taylor series of sin (to x^17) and cos (to x^18)
 // on |r| <= pi/4, whose truncation errors (< 1e-19) are below FP64 rounding.
 // Small and branch-light, unlike a general libm sincos with its large-argument path.
@@ -249,8 +237,9 @@ __device__ inline void sincos_small(double x, double* s, double* c)
 // rounded, and its low bits read, by adding 1.5 2^52); e^{i j pi/64} from a
 // table of one turn (tab[(j + 64) mod 128], normally in LDS) and e^{i b} from
 // its series to b^7 / b^6 (truncation < 1e-18 relative): 16 operations, within a
-// few ulp for |theta| up to ~1e13. Any theta (also NaN or inf) gives an index in
-// [0, 127].
+// few ulp for |theta| < 1e14 (2^51 pi/64; neighbouring doubles are 0.016 rad apart
+// there). Beyond, j is no longer rounded to whole numbers, and neither angle nor unit
+// modulus hold; the index stays in [0, 127] for any theta (also NaN or inf).
 constexpr double PI64_HI = 0.04908738521234052;     // pi / 64 rounded
 constexpr double PI64_LO = 1.9135106236677393e-18;  // pi / 64 - PI64_HI
 constexpr double ROUND_MAGIC = 6755399441055744.0;  // 1.5 2^52
@@ -274,7 +263,7 @@ __device__ inline cd cexpi_tab(double theta, const E* __restrict__ tab)
 
 // The same from a table of 1024 entries (tab[j mod 1024] = e^{i j pi/512}, built
 // by fill_etab1k): |b| <= pi/1024, so the series end at b^5 / b^4 (truncation
-// < 2e-18). For persistent kernels, which fill its 16 KB of LDS once.
+// < 2e-18), for |theta| < 1e13 (2^51 pi/512). For persistent kernels, which fill its 16 KB of LDS once.
 template <class E>
 __device__ inline cd cexpi_tab1k(double theta, const E* __restrict__ tab)
 {

@@ -907,7 +907,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADJ ? 3 : 4
     // following from a counter (dynamic: the items running at any time stay a window of
     // consecutive entries, i.e. the same dense bins). The counter takes some 8 ns per
     // wavefront, so with none left beyond the first ones it is not asked: 16 templates of
-    // 65536 bins, 8192 wavefronts for 4096 items: 180 -> 72 us.
+    // 65536 bins in 4096 items, 8192 wavefronts: 180 -> 72 us (56 in item_bins' items).
     const int waves = gridDim.x * (blockDim.x >> 6);
     int pi = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
     for (bool first = true;; first = false) {
@@ -1628,7 +1628,8 @@ extern "C" int bbhx_hip_direct_fused(bbhx_direct_plan* p, double* d_h, double* h
 // 0 and 1 are evaluated alike, in FP64, the faster form: FP32 instructions issue at
 // the FP64 rate without packed arithmetic, and an FP32 pass over the quiet
 // templates needs its own records, the split of the items and a second pass for the
-// loud ones (1024 uneven templates: 27.7 ms against 25.0).
+// loud ones. 1024 uneven templates: 27.7 ms with such a pass, which had the FP64 pass's
+// walker but not its later changes, 25.0 then without it, 23 now.
 extern "C" int bbhx_hip_direct_plan_set_precision(bbhx_direct_plan* p, int precision)
 {
     return p && (precision == 0 || precision == 1) ? OK : ERR_ARGS;

@@ -1,16 +1,23 @@
 // Not-a-knot spline systems by parallel cyclic reduction in a workgroup.
 //
 // One knot per lane, several quantities on the same knots together, the systems
-// and their transposes: with every row scaled to a unit diagonal, a step at distance d replaces the
-// couplings to rows i -+ d by ones to rows i -+ 2d. The rows are diagonally
-// dominant by two or more (the couplings' magnitudes add up to at most half of the
-// diagonal), so the couplings fall from 1/2 to at most 1/4, 1/16, 1/256, 2^-16,
-// 2^-32 and 2^-64 in six steps, after which each row is its solution. What lies
-// farther than that does not count either, so a grid longer than a workgroup is cut
-// into blocks that overlap by SPL_W rows on each side: a solution forgets by a
-// factor of about 0.27 per row (0.5 at worst) what a block's end leaves out, and
-// on a log-spaced grid over 4 decades the end's slopes, steeper by at most
-// r^(11/3) per row (r = the knots' ratio), weigh (0.28 r^(11/3))^48 < 1e-16 there.
+// and their transposes: with every row scaled to a unit diagonal, a step at distance d
+// replaces the couplings to rows i -+ d by ones to rows i -+ 2d, so that grids of up to 66
+// knots (64 rows) are solved exactly in six steps. In a longer one the system's inner
+// rows are diagonally dominant by two or more (the couplings' magnitudes add up to at most
+// half of the diagonal), and the couplings fall from 1/2 to at most 1/4, 1/16, 1/256,
+// 2^-16, 2^-32 and 2^-64 (evenly spaced knots: 5e-37), after which each row is its
+// solution. A row that a folded end row went into couples by h_end / (h_end + h), up to 1
+// where the end interval is much the longer, and by at most a half after the first step.
+// The transposed rows need not be dominant (8 on four knots over the default range of
+// frequencies), but a step of the transposed system is the transpose of the system's own:
+// its couplings are those times the ratio of the two rows' diagonals, below 10^4 on any
+// grid here and 10^(4 64 / n) on a log-spaced one of n knots over 4 decades. What lies
+// farther does not count either, so a grid longer than a workgroup is cut into blocks
+// that overlap by SPL_W rows on each side: a solution forgets by a factor of about 0.27
+// per row (0.5 at worst) what a block's end leaves out, and on a log-spaced grid over 4
+// decades the end's slopes, steeper by at most r^(11/3) per row (r = the knots' ratio),
+// weigh (0.28 r^(11/3))^48 < 1e-16 there.
 #pragma once
 
 #include "common.h"

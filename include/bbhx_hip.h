@@ -219,14 +219,14 @@ int bbhx_hip_hdyn_fused_grad(double* d_h, double* h_h, double* grad, const doubl
  * lengths L_b, in one sequence of launches with no host synchronisation
  * and no allocation, so that the call can be captured in a hipGraph. A plan
  * holds the sizes and the device buffers (sparse grids, the nine spline
- * quantities and their coefficients: 328 B per (knot, mode), plus per-binary
- * tables); plan_bytes returns their total. */
+ * quantities and their coefficients: 400 B per (knot, mode), plus tables
+ * per binary and per work item); plan_bytes returns their total. */
 typedef struct bbhx_direct_plan bbhx_direct_plan;
 
 /* lengths_host (B,): sparse grid length of each binary (>= 4, <= 6144).
- * data_length: N dense bins. min_chunk (>= 64): the smallest number of dense
- * bins per work item that bbhx_hip_direct_fused will be called with (sizes the
- * partial-sum buffer). */
+ * data_length: N dense bins. min_chunk (>= 64): the smallest chunk that
+ * bbhx_hip_direct_fused will be called with. It sizes the partial-sum buffer,
+ * for work items of min_chunk bins, of 128 if B N <= 2^26. */
 int bbhx_hip_direct_plan_create(bbhx_direct_plan** out, int numBinAll, const int* lengths_host, int numModes,
                                 int data_length, int min_chunk);
 int bbhx_hip_direct_plan_destroy(bbhx_direct_plan* p);
@@ -251,9 +251,11 @@ int bbhx_hip_direct_plan_set_precision(bbhx_direct_plan* p, int precision);
  * search at the low / high end failed for some mode (the reference raises
  * ValueError there, phenomhm.py:530-600). mf_min, mf_max: the default grid
  * Mf range (1e-4, 0.6 in the reference). Launch shape of the persistent
- * dense-band kernel: chunk (>= the plan's min_chunk) dense bins per work item,
- * block = 64, 128 or 256 threads, grid persistent workgroups; the result does
- * not depend on it beyond the order of the sums. */
+ * dense-band kernel: grid persistent workgroups of block = 64, 128 or 256 threads,
+ * each wavefront with work items of at most chunk / (block / 64) dense bins (rounded up
+ * to 128 or a multiple of 256; chunk >= the plan's min_chunk; never below min_chunk
+ * in a batch of B N > 2^26). A small batch is cut finer, down to 128 bins. The result
+ * does not depend on the shape beyond the order of the sums. */
 int bbhx_hip_direct_fused(bbhx_direct_plan* p, double* d_h, double* h_h, int* flags, const double* params,
                           const double* t_start, const double* t_end, const int* ells_host, const int* mms_host,
                           int numModes, const double* dataFreqs, const double* dataChannels,
