@@ -203,9 +203,10 @@ __device__ inline void node_weight(NodeW* __restrict__ nw, const double* __restr
 //
 // node_residual: r (out) of the node at frequency f (1 / h0: q, channel c's at q[c K]).
 // The modes k0 + kl, k0 + kd + kl, ... (k0, kd of the wavefront, kl of the lane); kd = 1:
-// all of them, in pairs where they go. One body for both, as its code, some 20 KB, is
-// fetched anew for each launch: with a second copy for kd > 1 16 templates took 36 us.
-template <class E>
+// all of them, in pairs where they go. One body for both within a kernel, as its code,
+// some 20 KB, is fetched anew for each launch: with a second copy for kd > 1 16 templates
+// took 36 us. Without SPLIT kd = 1 always.
+template <bool SPLIT, class E>
 __device__ inline void node_residual(cd out[3], const FusedRec* __restrict__ rb, int pairs, int M, int k0, int kd,
                                      int kl, const Window& win, double f, const NodeW* __restrict__ q, int K,
                                      const resp::OrbitTab& orb, int TDItag, int rescaled, int tdi2,
@@ -215,7 +216,7 @@ __device__ inline void node_residual(cd out[3], const FusedRec* __restrict__ rb,
     cd S[6];
     for (int k = 0; k < 6; k++) S[k] = mk(0.0, 0.0);
     for (int k = k0; k < M; k += kd) {
-        const FusedRec& r = rb[min(k + kl, M - 1)];
+        const FusedRec& r = rb[SPLIT ? min(k + kl, M - 1) : k];
         double amp, phase, tf, ad;
         phm::phm_eval(r.w, f, amp, phase, tf, &ad);
         // phenomhm.py:487-507: phase += 2 pi f (t_ref - t0); tf += t_ref
@@ -247,7 +248,7 @@ __device__ inline void node_residual(cd out[3], const FusedRec* __restrict__ rb,
         // link terms' relative phases must not carry the rounding of this
         // large phase (1e4-1e7 rad). Modes outside the observation window
         // contribute nothing (WaveformBuild.cu:50).
-        if (in_window(win, tf) && k + kl < M) {
+        if (in_window(win, tf) && (!SPLIT || k + kl < M)) {
             const cd ap = amp * cexpi_tab(phase + dphi, tab);
             for (int i = 0; i < 6; i++) S[i] += G[i] * ap;
         }
@@ -255,7 +256,7 @@ __device__ inline void node_residual(cd out[3], const FusedRec* __restrict__ rb,
     cd T[3];
     resp::tdi_combine(S, nr, TDItag, rescaled, tdi2, T);
     // r = h / h0 with h = conj(T) (likelihood.py:603), as h (1 / h0)
-    for (int c = 0; c < 3; c++) out[c] = k0 + kl < M ? conj(T[c]) * q[c * K].q : mk(0.0, 0.0);
+    for (int c = 0; c < 3; c++) out[c] = !SPLIT || k0 + kl < M ? conj(T[c]) * q[c * K].q : mk(0.0, 0.0);
 }
 
 // Whether the R nodes left over are too many for their modes to be spread over T lanes
@@ -288,7 +289,7 @@ __device__ inline void residuals(cd* rs, cd* part, const FusedRec* __restrict__ 
     if constexpr (!SPLIT) {
         for (int j = t; j < K; j += T) {
             cd r[3];
-            node_residual(r, rb, pairs, M, 0, 1, 0, win, freqs[j], nw + j, K, orb, TDItag, rescaled, tdi2, tab);
+            node_residual<false>(r, rb, pairs, M, 0, 1, 0, win, freqs[j], nw + j, K, orb, TDItag, rescaled, tdi2, tab);
             for (int c = 0; c < 3; c++) rs[c * K + j] = r[c];
         }
         return;
@@ -308,7 +309,7 @@ __device__ inline void residuals(cd* rs, cd* part, const FusedRec* __restrict__ 
         const int g = t / rows, n = t - g * rows, j = base + min(n, R - 1);
         cd r[3];
         if (one ? t < 64 : g < ng && (n < R || !full))
-            node_residual(r, rb, pairs, M, one ? 0 : __builtin_amdgcn_readfirstlane(g), ng, one ? g : 0, win, freqs[j], nw + j, K, orb, TDItag, rescaled, tdi2, tab);
+            node_residual<true>(r, rb, pairs, M, one ? 0 : __builtin_amdgcn_readfirstlane(g), ng, one ? g : 0, win, freqs[j], nw + j, K, orb, TDItag, rescaled, tdi2, tab);
         if (one) {
             if (t < 64)
                 for (int o = rows; o < 64; o <<= 1)
@@ -404,14 +405,16 @@ inline bool residual_split(int waves, int K)
 // Wavefronts per template of the residual pass (workgroup of 64 x that many
 // threads): enough for about 2048 wavefronts in the launch (two per SIMD of
 // MI355X's 1024), at most one per mode and 64 nodes (one per 64 nodes where the modes are
-// not spread, as the others would only wait) and at most MAX_RESIDUAL_WAVES.
+// not spread, as the others would only wait, and from four of these on, one for each
+// SIMD of the workgroup's CU: 100 templates of 200 nodes 20.7 us, 21.7 with their modes
+// spread over eight wavefronts) and at most MAX_RESIDUAL_WAVES.
 // One for up to 64 nodes, where a template's result so does not depend on the batch.
 // The forward and the gradient's weights pass use the same count, so their
 // sums agree bit for bit.
 inline int residual_waves(int B, int K, int M)
 {
     int nw = (2048 + B - 1) / B;
-    const int nodes = (K + 63) / 64, most = K > 64 ? nodes * M : 1;
+    const int nodes = (K + 63) / 64, most = nodes > 1 && nodes < 4 ? nodes * M : nodes;
     nw = nw < most ? nw : most;
     nw = nw < MAX_RESIDUAL_WAVES ? nw : MAX_RESIDUAL_WAVES;
     if (nw > nodes && !residual_split(nw, K)) nw = nodes;

@@ -107,8 +107,10 @@ def test_direct_grids_of_many_templates(record):
 
 @pytest.mark.parametrize("grad", [False, True])
 def test_heterodyned_wavefronts(record, grad):
-    """One wavefront per 64 nodes where the modes of the last nodes are not spread over others."""
-    sizes = [(16, 300, 6, 5), (16, 320, 1, 5), (16, 128, 6, 8), (16, 64, 6, 1), (16, 1000, 6, 8), (300, 448, 6, 7)]
+    """One wavefront per 64 nodes where the modes of the last nodes are not spread over others, or
+    where four have nodes already."""
+    sizes = [(16, 300, 6, 5), (16, 320, 1, 5), (16, 128, 6, 8), (16, 64, 6, 1), (16, 1000, 6, 8), (300, 448, 6, 7),
+             (16, 192, 6, 8), (16, 193, 6, 4), (16, 256, 6, 4)]
     for (batch, nodes, modes, waves), r in zip(sizes, record(*[("heterodyned", *s[:3], grad) for s in sizes])):
         (grid, block, _), = launches(r, "k_grad_weights" if grad else "k_fused_eval")
         assert (grid[0], block[0]) == (batch, 64 * waves)
