@@ -788,8 +788,8 @@ __device__ inline void mode_adjoint_per_lane(double* __restrict__ Ym, const SegR
 // over searches its own (mode_per_lane).
 //
 // Bound by FP64 issue: 55 vector instructions per (bin, mode) evaluation (24 of
-// the eight cubics, 14 of e^{i phase}, 12 of the mode sum), about 77 with the
-// walker and the inner products, vector units 82 % busy. 1024 uneven templates,
+// the eight cubics, 14 of e^{i phase}, 12 of the mode sum), 83 with the walker and
+// the inner products, the SIMDs issuing 84 % of the cycles (counters). 1024 uneven templates,
 // 1.58 M bins: 44.3 -> 20 ms (145 instructions per evaluation before, 65 %
 // busy: two rounds of scalar loads per segment and iteration, t_f for every bin,
 // a copy of one coefficient per cubic and bin, a 24-operation e^{i phase}).
@@ -803,8 +803,9 @@ __device__ inline void mode_adjoint_per_lane(double* __restrict__ Ym, const SegR
 // where the walker leaves it. At least 4 wavefronts per SIMD (at most 128 VGPRs), 3
 // with the adjoint pass, which takes one iteration per block: it holds Lam as well,
 // and more iterations spill (256 uneven templates of 1.58 M bins, 1, 2, 3 and 4 of
-// them: 23.4, 24.1, 33 and 37 ms). Bound by FP64 issue, some 1.2 x the forward's
-// instructions for the second pass over the modes. 32 sums over the wavefront by
+// them: 23.4, 24.1, 33 and 37 ms). Bound by instruction issue, 82 % of the cycles: 396
+// vector instructions per (mode, 64 bins), 134 of them FP64 arithmetic, 8 matrix
+// instructions, the rest moves, selections and the walker's. 32 sums over the wavefront by
 // exchanges between lanes in place of the matrix product, and a record loaded per
 // lane: 43.5 ms.
 
